@@ -434,6 +434,8 @@ def loop_text(mfma, cvt):
     del _sites[:]
     del _redo[:]
     lines = k_prereads(0)
+    # a wave whose walk is one tile has no second score tile to compute
+    lines += ["s_cmp_ge_i32 %s, %s" % (S_C, S_STOP), "s_cbranch_scc1 700f"]
     lines.append("200:")
     for i in range(UNROLL):
         lines += iteration(i, mfma, cvt)

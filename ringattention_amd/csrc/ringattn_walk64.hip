@@ -11,9 +11,8 @@
 //       matrix work and the vector work have no dependence on each other and interleave freely in
 //       the single instruction stream:
 //           iteration u :  S(u+1) = K(u+1) Q^T   |   P(u) = exp2(S(u) k2 - m k2), row sums   |   O += P(u-1) V(u-1)
-//       The reference max for tile u+1 is decided at the end of iteration u (wave-uniform branch,
-//       as in ring_walk_kernel); its rescale of acc-O (:226-232) is applied one iteration later,
-//       once P(u) -- computed against the old reference -- has been accumulated.
+//       The exponentials are taken against the reference max as it stands; out of line, and only when a sum of four of
+//       them came out above 2^14, the reference moves (rescale of l and acc-O, :226-232) and they are taken again.
 //       The KV chunks of a segment are walked as ONE sequence of 32-key tiles (the diagonal chunk
 //       last): a chunk boundary is only a jump of the load address.
 //       One wave per SIMD has nobody to wait behind, so nothing may be waited for: the K and V rings are eight
@@ -185,7 +184,6 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   constexpr int PIECES = TILE / 4096;  // 1 KB pieces of a tile per wave
   constexpr int KS = D / 16;       // contraction slices of QK^T
   constexpr int DB = D / 32;       // 32-wide blocks of the head dim in PV
-  constexpr float kLazyLog2 = 8.f;
   static_assert(BM == 64 * WAVES, "two 32-row blocks per wave");
   constexpr int kListAt = 2 * NBUF * TILE;  // behind the rings: the chunks of this q tile in walking order, (byte offset, tiles) each
   __shared__ __attribute__((aligned(1024))) unsigned char smem[kListAt + 8 * (kMaxParts + 4)];
@@ -316,9 +314,6 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   float m[2] = {-INFINITY, -INFINITY};  // reference max (raw score units)
   float ms[2] = {0.f, 0.f};             // m * k2, 0 while m is -inf (guard of csrc/ring_attention.cu:183)
   float ls[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  float cand[2] = {-INFINITY, -INFINITY};
-  float apend[2] = {1.f, 1.f};  // rescale of acc-O that is still to be applied
-  bool pend = false;
   f32x16 oacc[2][DB];
 #pragma unroll
   for (int b = 0; b < 2; ++b)
@@ -352,39 +347,6 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
       s[1] = E::mma(kfr, qf[1][ks], s[1]);
     }
   };
-  // O^T += V^T P^T of one 32-key tile for both blocks (csrc/ring_attention.cu:609): each V^T fragment feeds two MFMAs
-  auto pv = [&](int vbytes, const s16x8 (&p)[2][2]) {
-    const unsigned char* vs_lds = smem + vbytes;
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2) {
-      const unsigned char* vrow = vs_lds + 16 * t2 * ROWB;
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow + voff[db]));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow + 8 * ROWB + voff[db]));
-        const s16x8 vfr = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        oacc[0][db] = E::mma(vfr, p[0][t2], oacc[0][db]);
-        oacc[1][db] = E::mma(vfr, p[1][t2], oacc[1][db]);
-      }
-    }
-  };
-  // P^T = exp2(S^T k2 - m k2): row sum from the unrounded values (csrc/ring_attention.cu:242), MFMA operands
-  // rounded to the storage type (:604)
-  auto exps = [&](const f32x16 (&s)[2], s16x8 (&p)[2][2]) {
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
-        typename E::vec8 pv8;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(s[b][8 * t2 + e], a.scale_log2, -ms[b]));
-          ls[b][e & 3] += pe;
-          pv8[e] = (typename E::type)pe;
-        }
-        p[b][t2] = __builtin_bit_cast(s16x8, pv8);
-      }
-  };
   // max(m, row max of the tile): two chains of v_max3_f32, one exchange between the halves of the wave
   auto tile_max = [&](const f32x16& s, float mb) {
     float m0 = mb, m1 = mb;
@@ -407,82 +369,6 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
       }
     }
   };
-  // End of an iteration, seldom taken.  First the rescale of acc-O that was decided an iteration ago (the
-  // probabilities computed against the old reference are all in by now); then, if some row's cand = max(m, tile max)
-  // is far above its reference (or the reference is unset), the move of csrc/ring_attention.cu:226-232: l at once,
-  // acc-O after the next iteration.
-  auto settle = [&](bool far_any) {
-    if (pend) {
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int db = 0; db < DB; ++db) oacc[b][db] *= apend[b];
-      pend = false;
-    }
-    if (far_any) {
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const float cs = (cand[b] == -INFINITY) ? 0.f : cand[b] * a.scale_log2;
-        const float alpha = __builtin_amdgcn_exp2f(m[b] * a.scale_log2 - cs);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ls[b][i] *= alpha;
-        apend[b] = alpha;
-        m[b] = cand[b];
-        ms[b] = cs;
-      }
-      pend = true;
-    }
-  };
-  auto far_now = [&]() {
-    const bool far = (cand[0] - m[0]) * a.scale_log2 > kLazyLog2 || (cand[1] - m[1]) * a.scale_log2 > kLazyLog2;
-    return __builtin_amdgcn_ballot_w64(far) != 0;
-  };
-  // the barrier of a pair of iterations: every wave's loads of four and more iterations ago have landed (each
-  // iteration issues two tiles: 2 PIECES loads); the loads of the last three stay in flight
-  auto ring_barrier = [&]() {
-    if (PIECES == 2) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    __syncthreads();
-  };
-
-  // ---- any iteration: u from 0 to N; products and loads that fall outside the sequence (or outside this wave's
-  // share of the diagonal chunk) are left out, tiles of the diagonal chunk are masked
-  auto general = [&](int u) {
-    if ((u & 1) == 0) {
-      ring_barrier();
-      issue_k((u + 7) & 7);
-      issue_k(u & 7);
-    } else {
-      issue_v((u + 4) & 7);
-      issue_v((u + 5) & 7);
-    }
-    const bool do_qk = u + 1 < Ew, do_sm = u < Ew, do_pv = u >= 1 && u - 1 < Ew;
-    f32x16 snext[2];
-    s16x8 pf[2][2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      snext[b] = sacc[b];
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) pf[b][t2] = pprev[b][t2];
-    }
-    if (do_pv) pv((NBUF + ((u - 1) & 7)) * TILE, pprev);
-    if (do_sm) exps(sacc, pf);
-    if (do_qk) {
-      qk(((u + 1) & 7) * TILE, snext);
-      if (u + 1 >= Mw) mask_tile(snext, u + 1);
-      cand[0] = tile_max(snext[0], m[0]);
-      cand[1] = tile_max(snext[1], m[1]);
-    }
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      sacc[b] = snext[b];
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) pprev[b][t2] = pf[b][t2];
-    }
-    const bool far_any = do_qk && far_now();
-    if (far_any || pend) settle(far_any);
-  };
-
   // ---- prologue: K(0) .. K(6) and V(0) .. V(4) next to the Q loads; the scores of tile 0.  V ring slot 7 -- "tile
   // -1", which the first iteration multiplies with all-zero probabilities -- is cleared.
   if (first > 0) __syncthreads();  // every wave is done with the rings and the chunk list of the pass before
@@ -502,14 +388,13 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   __builtin_amdgcn_s_waitcnt(0);  // retire the Q loads with a wait the compiler can see (and the tiles)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (Ew > 0) {
-    qk(0, sacc);
-    if (0 >= Mw) mask_tile(sacc, 0);
-    cand[0] = tile_max(sacc[0], m[0]);
-    cand[1] = tile_max(sacc[1], m[1]);
-    settle(far_now());
-    // acc-O is still zero: the rescale that the first reference leaves pending is void
-    pend = false;
+  // (every wave has a tile: the first key of the sequence is visible to all rows)
+  qk(0, sacc);
+  if (0 >= Mw) mask_tile(sacc, 0);
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {  // the first reference: the row maxima of tile 0
+    m[b] = tile_max(sacc[b], m[b]);
+    ms[b] = (m[b] == -INFINITY) ? 0.f : m[b] * a.scale_log2;
   }
 
   // LDS addresses for the hand-scheduled loop: fragment offsets from the start of LDS, and where this wave's two
@@ -536,7 +421,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
     const unsigned asm_stop = uni((unsigned)(Ew - 1)), asm_mw1 = uni((unsigned)(Mw - 1));
     int vlim[2];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) vlim[b] = diag_rows + 64 * wave + 32 * b + n - 4 * h - (u + 1 - diag_base) * BN;
+    for (int b = 0; b < 2; ++b) vlim[b] = diag_rows + 64 * wave + 32 * b + n - 4 * h - (1 - diag_base) * BN;
     const uint64_t kp = (uint64_t)(uintptr_t)k_head + kst.off, vp = (uint64_t)(uintptr_t)v_head + vst.off;
     unsigned k_lo = uni((unsigned)kp), k_hi = uni((unsigned)(kp >> 32)), v_lo = uni((unsigned)vp), v_hi = uni((unsigned)(vp >> 32));
     unsigned k_left = uni((unsigned)kst.left), v_left = uni((unsigned)vst.left);
@@ -547,11 +432,8 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
     } else {
 #include "ringattn_walk64_loop_d64.inc"
     }
-  } else {
-    for (int u = 0; u <= N; ++u) general(u);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if (pend) settle(false);
 
   if (KEEP) {
     // ---- the rows' result: the reference's epilogue (csrc/ring_attention.cu:621-664), O = acc / l in the storage
