@@ -133,7 +133,7 @@ int ringattn_plan_destroy(ringattn_plan* plan);
 /*
  * The whole forward for all npes virtual ranks: replaces ring_attention()
  * (csrc/ring_attention.cu:706-722) run on every PE.  ONE block-attention launch: a workgroup
- * owns 256 query rows and walks every ring step of those rows with the running max, sum and
+ * owns 256 query rows and walks the keys of every ring step of those rows with the running max, sum and
  * acc-O in registers, like the reference's CTA (:439-443,456,597), then writes O = acc / sum
  * (:621-664) and the LSE.  (With RINGATTN_FLAG_STEP_PARTIALS: a partial (O, LSE) per step into
  * the workspace, merged at the end of the workgroup.)
@@ -215,10 +215,11 @@ int ringattn_rank_merge(ringattn_plan* plan, int rank, const void* o_parts, cons
  * kv_len), rows counted within a head.  diag_off < 0: every key visible; otherwise key kl
  * (local to the KV range) is visible to query ql (local to the query range) iff
  * kl <= ql + diag_off.  The partial result goes to slot `slot` (= the ring step).
- * step in [0, npes): the items ringattn_block_fwd(step) runs; step == -1: all items of
- * ringattn_fwd, row range by row range, in the order a workgroup runs them (a range that is
- * masked differently within a rank, as the two halves of a zigzag rank are, is listed as
- * separate items).  Writes min(n, capacity) items and stores n in *n_out.
+ * step in [0, npes): the items ringattn_block_fwd(step) runs; step == -1: all ring steps of
+ * ringattn_fwd, row range by row range, in the order a workgroup of a plan with
+ * RINGATTN_FLAG_STEP_PARTIALS runs them (a range that is masked differently within a rank, as the
+ * two halves of a zigzag rank are, is listed as separate items).  Without that flag a workgroup walks
+ * the same keys, those of adjacent steps as one range, in memory order.  Writes min(n, capacity) items and stores n in *n_out.
  */
 typedef struct ringattn_work_item {
   int q_start, q_len, kv_start, kv_len, diag_off, slot;
@@ -274,25 +275,16 @@ int ringattn_ring_attention(const void* q, const void* k, const void* v, void* o
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
  * reference (whose entry allocates on every call, csrc/ring_attention.cu:383-394).  Same
  * arguments and results as ringattn_ring_attention, plus the stream; it calls no hipMalloc,
- * hipFree, memcpy or other allocating routine and does not synchronise: the work (a
- * table-writing kernel, then the attention kernel) is queued on `stream`.  The table of ring steps
- * the attention kernel reads (32 bytes + 32 per visible step), which ringattn_ring_attention keeps
- * in a per-call allocation, lives in a static device array of ringattn_noalloc_scratch_bytes()
- * bytes (4 KiB, held by every GPU the library runs on until the process ends): enough for
- * RINGATTN_MAX_NPES steps, and a ring with more ranks is refused with RINGATTN_ERR_NPES like
- * everywhere else.  All calls on one GPU share that array.  A call's table takes the next slice of it, round
- * robin, and the attention kernel reads its slice for as long as it runs: calls on one stream are ordered by the
- * stream, and calls on several streams or threads may overlap as long as no more of them are in flight on a GPU
- * than slices fit (fourteen with 8-step rings, 288 bytes each; one when a table takes more than half the array).
- * Beyond that a running kernel may find another call's KV ranges in its table and read outside its K and V: do
- * not let that many calls overlap.  Nothing in the array needs clearing between calls.  The first call on a
- * device looks up the array's address (hipGetSymbolAddress): make it outside a stream capture.
+ * hipFree, memcpy or other allocating routine and does not synchronise: the attention kernel is
+ * queued on `stream`, one launch, with the call's key range among its arguments.  It holds no device
+ * memory beyond the caller's tensors, so calls on any number of streams and threads may overlap, and
+ * the call may be captured.
  */
 int ringattn_ring_attention_noalloc(const void* q, const void* k, const void* v, void* out, float* lse,
                                     int npes, int mype, const int* seqlen, int dim, int max_seq,
                                     int dtype, int causal, float softmax_scale, void* stream);
 
-/* Size in bytes of the static device scratch behind ringattn_ring_attention_noalloc. */
+/* The most device memory in bytes that ringattn_ring_attention_noalloc may keep for itself (at present it keeps none). */
 size_t ringattn_noalloc_scratch_bytes(void);
 
 /*

@@ -183,6 +183,39 @@ std::vector<HostSegment> forward_segments(const Derived& d, int P, bool causal) 
   return segs;
 }
 
+// What the forward that carries the softmax state walks.  The state runs from one ring step to the next, so a step's
+// boundary means nothing to it, and the key ranges that lie next to each other in memory are walked as one: without a
+// mask every row sees every key (one segment of all rows, one range of all keys), a causal ring in the contiguous layout
+// is causal attention over the whole sequence (one segment, one masked range), a zigzag rank's high half sees the
+// chunks of the ranks after it as one range.  Fewer, longer ranges: no q tile ends at a rank's end (ranks of 128 rows
+// filled half a tile), all q tiles of a head walk the keys in the same order and meet in L2, and ranks whose lengths
+// are no multiples of a key tile no longer break the walk up.
+std::vector<HostSegment> walk_segments(const Derived& d, int P, bool causal) {
+  if (!causal || !d.zigzag) {
+    HostSegment sg;
+    sg.len = (int)d.S;
+    sg.items.push_back(make_item(0, sg.len, 0, sg.len, causal ? 0 : -1, 0));
+    sg.active = 1;
+    sg.tile_work = d.S;
+    return {sg};
+  }
+  std::vector<HostSegment> segs = forward_segments(d, P, causal);
+  for (auto& sg : segs) {
+    std::sort(sg.items.begin(), sg.items.end(),
+              [](const ringattn::WorkItem& x, const ringattn::WorkItem& y) { return x.kv_start < y.kv_start; });
+    std::vector<ringattn::WorkItem> joined;
+    for (const auto& w : sg.items) {
+      if (!joined.empty() && w.diag_off < 0 && joined.back().diag_off < 0 &&
+          joined.back().kv_start + joined.back().kv_len == w.kv_start)
+        joined.back().kv_len += w.kv_len;
+      else
+        joined.push_back(w);
+    }
+    sg.items = joined;
+  }
+  return segs;
+}
+
 // Workspace of a forward that keeps per-step partials (RINGATTN_FLAG_STEP_PARTIALS; none
 // otherwise): one partial block [batch*heads, len] rows per (segment, item) -- only the
 // (rank, step) pairs the mask leaves visible -- partial O of every block first (fp32, or fp16
@@ -245,7 +278,8 @@ struct ringattn_plan {
   // [batch*heads, S] slot), one step of one rank on rank-local rows (ringattn_rank_step_fwd).
   std::vector<ringattn::Segment> h_segs;
   std::vector<ringattn::SegItem> h_segitems;
-  TableSlice fwd;
+  TableSlice fwd;                  // the ring steps of every row, one by one (RINGATTN_FLAG_STEP_PARTIALS)
+  TableSlice walk;                 // the same rows and keys as the forward that carries the state walks them
   std::vector<TableSlice> step;    // [npes]
   std::vector<TableSlice> local;   // [npes * npes]
   // the same schedule as plain work items, for ringattn_plan_work_items
@@ -257,10 +291,6 @@ struct ringattn_plan {
   int n_regions = 0;               // global ones; regions[n_regions + i] is regions[i] in local rows
   std::vector<int> region_rank;    // [n_regions]
   int region_max_len = 0;
-  // forward only: per XCD, the (segment, head) pairs its workgroups run, heads dealt round-robin
-  std::vector<int2> fwd_groups;
-  int fwd_groups_per_xcd = 0;
-  int2* d_groups = nullptr;
   ringattn::Segment* d_segs = nullptr;
   ringattn::SegItem* d_segitems = nullptr;
   ringattn::MergeRegion* d_regions = nullptr;
@@ -361,21 +391,10 @@ void build_schedule(ringattn_plan* pl) {
     }
   }
   pl->fwd_items = (int)pl->h_items.size();
-  // Workgroup order of the forward.  Heads are dealt to the 8 XCDs round-robin; an XCD runs
-  // the segments of one head after the other (busiest first within a head), so the ranks of
-  // a head, which read the same K and V, follow each other through that XCD's L2.  Only when
-  // the heads divide evenly; otherwise the kernel's arithmetic mapping spreads (segment,
-  // head) pairs over the XCDs.
-  if (d.BH % 8 == 0) {
-    const int heads_per_xcd = (int)(d.BH / 8);
-    pl->fwd_groups_per_xcd = heads_per_xcd * pl->fwd.seg_count;
-    pl->fwd_groups.assign((size_t)8 * pl->fwd_groups_per_xcd, int2{-1, -1});
-    for (int x = 0; x < 8; ++x) {
-      size_t pos = (size_t)x * pl->fwd_groups_per_xcd;
-      for (int hh = 0; hh < heads_per_xcd; ++hh)
-        for (int sgi = 0; sgi < pl->fwd.seg_count; ++sgi) pl->fwd_groups[pos++] = int2{sgi, hh * 8 + x};
-    }
-  }
+  // ---- the forward that carries the state: no partials, the ring steps joined where they can be
+  pl->walk.seg_begin = (int)pl->h_segs.size();
+  for (const auto& sg : walk_segments(d, P, causal))
+    push_segment(pl, pl->walk, sg.start, sg.len, sg.items, 0, [](int) { return (int64_t)0; }, 0);
 
   // ---- one ring step of every rank: partials at the rows of the queries in a [BH, S] slot
   for (int s = 0; s < P; ++s) {
@@ -441,11 +460,6 @@ int ensure_tables(ringattn_plan* pl) {
   if (!pl->d_segs) RA_HIP(hipMalloc((void**)&pl->d_segs, seg_bytes));
   if (!pl->d_segitems) RA_HIP(hipMalloc((void**)&pl->d_segitems, item_bytes));
   if (!pl->d_regions) RA_HIP(hipMalloc((void**)&pl->d_regions, reg_bytes));
-  if (!pl->fwd_groups.empty()) {
-    const size_t grp_bytes = pl->fwd_groups.size() * sizeof(int2);
-    if (!pl->d_groups) RA_HIP(hipMalloc((void**)&pl->d_groups, grp_bytes));
-    RA_HIP(hipMemcpy(pl->d_groups, pl->fwd_groups.data(), grp_bytes, hipMemcpyHostToDevice));
-  }
   RA_HIP(hipMemcpy(pl->d_segs, pl->h_segs.data(), seg_bytes, hipMemcpyHostToDevice));
   RA_HIP(hipMemcpy(pl->d_segitems, pl->h_segitems.data(), item_bytes, hipMemcpyHostToDevice));
   RA_HIP(hipMemcpy(pl->d_regions, pl->regions.data(), reg_bytes, hipMemcpyHostToDevice));
@@ -476,11 +490,29 @@ bool slice_takes_walk64(const ringattn_plan* pl, const TableSlice& sl, int mode)
   return pl->p.dim == 128 || (pl->p.dim == 64 && walk64_d64_enabled());
 }
 
+// the slice ringattn_fwd launches
+const TableSlice& forward_slice(const ringattn_plan* pl) { return step_partials(pl->p) ? pl->fwd : pl->walk; }
+
+// A launch of one segment with one key range carries both in its arguments: a forward without a mask or with the
+// contiguous causal layout, one step of one rank.  No table to upload before the first launch, and none to read -- a chain
+// of dependent memory round trips at the start of every workgroup.
+bool in_arguments(const ringattn_plan* pl, const TableSlice& sl, int mode) {
+  return mode != ringattn::kBlockPartialsMerged && sl.seg_count == 1 && pl->h_segs[(size_t)sl.seg_begin].item_count == 1;
+}
+
 // A block launch over a slice of the tables.
-int launch_slice(const ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a, hipStream_t stream) {
+int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a, hipStream_t stream) {
   if (sl.seg_count == 0) return RINGATTN_OK;
-  a.segs = pl->d_segs + sl.seg_begin;
-  a.items = pl->d_segitems;
+  if (in_arguments(pl, sl, a.mode)) {
+    a.one_seg = pl->h_segs[(size_t)sl.seg_begin];
+    a.one_item = pl->h_segitems[(size_t)a.one_seg.item_begin];
+    a.one_seg.item_begin = 0;  // the item's place is with the arguments now
+  } else {
+    const int rc = ensure_tables(pl);
+    if (rc != RINGATTN_OK) return rc;
+    a.segs = pl->d_segs + sl.seg_begin;
+    a.items = pl->d_segitems;
+  }
   a.n_segs = sl.seg_count;
   a.q_tiles_max = sl.q_tiles_max;
   if (slice_takes_walk64(pl, sl, a.mode))
@@ -507,10 +539,8 @@ int run_forward(ringattn_plan* pl, const void* q, const void* k, const void* v, 
   a.out = out;
   a.lse = lse;
   a.mode = step_partials(pl->p) ? ringattn::kBlockPartialsMerged : ringattn::kBlockCarryState;
-  a.groups = pl->d_groups;
-  a.groups_per_xcd = pl->fwd_groups_per_xcd;
   if (timing) RA_HIP(hipEventRecord(pl->ev_t0, stream));
-  const int rc = launch_slice(pl, pl->fwd, a, stream);
+  const int rc = launch_slice(pl, forward_slice(pl), a, stream);
   if (rc != RINGATTN_OK) return rc;
   if (timing) {
     RA_HIP(hipEventRecord(pl->ev_t1, stream));
@@ -534,15 +564,13 @@ inline bool plan_ok(const ringattn_plan* pl) {
 
 // ---- the reference-shaped call for one rank (ringattn_ring_attention and its variant that
 // allocates nothing) ------------------------------------------------------------------------
-// Device scratch of one call: the segment + item table the attention kernel reads (the softmax state
-// is carried in registers across the ring steps, so there are no partials to park).
+// One segment, one key range (the chunks a rank sees lie next to each other: all of them, or with the mask those up to
+// its own): the launch carries both in its arguments, so the call needs no device memory of its own.
 struct RankCall {
   ringattn_params p;
   Derived d;
-  ringattn::TablePack pack;  // the visible ring steps of the rank in ring order
-  int n_parts = 0;
-  int c = 0;                // rows of this rank
-  size_t scratch_bytes = 0;
+  ringattn::Segment seg;
+  ringattn::SegItem item;
 };
 
 int prepare_rank_call(RankCall* rc, const void* q, const void* k, const void* v, void* out, int npes, int mype,
@@ -565,45 +593,21 @@ int prepare_rank_call(RankCall* rc, const void* q, const void* k, const void* v,
   if (!q || !k || !v || !out) return RINGATTN_ERR_NULL;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) return RINGATTN_ERR_ALIGN;
   // the query rows are local to the caller's rank-sized q and out buffers
-  const int c = rc->c = d.start[mype + 1] - d.start[mype];
-  std::memset(&rc->pack, 0, sizeof(rc->pack));
-  ringattn::Segment& sg = rc->pack.seg;
-  sg.q_start = 0;
-  sg.q_len = c;
-  sg.item_begin = 0;
-  sg.last_item = -1;
-  rc->n_parts = 0;
-  for (int s = 0; s < npes; ++s) {
-    const int j = (mype + s) % npes;
-    if (causal && j > mype) continue;
-    ringattn::SegItem& it = rc->pack.items[rc->n_parts];
-    it.kv_start = d.start[j];
-    it.kv_len = d.start[j + 1] - d.start[j];
-    it.diag_off = (causal && j == mype) ? 0 : -1;
-    it.part_bh_stride = c;
-    it.part_base = (int64_t)rc->n_parts * c;
-    it.slot = s;
-    if (it.diag_off >= 0) {
-      sg.last_item = rc->n_parts;
-      sg.reverse_tiles = 1;
-    }
-    ++rc->n_parts;
-  }
-  sg.item_count = rc->n_parts;
-  if (rc->n_parts == 1) sg.last_item = -1;
-  rc->scratch_bytes = sizeof(ringattn::Segment) + (size_t)rc->n_parts * sizeof(ringattn::SegItem);
+  const int c = d.start[mype + 1] - d.start[mype];
+  std::memset(&rc->seg, 0, sizeof(rc->seg));
+  rc->seg.q_len = c;
+  rc->seg.item_count = 1;
+  rc->seg.last_item = -1;
+  rc->seg.reverse_tiles = causal ? 1 : 0;
+  std::memset(&rc->item, 0, sizeof(rc->item));
+  rc->item.kv_len = causal ? d.start[mype + 1] : (int)d.S;
+  rc->item.diag_off = causal ? d.start[mype] : -1;
   return RINGATTN_OK;
 }
 
-// The table (written by a kernel from its arguments), then the attention kernel: two launches on
-// `stream`, nothing is allocated or copied from the host.
-// `scratch`: rc.scratch_bytes of device memory, 32-byte aligned.
-int run_rank_call(const RankCall& rc, void* scratch, const void* q, const void* k, const void* v, void* out,
-                  float* lse, hipStream_t stream) {
-  const int dim = rc.p.dim, c = rc.c, n_parts = rc.n_parts;
-  ringattn::Segment* d_seg = (ringattn::Segment*)scratch;
-  ringattn::SegItem* d_items = (ringattn::SegItem*)(d_seg + 1);
-  RA_HIP(ringattn::launch_write_table(rc.pack, n_parts, d_seg, d_items, stream));
+// One launch on `stream`; nothing is allocated or copied from the host.
+int run_rank_call(const RankCall& rc, const void* q, const void* k, const void* v, void* out, float* lse, hipStream_t stream) {
+  const int dim = rc.p.dim, c = rc.seg.q_len;
   ringattn::BlockArgs a;
   fill_geometry(a, rc.p, rc.d);
   a.q = q;
@@ -612,51 +616,15 @@ int run_rank_call(const RankCall& rc, void* scratch, const void* q, const void* 
   a.out = out;
   a.lse = lse;  // may be NULL
   a.mode = ringattn::kBlockCarryState;
-  a.segs = d_seg;
-  a.items = d_items;
+  a.one_seg = rc.seg;
+  a.one_item = rc.item;
   a.n_segs = 1;
   a.q_tiles_max = q_tiles_of(c);
   a.bh_stride = (int64_t)c * dim;  // q and out hold this rank's rows only; k and v the whole sequence
   a.S = c;
-  bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled();
-  for (int i = 0; i < n_parts; ++i) wide = wide && walk64_takes(rc.pack.items[i]);
+  const bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled() && walk64_takes(rc.item);
   if (wide) RA_HIP(ringattn::launch_walk64(a, rc.p.dtype, dim, stream));
   else RA_HIP(ringattn::launch_walk(a, rc.p.dtype, dim, stream));
-  return RINGATTN_OK;
-}
-
-// Static device scratch of ringattn_ring_attention_noalloc.  In host code the array's name is
-// only a handle for hipGetSymbolAddress; the device address is looked up once per device
-// (each GPU holds its own copy of the array) and kept.
-// A call's table (32 bytes + 32 per visible ring step) takes the next slice of the array, round robin: the walk
-// kernel reads its table for as long as it runs, so a later call must not overwrite it while an earlier one is still
-// in flight on another stream.  With the tables of an 8-step ring (288 bytes) fourteen calls can be in flight
-// before a slice is used again; a call whose table needs more than half the array has it to itself.
-constexpr size_t kScratchBytes = 4096;
-static_assert(kScratchBytes >= sizeof(ringattn::Segment) + RINGATTN_MAX_NPES * sizeof(ringattn::SegItem),
-              "the table of the largest ring fits");
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
-constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mu;
-void* g_scratch_ptr[kMaxDevices] = {};
-size_t g_scratch_next[kMaxDevices] = {};
-
-int device_scratch(size_t bytes, void** slice) {
-  int dev = -1;
-  RA_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kMaxDevices) return RINGATTN_ERR_SHAPE;
-  if (bytes > kScratchBytes) return RINGATTN_ERR_WORKSPACE;
-  std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (!g_scratch_ptr[dev]) {
-    void* ptr = nullptr;
-    RA_HIP(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
-    if (!ptr) return RINGATTN_ERR_HIP;
-    g_scratch_ptr[dev] = ptr;
-  }
-  const size_t need = (bytes + 31) & ~(size_t)31;   // tables are read with 16-byte scalar loads
-  if (g_scratch_next[dev] + need > kScratchBytes) g_scratch_next[dev] = 0;
-  *slice = (char*)g_scratch_ptr[dev] + g_scratch_next[dev];
-  g_scratch_next[dev] += need;
   return RINGATTN_OK;
 }
 
@@ -748,7 +716,6 @@ int ringattn_plan_destroy(ringattn_plan* plan) {
   if (plan->d_segs) (void)hipFree(plan->d_segs);
   if (plan->d_segitems) (void)hipFree(plan->d_segitems);
   if (plan->d_regions) (void)hipFree(plan->d_regions);
-  if (plan->d_groups) (void)hipFree(plan->d_groups);
   if (plan->own_ws && plan->ws) {
     hipError_t e = hipFree(plan->ws);
     if (e != hipSuccess) rc = hip_fail(e);
@@ -763,8 +730,10 @@ int ringattn_fwd(ringattn_plan* plan, const void* q, const void* k, const void* 
   if (!q || !k || !v || !out || !lse) return RINGATTN_ERR_NULL;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || ((uintptr_t)lse & 3u)) return RINGATTN_ERR_ALIGN;
   hipStream_t stream = (hipStream_t)stream_;
-  int rc0 = ensure_tables(plan);
-  if (rc0 != RINGATTN_OK) return rc0;
+  if ((plan->p.flags & (RINGATTN_FLAG_TIMING | RINGATTN_FLAG_GRAPH)) || step_partials(plan->p)) {
+    const int rc0 = ensure_tables(plan);  // the timing events too; and nothing may be allocated during the capture
+    if (rc0 != RINGATTN_OK) return rc0;
+  }
   if (!(plan->p.flags & RINGATTN_FLAG_GRAPH)) return run_forward(plan, q, k, v, out, lse, stream);
 
   // hipGraph replay: the launch of a forward is captured once per pointer set on a private
@@ -803,8 +772,6 @@ int ringattn_block_fwd(ringattn_plan* plan, int step, const void* q, const void*
   if (!q || !k || !v || !o_part || !lse_part) return RINGATTN_ERR_NULL;
   if (step < 0 || step >= plan->p.npes) return RINGATTN_ERR_RANK;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o_part) || ((uintptr_t)lse_part & 3u)) return RINGATTN_ERR_ALIGN;
-  int rc = ensure_tables(plan);
-  if (rc != RINGATTN_OK) return rc;
   ringattn::BlockArgs a;
   fill_geometry(a, plan->p, plan->d);
   a.q = q;
@@ -834,8 +801,6 @@ int ringattn_rank_step_fwd(ringattn_plan* plan, int rank, int step, const void* 
   const int P = plan->p.npes;
   if (rank < 0 || rank >= P || step < 0 || step >= P) return RINGATTN_ERR_RANK;
   if (!aligned16(q) || !aligned16(k_chunk) || !aligned16(v_chunk) || !aligned16(o_part) || ((uintptr_t)lse_part & 3u)) return RINGATTN_ERR_ALIGN;
-  int rc = ensure_tables(plan);
-  if (rc != RINGATTN_OK) return rc;
   const Derived& d = plan->d;
   const int j = (rank + step) % P;
   const int64_t q_rows = d.start[rank + 1] - d.start[rank], kv_rows = d.start[j + 1] - d.start[j];
@@ -904,7 +869,7 @@ int ringattn_plan_launch_times(ringattn_plan* plan, float* ms, int capacity, int
 const char* ringattn_plan_forward_kernel(const ringattn_plan* plan) {
   if (!plan_ok(plan)) return nullptr;
   const int mode = step_partials(plan->p) ? ringattn::kBlockPartialsMerged : ringattn::kBlockCarryState;
-  return slice_takes_walk64(plan, plan->fwd, mode) ? "ring_walk64_kernel" : "ring_walk_kernel";
+  return slice_takes_walk64(plan, forward_slice(plan), mode) ? "ring_walk64_kernel" : "ring_walk_kernel";
 }
 
 int ringattn_plan_merge_regions(const ringattn_plan* plan, int* start, int* len, uint64_t* active, int capacity, int* n_out) {
@@ -956,17 +921,14 @@ int ringattn_ring_attention(const void* q, const void* k, const void* v, void* o
   RankCall rc_;
   int rc = prepare_rank_call(&rc_, q, k, v, out, npes, mype, seqlen, dim, max_seq, dtype, causal, softmax_scale);
   if (rc != RINGATTN_OK) return rc;
-  // per-call scratch, like the reference's per-call allocations (:383-394) but freed
-  void* ws = nullptr;
-  RA_HIP(hipMalloc(&ws, rc_.scratch_bytes));
-  rc = run_rank_call(rc_, ws, q, k, v, out, lse, nullptr);
+  rc = run_rank_call(rc_, q, k, v, out, lse, nullptr);
   hipError_t e = hipDeviceSynchronize();  // blocking, as csrc/ring_attention.cu:721
   if (rc == RINGATTN_OK && e != hipSuccess) rc = hip_fail(e);
-  (void)hipFree(ws);
   return rc;
 }
 
-size_t ringattn_noalloc_scratch_bytes(void) { return kScratchBytes; }
+// (an upper bound since the launch carries its one range in its arguments: nothing of it is used)
+size_t ringattn_noalloc_scratch_bytes(void) { return 4096; }
 
 int ringattn_ring_attention_noalloc(const void* q, const void* k, const void* v, void* out, float* lse,
                                     int npes, int mype, const int* seqlen, int dim, int max_seq,
@@ -974,10 +936,7 @@ int ringattn_ring_attention_noalloc(const void* q, const void* k, const void* v,
   RankCall rc_;
   int rc = prepare_rank_call(&rc_, q, k, v, out, npes, mype, seqlen, dim, max_seq, dtype, causal, softmax_scale);
   if (rc != RINGATTN_OK) return rc;
-  void* slice = nullptr;
-  rc = device_scratch(rc_.scratch_bytes, &slice);
-  if (rc != RINGATTN_OK) return rc;
-  return run_rank_call(rc_, slice, q, k, v, out, lse, (hipStream_t)stream);
+  return run_rank_call(rc_, q, k, v, out, lse, (hipStream_t)stream);
 }
 
 const char* ringattn_strerror(int code) {

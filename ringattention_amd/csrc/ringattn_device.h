@@ -3,6 +3,8 @@
 #pragma once
 #include "ringattn_kernels.h"
 
+#include <cstddef>
+
 namespace ringattn {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -85,30 +87,51 @@ template <int D> static __device__ __forceinline__ int v_swizzle(int row) {
                   : ((((row >> 1) & 1) << 2) | (((row >> 2) & 1) << 1));
 }
 
-// workgroup -> job (segment, head, q tile); false for the holes of the grid.  blockIdx mod 8 is
-// the XCD: the q tiles of a (segment, head) group are consecutive workgroups of one XCD and share
-// its K and V in that L2.  With a group table the host has dealt the heads to the XCDs and
-// listed, per XCD, the segments of one head after the other (busiest first): ranks of a head
-// follow each other through the same K and V, which then stay in that XCD's L2 / the
-// memory-side cache.  Without one, groups are dealt to the XCDs in segment-major order.
+// The segments and items of a launch: the tables in memory, or the one of each that came with the kernel arguments (the
+// single parameter of every kernel of this library sits at the start of the argument segment).  Pointers to constant
+// memory either way: a table is not written while a kernel runs, and the loads are then scalar ones.
+typedef const __attribute__((address_space(4))) SegItem* ItemPtr;
+typedef const __attribute__((address_space(4))) Segment* SegPtr;
+static __device__ __forceinline__ ItemPtr items_of(const BlockArgs& a) {
+  const auto* args = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+  return a.items ? (ItemPtr)(uintptr_t)a.items : (ItemPtr)(args + offsetof(BlockArgs, one_item));
+}
+static __device__ __forceinline__ SegPtr segs_of(const BlockArgs& a) {
+  const auto* args = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+  return a.items ? (SegPtr)(uintptr_t)a.segs : (SegPtr)(args + offsetof(BlockArgs, one_seg));
+}
+
+// workgroup -> job (segment, head, q tile); false for the holes of the grid.  blockIdx mod 8 is the XCD.  Heads are dealt
+// to the XCDs round-robin, and an XCD runs the segments of a head one after the other (busiest first), the q tiles of a
+// segment as consecutive workgroups: everything that reads a head's K and V follows each other through that XCD's L2.
+// The batch * heads mod 8 heads that do not deal out evenly are shared: with rem of them, gcd(8, rem) sets of XCDs take
+// rem / gcd heads each and split their tiles round-robin, so that one head (or any number) still fills all XCDs.
 template <int TILE_ROWS>
 static __device__ __forceinline__ bool decode_job(const BlockArgs& a, Segment& seg, int& bh, int& qt) {
   const int q_tiles = a.q_tiles_max;
-  const int xcd = blockIdx.x & 7, wslot = blockIdx.x >> 3;
-  int sg;
-  if (a.groups) {
-    const int2 g = a.groups[xcd * a.groups_per_xcd + wslot / q_tiles];
-    sg = g.x;
-    bh = g.y;
-    if (sg < 0) return false;
+  const int per_head = a.n_segs * q_tiles;
+  const int xcd = blockIdx.x & 7, w = blockIdx.x >> 3;
+  const int even_jobs = (a.BH >> 3) * per_head;
+  int head_jobs;  // the job's number among those of its head
+  if (w < even_jobs) {
+    bh = (w / per_head) * 8 + xcd;
+    head_jobs = w % per_head;
   } else {
-    const int group = (wslot / q_tiles) * 8 + xcd;
-    if (group >= a.n_segs * a.BH) return false;
-    sg = group / a.BH;
-    bh = group % a.BH;
+    const int rem = a.BH & 7, sets = rem & -rem;
+    const int j = (w - even_jobs) * (8 / sets) + xcd / sets;
+    const int i = j / per_head;
+    if (i >= rem / sets) return false;
+    bh = (a.BH & ~7) + (xcd & (sets - 1)) + sets * i;
+    head_jobs = j % per_head;
   }
-  seg = a.segs[sg];
-  qt = wslot % q_tiles;
+  const SegPtr sp = segs_of(a) + head_jobs / q_tiles;
+  seg.q_start = sp->q_start;
+  seg.q_len = sp->q_len;
+  seg.item_begin = sp->item_begin;
+  seg.item_count = sp->item_count;
+  seg.last_item = sp->last_item;
+  seg.reverse_tiles = sp->reverse_tiles;
+  qt = head_jobs % q_tiles;
   if (qt * TILE_ROWS >= seg.q_len) return false;  // segments shorter than the longest one
   if (seg.reverse_tiles) qt = (seg.q_len + TILE_ROWS - 1) / TILE_ROWS - 1 - qt;  // most keys first
   return true;

@@ -69,11 +69,8 @@ struct BlockArgs {
   float* lse_part;     // partial LSE rows (natural log), same row numbering; both unused with kBlockCarryState
   void* out;           // unless kBlockPartials: [BH, S, D] storage dtype
   float* lse;          // unless kBlockPartials: [BH, S]; may be NULL with kBlockCarryState
-  const Segment* segs; // device arrays
-  const SegItem* items;
-  const int2* groups;  // NULL, or [8][groups_per_xcd] (segment, head) pairs: what the workgroups of each XCD run,
-                       // in order; segment < 0 marks an unused entry
-  int groups_per_xcd;
+  const Segment* segs; // device arrays; both NULL: the launch has the one segment and the one item below, which then come
+  const SegItem* items;  // with the kernel arguments and not from memory
   int64_t bh_stride;   // elements between heads of q and out (= S * D)
   int64_t kv_bh_stride;      // elements between heads of k and v
   int S;               // rows per head of q, out and lse
@@ -85,7 +82,23 @@ struct BlockArgs {
   float scale_log2;    // softmax_scale * log2(e)
   int half_partials;   // partial O stored as fp16 instead of fp32
   int mode;            // BlockMode
+  Segment one_seg;
+  SegItem one_item;
 };
+
+// Workgroups of a launch: 8 x the jobs (head, segment, q tile) of the busiest XCD.  Heads are dealt to the eight XCDs
+// (decode_job in ringattn_device.h is the other half of this); what is left of them, batch * heads mod 8, is shared
+// out tile by tile.
+inline int64_t job_grid(const BlockArgs& a) {
+  const int64_t per_head = (int64_t)a.n_segs * a.q_tiles_max;
+  int64_t per_xcd = (a.BH / 8) * per_head;
+  const int rem = a.BH & 7;
+  if (rem) {
+    const int sets = rem & -rem;  // gcd(8, rem): groups of 8 / sets XCDs with rem / sets heads each
+    per_xcd += ((rem / sets) * per_head * sets + 7) / 8;
+  }
+  return 8 * per_xcd;
+}
 
 // Merge of (O, LSE) partials into the final O (storage dtype) and LSE, for row ranges of every
 // head: a region covers rows [start, start + len) and reads the slots whose bit is set in `active`.
@@ -111,21 +124,11 @@ struct MergeArgs {
   int row_mul;            // 0: slot-major partials as above; n > 0: [heads * S, n, D] / [heads * S, n], a row's slots adjacent
 };
 
-// Up to kMaxParts table entries passed BY VALUE to a small kernel that writes them to device
-// memory: an item table for callers that may not copy from the host (no allocation, no
-// memcpy node: a plain kernel launch).
-struct TablePack {
-  Segment seg;
-  SegItem items[kMaxParts];
-};
-
 // dtype: 0 = fp16, 1 = bf16.  Return hipSuccess or the launch error.
 hipError_t launch_walk(const BlockArgs& a, int dtype, int dim, hipStream_t stream);  // ring_walk_kernel, any BlockMode
 // ring_walk64_kernel: the carried-state forward at d = 128 with 64 query rows per wave; only for tables that
 // walk64_takes() accepts
 hipError_t launch_walk64(const BlockArgs& a, int dtype, int dim, hipStream_t stream);
 hipError_t launch_merge(const MergeArgs& a, int dtype, int dim, hipStream_t stream);
-// writes pack.seg to *seg_dst and pack.items[0..n) to item_dst
-hipError_t launch_write_table(const TablePack& pack, int n, Segment* seg_dst, SegItem* item_dst, hipStream_t stream);
 
 }  // namespace ringattn

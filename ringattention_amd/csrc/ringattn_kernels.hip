@@ -4,8 +4,6 @@
 //       has no such function: it carries (max, sum, acc-O) in registers across ring steps
 //       (csrc/ring_attention.cu:439-443,597).  The merge is the algebraic equivalent on
 //       (O, LSE) pairs (:207-245,621-633).
-//   write_table_kernel : a segment + item table from kernel arguments to device memory, for
-//       callers that may not copy from the host.
 #include "ringattn_device.h"
 
 #include <type_traits>
@@ -100,20 +98,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
   merge_row<DT, D, HP>(parts, a.o_parts, a.lse_parts, a.out, a.lse, row, threadIdx.x % TPR);
 }
 
-// ---- segment + item table from kernel arguments -------------------------------------
-__global__ __launch_bounds__(64) void write_table_kernel(const TablePack pack, int n, Segment* seg_dst, SegItem* item_dst) {
-  const int i = threadIdx.x;
-  if (i < n) item_dst[i] = pack.items[i];
-  if (i == 0) *seg_dst = pack.seg;
-}
-
 // ---- host launchers -----------------------------------------------------------------
-hipError_t launch_write_table(const TablePack& pack, int n, Segment* seg_dst, SegItem* item_dst, hipStream_t stream) {
-  if (n <= 0 || n > kMaxParts) return hipErrorInvalidValue;
-  write_table_kernel<<<1, 64, 0, stream>>>(pack, n, seg_dst, item_dst);
-  return hipGetLastError();
-}
-
 hipError_t launch_merge(const MergeArgs& a, int dtype, int dim, hipStream_t stream) {
   if (a.n_regions <= 0 || a.max_len <= 0 || a.heads <= 0) return hipSuccess;
   const int rows_per_block = 256 / (dim / 8);

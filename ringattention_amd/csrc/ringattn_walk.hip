@@ -86,11 +86,12 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
   if (!decode_job<BM>(a, seg, bh, qt)) return;
   const int q_start = seg.q_start, q_len = seg.q_len;
   const int n_items = seg.item_count;
+  const ItemPtr items = items_of(a);
   // items in run order: table order, except that item `last_item` is moved to the end
-  auto item_at = [&](int i) -> const SegItem* {
+  auto item_at = [&](int i) -> ItemPtr {
     int idx = i;
     if (seg.last_item >= 0) idx = (i == n_items - 1) ? seg.last_item : (i >= seg.last_item ? i + 1 : i);
-    return a.items + seg.item_begin + idx;
+    return items + seg.item_begin + idx;
   };
 
   const int64_t head_off = (int64_t)bh * a.bh_stride;
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
   int past_stride = 0;
   int kv_len = 0, n_tiles = 0, first_masked = 0, kv_tail = -1, diag_rows = 0;
   bool diag = false;
-  auto set_chunk = [&](const SegItem* w) {
+  auto set_chunk = [&](ItemPtr w) {
     diag = w->diag_off >= 0;
     kv_len = w->kv_len;
     diag_rows = w->diag_off + qt * BM;  // keys below this local index are visible to the whole q tile
@@ -349,7 +350,7 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
     __syncthreads();
   };
   // a chunk's partial (csrc/ring_attention.cu:621-633): normalise, emit O and LSE
-  auto emit_partial = [&](const SegItem* w) {
+  auto emit_partial = [&](ItemPtr w) {
     const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
     const float inv = (l > 0.f) ? 1.f / l : 0.f;
     const int row_l = qt * BM + 32 * wave + n;
@@ -468,14 +469,14 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
 
     bool carried = false;  // the previous chunk's pipeline ran on into this one
     for (int it = 0; it < n_items; ++it) {
-      const SegItem* w = item_at(it);
+      const ItemPtr w = item_at(it);
       set_chunk(w);
       // The pipeline carries over into the next chunk when this one ends in plain steady groups
       // on a multiple of four tiles (ring slots then line up with a fresh start) and the next
       // chunk has its first three tiles in full.
       bool carry = false;
       if (it + 1 < n_items) {
-        const SegItem* wn = item_at(it + 1);
+        const ItemPtr wn = item_at(it + 1);
         carry = !diag && kv_tail < 0 && (n_tiles & 3) == 0 && wn->kv_len >= 4 * BN;
         if (carry) {
           past_delta = ((int64_t)wn->kv_start - w->kv_start) * ROWB - (int64_t)n_tiles * TILE;
@@ -591,8 +592,7 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
 hipError_t launch_walk(const BlockArgs& a, int dtype, int dim, hipStream_t stream) {
   if (a.n_segs <= 0) return hipSuccess;
   const int q_tiles = a.q_tiles_max;  // kWalkM-row tiles of the longest segment
-  const int64_t groups = (int64_t)a.n_segs * a.BH;
-  const int64_t blocks = (a.groups ? (int64_t)a.groups_per_xcd : (groups + 7) / 8) * 8 * q_tiles;
+  const int64_t blocks = job_grid(a);
   if (q_tiles <= 0 || blocks > INT32_MAX) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)blocks;
   if (a.mode != kBlockCarryState && a.mode != kBlockPartials && a.mode != kBlockPartialsMerged) return hipErrorInvalidValue;

@@ -198,11 +198,12 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   if (!decode_job<BM>(a, seg, bh, qt)) return;
   const int q_start = seg.q_start, q_len = seg.q_len;
   const int all_items = seg.item_count;
+  const ItemPtr items = items_of(a);
   // items in run order: table order, except that item `last_item` (the diagonal one) is moved to the end
-  auto item_in_order = [&](int i) -> const SegItem* {
+  auto item_in_order = [&](int i) -> ItemPtr {
     int idx = i;
     if (seg.last_item >= 0) idx = (i == all_items - 1) ? seg.last_item : (i >= seg.last_item ? i + 1 : i);
-    return a.items + seg.item_begin + idx;
+    return items + seg.item_begin + idx;
   };
   const int64_t head_off = (int64_t)bh * a.bh_stride;
   const int kv_bh = (bh / a.heads) * (a.heads / a.kv_group) + (bh % a.heads) / a.kv_group;
@@ -245,10 +246,10 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   // ---- a pass walks n_items chunks from item `first` on as one sequence: all of them (KEEP), or one
   const int n_items = KEEP ? all_items : 1;
   for (int first = 0; first < all_items; first += n_items) {
-  auto item_at = [&](int i) -> const SegItem* { return item_in_order(first + i); };
+  auto item_at = [&](int i) -> ItemPtr { return item_in_order(first + i); };
   // ---- the flattened tile sequence of the pass: item i contributes tiles_of(i) tiles
   const int diag_item = (n_items > 0 && item_at(n_items - 1)->diag_off >= 0) ? n_items - 1 : -1;
-  auto tiles_of = [&](const SegItem* w) {
+  auto tiles_of = [&](ItemPtr w) {
     const int kv_tiles = w->kv_len / BN;
     return w->diag_off >= 0 ? min(kv_tiles, (w->diag_off + qt * BM + BM - 1) / BN + 1) : kv_tiles;
   };
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   // this wave's share of the diagonal chunk: tiles below Mw are visible to all its rows, tiles from Ew on to none
   int Mw = N, Ew = N, diag_base = 0, diag_rows = 0;
   if (diag_item >= 0) {
-    const SegItem* w = item_at(diag_item);
+    const ItemPtr w = item_at(diag_item);
     const int n_last = tiles_of(w);
     diag_base = N - n_last;
     diag_rows = w->diag_off + qt * BM;  // keys below this local index are visible to the whole q tile
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   };
   auto chunk_of = [&](int i, unsigned& off, int& cnt) {
     if (i < n_items) {
-      const SegItem* w = item_at(i);
+      const ItemPtr w = item_at(i);
       off = (unsigned)w->kv_start * ROWB;
       cnt = tiles_of(w);
     } else {
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
     }
   } else {
     // ---- the chunk's partial (csrc/ring_attention.cu:621-633): normalised O and LSE at the rows of the queries
-    const SegItem* w = item_at(0);
+    const ItemPtr w = item_at(0);
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
       const float l = cross_half_sum((ls[b][0] + ls[b][1]) + (ls[b][2] + ls[b][3]));
@@ -505,8 +506,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
 hipError_t launch_walk64(const BlockArgs& a, int dtype, int dim, hipStream_t stream) {
   if (a.n_segs <= 0) return hipSuccess;
   const int q_tiles = a.q_tiles_max;
-  const int64_t groups = (int64_t)a.n_segs * a.BH;
-  const int64_t blocks = (a.groups ? (int64_t)a.groups_per_xcd : (groups + 7) / 8) * 8 * q_tiles;
+  const int64_t blocks = job_grid(a);
   if (q_tiles <= 0 || blocks > INT32_MAX) return hipErrorInvalidValue;
   if (a.mode != kBlockCarryState && a.mode != kBlockPartials && a.mode != kBlockPartialsMerged) return hipErrorInvalidValue;
   if (dtype != 0 && dtype != 1) return hipErrorInvalidValue;
