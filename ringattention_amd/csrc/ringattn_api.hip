@@ -238,14 +238,39 @@ size_t workspace_bytes_of(const ringattn_params* p, const Derived& d) {
 // A slice of the device tables: what one block launch runs.
 struct TableSlice {
   int seg_begin = 0, seg_count = 0;
-  int q_tiles_max = 0;  // kWalkM-row tiles of the longest segment
+  int q_len_max = 0;    // rows of the longest segment
   bool wide = false;    // every KV range of the slice suits ring_walk64_kernel
   int min_kv = 0;       // the shortest KV range of the slice
+  bool split = false;   // few enough rows for ring_split_kernel
 };
 
 // ring_walk64_kernel walks whole 32-key tiles, and past the end of its sequence its load streams go round the first
 // four tiles of a head: a KV range must be a multiple of 32 keys and hold at least 128.
 static bool walk64_takes(const ringattn::SegItem& it) { return it.kv_len % 32 == 0 && it.kv_len >= 128; }
+// ---- which kernel runs a launch that carries the softmax state ---------------------------------------------------------
+// The keys an R-row q tile of `seg` visits, in 32-key tiles: what a launch costs is the longest of its tiles' walks while
+// there are compute units to spare, and their sum over the compute units when there are not.
+struct WalkCost {
+  int64_t tiles = 0;   // of the longest walk
+  int64_t total = 0;   // of all walks
+};
+template <class ItemFn>
+static void add_walks(WalkCost& c, const ringattn::Segment& seg, int rows, int64_t heads, ItemFn item) {
+  const int q_tiles = (seg.q_len + rows - 1) / rows;
+  int64_t fixed = 0, first = 0, last = 0;  // keys of the unmasked ranges; of the masked one for the first and the last q tile
+  for (int i = 0; i < seg.item_count; ++i) {
+    const ringattn::SegItem& it = item(i);
+    if (it.diag_off < 0) fixed += (it.kv_len + 31) / 32;
+    else {
+      first += (std::min(it.kv_len, it.diag_off + rows) + 31) / 32;
+      last += (std::min(it.kv_len, it.diag_off + seg.q_len) + 31) / 32;
+    }
+  }
+  c.tiles = std::max(c.tiles, fixed + std::max(first, last));
+  c.total += heads * q_tiles * (fixed + (first + last) / 2);
+}
+constexpr int kComputeUnits = 256;
+
 // RINGATTN_WIDE=0 in the environment keeps every forward on ring_walk_kernel (for comparisons)
 static bool walk64_enabled() {
   const char* e = std::getenv("RINGATTN_WIDE");
@@ -261,6 +286,28 @@ static bool walk64_d64_enabled() {
 static int walk64_partials_choice() {
   const char* e = std::getenv("RINGATTN_WIDE_PARTIALS");
   return !e ? -1 : (e[0] == '0' ? 0 : 1);
+}
+
+// ring_split_kernel splits the keys of 32 query rows over the eight waves of a workgroup: eight times the workgroups of
+// the 256-row kernels with walks an eighth as long, but only 55-60 % of their rate when the whole device is busy, because a
+// K/V tile fetched from L2 serves 32 rows and not 256.  Measured: a 32-key tile of a 256-row walk takes 0.58 us at d = 128
+// and 0.44 us at d = 64; eight tiles of a 32-row walk take 1.6 us at d = 128 (one workgroup per compute unit) and 1.0 us at
+// d = 64 (1.7 us for the two that a compute unit then holds).  Start and end are 5 us either way.  One head of 8192 tokens
+// (32 workgroups of 256 rows): 152 -> 54 us at d = 128, 114 -> 38 us at d = 64; four heads of it (128 workgroups) 166 -> 209
+// at d = 128, 120 -> 113 at d = 64; with the causal mask, where the longest of the 256-row walks sets the time, 157 -> 120
+// and 119 -> 64.
+// RINGATTN_SPLIT=0 in the environment keeps every launch on the 256-row kernels, and so do RINGATTN_WIDE=0 and
+// RINGATTN_WIDE_PARTIALS=1, which name one of these (comparisons, tests).
+static bool split_enabled() {
+  const char* e = std::getenv("RINGATTN_SPLIT");
+  return !(e && e[0] == '0') && walk64_enabled() && walk64_partials_choice() != 1;
+}
+static bool split_pays(const WalkCost& wide, const WalkCost& narrow, int dim) {
+  const double c_wide = dim == 128 ? 0.58 : 0.44;
+  const double alone = dim == 128 ? 1.6 : 1.0, shared = dim == 128 ? 1.6 : 0.86;
+  const double t_wide = c_wide * std::max((double)wide.tiles, (double)wide.total / kComputeUnits);
+  const double t_narrow = std::max(alone * (double)narrow.tiles, shared * (double)narrow.total / kComputeUnits) / 8;
+  return t_narrow < t_wide;
 }
 
 struct ringattn_plan {
@@ -321,7 +368,7 @@ void fill_geometry(ringattn::BlockArgs& a, const ringattn_params& p, const Deriv
   a.half_partials = half_partials(p) ? 1 : 0;
 }
 
-inline int q_tiles_of(int len) { return (len + ringattn::kWalkM - 1) / ringattn::kWalkM; }
+inline int q_tiles_of(int len, int tile = ringattn::kWalkM) { return (len + tile - 1) / tile; }
 
 // Appends one segment with its items to the tables.  part_base(i) / stride: where item i's
 // partial block lives.  A masked (diagonal) item runs last and the q tiles go busiest first.
@@ -363,7 +410,7 @@ void push_segment(ringattn_plan* pl, TableSlice& slice, int q_start, int q_len,
     slice.min_kv = (slice.seg_count == 0 && i == 0) ? kv : std::min(slice.min_kv, kv);
   }
   ++slice.seg_count;
-  slice.q_tiles_max = std::max(slice.q_tiles_max, q_tiles_of(q_len));
+  slice.q_len_max = std::max(slice.q_len_max, q_len);
 }
 
 // The tables of a plan (host side; nothing here touches the GPU).
@@ -395,6 +442,14 @@ void build_schedule(ringattn_plan* pl) {
   pl->walk.seg_begin = (int)pl->h_segs.size();
   for (const auto& sg : walk_segments(d, P, causal))
     push_segment(pl, pl->walk, sg.start, sg.len, sg.items, 0, [](int) { return (int64_t)0; }, 0);
+  WalkCost whole, split;
+  for (int i = 0; i < pl->walk.seg_count; ++i) {
+    const ringattn::Segment& sg = pl->h_segs[(size_t)(pl->walk.seg_begin + i)];
+    auto item = [&](int k) -> const ringattn::SegItem& { return pl->h_segitems[(size_t)(sg.item_begin + k)]; };
+    add_walks(whole, sg, ringattn::kWalkM, d.BH, item);
+    add_walks(split, sg, ringattn::kSplitM, d.BH, item);
+  }
+  pl->walk.split = split_pays(whole, split, pl->p.dim);
 
   // ---- one ring step of every rank: partials at the rows of the queries in a [BH, S] slot
   for (int s = 0; s < P; ++s) {
@@ -514,7 +569,12 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
     a.items = pl->d_segitems;
   }
   a.n_segs = sl.seg_count;
-  a.q_tiles_max = sl.q_tiles_max;
+  if (a.mode == ringattn::kBlockCarryState && sl.split && split_enabled()) {
+    a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kSplitM);
+    RA_HIP(ringattn::launch_split(a, pl->p.dtype, pl->p.dim, stream));
+    return RINGATTN_OK;
+  }
+  a.q_tiles_max = q_tiles_of(sl.q_len_max);
   if (slice_takes_walk64(pl, sl, a.mode))
     RA_HIP(ringattn::launch_walk64(a, pl->p.dtype, pl->p.dim, stream));
   else
@@ -623,6 +683,14 @@ int run_rank_call(const RankCall& rc, const void* q, const void* k, const void* 
   a.bh_stride = (int64_t)c * dim;  // q and out hold this rank's rows only; k and v the whole sequence
   a.S = c;
   const bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled() && walk64_takes(rc.item);
+  WalkCost whole, split;
+  add_walks(whole, rc.seg, ringattn::kWalkM, 1, [&](int) -> const ringattn::SegItem& { return rc.item; });
+  add_walks(split, rc.seg, ringattn::kSplitM, 1, [&](int) -> const ringattn::SegItem& { return rc.item; });
+  if (split_pays(whole, split, dim) && split_enabled()) {
+    a.q_tiles_max = q_tiles_of(c, ringattn::kSplitM);
+    RA_HIP(ringattn::launch_split(a, rc.p.dtype, dim, stream));
+    return RINGATTN_OK;
+  }
   if (wide) RA_HIP(ringattn::launch_walk64(a, rc.p.dtype, dim, stream));
   else RA_HIP(ringattn::launch_walk(a, rc.p.dtype, dim, stream));
   return RINGATTN_OK;
@@ -869,6 +937,7 @@ int ringattn_plan_launch_times(ringattn_plan* plan, float* ms, int capacity, int
 const char* ringattn_plan_forward_kernel(const ringattn_plan* plan) {
   if (!plan_ok(plan)) return nullptr;
   const int mode = step_partials(plan->p) ? ringattn::kBlockPartialsMerged : ringattn::kBlockCarryState;
+  if (mode == ringattn::kBlockCarryState && plan->walk.split && split_enabled()) return "ring_split_kernel";
   return slice_takes_walk64(plan, forward_slice(plan), mode) ? "ring_walk64_kernel" : "ring_walk_kernel";
 }
 

@@ -7,6 +7,7 @@
 namespace ringattn {
 
 constexpr int kWalkM = 256;   // query rows per workgroup of ring_walk_kernel (8 waves x 32 rows)
+constexpr int kSplitM = 32;   // query rows per workgroup of ring_split_kernel
 constexpr int kMaxParts = 64; // partial slots a merge can combine
 
 // One unit of block-attention work as the host layer lists it: the queries
@@ -129,6 +130,9 @@ hipError_t launch_walk(const BlockArgs& a, int dtype, int dim, hipStream_t strea
 // ring_walk64_kernel: the carried-state forward at d = 128 with 64 query rows per wave; only for tables that
 // walk64_takes() accepts
 hipError_t launch_walk64(const BlockArgs& a, int dtype, int dim, hipStream_t stream);
+// ring_split_kernel: kSplitM query rows per workgroup (a.q_tiles_max counts tiles of that many rows), the keys split over
+// its waves; kBlockCarryState
+hipError_t launch_split(const BlockArgs& a, int dtype, int dim, hipStream_t stream);
 hipError_t launch_merge(const MergeArgs& a, int dtype, int dim, hipStream_t stream);
 
 }  // namespace ringattn

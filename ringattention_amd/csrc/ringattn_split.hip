@@ -1,0 +1,327 @@
+// gfx950 (CDNA4) kernel: block attention for launches with few query rows.
+//
+//   ring_split_kernel : the forward of ring_walk_kernel and ring_walk64_kernel (the reference's CTA that walks its ring
+//       steps with max / sum / acc-O in registers, csrc/ring_attention.cu:439-443,456-620, epilogue :621-664) with the
+//       work split over the KEYS inside a workgroup: all EIGHT waves own the same 32 query rows, wave w takes the
+//       32-key tiles w, w + 8, w + 16, ... of the rows' key ranges with a softmax state of its own, and the eight
+//       states are combined through LDS at the end (the rescale of :226-232 once more, across waves instead of tiles).
+//       A workgroup of the other kernels owns 256 rows, so a launch of 8192 rows has 32 workgroups on 256 compute units;
+//       here it has 256, and the walk of a workgroup is an eighth as long.
+//
+//       Nothing is shared between the waves until the end, so there is no barrier in the loop: a wave loads its own
+//       tiles (one K and one V tile of LDS per wave).  One buffer each is enough: the next K tile is fetched as soon as
+//       the fragments of this one are in registers and has the softmax and the PV product to arrive in, the next V tile
+//       has the QK^T product and the softmax; two (d = 64: four) waves per SIMD overlap one another's matrix and vector
+//       phases without any coordination.
+//       What bounds it: a K/V tile fetched from L2 feeds 32 query rows instead of 256.  At d = 128 a compute unit would
+//       have to take in 128 B per clock to keep its matrix pipes full, twice what its path to L2 carries; without the
+//       loads (timing only) the loop runs 25 % faster.  A full device reaches 690 TFLOP/s at d = 128 and 640 at d = 64
+//       (ring_walk64_kernel 1260 and 940), so this kernel is for launches that leave it compute units idle: the host
+//       weighs the two (split_pays in ringattn_api.hip).  One head of 8192 tokens, us: 152 -> 54 at d = 128, 114 -> 38 at
+//       d = 64; one head of 512 tokens 19.2 -> 10.2 and 13.6 -> 10.7 (with the host's share of the launch).
+#include "ringattn_device.h"
+
+namespace ringattn {
+
+template <int DT, int D>
+__global__ __launch_bounds__(512, D == 64 ? 4 : 2) void ring_split_kernel(const BlockArgs a) {
+  using E = Elem<DT>;
+  constexpr int WAVES = 8;
+  constexpr int BM = kSplitM;      // query rows per workgroup, all of them in every wave
+  constexpr int BN = 32;           // keys per tile
+  constexpr int CPR = D / 8;       // 16-byte chunks per row
+  constexpr int ROWB = D * 2;      // bytes per row
+  constexpr int TILE = BN * ROWB;  // bytes per tile
+  constexpr int KS = D / 16;       // contraction slices of QK^T
+  constexpr int DB = D / 32;       // 32-wide blocks of the head dim in PV
+  constexpr int PIECES = TILE / 1024;  // 1 KB wave-loads per tile
+  constexpr int RPP = 1024 / ROWB;     // rows per piece
+  static_assert(BM == 32, "one 32-row block");
+  constexpr int WREG = 2 * TILE;   // LDS per wave: its K tile and its V tile; at the end its acc-O
+  static_assert(WREG == BM * D * 4, "acc-O of a wave as fp32 takes the place of its tiles");
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[WAVES * WREG];
+  __shared__ float2 stat[WAVES][BM];  // (reference max * k2, row sum) of every wave
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, h = lane >> 5;
+
+  Segment seg;
+  int bh, qt;
+  if (!decode_job<BM>(a, seg, bh, qt)) return;
+  const int n_items = seg.item_count;
+  const int q0 = qt * BM;  // first row of the tile within the segment
+  const int q_last = min(q0 + BM, seg.q_len) - 1;
+  // lane i keeps item i of the segment (kMaxParts = 64 at most); the order they are walked in does not matter here
+  int it_start = 0, it_len = 0, it_diag = -1;
+  if (lane < n_items) {
+    const ItemPtr w = items_of(a) + seg.item_begin + lane;
+    it_start = w->kv_start;
+    it_len = w->kv_len;
+    it_diag = w->diag_off;
+  }
+  int it_tiles = (it_len + BN - 1) / BN;
+  if (it_diag >= 0) it_tiles = min(it_tiles, (it_diag + q_last) / BN + 1);
+
+  const int64_t head_off = (int64_t)bh * a.bh_stride;
+  // grouped-query attention: query head h of a batch entry reads KV head h / kv_group
+  const int kv_bh = (bh / a.heads) * (a.heads / a.kv_group) + (bh % a.heads) / a.kv_group;
+  const char* k_head = (const char*)a.k + (int64_t)kv_bh * a.kv_bh_stride * 2;
+  const char* v_head = (const char*)a.v + (int64_t)kv_bh * a.kv_bh_stride * 2;
+
+  // Q of this lane's row (B operands for the whole launch); rows beyond the range read the last valid row
+  s16x8 qf[KS];
+  {
+    const char* qrow = (const char*)a.q + (head_off + (int64_t)(seg.q_start + min(q0 + n, q_last)) * D) * 2 + h * 16;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const s16x8*)(qrow + ks * 32);
+  }
+
+  // ---- LDS of this wave, fragment offsets, load offsets
+  unsigned char* my = smem + wave * WREG;
+  const unsigned k_lds = lds_offset(smem) + wave * WREG;
+  int koff[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) koff[ks] = n * ROWB + (((2 * ks + h) ^ k_swizzle<D>(n)) << 4);
+  int voff[DB];
+  {
+    const int s = lane & 15, g1 = (lane >> 4) & 1;
+    const int row8 = 4 * h + (s >> 2);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+      const int c = 2 * (2 * db + g1) + ((s & 3) >> 1);
+      voff[db] = TILE + row8 * ROWB + ((c ^ v_swizzle<D>(row8)) << 4) + ((s & 1) << 3);
+    }
+  }
+  // offsets of this lane's 16 bytes within a 1 KB piece of a tile; the swizzles repeat after a few pieces
+  constexpr int NPK = D == 128 ? 4 : 2, NPV = D == 128 ? 2 : 1;
+  const int prow = lane / CPR;
+  int goff_k[NPK], goff_v[NPV];
+#pragma unroll
+  for (int j = 0; j < NPK; ++j) goff_k[j] = prow * ROWB + (((lane % CPR) ^ k_swizzle<D>(RPP * j + prow)) << 4);
+#pragma unroll
+  for (int j = 0; j < NPV; ++j) goff_v[j] = prow * ROWB + (((lane % CPR) ^ v_swizzle<D>(RPP * j + prow)) << 4);
+  // the tile at `base` to `dst`; `rows` of it exist (if fewer than 32, the others read the last one of them)
+  auto load_tile = [&](const char* base, unsigned dst, int rows, const auto& goff) {
+    constexpr int NP = sizeof(goff) / sizeof(int);
+    if (rows >= BN) {
+#pragma unroll
+      for (int j = 0; j < PIECES; ++j)
+        load_lds_16_settled(base + 1024 * j, goff[j % NP], __builtin_amdgcn_readfirstlane(dst + 1024 * j));
+    } else {
+      int row = prow;
+      asm volatile("" : "+v"(row));  // (keeps this seldom taken arithmetic from being done ahead of the loop, in registers)
+#pragma unroll
+      for (int j = 0; j < PIECES; ++j)
+        load_lds_16_settled(base, goff[j % NP] + 1024 * j - max(0, RPP * j + row - (rows - 1)) * ROWB,
+                            __builtin_amdgcn_readfirstlane(dst + 1024 * j));
+    }
+  };
+
+  // ---- the tiles of this wave: numbers wave, wave + 8, ... of the items' tiles laid end to end
+  struct Pos {
+    int item, t;  // item, tile within it
+    int start, len, diag;
+  };
+  auto settle = [&](Pos& p) {  // p.t may lie beyond the item: on to the item that holds it; false past the last one
+    while (p.item < n_items) {
+      const int tiles = __builtin_amdgcn_readlane(it_tiles, p.item);
+      if (p.t < tiles) {
+        p.start = __builtin_amdgcn_readlane(it_start, p.item);
+        p.len = __builtin_amdgcn_readlane(it_len, p.item);
+        p.diag = __builtin_amdgcn_readlane(it_diag, p.item);
+        return true;
+      }
+      p.t -= tiles;
+      ++p.item;
+    }
+    return false;
+  };
+  auto issue_k = [&](const Pos& p) {
+    load_tile(k_head + ((int64_t)p.start + p.t * BN) * ROWB, k_lds, p.len - p.t * BN, goff_k);
+  };
+  auto issue_v = [&](const Pos& p) {
+    load_tile(v_head + ((int64_t)p.start + p.t * BN) * ROWB, k_lds + TILE, p.len - p.t * BN, goff_v);
+  };
+
+  float m = -INFINITY;  // reference max (raw score units)
+  float ms = 0.f;       // m * k2, 0 while m is -inf (guard of csrc/ring_attention.cu:183)
+  float ls[4] = {0.f, 0.f, 0.f, 0.f};
+  f32x16 oacc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) oacc[db][e] = 0.f;
+
+  Pos cur;
+  cur.item = 0;
+  cur.t = wave;
+  bool have = settle(cur);
+  bool fresh = true;  // no tile done yet: no reference to take exponentials against
+  if (have) {
+    issue_k(cur);
+    issue_v(cur);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // retire the Q loads with a wait the compiler can see (and the first tiles)
+  while (have) {
+    Pos nxt = cur;
+    nxt.t += WAVES;
+    const bool more = settle(nxt);
+    // ---- S^T = K Q^T (csrc/ring_attention.cu:565): K(t) is in, V(t) may still be on its way
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
+    f32x16 sacc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sacc[e] = 0.f;
+    {
+      s16x8 kfr[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kfr[ks] = *(const s16x8*)(my + koff[ks]);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) sacc = E::mma(kfr[ks], qf[ks], sacc);
+    }
+    // the fragments are in registers: the K buffer takes the next tile
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (more) issue_k(nxt);
+    // key visible iff inside the KV range and key_local <= query_local + diag_off
+    const int t0 = cur.t * BN;
+    if (t0 + BN > cur.len || (cur.diag >= 0 && t0 + BN - 1 > cur.diag + q0)) {
+      int lim = cur.len - 1 - t0 - 4 * h;
+      if (cur.diag >= 0) lim = min(lim, cur.diag + q0 + n - t0 - 4 * h);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int key = 8 * (e >> 2) + (e & 3);
+        if (key > lim) sacc[e] = -INFINITY;
+      }
+    }
+    // ---- softmax (:194-245): exponentials against the reference as it stands; the row maximum is only looked at when a
+    // sum of four exponentials is above 2^14 (or not a number), or a row has no reference yet
+    s16x8 pf[2];
+    float sums[4];
+    bool move = fresh;
+    fresh = false;
+#pragma unroll 1
+    for (;;) {
+      if (move) {  // rescale of l and acc-O as in :226-232
+        float m0 = m, m1 = m;
+#pragma unroll
+        for (int e = 0; e < 16; e += 4) {
+          m0 = fmaxf(fmaxf(m0, sacc[e]), sacc[e + 1]);
+          m1 = fmaxf(fmaxf(m1, sacc[e + 2]), sacc[e + 3]);
+        }
+        const float cand = cross_half_max(fmaxf(m0, m1));
+        const float cs = (cand == -INFINITY) ? 0.f : cand * a.scale_log2;
+        const float alpha = __builtin_amdgcn_exp2f(m * a.scale_log2 - cs);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ls[i] *= alpha;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
+        m = cand;
+        ms = cs;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sums[i] = 0.f;
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2) {
+        typename E::vec8 pv;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[8 * t2 + e], a.scale_log2, -ms));
+          sums[e & 3] += p;             // from the unrounded p (:242)
+          pv[e] = (typename E::type)p;  // rounded for the MFMA (:604)
+        }
+        pf[t2] = __builtin_bit_cast(s16x8, pv);
+      }
+      const bool again = !(fmaxf(fmaxf(sums[0], sums[1]), fmaxf(sums[2], sums[3])) <= 16384.f) || m == -INFINITY;
+      if (move || __builtin_amdgcn_ballot_w64(again) == 0) break;
+      move = true;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ls[i] += sums[i];
+    // ---- O^T += V^T P^T (:609): V(t) is in, K of the next tile may still be on its way
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const unsigned char* vrow = my + 16 * t2 * ROWB + voff[db];
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow + 8 * ROWB));
+        oacc[db] = E::mma(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pf[t2], oacc[db]);
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (more) issue_v(nxt);
+    cur = nxt;
+    have = more;
+  }
+
+  // ---- combine the eight states: a common reference, every wave's factor against it, and the sums
+  {
+    const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
+    if (h == 0) stat[wave][n] = float2{l > 0.f ? ms : -INFINITY, l};
+  }
+  __syncthreads();
+  {
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) top = fmaxf(top, stat[w][n].x);
+    const float mine = stat[wave][n].x;
+    const float f = mine == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mine - top);
+    // this wave's acc-O, scaled, as fp32 over its own tiles: 16-byte chunk c of row n at chunk c ^ n, so that neither these
+    // writes (32 rows at once) nor the reads below (a few whole rows at once) meet in a bank
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        f32x4 val;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) val[e] = oacc[db][4 * q4 + e] * f;
+        const int c = 8 * db + 2 * q4 + h;
+        *(f32x4*)(my + n * (D * 4) + ((c ^ (n & (D / 4 - 1))) << 4)) = val;
+      }
+  }
+  __syncthreads();
+  // a thread owns eight columns of a row (at d = 64 half the threads have none)
+  const int row = tid / (D / 8), c8 = tid % (D / 8);
+  if (row >= BM || q0 + row > q_last) return;  // (or the row lies beyond the query range)
+  float top = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) top = fmaxf(top, stat[w][row].x);
+  float o[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = 0.f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    const float2 st = stat[w][row];
+    l += st.x == -INFINITY ? 0.f : st.y * __builtin_amdgcn_exp2f(st.x - top);
+    const unsigned char* src = smem + w * WREG + row * (D * 4);
+    const f32x4 x0 = *(const f32x4*)(src + (((2 * c8) ^ (row & (D / 4 - 1))) << 4));
+    const f32x4 x1 = *(const f32x4*)(src + (((2 * c8 + 1) ^ (row & (D / 4 - 1))) << 4));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] += x0[e];
+      o[4 + e] += x1[e];
+    }
+  }
+  const float inv = (l > 0.f) ? 1.f / l : 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] *= inv;
+  const int64_t orow = (int64_t)bh * a.S + seg.q_start + q0 + row;
+  Store8<DT>::st((char*)a.out + (orow * D + c8 * 8) * 2, o);
+  if (c8 == 0 && a.lse) a.lse[orow] = (l > 0.f) ? (top + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
+}
+
+hipError_t launch_split(const BlockArgs& a, int dtype, int dim, hipStream_t stream) {
+  if (a.n_segs <= 0) return hipSuccess;
+  const int64_t blocks = job_grid(a);
+  if (a.q_tiles_max <= 0 || blocks > INT32_MAX || a.mode != kBlockCarryState) return hipErrorInvalidValue;
+  const unsigned grid = (unsigned)blocks;
+  if (dtype == 0 && dim == 64) ring_split_kernel<0, 64><<<grid, 512, 0, stream>>>(a);
+  else if (dtype == 1 && dim == 64) ring_split_kernel<1, 64><<<grid, 512, 0, stream>>>(a);
+  else if (dtype == 0 && dim == 128) ring_split_kernel<0, 128><<<grid, 512, 0, stream>>>(a);
+  else if (dtype == 1 && dim == 128) ring_split_kernel<1, 128><<<grid, 512, 0, stream>>>(a);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+}  // namespace ringattn

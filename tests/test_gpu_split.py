@@ -1,0 +1,67 @@
+"""ring_split_kernel (ringattn_split.hip: 32 query rows per workgroup, the keys split over its eight waves) against the
+CPU oracle where it can go wrong: fewer tiles than waves, one tile more or less than a round of eight, a last tile of one
+key, rows of a tile that see nothing of a wave's first tile (causal), several key ranges (zigzag), grouped heads, heads
+that the eight XCDs share unevenly, and logits that make every wave move its reference again and again.  Bounds: those of
+test_gpu_parity.check_rows, which derive from the roundings of P and O to the storage type."""
+import numpy as np
+import pytest
+import torch
+
+from ringattention_amd import api
+from ringattention_amd.configs import Workload
+from test_gpu_parity import check_rows
+from test_gpu_walk64 import rising_logits
+from test_kernel_resources import test_no_lds_transfer_reads_a_scalar_register_fresh_from_a_vector_instruction as _hazards
+from test_kernel_resources import compile_to_asm
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("lens,B,H,hkv,dtype,causal,zigzag,slope", [
+    ((1,), 1, 1, 1, "fp16", True, False, 0),
+    ((33,), 1, 2, 1, "bf16", False, False, 0),                    # a second tile of one key
+    ((255, 1), 1, 1, 1, "fp16", False, False, 0),                 # eight tiles: one per wave
+    ((257,), 2, 3, 3, "bf16", True, False, 0),                    # nine tiles; six heads over eight XCDs
+    ((200, 313), 1, 9, 3, "fp16", True, False, 0),                # one head more than the XCDs, grouped
+    ((130, 70, 2, 258), 1, 2, 2, "bf16", True, True, 0),          # two segments per rank, ranges of one tile and less
+    ((640, 384), 1, 2, 2, "fp16", False, False, 0.3),             # the row maximum keeps climbing
+    ((640, 385), 1, 2, 2, "bf16", True, False, 0.3),
+    ((1024,), 1, 1, 1, "fp16", True, False, 4.0),                 # steep enough to overflow a stale reference
+])
+def test_split_kernel_against_oracle(oracle, monkeypatch, lens, B, H, hkv, dtype, causal, zigzag, slope, d):
+    for name in ("RINGATTN_WIDE", "RINGATTN_WIDE_PARTIALS", "RINGATTN_SPLIT"):
+        monkeypatch.delenv(name, raising=False)
+    S = sum(lens)
+    w = Workload("split", B, H, d, 1, S, dtype, 900 + S, causal)
+    q, _, _ = rising_logits(w, slope) if slope else api.make_qkv_bits(w)
+    wk = Workload("split_kv", B, hkv, d, 1, S, dtype, 1900 + S, causal)
+    _, k, v = rising_logits(wk, slope) if slope else api.make_qkv_bits(wk)
+    order = api.zigzag_order(lens) if zigzag else np.arange(S)
+    inv = torch.from_numpy(np.argsort(order)).cuda()
+    qd, kd, vd = (api.bits_to_tensor(np.ascontiguousarray(x[:, :, order]), dtype) for x in (q, k, v))
+    plan = api.RingAttention(len(lens), list(lens), d, B, H, dtype, causal, kv_heads=hkv, layout="zigzag" if zigzag else "contiguous")
+    try:
+        assert plan.forward_kernel() == "ring_split_kernel"
+        out_buf = torch.full((B * H * S + 64, d), 7.0, dtype=qd.dtype, device="cuda")
+        lse_buf = torch.full((B * H * S + 64,), 7.0, dtype=torch.float32, device="cuda")
+        out, lse = plan.forward(qd, kd, vd, out_buf[:B * H * S].view(B, H, S, d), lse_buf[:B * H * S].view(B, H, S))
+        torch.cuda.synchronize()
+    finally:
+        plan.close()
+    assert bool((out_buf[B * H * S:] == 7.0).all()) and bool((lse_buf[B * H * S:] == 7.0).all())
+    k_full, v_full = (np.repeat(x, H // hkv, axis=1) for x in (k, v))
+    check_rows(oracle, w, q, k_full, v_full, out[:, :, inv].contiguous(), lse[:, :, inv].contiguous(), np.arange(w.rows))
+
+
+def test_split_kernel_resources_and_hazards(tmp_path):
+    """Two waves per SIMD at d = 128, four (two workgroups per compute unit) at d = 64, no scratch; and the wait states in
+    front of the direct-to-LDS loads."""
+    _, usage = compile_to_asm("ringattn_split.hip", tmp_path / "split.s")
+    kernels = {n: u for n, u in usage.items() if "ring_split_kernel" in n}
+    assert len(kernels) == 4
+    for n, u in kernels.items():
+        d64 = "ELi64E" in n
+        assert u["ScratchSize [bytes/lane]"] == 0, (n, u)
+        assert u["VGPRs"] <= (128 if d64 else 256), (n, u)
+        assert 2 * u["LDS Size [bytes/block]"] <= 160 * 1024 if d64 else u["LDS Size [bytes/block]"] <= 160 * 1024, (n, u)
+    _hazards("ringattn_split.hip", tmp_path)
