@@ -366,6 +366,7 @@ void fill_geometry(ringattn::BlockArgs& a, const ringattn_params& p, const Deriv
   a.kv_group = p.kv_heads > 0 ? p.heads / p.kv_heads : 1;
   a.scale_log2 = d.scale * kLog2e;
   a.half_partials = half_partials(p) ? 1 : 0;
+  a.causal = p.causal != 0;
 }
 
 inline int q_tiles_of(int len, int tile = ringattn::kWalkM) { return (len + tile - 1) / tile; }

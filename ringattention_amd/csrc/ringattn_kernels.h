@@ -83,17 +83,26 @@ struct BlockArgs {
   float scale_log2;    // softmax_scale * log2(e)
   int half_partials;   // partial O stored as fp16 instead of fp32
   int mode;            // BlockMode
+  int causal;          // some item is masked
+  int tail_heads;      // see job_grid
   Segment one_seg;
   SegItem one_item;
 };
 
-// Workgroups of a launch: 8 x the jobs (head, segment, q tile) of the busiest XCD.  Heads are dealt to the eight XCDs
-// (decode_job in ringattn_device.h is the other half of this); what is left of them, batch * heads mod 8, is shared
-// out tile by tile.
-inline int64_t job_grid(const BlockArgs& a) {
+// Workgroups of a launch: 8 x the jobs (head, segment, q tile) of the busiest XCD (decode_job in ringattn_device.h is the
+// other half of this).  Heads are dealt to the eight XCDs and run one after the other; what is left of them, batch * heads
+// mod 8, is shared out tile by tile.  `masked`: the q tiles of a head differ in length, longest first.  Then the last heads
+// of an XCD, as many as make up 64 jobs (two for each of its 32 compute units), and its part of the shared ones go through
+// their tiles together: one after the other, the longest tile of the last head would start when little else is left.
+inline int64_t job_grid(BlockArgs& a, bool masked) {
   const int64_t per_head = (int64_t)a.n_segs * a.q_tiles_max;
-  int64_t per_xcd = (a.BH / 8) * per_head;
-  const int rem = a.BH & 7;
+  const int full = a.BH / 8, rem = a.BH & 7;
+  a.tail_heads = 0;
+  if (masked && per_head > 0) {
+    const int64_t g = (64 + per_head - 1) / per_head;
+    a.tail_heads = (int)(g < full ? g : full);
+  }
+  int64_t per_xcd = full * per_head;
   if (rem) {
     const int sets = rem & -rem;  // gcd(8, rem): groups of 8 / sets XCDs with rem / sets heads each
     per_xcd += ((rem / sets) * per_head * sets + 7) / 8;
@@ -126,13 +135,13 @@ struct MergeArgs {
 };
 
 // dtype: 0 = fp16, 1 = bf16.  Return hipSuccess or the launch error.
-hipError_t launch_walk(const BlockArgs& a, int dtype, int dim, hipStream_t stream);  // ring_walk_kernel, any BlockMode
+hipError_t launch_walk(BlockArgs a, int dtype, int dim, hipStream_t stream);  // ring_walk_kernel, any BlockMode
 // ring_walk64_kernel: the carried-state forward at d = 128 with 64 query rows per wave; only for tables that
 // walk64_takes() accepts
-hipError_t launch_walk64(const BlockArgs& a, int dtype, int dim, hipStream_t stream);
+hipError_t launch_walk64(BlockArgs a, int dtype, int dim, hipStream_t stream);
 // ring_split_kernel: kSplitM query rows per workgroup (a.q_tiles_max counts tiles of that many rows), the keys split over
 // its waves; kBlockCarryState
-hipError_t launch_split(const BlockArgs& a, int dtype, int dim, hipStream_t stream);
+hipError_t launch_split(BlockArgs a, int dtype, int dim, hipStream_t stream);
 hipError_t launch_merge(const MergeArgs& a, int dtype, int dim, hipStream_t stream);
 
 }  // namespace ringattn

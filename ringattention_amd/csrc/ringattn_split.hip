@@ -311,9 +311,9 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void ring_split_kernel(const 
   if (c8 == 0 && a.lse) a.lse[orow] = (l > 0.f) ? (top + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
 }
 
-hipError_t launch_split(const BlockArgs& a, int dtype, int dim, hipStream_t stream) {
+hipError_t launch_split(BlockArgs a, int dtype, int dim, hipStream_t stream) {
   if (a.n_segs <= 0) return hipSuccess;
-  const int64_t blocks = job_grid(a);
+  const int64_t blocks = job_grid(a, a.causal != 0);
   if (a.q_tiles_max <= 0 || blocks > INT32_MAX || a.mode != kBlockCarryState) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)blocks;
   if (dtype == 0 && dim == 64) ring_split_kernel<0, 64><<<grid, 512, 0, stream>>>(a);

@@ -589,10 +589,10 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
   }
 }
 
-hipError_t launch_walk(const BlockArgs& a, int dtype, int dim, hipStream_t stream) {
+hipError_t launch_walk(BlockArgs a, int dtype, int dim, hipStream_t stream) {
   if (a.n_segs <= 0) return hipSuccess;
   const int q_tiles = a.q_tiles_max;  // kWalkM-row tiles of the longest segment
-  const int64_t blocks = job_grid(a);
+  const int64_t blocks = job_grid(a, a.causal != 0);
   if (q_tiles <= 0 || blocks > INT32_MAX) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)blocks;
   if (a.mode != kBlockCarryState && a.mode != kBlockPartials && a.mode != kBlockPartialsMerged) return hipErrorInvalidValue;

@@ -503,10 +503,10 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   }
 }
 
-hipError_t launch_walk64(const BlockArgs& a, int dtype, int dim, hipStream_t stream) {
+hipError_t launch_walk64(BlockArgs a, int dtype, int dim, hipStream_t stream) {
   if (a.n_segs <= 0) return hipSuccess;
   const int q_tiles = a.q_tiles_max;
-  const int64_t blocks = job_grid(a);
+  const int64_t blocks = job_grid(a, a.causal != 0);
   if (q_tiles <= 0 || blocks > INT32_MAX) return hipErrorInvalidValue;
   if (a.mode != kBlockCarryState && a.mode != kBlockPartials && a.mode != kBlockPartialsMerged) return hipErrorInvalidValue;
   if (dtype != 0 && dtype != 1) return hipErrorInvalidValue;
