@@ -353,6 +353,17 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
   auto emit_partial = [&](ItemPtr w) {
     const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
     const float inv = (l > 0.f) ? 1.f / l : 0.f;
+    if constexpr (HP) {  // fp16 partials: |O_part| <= max |V|, the caller vouches that this fits
+      const int row0 = qt * BM + 32 * wave;
+      const int step = w->part_row_mul > 0 ? w->part_row_mul : 1;  // n: a row's steps next to each other
+      const int64_t prow = (w->part_base + (int64_t)bh * w->part_bh_stride + row0) * step + (w->part_row_mul > 0 ? w->slot : 0);
+      store_block<0, D>(oacc, inv, (char*)a.o_part + prow * (D * 2), (int64_t)step * (D * 2), q_len - row0);
+      if (h == 0 && row0 + n < q_len)
+        a.lse_part[prow + (int64_t)n * step] = (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
+      return;
+    }
+    // fp32 rows come out 32 bytes at a time as they are; with store_block's 64 a forward over many chunks of a few tiles
+    // (ranks of 32 to 192 tokens, d = 64) measured 127 -> 133 us, longer chunks the same
     const int row_l = qt * BM + 32 * wave + n;
     if (row_l >= q_len) return;  // a row beyond the query range
     int64_t prow = w->part_base + (int64_t)bh * w->part_bh_stride + row_l;
@@ -365,14 +376,7 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
         f32x4 val;
 #pragma unroll
         for (int e = 0; e < 4; ++e) val[e] = oacc[db][4 * q4 + e] * inv;
-        if (HP) {  // fp16 partials: |O_part| <= max |V|, the caller vouches that this fits
-          f16x4 hv;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) hv[e] = (_Float16)val[e];
-          *(f16x4*)((_Float16*)a.o_part + opos + 32 * db + 8 * q4 + 4 * h) = hv;
-        } else {
-          *(f32x4*)((float*)a.o_part + opos + 32 * db + 8 * q4 + 4 * h) = val;
-        }
+        *(f32x4*)((float*)a.o_part + opos + 32 * db + 8 * q4 + 4 * h) = val;
       }
     if (h == 0) a.lse_part[prow] = (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
   };
@@ -571,21 +575,11 @@ __global__ __launch_bounds__(512, 1) void ring_walk_kernel(const BlockArgs a) {
   if (keep_state) {
     const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
     const float inv = (l > 0.f) ? 1.f / l : 0.f;
-    const int row_l = qt * BM + 32 * wave + n;
-    if (row_l < q_len) {  // not a row beyond the query range
-      const int64_t row = (int64_t)bh * a.S + q_start + row_l;
-      typename E::type* orow = (typename E::type*)a.out + row * D;
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          typename E::vec4 val;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) val[e] = (typename E::type)(oacc[db][4 * q4 + e] * inv);
-          *(typename E::vec4*)(orow + 32 * db + 8 * q4 + 4 * h) = val;
-        }
-      if (h == 0 && a.lse) a.lse[row] = (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
-    }
+    const int row0 = qt * BM + 32 * wave;
+    const int64_t row = (int64_t)bh * a.S + q_start + row0;  // the wave's first row
+    store_block<DT, D>(oacc, inv, (char*)a.out + row * ROWB, ROWB, q_len - row0);
+    if (h == 0 && row0 + n < q_len && a.lse)
+      a.lse[row + n] = (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
   }
 }
 

@@ -443,21 +443,11 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
     for (int b = 0; b < 2; ++b) {
       const float l = cross_half_sum((ls[b][0] + ls[b][1]) + (ls[b][2] + ls[b][3]));
       const float inv = (l > 0.f) ? 1.f / l : 0.f;
-      const int row_l = qt * BM + 64 * wave + 32 * b + n;
-      if (row_l < q_len) {  // not a row beyond the query range
-        const int64_t row = (int64_t)bh * a.S + q_start + row_l;
-        typename E::type* orow = (typename E::type*)a.out + row * D;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            typename E::vec4 val;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) val[e] = (typename E::type)(oacc[b][db][4 * q4 + e] * inv);
-            *(typename E::vec4*)(orow + 32 * db + 8 * q4 + 4 * h) = val;
-          }
-        if (h == 0 && a.lse) a.lse[row] = (l > 0.f) ? (ms[b] + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
-      }
+      const int row0 = qt * BM + 64 * wave + 32 * b;
+      const int64_t row = (int64_t)bh * a.S + q_start + row0;  // the block's first row
+      store_block<DT, D>(oacc[b], inv, (char*)a.out + row * ROWB, ROWB, q_len - row0);
+      if (h == 0 && row0 + n < q_len && a.lse)
+        a.lse[row + n] = (l > 0.f) ? (ms[b] + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
     }
   } else {
     // ---- the chunk's partial (csrc/ring_attention.cu:621-633): normalised O and LSE at the rows of the queries
@@ -466,29 +456,14 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
     for (int b = 0; b < 2; ++b) {
       const float l = cross_half_sum((ls[b][0] + ls[b][1]) + (ls[b][2] + ls[b][3]));
       const float inv = (l > 0.f) ? 1.f / l : 0.f;
-      const int row_l = qt * BM + 64 * wave + 32 * b + n;
-      if (row_l < q_len) {
-        int64_t prow = w->part_base + (int64_t)bh * w->part_bh_stride + row_l;
-        if (w->part_row_mul > 0) prow = prow * w->part_row_mul + w->slot;  // a row's steps next to each other
-        const int64_t opos = prow * D;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            f32x4 val;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) val[e] = oacc[b][db][4 * q4 + e] * inv;
-            if (HP) {  // fp16 partials: |O_part| <= max |V|, the caller vouches that this fits
-              f16x4 hv;
-#pragma unroll
-              for (int e = 0; e < 4; ++e) hv[e] = (_Float16)val[e];
-              *(f16x4*)((_Float16*)a.o_part + opos + 32 * db + 8 * q4 + 4 * h) = hv;
-            } else {
-              *(f32x4*)((float*)a.o_part + opos + 32 * db + 8 * q4 + 4 * h) = val;
-            }
-          }
-        if (h == 0) a.lse_part[prow] = (l > 0.f) ? (ms[b] + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
-      }
+      const int row0 = qt * BM + 64 * wave + 32 * b;
+      int64_t prow = w->part_base + (int64_t)bh * w->part_bh_stride + row0;  // of the block's first row
+      const int step = w->part_row_mul > 0 ? w->part_row_mul : 1;            // n: a row's steps next to each other
+      if (w->part_row_mul > 0) prow = prow * step + w->slot;
+      constexpr int PB = HP ? 2 : 4;  // fp16 partials: |O_part| <= max |V|, the caller vouches that this fits
+      store_block<HP ? 0 : 2, D>(oacc[b], inv, (char*)a.o_part + prow * (D * PB), (int64_t)step * (D * PB), q_len - row0);
+      if (h == 0 && row0 + n < q_len)
+        a.lse_part[prow + (int64_t)n * step] = (l > 0.f) ? (ms[b] + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
     }
   }
   }  // passes
