@@ -1,8 +1,10 @@
 #!/usr/bin/env python3
 """Generates ringattn_walk64_loop.inc: the steady loop of ring_walk64_kernel (ringattn_walk64.hip) as ONE
-inline-assembly statement with hand-allocated registers and a hand-made instruction order.
+inline-assembly statement with hand-allocated registers and a hand-made instruction order; and ringattn_pair_loop.inc, the
+same loop for ring_pair_kernel (ringattn_pair.hip).
 
-    python3 gen_walk64_loop.py            # rewrites ringattn_walk64_loop.inc (d = 128) and ringattn_walk64_loop_d64.inc next to this file
+    python3 gen_walk64_loop.py            # rewrites ringattn_walk64_loop.inc (d = 128), ringattn_walk64_loop_d64.inc and their two
+                                          # ringattn_pair_loop counterparts next to this file
     python3 gen_walk64_loop.py --check    # exit status 1 if a committed file differs
 
 Why by hand: one wave per SIMD has nobody to hide behind.  Within an iteration the matrix work (S(u+1) = K(u+1) Q^T
@@ -14,6 +16,15 @@ MFMA, serialises the fragment reads behind waits and puts the exponentials after
 
 At d = 64 a tile has half the MFMAs (16) for the same vector work, seven to eight vector instructions go behind each, a
 K or V tile is 4 KB (one 1 KB piece per wave), acc-O takes a[0:63] and Q a[64:95]; everything else is the same text.
+
+For ring_pair_kernel the keys are dealt to two groups of two waves, tile by tile.  A group has rings of its own, four tiles
+deep; each of its waves loads half of a tile (at d = 128 four pieces) and steps on by two tiles.  With four slots a K tile has to be
+loaded per iteration, so there is a barrier in every iteration: in front of iteration u every wave has read K(u) and V(u-2),
+K(u+4) and V(u+2) take their places, and what the iteration reads -- V(u-1), and K(u+2) ahead of the next one -- was issued two
+and three iterations before (three tiles' loads may be in flight).
+
+The last tile of a range that is no multiple of 32 keys is a list entry of its own, marked in bit 0 of its offset: the rows past
+the end are read from the last row (the lanes' offsets into their pieces step back), and the mask hides them.
 
 Register map (d = 128; fixed; the C++ side hands its values over in exactly these registers):
     a[0:127]    acc-O: block b, head-dim block db at a[64 b + 16 db .. +15]
@@ -29,6 +40,8 @@ Register map (d = 128; fixed; the C++ side hands its values over in exactly thes
     wave's first piece in K / V ring slot 0, s51 the iteration u, s52 the first u whose score tile u+1 is not computed,
     s53 set to 2 when the workgroup's last iteration is done, s54 the first u whose score tile gets the causal mask, s55 the last iteration;
     v[190:191] mask limits of the two blocks
+    ring_pair_kernel at d = 128: v[240:243] / v[244:247] global offsets of the wave's four pieces of a K / V tile, v[248:251] what
+    they step back by in the last tile of a ragged range
 """
 import os
 import sys
@@ -37,22 +50,24 @@ def _knob(name, default):
     return int(os.environ.get("W64_" + name, default))
 
 
-NBUF = 8
-UNROLL = 8      # iterations per trip: ring slots are immediates
 LEAD = _knob('LEAD', 3)        # a fragment read is issued this many MFMAs ahead of the MFMA that needs it
 HEAD_VALU = _knob('HEAD', 4)   # vector instructions in front of the first MFMA of an iteration
 PREREAD = _knob('PREREAD', 4)     # K fragments of the next iteration read at the end of this one
 
 
-def configure(d):
-    """The head dimension the text is generated for."""
-    global D, KS, DB, ROWB, TILE, PIECES, LOADS_IN_FLIGHT, SHARE, MASK_AT
-    D = d
+def configure(d, groups=1):
+    """The head dimension the text is generated for, and the groups of waves the keys are dealt to."""
+    global D, KS, DB, ROWB, TILE, PIECES, LOADS_IN_FLIGHT, SHARE, MASK_AT, GROUPS, NBUF, UNROLL, TAIL
+    D, GROUPS = d, groups
+    NBUF = 8 if groups == 1 else 4     # ring depth in tiles
+    UNROLL = NBUF                      # iterations per trip: ring slots are immediates
+    TAIL = groups > 1                  # the last tile of a chunk list may be a ragged one
     KS, DB = d // 16, d // 32          # contraction slices of QK^T, 32-wide blocks of the head dim in PV
     ROWB = 2 * d                       # bytes per row
     TILE = 32 * ROWB                   # bytes per tile
-    PIECES = TILE // 4096              # 1 KB pieces of a tile per wave
-    LOADS_IN_FLIGHT = 3 * 2 * PIECES   # at the barrier: the loads of the last three iterations (two tiles each)
+    PIECES = groups * TILE // 4096     # 1 KB pieces of a tile per wave
+    # at the barrier: the loads of the last three iterations (two tiles each); or of the last one and the V tile before them
+    LOADS_IN_FLIGHT = (6 if groups == 1 else 3) * PIECES
     # vector instructions behind an even / odd MFMA
     SHARE = (_knob('SHARE_A', 3), _knob('SHARE_B', 4)) if d == 128 else (_knob('SHARE_A', 7), _knob('SHARE_B', 8))
     MASK_AT = 2 * KS + 3    # the mask of tile u+1 is applied (if at all) behind this MFMA: the last QK MFMA is index 2 KS - 1
@@ -105,8 +120,9 @@ def VFhi(i):
 
 KOFF = lambda ks: "v%d" % (160 + ks)
 VOFF = lambda db: "v%d" % (168 + db)
-GOFFK = lambda j: "v%d" % (172 + j)
-GOFFV = lambda j: "v%d" % (174 + j)
+GOFFK = lambda j: "v%d" % ((172 if PIECES <= 2 else 240) + j)
+GOFFV = lambda j: "v%d" % ((174 if PIECES <= 2 else 244) + j)
+BACK = lambda j: "v%d" % (248 + j)
 M = lambda b: "v%d" % (176 + b)
 MS = lambda b: "v%d" % (178 + b)
 LS = lambda b, i: "v%d" % (180 + 4 * b + i)
@@ -156,14 +172,14 @@ def tile_load(st, slot, goff):
         "s_sub_u32 %s, %s, 1" % (st.left, st.left),
         ld + "global_load_lds_dwordx4 %s, %s" % (goff(0), st.ptr),
     ]
-    if PIECES == 2:
+    for j in range(1, PIECES):
         out += [
-            "s_add_u32 m0, %s, %d" % (st.lds, slot * TILE + 1024),
+            "s_add_u32 m0, %s, %d" % (st.lds, slot * TILE + 1024 * j),
             "s_nop 0",
-            ld + "global_load_lds_dwordx4 %s, %s" % (goff(1), st.ptr),
+            ld + "global_load_lds_dwordx4 %s, %s" % (goff(j), st.ptr),
         ]
     out += [
-        "s_add_u32 %s, %s, %d" % (st.lo, st.lo, TILE),
+        "s_add_u32 %s, %s, %d" % (st.lo, st.lo, GROUPS * TILE),
         "s_addc_u32 %s, %s, 0" % (st.hi, st.hi),
         "s_cmp_eq_u32 %s, 0" % st.left,
         "s_cbranch_scc1 3%02df" % site,
@@ -184,8 +200,13 @@ def chunk_changes():
                 "s_waitcnt lgkmcnt(0)",
                 "v_readfirstlane_b32 %s, %s" % (S_T(0), TMP(6)),
                 "v_readfirstlane_b32 %s, %s" % (st.left, TMP(7)),
-                "s_nop 3",
-                "s_add_u32 %s, %s, %s" % (st.lo, st.head[0], S_T(0)),
+                "s_nop 3"]
+        if TAIL:
+            goff = GOFFK if st is KST else GOFFV
+            out += ["s_bitcmp1_b32 %s, 0" % S_T(0), "s_cbranch_scc0 12%02df" % site, "s_bitset0_b32 %s, 0" % S_T(0)]
+            out += ["v_sub_u32_e32 %s, %s, %s" % (goff(j), goff(j), BACK(j)) for j in range(PIECES)]
+            out.append("12%02d:" % site)
+        out += ["s_add_u32 %s, %s, %s" % (st.lo, st.head[0], S_T(0)),
                 "s_addc_u32 %s, %s, 0" % (st.hi, st.head[1]),
                 "s_branch 4%02db" % site]
     return out
@@ -289,7 +310,11 @@ def iteration(i, mfma, cvt, do_qk=True, do_sm=True, do_pv=True):
     # full iterations only) worked in behind the first MFMAs.  The K fragments the first MFMAs use were landed a
     # barrier ago; the V fragments of this iteration are only read behind this barrier.
     misc = []
-    if i % 2 == 0:
+    if GROUPS > 1:
+        misc += ["s_waitcnt vmcnt(%d)" % LOADS_IN_FLIGHT, "s_barrier"]
+        misc += tile_load(KST, i % NBUF, GOFFK)
+        misc += tile_load(VST, (i + 2) % NBUF, GOFFV)
+    elif i % 2 == 0:
         misc += ["s_waitcnt vmcnt(%d)" % LOADS_IN_FLIGHT] + ([] if _knob('NOBARRIER', 0) else ["s_barrier"])
         misc += tile_load(KST, (i + 7) % NBUF, GOFFK)
         misc += tile_load(KST, i % NBUF, GOFFK)
@@ -337,7 +362,7 @@ def iteration(i, mfma, cvt, do_qk=True, do_sm=True, do_pv=True):
     tail = []
     if do_qk:   # the mask limits move on by a tile
         for b in range(2):
-            valu.append("v_subrev_u32_e32 %s, 32, %s" % (VLIM(b), VLIM(b)))
+            valu.append("v_subrev_u32_e32 %s, %d, %s" % (VLIM(b), 32 * GROUPS, VLIM(b)))
 
     # ---- interleave
     issued = min(PREREAD, KS) if do_qk else 0   # the first K fragments are on their way (read at the end of the previous iteration)
@@ -490,6 +515,9 @@ def operands():
     for st, n in ((KST, "k"), (VST, "v")):
         outs += ['"+{%s}"(%s_lo)' % (st.lo, n), '"+{%s}"(%s_hi)' % (st.hi, n), '"+{%s}"(%s_left)' % (st.left, n),
                  '"+{%s}"(%s_next)' % (st.next, n)]
+    if TAIL:   # (the last tile moves these)
+        for goff, n in ((GOFFK, "goff_k"), (GOFFV, "goff_v")):
+            outs += ['"+{%s}"(%s[%d])' % (goff(j), n, j) for j in range(PIECES)]
     outs += ['"+{%s}"(asm_u)' % S_C, '"+{%s}"(asm_far)' % S_FAR]
     for b in range(2):
         outs.append('"+{%s}"(vlim[%d])' % (VLIM(b), b))
@@ -500,10 +528,11 @@ def operands():
         ins.append('"{%s}"(koff_a[%d])' % (KOFF(ks), ks))
     for db in range(DB):
         ins.append('"{%s}"(voff_a[%d])' % (VOFF(db), db))
-    for j in range(PIECES):
-        ins.append('"{%s}"(goff_k[%d])' % (GOFFK(j), j))
-    for j in range(PIECES):
-        ins.append('"{%s}"(goff_v[%d])' % (GOFFV(j), j))
+    if TAIL:
+        ins += ['"{%s}"(back[%d])' % (BACK(j), j) for j in range(PIECES)]
+    else:
+        for goff, n in ((GOFFK, "goff_k"), (GOFFV, "goff_v")):
+            ins += ['"{%s}"(%s[%d])' % (goff(j), n, j) for j in range(PIECES)]
     ins += ['"{%s}"(kh_lo)' % KST.head[0], '"{%s}"(kh_hi)' % KST.head[1], '"{%s}"(vh_lo)' % VST.head[0], '"{%s}"(vh_hi)' % VST.head[1],
             '"{%s}"(k2_bits)' % S_K2, '"{%s}"(lds_dst_k)' % S_LDSK, '"{%s}"(lds_dst_v)' % S_LDSV,
             '"{%s}"(asm_stop)' % S_STOP, '"{%s}"(asm_mw1)' % S_MW1, '"{%s}"(asm_n)' % S_N]
@@ -512,9 +541,10 @@ def operands():
     return outs, ins, clob
 
 
-def render(d=128):
-    configure(d)
-    res = ["// Generated by gen_walk64_loop.py -- do not edit.  The steady loop of ring_walk64_kernel: see the generator for the",
+def render(d=128, groups=1):
+    configure(d, groups)
+    res = ["// Generated by gen_walk64_loop.py -- do not edit.  The steady loop of %s: see the generator for the"
+           % ("ring_walk64_kernel" if groups == 1 else "ring_pair_kernel"),
            "// register map and the instruction order.  Expects the kernel's variables by name.", ""]
     for dt, (mfma, cvt) in enumerate((("v_mfma_f32_32x32x16_f16", "v_cvt_pk_f16_f32"),
                                       ("v_mfma_f32_32x32x16_bf16", "v_cvt_pk_bf16_f32"))):
@@ -531,15 +561,16 @@ def render(d=128):
 
 
 FILES = {128: "ringattn_walk64_loop.inc", 64: "ringattn_walk64_loop_d64.inc"}
+PAIR_FILES = {128: "ringattn_pair_loop.inc", 64: "ringattn_pair_loop_d64.inc"}
 
 if __name__ == "__main__":
     here = os.environ.get("W64_OUT_DIR") or os.path.dirname(os.path.abspath(__file__))
     status = 0
-    for d, name in FILES.items():
+    for d, groups, name in [(d, 1, n) for d, n in FILES.items()] + [(d, 2, n) for d, n in PAIR_FILES.items()]:
         path = os.path.join(here, name)
-        if d == 128 and os.environ.get("W64_OUT"):
+        if (d, groups) == (128, 1) and os.environ.get("W64_OUT"):
             path = os.environ["W64_OUT"]
-        text = render(d)
+        text = render(d, groups)
         if "--check" in sys.argv:
             with open(path) as f:
                 status |= 0 if f.read() == text else 1

@@ -235,24 +235,13 @@ size_t workspace_bytes_of(const ringattn_params* p, const Derived& d) {
 
 }  // namespace
 
-// A slice of the device tables: what one block launch runs.
-struct TableSlice {
-  int seg_begin = 0, seg_count = 0;
-  int q_len_max = 0;    // rows of the longest segment
-  bool wide = false;    // every KV range of the slice suits ring_walk64_kernel
-  int min_kv = 0;       // the shortest KV range of the slice
-  bool split = false;   // few enough rows for ring_split_kernel
-};
-
-// ring_walk64_kernel walks whole 32-key tiles, and past the end of its sequence its load streams go round the first
-// four tiles of a head: a KV range must be a multiple of 32 keys and hold at least 128.
-static bool walk64_takes(const ringattn::SegItem& it) { return it.kv_len % 32 == 0 && it.kv_len >= 128; }
 // ---- which kernel runs a launch that carries the softmax state ---------------------------------------------------------
 // The keys an R-row q tile of `seg` visits, in 32-key tiles: what a launch costs is the longest of its tiles' walks while
 // there are compute units to spare, and their sum over the compute units when there are not.
 struct WalkCost {
   int64_t tiles = 0;   // of the longest walk
   int64_t total = 0;   // of all walks
+  int64_t jobs = 0;    // walks
 };
 template <class ItemFn>
 static void add_walks(WalkCost& c, const ringattn::Segment& seg, int rows, int64_t heads, ItemFn item) {
@@ -268,9 +257,41 @@ static void add_walks(WalkCost& c, const ringattn::Segment& seg, int rows, int64
   }
   c.tiles = std::max(c.tiles, fixed + std::max(first, last));
   c.total += heads * q_tiles * (fixed + (first + last) / 2);
+  c.jobs += heads * q_tiles;
 }
 constexpr int kComputeUnits = 256;
+struct CarryCosts {
+  WalkCost whole, halves, thin;  // with q tiles of kWalkM, kPairM and kSplitM rows
+  bool pair = true;              // every segment suits ring_pair_kernel
+  bool masked = false;           // the walks differ in length
+  template <class ItemFn>
+  void add(const ringattn::Segment& seg, int64_t heads, ItemFn item) {
+    add_walks(whole, seg, ringattn::kWalkM, heads, item);
+    add_walks(halves, seg, ringattn::kPairM, heads, item);
+    add_walks(thin, seg, ringattn::kSplitM, heads, item);
+    // ring_pair_kernel: what runs past the end of a walk goes round the first rows of a head, so a KV range holds at least
+    // 128 keys; only the range walked last may end in a tile of fewer than 32 keys, whose place the kernel keeps in 32 bits
+    const int last = seg.last_item >= 0 ? seg.last_item : seg.item_count - 1;
+    for (int i = 0; i < seg.item_count; ++i) {
+      const ringattn::SegItem& it = item(i);
+      masked = masked || it.diag_off >= 0;
+      pair = pair && it.kv_len >= 128 && (it.kv_len % 32 == 0 || (i == last && it.kv_start + it.kv_len <= 1 << 24));
+    }
+  }
+};
 
+// A slice of the device tables: what one block launch runs.
+struct TableSlice {
+  int seg_begin = 0, seg_count = 0;
+  int q_len_max = 0;    // rows of the longest segment
+  bool wide = false;    // every KV range of the slice suits ring_walk64_kernel
+  int min_kv = 0;       // the shortest KV range of the slice
+  CarryCosts costs;     // pl->walk only
+};
+
+// ring_walk64_kernel walks whole 32-key tiles, and past the end of its sequence its load streams go round the first
+// four tiles of a head: a KV range must be a multiple of 32 keys and hold at least 128.
+static bool walk64_takes(const ringattn::SegItem& it) { return it.kv_len % 32 == 0 && it.kv_len >= 128; }
 // RINGATTN_WIDE=0 in the environment keeps every forward on ring_walk_kernel (for comparisons)
 static bool walk64_enabled() {
   const char* e = std::getenv("RINGATTN_WIDE");
@@ -288,26 +309,68 @@ static int walk64_partials_choice() {
   return !e ? -1 : (e[0] == '0' ? 0 : 1);
 }
 
-// ring_split_kernel splits the keys of 32 query rows over the eight waves of a workgroup: eight times the workgroups of
-// the 256-row kernels with walks an eighth as long, but only 55-60 % of their rate when the whole device is busy, because a
-// K/V tile fetched from L2 serves 32 rows and not 256.  Measured: a 32-key tile of a 256-row walk takes 0.58 us at d = 128
-// and 0.44 us at d = 64; eight tiles of a 32-row walk take 1.6 us at d = 128 (one workgroup per compute unit) and 1.0 us at
-// d = 64 (1.7 us for the two that a compute unit then holds).  Start and end are 5 us either way.  One head of 8192 tokens
-// (32 workgroups of 256 rows): 152 -> 54 us at d = 128, 114 -> 38 us at d = 64; four heads of it (128 workgroups) 166 -> 209
-// at d = 128, 120 -> 113 at d = 64; with the causal mask, where the longest of the 256-row walks sets the time, 157 -> 120
-// and 119 -> 64.
-// RINGATTN_SPLIT=0 in the environment keeps every launch on the 256-row kernels, and so do RINGATTN_WIDE=0 and
-// RINGATTN_WIDE_PARTIALS=1, which name one of these (comparisons, tests).
+// RINGATTN_SPLIT=0 and RINGATTN_PAIR=0 in the environment take ring_split_kernel and ring_pair_kernel out of the choice below,
+// RINGATTN_PAIR=1 takes the latter whenever the shapes allow; RINGATTN_WIDE=0 and RINGATTN_WIDE_PARTIALS=1, which name one
+// of the 256-row kernels, keep every launch on these (comparisons, tests).
 static bool split_enabled() {
   const char* e = std::getenv("RINGATTN_SPLIT");
-  return !(e && e[0] == '0') && walk64_enabled() && walk64_partials_choice() != 1;
+  return !(e && e[0] == '0');
 }
-static bool split_pays(const WalkCost& wide, const WalkCost& narrow, int dim) {
-  const double c_wide = dim == 128 ? 0.58 : 0.44;
-  const double alone = dim == 128 ? 1.6 : 1.0, shared = dim == 128 ? 1.6 : 0.86;
-  const double t_wide = c_wide * std::max((double)wide.tiles, (double)wide.total / kComputeUnits);
-  const double t_narrow = std::max(alone * (double)narrow.tiles, shared * (double)narrow.total / kComputeUnits) / 8;
-  return t_narrow < t_wide;
+static int pair_choice() {
+  const char* e = std::getenv("RINGATTN_PAIR");
+  return !e ? -1 : (e[0] == '0' ? 0 : 1);
+}
+
+// Three kernels carry the state, with 256, 128 and 32 query rows per workgroup (kWalkM, kPairM, kSplitM), a workgroup per
+// compute unit: the fewer the rows, the shorter the walks (the waves that do not own rows of their own share out the
+// keys) and the more of them, but the more often a K/V tile is fetched from L2.  A launch of few q tiles takes as long as
+// its longest walk, one of many as all of them over the compute units, at a lower clock.  Each kernel by three measured
+// numbers: us per step of a walk (one, two and eight key tiles) with most compute units idle and with all of them busy,
+// and us per workgroup besides (Q, first tiles, result).  They give the time of 150 launches -- heads 1 to 64, sequences of
+// 320 to 32768, with and without the causal mask -- to 2-4 % rms; us measured on the 256-, 128- and 32-row kernel at
+// d = 128, and at d = 64:
+//     1 head x 2048                         44, 28, 17        34, 22, 13
+//     8 heads x 2048                        43, 29, 33        34, 22, 19
+//     8 heads x 4096, causal                79, 50, 65        61, 38, 35
+//     16 heads x 4096, causal               85, 69, 127       62, 46, 62
+//     4 heads x 8192                       151, 117, 197     118, 77, 103
+//     8 heads x 8192                       211, 230, 389     131, 145, 198
+//     9 heads x 8192 (288 q tiles of 256)  355, 310, 437     244, 208, 223
+//     16 heads x 8192, causal              221, 245, 424     142, 159, 209
+enum class CarryKernel { kWhole, kPair, kSplit };
+struct KernelRate {
+  int tiles_per_step;
+  double lone, busy, job;
+};
+constexpr KernelRate kRates128[3] = {{1, 0.55, 0.79, 5.3}, {2, 0.60, 0.84, 6.0}, {8, 1.15, 1.35, 4.9}};
+constexpr KernelRate kRates64[3] = {{1, 0.42, 0.49, 3.2}, {2, 0.46, 0.53, 4.0}, {8, 0.96, 0.71, 1.9}};
+
+static double carry_time(const WalkCost& w, const KernelRate& r, bool equal_walks) {
+  const double longest = (double)w.tiles / r.tiles_per_step;
+  if (equal_walks) {  // round after round, the last one on what compute units it needs
+    const int64_t rounds = w.jobs / kComputeUnits, rest = w.jobs % kComputeUnits;
+    const double t = (double)rounds * (r.busy * longest + r.job);
+    return rest == 0 ? t : t + r.job + longest * std::max(r.lone, r.busy * (double)rest / kComputeUnits);
+  }
+  // the longest walk and the even share of all of them; where these are alike, what is left at the end adds to both
+  const double x = r.lone * longest + r.job;
+  const double y = (r.busy * (double)w.total / r.tiles_per_step + r.job * (double)w.jobs) / kComputeUnits;
+  return std::sqrt(std::sqrt(x * x * x * x + y * y * y * y));
+}
+
+static CarryKernel carry_kernel(const CarryCosts& c, int dim) {
+  if (!walk64_enabled() || walk64_partials_choice() == 1) return CarryKernel::kWhole;
+  if (c.pair && pair_choice() == 1) return CarryKernel::kPair;
+  const KernelRate* r = dim == 128 ? kRates128 : kRates64;
+  // the 256-row kernels unless another is ahead by more than these times are good for
+  double best = carry_time(c.whole, r[0], !c.masked) * 0.95;
+  CarryKernel kernel = CarryKernel::kWhole;
+  if (c.pair && pair_choice() != 0) {
+    const double t = carry_time(c.halves, r[1], !c.masked);
+    if (t < best) best = t, kernel = CarryKernel::kPair;
+  }
+  if (split_enabled() && carry_time(c.thin, r[2], false) < best) kernel = CarryKernel::kSplit;
+  return kernel;
 }
 
 struct ringattn_plan {
@@ -443,14 +506,10 @@ void build_schedule(ringattn_plan* pl) {
   pl->walk.seg_begin = (int)pl->h_segs.size();
   for (const auto& sg : walk_segments(d, P, causal))
     push_segment(pl, pl->walk, sg.start, sg.len, sg.items, 0, [](int) { return (int64_t)0; }, 0);
-  WalkCost whole, split;
   for (int i = 0; i < pl->walk.seg_count; ++i) {
     const ringattn::Segment& sg = pl->h_segs[(size_t)(pl->walk.seg_begin + i)];
-    auto item = [&](int k) -> const ringattn::SegItem& { return pl->h_segitems[(size_t)(sg.item_begin + k)]; };
-    add_walks(whole, sg, ringattn::kWalkM, d.BH, item);
-    add_walks(split, sg, ringattn::kSplitM, d.BH, item);
+    pl->walk.costs.add(sg, d.BH, [&](int k) -> const ringattn::SegItem& { return pl->h_segitems[(size_t)(sg.item_begin + k)]; });
   }
-  pl->walk.split = split_pays(whole, split, pl->p.dim);
 
   // ---- one ring step of every rank: partials at the rows of the queries in a [BH, S] slot
   for (int s = 0; s < P; ++s) {
@@ -556,6 +615,21 @@ bool in_arguments(const ringattn_plan* pl, const TableSlice& sl, int mode) {
   return mode != ringattn::kBlockPartialsMerged && sl.seg_count == 1 && pl->h_segs[(size_t)sl.seg_begin].item_count == 1;
 }
 
+// the launch of `kernel` over q tiles of its size; `wide`: kWhole is ring_walk64_kernel
+hipError_t launch_q_tiles(ringattn::BlockArgs& a, CarryKernel kernel, bool wide, int q_len, int dtype, int dim, hipStream_t stream) {
+  switch (kernel) {
+    case CarryKernel::kPair:
+      a.q_tiles_max = q_tiles_of(q_len, ringattn::kPairM);
+      return ringattn::launch_pair(a, dtype, dim, stream);
+    case CarryKernel::kSplit:
+      a.q_tiles_max = q_tiles_of(q_len, ringattn::kSplitM);
+      return ringattn::launch_split(a, dtype, dim, stream);
+    default:
+      a.q_tiles_max = q_tiles_of(q_len);
+      return wide ? ringattn::launch_walk64(a, dtype, dim, stream) : ringattn::launch_walk(a, dtype, dim, stream);
+  }
+}
+
 // A block launch over a slice of the tables.
 int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a, hipStream_t stream) {
   if (sl.seg_count == 0) return RINGATTN_OK;
@@ -570,16 +644,9 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
     a.items = pl->d_segitems;
   }
   a.n_segs = sl.seg_count;
-  if (a.mode == ringattn::kBlockCarryState && sl.split && split_enabled()) {
-    a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kSplitM);
-    RA_HIP(ringattn::launch_split(a, pl->p.dtype, pl->p.dim, stream));
-    return RINGATTN_OK;
-  }
-  a.q_tiles_max = q_tiles_of(sl.q_len_max);
-  if (slice_takes_walk64(pl, sl, a.mode))
-    RA_HIP(ringattn::launch_walk64(a, pl->p.dtype, pl->p.dim, stream));
-  else
-    RA_HIP(ringattn::launch_walk(a, pl->p.dtype, pl->p.dim, stream));
+  const CarryKernel kernel =
+      a.mode == ringattn::kBlockCarryState ? carry_kernel(sl.costs, pl->p.dim) : CarryKernel::kWhole;
+  RA_HIP(launch_q_tiles(a, kernel, slice_takes_walk64(pl, sl, a.mode), sl.q_len_max, pl->p.dtype, pl->p.dim, stream));
   return RINGATTN_OK;
 }
 
@@ -680,20 +747,12 @@ int run_rank_call(const RankCall& rc, const void* q, const void* k, const void* 
   a.one_seg = rc.seg;
   a.one_item = rc.item;
   a.n_segs = 1;
-  a.q_tiles_max = q_tiles_of(c);
   a.bh_stride = (int64_t)c * dim;  // q and out hold this rank's rows only; k and v the whole sequence
   a.S = c;
   const bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled() && walk64_takes(rc.item);
-  WalkCost whole, split;
-  add_walks(whole, rc.seg, ringattn::kWalkM, 1, [&](int) -> const ringattn::SegItem& { return rc.item; });
-  add_walks(split, rc.seg, ringattn::kSplitM, 1, [&](int) -> const ringattn::SegItem& { return rc.item; });
-  if (split_pays(whole, split, dim) && split_enabled()) {
-    a.q_tiles_max = q_tiles_of(c, ringattn::kSplitM);
-    RA_HIP(ringattn::launch_split(a, rc.p.dtype, dim, stream));
-    return RINGATTN_OK;
-  }
-  if (wide) RA_HIP(ringattn::launch_walk64(a, rc.p.dtype, dim, stream));
-  else RA_HIP(ringattn::launch_walk(a, rc.p.dtype, dim, stream));
+  CarryCosts costs;
+  costs.add(rc.seg, 1, [&](int) -> const ringattn::SegItem& { return rc.item; });
+  RA_HIP(launch_q_tiles(a, carry_kernel(costs, dim), wide, c, rc.p.dtype, dim, stream));
   return RINGATTN_OK;
 }
 
@@ -938,7 +997,10 @@ int ringattn_plan_launch_times(ringattn_plan* plan, float* ms, int capacity, int
 const char* ringattn_plan_forward_kernel(const ringattn_plan* plan) {
   if (!plan_ok(plan)) return nullptr;
   const int mode = step_partials(plan->p) ? ringattn::kBlockPartialsMerged : ringattn::kBlockCarryState;
-  if (mode == ringattn::kBlockCarryState && plan->walk.split && split_enabled()) return "ring_split_kernel";
+  if (mode == ringattn::kBlockCarryState) {
+    const CarryKernel kernel = carry_kernel(plan->walk.costs, plan->p.dim);
+    if (kernel != CarryKernel::kWhole) return kernel == CarryKernel::kPair ? "ring_pair_kernel" : "ring_split_kernel";
+  }
   return slice_takes_walk64(plan, forward_slice(plan), mode) ? "ring_walk64_kernel" : "ring_walk_kernel";
 }
 

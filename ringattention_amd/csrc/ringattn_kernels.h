@@ -8,6 +8,7 @@ namespace ringattn {
 
 constexpr int kWalkM = 256;   // query rows per workgroup of ring_walk_kernel (8 waves x 32 rows)
 constexpr int kSplitM = 32;   // query rows per workgroup of ring_split_kernel
+constexpr int kPairM = 128;  // query rows per workgroup of ring_pair_kernel
 constexpr int kMaxParts = 64; // partial slots a merge can combine
 
 // One unit of block-attention work as the host layer lists it: the queries
@@ -142,6 +143,9 @@ hipError_t launch_walk64(BlockArgs a, int dtype, int dim, hipStream_t stream);
 // ring_split_kernel: kSplitM query rows per workgroup (a.q_tiles_max counts tiles of that many rows), the keys split over
 // its waves; kBlockCarryState
 hipError_t launch_split(BlockArgs a, int dtype, int dim, hipStream_t stream);
+// ring_pair_kernel: kPairM query rows per workgroup (a.q_tiles_max counts tiles of that many rows), the keys dealt to two
+// pairs of waves; kBlockCarryState, tables that CarryCosts::add finds fit for it
+hipError_t launch_pair(BlockArgs a, int dtype, int dim, hipStream_t stream);
 hipError_t launch_merge(const MergeArgs& a, int dtype, int dim, hipStream_t stream);
 
 }  // namespace ringattn

@@ -17,7 +17,7 @@
 //       have to take in 128 B per clock to keep its matrix pipes full, twice what its path to L2 carries; without the
 //       loads (timing only) the loop runs 25 % faster.  A full device reaches 690 TFLOP/s at d = 128 and 640 at d = 64
 //       (ring_walk64_kernel 1260 and 940), so this kernel is for launches that leave it compute units idle: the host
-//       weighs the two (split_pays in ringattn_api.hip).  One head of 8192 tokens, us: 152 -> 54 at d = 128, 114 -> 38 at
+//       weighs the kernels (carry_kernel in ringattn_api.hip).  One head of 8192 tokens, us: 152 -> 54 at d = 128, 114 -> 38 at
 //       d = 64; one head of 512 tokens 19.2 -> 10.2 and 13.6 -> 10.7 (with the host's share of the launch).
 #include "ringattn_device.h"
 
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void ring_split_kernel(const 
   // ---- combine the eight states: a common reference, every wave's factor against it, and the sums
   {
     const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
-    if (h == 0) stat[wave][n] = float2{l > 0.f ? ms : -INFINITY, l};
+    if (h == 0) stat[wave][n] = float2{l == 0.f ? -INFINITY : ms, l};  // (0: nothing seen; a NaN stays one)
   }
   __syncthreads();
   {
