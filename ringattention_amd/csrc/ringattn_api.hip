@@ -310,11 +310,12 @@ static int walk64_partials_choice() {
 }
 
 // RINGATTN_SPLIT=0 and RINGATTN_PAIR=0 in the environment take ring_split_kernel and ring_pair_kernel out of the choice below,
-// RINGATTN_PAIR=1 takes the latter whenever the shapes allow; RINGATTN_WIDE=0 and RINGATTN_WIDE_PARTIALS=1, which name one
-// of the 256-row kernels, keep every launch on these (comparisons, tests).
-static bool split_enabled() {
+// RINGATTN_PAIR=1 takes the latter whenever the shapes allow, RINGATTN_SPLIT=8 or 16 the former with that many waves (16 at
+// d = 64 only); RINGATTN_WIDE=0 and RINGATTN_WIDE_PARTIALS=1, which name one of the 256-row kernels, keep every launch on
+// these (comparisons, tests).
+static int split_choice() {  // -1: unset
   const char* e = std::getenv("RINGATTN_SPLIT");
-  return !(e && e[0] == '0');
+  return e ? std::atoi(e) : -1;
 }
 static int pair_choice() {
   const char* e = std::getenv("RINGATTN_PAIR");
@@ -337,7 +338,7 @@ static int pair_choice() {
 //     8 heads x 8192                       211, 230, 389     131, 145, 198
 //     9 heads x 8192 (288 q tiles of 256)  355, 310, 437     244, 208, 223
 //     16 heads x 8192, causal              221, 245, 424     142, 159, 209
-enum class CarryKernel { kWhole, kPair, kSplit };
+enum class CarryKernel { kWhole, kPair, kSplit, kSplit16 };
 struct KernelRate {
   int tiles_per_step;
   double lone, busy, job;
@@ -361,6 +362,8 @@ static double carry_time(const WalkCost& w, const KernelRate& r, bool equal_walk
 static CarryKernel carry_kernel(const CarryCosts& c, int dim) {
   if (!walk64_enabled() || walk64_partials_choice() == 1) return CarryKernel::kWhole;
   if (c.pair && pair_choice() == 1) return CarryKernel::kPair;
+  const int split = split_choice();
+  if (split == 8 || split == 16) return split == 16 && dim == 64 ? CarryKernel::kSplit16 : CarryKernel::kSplit;
   const KernelRate* r = dim == 128 ? kRates128 : kRates64;
   // the 256-row kernels unless another is ahead by more than these times are good for
   double best = carry_time(c.whole, r[0], !c.masked) * 0.95;
@@ -369,7 +372,14 @@ static CarryKernel carry_kernel(const CarryCosts& c, int dim) {
     const double t = carry_time(c.halves, r[1], !c.masked);
     if (t < best) best = t, kernel = CarryKernel::kPair;
   }
-  if (split_enabled() && carry_time(c.thin, r[2], false) < best) kernel = CarryKernel::kSplit;
+  if (split != 0 && carry_time(c.thin, r[2], false) < best) kernel = CarryKernel::kSplit;
+  // At d = 64 two workgroups of ring_split_kernel fit on a compute unit.  A launch of no more workgroups than there are
+  // compute units fills the other half with waves of the same workgroup, sixteen of them instead of eight, where the walk
+  // is long enough to pay for the combination of twice the states.  us with eight and with sixteen waves, at 64, 128, 256
+  // and 512 tiles: 2048 rows 12.8, 13.7; 4096 rows 20.4, 18.9; 8192 rows 36.9, 33.1; 8192 rows x 16384 keys 64.1, 58.2, 4096 of
+  // them 63.1, 48.5; causal 4096 rows 19.8, 18.6.  More workgroups than compute units: 8 heads x 2048 19.2, 25.6.
+  if (kernel == CarryKernel::kSplit && dim == 64 && c.thin.jobs <= kComputeUnits && c.thin.tiles >= 96)
+    kernel = CarryKernel::kSplit16;
   return kernel;
 }
 
@@ -622,8 +632,9 @@ hipError_t launch_q_tiles(ringattn::BlockArgs& a, CarryKernel kernel, bool wide,
       a.q_tiles_max = q_tiles_of(q_len, ringattn::kPairM);
       return ringattn::launch_pair(a, dtype, dim, stream);
     case CarryKernel::kSplit:
+    case CarryKernel::kSplit16:
       a.q_tiles_max = q_tiles_of(q_len, ringattn::kSplitM);
-      return ringattn::launch_split(a, dtype, dim, stream);
+      return ringattn::launch_split(a, dtype, dim, kernel == CarryKernel::kSplit16, stream);
     default:
       a.q_tiles_max = q_tiles_of(q_len);
       return wide ? ringattn::launch_walk64(a, dtype, dim, stream) : ringattn::launch_walk(a, dtype, dim, stream);

@@ -141,8 +141,8 @@ hipError_t launch_walk(BlockArgs a, int dtype, int dim, hipStream_t stream);  //
 // walk64_takes() accepts
 hipError_t launch_walk64(BlockArgs a, int dtype, int dim, hipStream_t stream);
 // ring_split_kernel: kSplitM query rows per workgroup (a.q_tiles_max counts tiles of that many rows), the keys split over
-// its waves; kBlockCarryState
-hipError_t launch_split(BlockArgs a, int dtype, int dim, hipStream_t stream);
+// its waves (eight; `many_waves`, d = 64 only: sixteen); kBlockCarryState
+hipError_t launch_split(BlockArgs a, int dtype, int dim, bool many_waves, hipStream_t stream);
 // ring_pair_kernel: kPairM query rows per workgroup (a.q_tiles_max counts tiles of that many rows), the keys dealt to two
 // pairs of waves; kBlockCarryState, tables that CarryCosts::add finds fit for it
 hipError_t launch_pair(BlockArgs a, int dtype, int dim, hipStream_t stream);

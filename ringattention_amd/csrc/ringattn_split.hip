@@ -2,9 +2,9 @@
 //
 //   ring_split_kernel : the forward of ring_walk_kernel and ring_walk64_kernel (the reference's CTA that walks its ring
 //       steps with max / sum / acc-O in registers, csrc/ring_attention.cu:439-443,456-620, epilogue :621-664) with the
-//       work split over the KEYS inside a workgroup: all EIGHT waves own the same 32 query rows, wave w takes the
-//       32-key tiles w, w + 8, w + 16, ... of the rows' key ranges with a softmax state of its own, and the eight
-//       states are combined through LDS at the end (the rescale of :226-232 once more, across waves instead of tiles).
+//       work split over the KEYS inside a workgroup: all WAVES (eight; sixteen at d = 64 where a compute unit
+//       has only one workgroup) own the same 32 query rows, wave w takes the 32-key tiles w, w + WAVES, ...
+//       of the rows' key ranges with a softmax state of its own, and the states are combined through LDS at the end (the rescale of :226-232 once more, across waves instead of tiles).
 //       A workgroup of the other kernels owns 256 rows, so a launch of 8192 rows has 32 workgroups on 256 compute units;
 //       here it has 256, and the walk of a workgroup is an eighth as long.
 //
@@ -18,15 +18,15 @@
 //       loads (timing only) the loop runs 25 % faster.  A full device reaches 690 TFLOP/s at d = 128 and 640 at d = 64
 //       (ring_walk64_kernel 1260 and 940), so this kernel is for launches that leave it compute units idle: the host
 //       weighs the kernels (carry_kernel in ringattn_api.hip).  One head of 8192 tokens, us: 152 -> 54 at d = 128, 114 -> 38 at
-//       d = 64; one head of 512 tokens 19.2 -> 10.2 and 13.6 -> 10.7 (with the host's share of the launch).
+//       d = 64; one head of 512 tokens 19.2 -> 10.2 and 13.6 -> 10.7 (with the host's share of the launch).  With sixteen waves, four
+//       per SIMD, for the 256 workgroups of 8192 rows x 16384 keys at d = 64: 64.1 -> 58.2, and for half as many rows 63.1 -> 48.5.
 #include "ringattn_device.h"
 
 namespace ringattn {
 
-template <int DT, int D>
-__global__ __launch_bounds__(512, D == 64 ? 4 : 2) void ring_split_kernel(const BlockArgs a) {
+template <int DT, int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel(const BlockArgs a) {
   using E = Elem<DT>;
-  constexpr int WAVES = 8;
   constexpr int BM = kSplitM;      // query rows per workgroup, all of them in every wave
   constexpr int BN = 32;           // keys per tile
   constexpr int CPR = D / 8;       // 16-byte chunks per row
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void ring_split_kernel(const 
     have = more;
   }
 
-  // ---- combine the eight states: a common reference, every wave's factor against it, and the sums
+  // ---- combine the states: a common reference, every wave's factor against it, and the sums
   {
     const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
     if (h == 0) stat[wave][n] = float2{l == 0.f ? -INFINITY : ms, l};  // (0: nothing seen; a NaN stays one)
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void ring_split_kernel(const 
   float o[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = 0.f;
-#pragma unroll
+#pragma unroll(WAVES > 8 ? 4 : 8)  // (sixteen waves' worth of reads in flight would not fit the registers)
   for (int w = 0; w < WAVES; ++w) {
     const float2 st = stat[w][row];
     l += st.x == -INFINITY ? 0.f : st.y * __builtin_amdgcn_exp2f(st.x - top);
@@ -311,15 +311,18 @@ __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void ring_split_kernel(const 
   if (c8 == 0 && a.lse) a.lse[orow] = (l > 0.f) ? (top + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
 }
 
-hipError_t launch_split(BlockArgs a, int dtype, int dim, hipStream_t stream) {
+hipError_t launch_split(BlockArgs a, int dtype, int dim, bool many_waves, hipStream_t stream) {
   if (a.n_segs <= 0) return hipSuccess;
   const int64_t blocks = job_grid(a, a.causal != 0);
   if (a.q_tiles_max <= 0 || blocks > INT32_MAX || a.mode != kBlockCarryState) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)blocks;
-  if (dtype == 0 && dim == 64) ring_split_kernel<0, 64><<<grid, 512, 0, stream>>>(a);
-  else if (dtype == 1 && dim == 64) ring_split_kernel<1, 64><<<grid, 512, 0, stream>>>(a);
-  else if (dtype == 0 && dim == 128) ring_split_kernel<0, 128><<<grid, 512, 0, stream>>>(a);
-  else if (dtype == 1 && dim == 128) ring_split_kernel<1, 128><<<grid, 512, 0, stream>>>(a);
+  if (many_waves && dim != 64) return hipErrorInvalidValue;
+  if (dtype == 0 && many_waves) ring_split_kernel<0, 64, 16><<<grid, 1024, 0, stream>>>(a);
+  else if (dtype == 1 && many_waves) ring_split_kernel<1, 64, 16><<<grid, 1024, 0, stream>>>(a);
+  else if (dtype == 0 && dim == 64) ring_split_kernel<0, 64, 8><<<grid, 512, 0, stream>>>(a);
+  else if (dtype == 1 && dim == 64) ring_split_kernel<1, 64, 8><<<grid, 512, 0, stream>>>(a);
+  else if (dtype == 0 && dim == 128) ring_split_kernel<0, 128, 8><<<grid, 512, 0, stream>>>(a);
+  else if (dtype == 1 && dim == 128) ring_split_kernel<1, 128, 8><<<grid, 512, 0, stream>>>(a);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

@@ -1,4 +1,4 @@
-"""ring_split_kernel (ringattn_split.hip: 32 query rows per workgroup, the keys split over its eight waves) against the
+"""ring_split_kernel (ringattn_split.hip: 32 query rows per workgroup, the keys split over its eight or sixteen waves) against the
 CPU oracle where it can go wrong: fewer tiles than waves, one tile more or less than a round of eight, a last tile of one
 key, rows of a tile that see nothing of a wave's first tile (causal), several key ranges (zigzag), grouped heads, heads
 that the eight XCDs share unevenly, and logits that make every wave move its reference again and again.  Bounds: those of
@@ -31,6 +31,10 @@ from test_kernel_resources import compile_to_asm
 def test_split_kernel_against_oracle(oracle, monkeypatch, lens, B, H, hkv, dtype, causal, zigzag, slope, d):
     for name in ("RINGATTN_WIDE", "RINGATTN_WIDE_PARTIALS", "RINGATTN_SPLIT"):
         monkeypatch.delenv(name, raising=False)
+    check_forward(oracle, lens, B, H, hkv, dtype, causal, zigzag, slope, d)
+
+
+def check_forward(oracle, lens, B, H, hkv, dtype, causal, zigzag, slope, d):
     S = sum(lens)
     w = Workload("split", B, H, d, 1, S, dtype, 900 + S, causal)
     q, _, _ = rising_logits(w, slope) if slope else api.make_qkv_bits(w)
@@ -53,15 +57,34 @@ def test_split_kernel_against_oracle(oracle, monkeypatch, lens, B, H, hkv, dtype
     check_rows(oracle, w, q, k_full, v_full, out[:, :, inv].contiguous(), lse[:, :, inv].contiguous(), np.arange(w.rows))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,B,H,hkv,dtype,causal,zigzag,slope,forced", [
+    ((1,), 1, 1, 1, "fp16", True, False, 0, True),                       # fifteen waves see nothing
+    ((480,), 1, 2, 1, "bf16", False, False, 0, True),                    # fifteen tiles
+    ((300, 212), 1, 2, 2, "fp16", True, False, 0, True),                 # sixteen: one per wave
+    ((513,), 2, 3, 3, "fp16", False, False, 0, True),                    # a seventeenth tile of one key
+    ((130, 70, 2, 258), 1, 2, 2, "bf16", True, True, 0, True),           # several ranges
+    ((1024, 1025), 1, 1, 1, "fp16", True, False, 0.3, True),             # the row maximum keeps climbing
+    ((1536, 1601), 1, 2, 1, "fp16", True, False, 0, False),              # 99 tiles, 198 workgroups: chosen without being asked
+])
+def test_split_kernel_with_sixteen_waves(oracle, monkeypatch, lens, B, H, hkv, dtype, causal, zigzag, slope, forced):
+    for name in ("RINGATTN_WIDE", "RINGATTN_WIDE_PARTIALS", "RINGATTN_SPLIT"):
+        monkeypatch.delenv(name, raising=False)
+    if forced:
+        monkeypatch.setenv("RINGATTN_SPLIT", "16")
+    check_forward(oracle, lens, B, H, hkv, dtype, causal, zigzag, slope, 64)
+
+
 def test_split_kernel_resources_and_hazards(tmp_path):
     """Two waves per SIMD at d = 128, four (two workgroups per compute unit) at d = 64, no scratch; and the wait states in
     front of the direct-to-LDS loads."""
     _, usage = compile_to_asm("ringattn_split.hip", tmp_path / "split.s")
     kernels = {n: u for n, u in usage.items() if "ring_split_kernel" in n}
-    assert len(kernels) == 4
+    assert len(kernels) == 6
     for n, u in kernels.items():
         d64 = "ELi64E" in n
         assert u["ScratchSize [bytes/lane]"] == 0, (n, u)
         assert u["VGPRs"] <= (128 if d64 else 256), (n, u)
-        assert 2 * u["LDS Size [bytes/block]"] <= 160 * 1024 if d64 else u["LDS Size [bytes/block]"] <= 160 * 1024, (n, u)
+        share = 2 if d64 and "ELi8E" in n else 1  # (sixteen waves at d = 64: one workgroup, four waves per SIMD)
+        assert share * u["LDS Size [bytes/block]"] <= 160 * 1024, (n, u)
     _hazards("ringattn_split.hip", tmp_path)
