@@ -133,7 +133,7 @@ int ringattn_plan_destroy(ringattn_plan* plan);
 /*
  * The whole forward for all npes virtual ranks: replaces ring_attention()
  * (csrc/ring_attention.cu:706-722) run on every PE.  ONE block-attention launch: a workgroup
- * owns 256 query rows and walks the keys of every ring step of those rows with the running max, sum and
+ * owns 256, 128 or 32 query rows and walks the keys of every ring step of those rows with the running max, sum and
  * acc-O in registers, like the reference's CTA (:439-443,456,597), then writes O = acc / sum
  * (:621-664) and the LSE.  (With RINGATTN_FLAG_STEP_PARTIALS: a partial (O, LSE) per step into
  * the workspace, merged at the end of the workgroup.)
