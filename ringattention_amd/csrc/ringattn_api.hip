@@ -259,13 +259,18 @@ static void add_walks(WalkCost& c, const ringattn::Segment& seg, int rows, int64
   c.total += heads * q_tiles * (fixed + (first + last) / 2);
   c.jobs += heads * q_tiles;
 }
+// The generated loops (ring_walk64_kernel, ring_pair_kernel) keep the place of a key range -- and the place of its last
+// tile, where that one is ragged -- as a byte offset within the head, in 32 bits: tile 1 of the range has to begin within 4 GiB.
+// (A range may reach beyond that: the loops add whole tiles to 64-bit addresses.)
+static bool begins_within_4g(const ringattn::SegItem& it, int dim) { return ((int64_t)it.kv_start + 32) * 2 * dim <= UINT32_MAX; }
+
 constexpr int kComputeUnits = 256;
 struct CarryCosts {
   WalkCost whole, halves, thin;  // with q tiles of kWalkM, kPairM and kSplitM rows
   bool pair = true;              // every segment suits ring_pair_kernel
   bool masked = false;           // the walks differ in length
   template <class ItemFn>
-  void add(const ringattn::Segment& seg, int64_t heads, ItemFn item) {
+  void add(const ringattn::Segment& seg, int64_t heads, int dim, ItemFn item) {
     add_walks(whole, seg, ringattn::kWalkM, heads, item);
     add_walks(halves, seg, ringattn::kPairM, heads, item);
     add_walks(thin, seg, ringattn::kSplitM, heads, item);
@@ -275,7 +280,7 @@ struct CarryCosts {
     for (int i = 0; i < seg.item_count; ++i) {
       const ringattn::SegItem& it = item(i);
       masked = masked || it.diag_off >= 0;
-      pair = pair && it.kv_len >= 128 && (it.kv_len % 32 == 0 || (i == last && it.kv_start + it.kv_len <= 1 << 24));
+      pair = pair && begins_within_4g(it, dim) && it.kv_len >= 128 && (it.kv_len % 32 == 0 || (i == last && it.kv_start + it.kv_len <= 1 << 24));
     }
   }
 };
@@ -291,7 +296,9 @@ struct TableSlice {
 
 // ring_walk64_kernel walks whole 32-key tiles, and past the end of its sequence its load streams go round the first
 // four tiles of a head: a KV range must be a multiple of 32 keys and hold at least 128.
-static bool walk64_takes(const ringattn::SegItem& it) { return it.kv_len % 32 == 0 && it.kv_len >= 128; }
+static bool walk64_takes(const ringattn::SegItem& it, int dim) {
+  return it.kv_len % 32 == 0 && it.kv_len >= 128 && begins_within_4g(it, dim);
+}
 // RINGATTN_WIDE=0 in the environment keeps every forward on ring_walk_kernel (for comparisons)
 static bool walk64_enabled() {
   const char* e = std::getenv("RINGATTN_WIDE");
@@ -477,7 +484,7 @@ void push_segment(ringattn_plan* pl, TableSlice& slice, int q_start, int q_len,
   if (sg.item_count == 1) sg.last_item = -1;
   pl->h_segs.push_back(sg);
   bool wide = true;
-  for (size_t i = 0; i < items.size(); ++i) wide = wide && walk64_takes(pl->h_segitems[(size_t)sg.item_begin + i]);
+  for (size_t i = 0; i < items.size(); ++i) wide = wide && walk64_takes(pl->h_segitems[(size_t)sg.item_begin + i], pl->p.dim);
   slice.wide = slice.seg_count == 0 ? wide : (slice.wide && wide);
   for (size_t i = 0; i < items.size(); ++i) {
     const int kv = pl->h_segitems[(size_t)sg.item_begin + i].kv_len;
@@ -518,7 +525,7 @@ void build_schedule(ringattn_plan* pl) {
     push_segment(pl, pl->walk, sg.start, sg.len, sg.items, 0, [](int) { return (int64_t)0; }, 0);
   for (int i = 0; i < pl->walk.seg_count; ++i) {
     const ringattn::Segment& sg = pl->h_segs[(size_t)(pl->walk.seg_begin + i)];
-    pl->walk.costs.add(sg, d.BH, [&](int k) -> const ringattn::SegItem& { return pl->h_segitems[(size_t)(sg.item_begin + k)]; });
+    pl->walk.costs.add(sg, d.BH, pl->p.dim, [&](int k) -> const ringattn::SegItem& { return pl->h_segitems[(size_t)(sg.item_begin + k)]; });
   }
 
   // ---- one ring step of every rank: partials at the rows of the queries in a [BH, S] slot
@@ -760,9 +767,9 @@ int run_rank_call(const RankCall& rc, const void* q, const void* k, const void* 
   a.n_segs = 1;
   a.bh_stride = (int64_t)c * dim;  // q and out hold this rank's rows only; k and v the whole sequence
   a.S = c;
-  const bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled() && walk64_takes(rc.item);
+  const bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled() && walk64_takes(rc.item, dim);
   CarryCosts costs;
-  costs.add(rc.seg, 1, [&](int) -> const ringattn::SegItem& { return rc.item; });
+  costs.add(rc.seg, 1, dim, [&](int) -> const ringattn::SegItem& { return rc.item; });
   RA_HIP(launch_q_tiles(a, carry_kernel(costs, dim), wide, c, rc.p.dtype, dim, stream));
   return RINGATTN_OK;
 }
