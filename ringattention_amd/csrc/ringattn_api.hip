@@ -318,8 +318,8 @@ static int walk64_partials_choice() {
 
 // RINGATTN_SPLIT=0 and RINGATTN_PAIR=0 in the environment take ring_split_kernel and ring_pair_kernel out of the choice below,
 // RINGATTN_PAIR=1 takes the latter whenever the shapes allow, RINGATTN_SPLIT=8 or 16 the former with that many waves (16 at
-// d = 64 only); RINGATTN_WIDE=0 and RINGATTN_WIDE_PARTIALS=1, which name one of the 256-row kernels, keep every launch on
-// these (comparisons, tests).
+// d = 64 only); RINGATTN_WIDE=0, RINGATTN_WIDE_D64=0 (d = 64) and RINGATTN_WIDE_PARTIALS=1, which name one of the 256-row
+// kernels, keep every launch on these (comparisons, tests).
 static int split_choice() {  // -1: unset
   const char* e = std::getenv("RINGATTN_SPLIT");
   return e ? std::atoi(e) : -1;
@@ -367,7 +367,7 @@ static double carry_time(const WalkCost& w, const KernelRate& r, bool equal_walk
 }
 
 static CarryKernel carry_kernel(const CarryCosts& c, int dim) {
-  if (!walk64_enabled() || walk64_partials_choice() == 1) return CarryKernel::kWhole;
+  if (!walk64_enabled() || (dim == 64 && !walk64_d64_enabled()) || walk64_partials_choice() == 1) return CarryKernel::kWhole;
   if (c.pair && pair_choice() == 1) return CarryKernel::kPair;
   const int split = split_choice();
   if (split == 8 || split == 16) return split == 16 && dim == 64 ? CarryKernel::kSplit16 : CarryKernel::kSplit;

@@ -38,3 +38,13 @@ def test_per_step_partials_of_chunks_that_begin_beyond_4_gib(monkeypatch):
     for lens, kernel in (((rows // 2, rows // 2), "ring_walk64_kernel"), ((rows // 2, rows // 2, 4096), "ring_walk_kernel")):
         assert chosen(monkeypatch, lens, 128, causal=True, env={"RINGATTN_WIDE_PARTIALS": "1"}, step_partials=True,
                       workspace=(1 << 20, 1 << 60)) == kernel
+
+
+@pytest.mark.parametrize("lens,heads,causal", [((2048,), 1, False), ((8192,), 4, False), ((4400,), 16, True), ((1024,) * 8, 8, False)])
+def test_switches_that_name_a_256_row_kernel(monkeypatch, lens, heads, causal):
+    """RINGATTN_WIDE=0 and, at d = 64, RINGATTN_WIDE_D64=0 keep a forward on ring_walk_kernel whatever its size; the latter
+    says nothing about d = 128."""
+    for d in (64, 128):
+        assert chosen(monkeypatch, lens, d, heads, causal, env={"RINGATTN_WIDE": "0"}) == "ring_walk_kernel"
+    assert chosen(monkeypatch, lens, 64, heads, causal, env={"RINGATTN_WIDE_D64": "0"}) == "ring_walk_kernel"
+    assert chosen(monkeypatch, lens, 128, heads, causal, env={"RINGATTN_WIDE_D64": "0"}) == chosen(monkeypatch, lens, 128, heads, causal)
