@@ -253,7 +253,9 @@ def redo_routine(cur, cvt):
     """Out of line: the exponentials of the tile in score buffer `cur` came out too large for the standing reference
     (a sum of four above 2^14).  All MFMAs of the iteration are issued and acc-O holds the tiles before this one, so
     the reference moves to the row maximum at once -- l and acc-O rescaled as in csrc/ring_attention.cu:226-232 -- and
-    the exponentials are taken again.  s57 says where to go back to."""
+    the exponentials are taken again.  s57 says where to go back to.
+    A row whose scores so far are all -inf has m = -inf and, for m k2, the lowest finite value (kNoReference in
+    ringattn_device.h): its probabilities stay 0, and its first finite score overflows and leads here."""
     out = ["85%d:" % cur, "s_nop 15"]
     for stp in range(4):
         for b in range(2):
@@ -272,6 +274,8 @@ def redo_routine(cur, cvt):
         out.append("v_max_f32 %s, %s, %s" % (M(b), TMP(2 * b), TMP(2 * b + 1)))        # the new reference
     for b in range(2):
         out.append("v_mul_f32 %s, %s, %s" % (TMP(4 + b), S_K2, M(b)))                  # m k2
+    for b in range(2):
+        out.append("v_max_f32 %s, 0xff7fffff, %s" % (TMP(4 + b), TMP(4 + b)))          # (a row that has seen nothing: kNoReference)
     for b in range(2):
         out.append("v_sub_f32 %s, %s, %s" % (TMP(6 + b), MS(b), TMP(4 + b)))           # old m k2 - new m k2
     for b in range(2):

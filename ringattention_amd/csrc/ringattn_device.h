@@ -87,6 +87,11 @@ template <int D> static __device__ __forceinline__ int v_swizzle(int row) {
                   : ((((row >> 1) & 1) << 2) | (((row >> 2) & 1) << 1));
 }
 
+// m * k2 of a row in the generated loops while its scores so far are all -inf (keys that a coordinate of -inf hides: left
+// padding): the exponential of such a score against it is 0, and that of the first finite one infinite, which is what makes the
+// loops look at the row maximum (redo_routine in gen_walk64_loop.py).
+constexpr float kNoReference = -3.402823466e38f;
+
 // The segments and items of a launch: the tables in memory, or the one of each that came with the kernel arguments (the
 // single parameter of every kernel of this library sits at the start of the argument segment).  Pointers to constant
 // memory either way: a table is not written while a kernel runs, and the loads are then scalar ones.

@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256, 1) void ring_pair_kernel(const BlockArgs a) {
   __syncthreads();
 
   // ---- softmax state of the two blocks
-  float m[2], ms[2];  // reference max (raw score units); m * k2, 0 while m is -inf (guard of csrc/ring_attention.cu:183)
+  float m[2], ms[2];  // reference max (raw score units); m * k2, kNoReference while m is -inf (guard of csrc/ring_attention.cu:183)
   float ls[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   f32x16 oacc[2][DB];
   f32x16 sacc[2];     // scores of tile u, consumed by the exponentials of iteration u
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(256, 1) void ring_pair_kernel(const BlockArgs a) {
       m1 = fmaxf(fmaxf(m1, sacc[b][e + 2]), sacc[b][e + 3]);
     }
     m[b] = cross_half_max(fmaxf(m0, m1));
-    ms[b] = (m[b] == -INFINITY) ? 0.f : m[b] * a.scale_log2;
+    ms[b] = (m[b] == -INFINITY) ? kNoReference : m[b] * a.scale_log2;
   }
   if (grp == 1) scores(1, 1, before_last == 0 && clear <= 1);
 

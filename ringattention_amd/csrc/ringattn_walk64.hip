@@ -313,7 +313,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
 
   // ---- softmax state of the two blocks
   float m[2] = {-INFINITY, -INFINITY};  // reference max (raw score units)
-  float ms[2] = {0.f, 0.f};             // m * k2, 0 while m is -inf (guard of csrc/ring_attention.cu:183)
+  float ms[2] = {0.f, 0.f};             // m * k2, kNoReference while m is -inf (guard of csrc/ring_attention.cu:183)
   float ls[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   f32x16 oacc[2][DB];
 #pragma unroll
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
 #pragma unroll
   for (int b = 0; b < 2; ++b) {  // the first reference: the row maxima of tile 0
     m[b] = tile_max(sacc[b], m[b]);
-    ms[b] = (m[b] == -INFINITY) ? 0.f : m[b] * a.scale_log2;
+    ms[b] = (m[b] == -INFINITY) ? kNoReference : m[b] * a.scale_log2;
   }
 
   // LDS addresses for the hand-scheduled loop: fragment offsets from the start of LDS, and where this wave's two
