@@ -414,10 +414,10 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
 
   // The hand-scheduled loop (ringattn_walk64_loop.inc) runs all iterations of the workgroup, 0 to N: every iteration
   // whose score tile u+1 this wave computes -- masking the tiles of the diagonal chunk that need it --, the wave's last
-  // two iterations, and then only the wave's share of the loads and the barriers.  A wave with no second score tile
-  // walks the iterations in plain code.
-  if (1 < Ew) {
-    const int u = 0;  // where the loop starts
+  // two iterations, and then only the wave's share of the loads and the barriers.  Every wave goes through it: the
+  // barriers and tile loads in it are the workgroup's.  (A wave has two tiles at least: a range is four, and of a diagonal
+  // one the first 64 keys are visible to some row of every wave.  The loop would do with one.)
+  {
     unsigned asm_u = 0, asm_far = 0;
     const unsigned asm_stop = uni((unsigned)(Ew - 1)), asm_mw1 = uni((unsigned)(Mw - 1));
     int vlim[2];

@@ -122,6 +122,24 @@ def test_walk64_kernel_runs_one_wave_per_simd(tmp_path):
         assert "scratch_" not in loop
 
 
+def test_every_wave_of_the_workgroup_enters_the_hand_scheduled_loop(tmp_path):
+    """The loop holds the workgroup's barriers and each wave's share of the tile loads: from the last barrier in front of it on
+    no branch may lead past it."""
+    for source, kernel in (("ringattn_walk64.hip", "ring_walk64_kernel"), ("ringattn_pair.hip", "ring_pair_kernel")):
+        asm, usage = compile_to_asm(source, tmp_path / "loop.s")
+        for n in (n for n in usage if kernel in n):
+            start = asm.index("\n" + n + ":")
+            lines = asm[start:asm.index(".amdhsa_kernel " + n, start)].split("\n")
+            at = {m.group(1): i for i, m in enumerate(re.match(r"(\.LBB\d+_\d+):", l) for l in lines) if m}
+            begins = [i for i, l in enumerate(lines) if ";;#ASMSTART" in l]
+            ends = [next(j for j in range(i, len(lines)) if ";;#ASMEND" in lines[j]) for i in begins]
+            begin, end = max(zip(begins, ends), key=lambda x: x[1] - x[0])
+            barrier = max(i for i in range(begin) if lines[i].strip() == "s_barrier")
+            for l in lines[barrier:begin]:
+                m = re.match(r"\s*s_c?branch\S*\s+(\.LBB\d+_\d+)", l)
+                assert not m or at[m.group(1)] < end, (n, l)
+
+
 @pytest.mark.parametrize("source", ["ringattn_walk.hip", "ringattn_walk64.hip"])
 def test_no_lds_transfer_reads_a_scalar_register_fresh_from_a_vector_instruction(source, tmp_path):
     """A vector instruction that writes a scalar register (v_readfirstlane, v_readlane, a compare into a register
