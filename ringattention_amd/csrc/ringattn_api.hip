@@ -399,7 +399,7 @@ struct ringattn_plan {
   bool own_ws = false;
   void* o_parts = nullptr;     // partial O rows, fp32 (fp16 with RINGATTN_FLAG_HALF_PARTIALS)
   float* lse_parts = nullptr;  // partial LSE rows
-  // Segment / item tables (host copies + device copies made at the first launch).  Three
+  // Segment / item tables (host copies; device copies made by ensure_tables).  Three
   // families of slices: the forward (all ring steps of every rank, one launch, partials in the
   // workspace), one ring step of every rank (ringattn_block_fwd, partials in the caller's
   // [batch*heads, S] slot), one step of one rank on rank-local rows (ringattn_rank_step_fwd).
@@ -582,19 +582,46 @@ void build_schedule(ringattn_plan* pl) {
   }
 }
 
-// Device copies of the tables and the timing events: made at the first launch, outside any capture.
-int ensure_tables(ringattn_plan* pl) {
-  if (pl->tables_ready) return RINGATTN_OK;
+// The copies of ensure_tables, by way of `copies`: NULL, or a stream of its own next to one that is being captured.
+int upload_tables(ringattn_plan* pl, hipStream_t copies) {
   // a call that failed half way is resumed: nothing is created twice
-  const size_t seg_bytes = pl->h_segs.size() * sizeof(ringattn::Segment);
-  const size_t item_bytes = pl->h_segitems.size() * sizeof(ringattn::SegItem);
-  const size_t reg_bytes = pl->regions.size() * sizeof(ringattn::MergeRegion);
-  if (!pl->d_segs) RA_HIP(hipMalloc((void**)&pl->d_segs, seg_bytes));
-  if (!pl->d_segitems) RA_HIP(hipMalloc((void**)&pl->d_segitems, item_bytes));
-  if (!pl->d_regions) RA_HIP(hipMalloc((void**)&pl->d_regions, reg_bytes));
-  RA_HIP(hipMemcpy(pl->d_segs, pl->h_segs.data(), seg_bytes, hipMemcpyHostToDevice));
-  RA_HIP(hipMemcpy(pl->d_segitems, pl->h_segitems.data(), item_bytes, hipMemcpyHostToDevice));
-  RA_HIP(hipMemcpy(pl->d_regions, pl->regions.data(), reg_bytes, hipMemcpyHostToDevice));
+  auto upload = [&](void** dst, const void* src, size_t bytes) -> int {
+    if (!*dst) RA_HIP(hipMalloc(dst, bytes));
+    if (copies) RA_HIP(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, copies));
+    else RA_HIP(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
+    return RINGATTN_OK;
+  };
+  int rc = upload((void**)&pl->d_segs, pl->h_segs.data(), pl->h_segs.size() * sizeof(ringattn::Segment));
+  if (rc == RINGATTN_OK) rc = upload((void**)&pl->d_segitems, pl->h_segitems.data(), pl->h_segitems.size() * sizeof(ringattn::SegItem));
+  if (rc == RINGATTN_OK) rc = upload((void**)&pl->d_regions, pl->regions.data(), pl->regions.size() * sizeof(ringattn::MergeRegion));
+  return rc;
+}
+
+// Device copies of the tables and the timing events: made by the first call of a step or a merge, and by the first forward
+// whose launch does not carry its only range in its arguments.  That call may sit in a capture of `stream` (the forwards
+// that warmed the plan up needed no tables): the copies are then made beside the captured work, at once, on a stream of
+// their own, in the capture mode that allows the thread to allocate.
+int ensure_tables(ringattn_plan* pl, hipStream_t stream) {
+  if (pl->tables_ready) return RINGATTN_OK;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (stream) RA_HIP(hipStreamIsCapturing(stream, &capture));
+  if (capture == hipStreamCaptureStatusNone) {
+    const int rc = upload_tables(pl, nullptr);
+    if (rc != RINGATTN_OK) return rc;
+  } else {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    hipStream_t copies = nullptr;
+    hipError_t e = hipStreamCreateWithFlags(&copies, hipStreamNonBlocking);
+    int rc = e == hipSuccess ? upload_tables(pl, copies) : hip_fail(e);
+    if (copies) {
+      e = hipStreamSynchronize(copies);
+      if (rc == RINGATTN_OK && e != hipSuccess) rc = hip_fail(e);
+      (void)hipStreamDestroy(copies);
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (rc != RINGATTN_OK) return rc;
+  }
   if (pl->p.flags & RINGATTN_FLAG_TIMING) {
     if (!pl->ev_t0) RA_HIP(hipEventCreate(&pl->ev_t0));
     if (!pl->ev_t1) RA_HIP(hipEventCreate(&pl->ev_t1));
@@ -656,7 +683,7 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
     a.one_item = pl->h_segitems[(size_t)a.one_seg.item_begin];
     a.one_seg.item_begin = 0;  // the item's place is with the arguments now
   } else {
-    const int rc = ensure_tables(pl);
+    const int rc = ensure_tables(pl, stream);
     if (rc != RINGATTN_OK) return rc;
     a.segs = pl->d_segs + sl.seg_begin;
     a.items = pl->d_segitems;
@@ -877,7 +904,7 @@ int ringattn_fwd(ringattn_plan* plan, const void* q, const void* k, const void* 
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || ((uintptr_t)lse & 3u)) return RINGATTN_ERR_ALIGN;
   hipStream_t stream = (hipStream_t)stream_;
   if ((plan->p.flags & (RINGATTN_FLAG_TIMING | RINGATTN_FLAG_GRAPH)) || step_partials(plan->p)) {
-    const int rc0 = ensure_tables(plan);  // the timing events too; and nothing may be allocated during the capture
+    const int rc0 = ensure_tables(plan, stream);  // the timing events too; and nothing may be allocated during the capture
     if (rc0 != RINGATTN_OK) return rc0;
   }
   if (!(plan->p.flags & RINGATTN_FLAG_GRAPH)) return run_forward(plan, q, k, v, out, lse, stream);
@@ -918,6 +945,8 @@ int ringattn_block_fwd(ringattn_plan* plan, int step, const void* q, const void*
   if (!q || !k || !v || !o_part || !lse_part) return RINGATTN_ERR_NULL;
   if (step < 0 || step >= plan->p.npes) return RINGATTN_ERR_RANK;
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o_part) || ((uintptr_t)lse_part & 3u)) return RINGATTN_ERR_ALIGN;
+  const int rc = ensure_tables(plan, (hipStream_t)stream);  // whether or not this step reads them: the merge will
+  if (rc != RINGATTN_OK) return rc;
   ringattn::BlockArgs a;
   fill_geometry(a, plan->p, plan->d);
   a.q = q;
@@ -933,7 +962,7 @@ int ringattn_merge_ring(ringattn_plan* plan, const void* o_parts, const float* l
   if (!plan_ok(plan)) return RINGATTN_ERR_PLAN;
   if (!o_parts || !lse_parts || !out || !lse) return RINGATTN_ERR_NULL;
   if (!aligned16(o_parts) || !aligned16(out) || ((uintptr_t)lse_parts & 3u) || ((uintptr_t)lse & 3u)) return RINGATTN_ERR_ALIGN;
-  int rc = ensure_tables(plan);
+  int rc = ensure_tables(plan, (hipStream_t)stream);
   if (rc != RINGATTN_OK) return rc;
   // ONE launch: a grid row per region
   return launch_regions(plan, 0, plan->n_regions, plan->region_max_len, (int)plan->d.S, plan->d.rows, o_parts, lse_parts,
@@ -947,6 +976,8 @@ int ringattn_rank_step_fwd(ringattn_plan* plan, int rank, int step, const void* 
   const int P = plan->p.npes;
   if (rank < 0 || rank >= P || step < 0 || step >= P) return RINGATTN_ERR_RANK;
   if (!aligned16(q) || !aligned16(k_chunk) || !aligned16(v_chunk) || !aligned16(o_part) || ((uintptr_t)lse_part & 3u)) return RINGATTN_ERR_ALIGN;
+  const int rc = ensure_tables(plan, (hipStream_t)stream);  // whether or not this step reads them: the merge will
+  if (rc != RINGATTN_OK) return rc;
   const Derived& d = plan->d;
   const int j = (rank + step) % P;
   const int64_t q_rows = d.start[rank + 1] - d.start[rank], kv_rows = d.start[j + 1] - d.start[j];
@@ -970,7 +1001,7 @@ int ringattn_rank_merge(ringattn_plan* plan, int rank, const void* o_parts, cons
   if (!o_parts || !lse_parts || !out || !lse) return RINGATTN_ERR_NULL;
   if (rank < 0 || rank >= plan->p.npes) return RINGATTN_ERR_RANK;
   if (!aligned16(o_parts) || !aligned16(out) || ((uintptr_t)lse_parts & 3u) || ((uintptr_t)lse & 3u)) return RINGATTN_ERR_ALIGN;
-  int rc = ensure_tables(plan);
+  int rc = ensure_tables(plan, (hipStream_t)stream);
   if (rc != RINGATTN_OK) return rc;
   const Derived& d = plan->d;
   const int rows = d.start[rank + 1] - d.start[rank];
