@@ -4,6 +4,7 @@
 #include "ringattn_kernels.h"
 
 #include <cstddef>
+#include <type_traits>
 
 namespace ringattn {
 
@@ -261,7 +262,7 @@ static __device__ __forceinline__ void store_block(const f32x16 (&acc)[D / 32], 
 // arranged differently: the attention kernel, which runs this at the end of a workgroup, has just two
 // waves per SIMD to hide memory latency with, and every round trip it waits for is time its
 // compute unit runs half empty.  So all partial LSEs are fetched in one sweep and parked in LDS
-// (lse_s: [items][128] floats), and the partial O rows move in batches of 256 bytes per thread
+// (lse_s: [items][BM] floats), and the partial O rows move in batches of 256 bytes per thread
 // (two output rows x four or eight parts), three batches in flight at any time.
 typedef __attribute__((address_space(3))) float lds_float;
 template <int DT, int D, bool HP, int BM, int THREADS>
@@ -271,8 +272,6 @@ static __device__ __forceinline__ void merge_job_rows(const void* o_part, const 
   constexpr int WAVES = THREADS / 64;
   constexpr int TPR = D / 8;  // threads per row, 8 columns each
   constexpr int ROWS = THREADS / TPR;
-  constexpr int R = 2, G = HP ? 8 : 4;  // rows per thread and parts per batch: 64 registers a batch
-  constexpr int RSTEP = R * ROWS;
   constexpr int KMAX = kMaxParts / WAVES;  // parts per wave in the LSE sweep
   constexpr int LR = BM / 64;              // rows per lane in the LSE sweep
   const int tid = threadIdx.x, lane = tid & 63;
@@ -316,112 +315,124 @@ static __device__ __forceinline__ void merge_job_rows(const void* o_part, const 
   // this thread's 8 columns of a partial row: 16 bytes as fp16, 32 as fp32
   constexpr int PB = HP ? 16 : 32;
   constexpr int NV = PB / 16;
-  const int n_groups = (n_parts + G - 1) / G;
-  const int n_batches = (BM / RSTEP) * n_groups;  // batch b: rows of b / n_groups, parts of b % n_groups
-  struct Batch {
-    f32x4 raw[R][G][NV];  // as loaded; fp16 partials are widened when they are used
-  };
-  auto row_of = [&](int b, int j) { return (b / n_groups) * RSTEP + j * ROWS + rsub; };  // within the job
-  // Every load of a batch is made, those of parts and rows that do not exist from the last one that does: with loads under
-  // conditions the compiler cannot count those in flight, and waits for the batches fetched ahead as well.  Where the parts
-  // lie comes from a lane of first_row and not from the table, a scalar round trip for each.  Together, and past the
-  // cache's retention (fp16; fp32 rows measured 1.6 % slower that way): forward with fp16 partials, 64 heads x 32 x 512, d = 128
-  // 11.74 -> 10.70 ms, of which the merge was 2.4 ms; fp32 partials, 16 heads 3.74 -> 3.64 ms.
-  auto fetch = [&](int b, Batch& t) {
-    const int i0 = (b % n_groups) * G;
-    int at[R];
+  // R rows and G parts of a thread per batch
+  auto merge_in = [&](auto rows_c, auto parts_c) {
+    constexpr int R = decltype(rows_c)::value, G = decltype(parts_c)::value;
+    constexpr int RSTEP = R * ROWS;
+    const int n_groups = (n_parts + G - 1) / G;
+    const int n_batches = (BM / RSTEP) * n_groups;  // batch b: rows of b / n_groups, parts of b % n_groups
+    struct Batch {
+      f32x4 raw[R][G][NV];  // as loaded; fp16 partials are widened when they are used
+    };
+    auto row_of = [&](int b, int j) { return (b / n_groups) * RSTEP + j * ROWS + rsub; };  // within the job
+    // Every load of a batch is made, those of parts and rows that do not exist from the last one that does: with loads under
+    // conditions the compiler cannot count those in flight, and waits for the batches fetched ahead as well.  Where the parts
+    // lie comes from a lane of first_row and not from the table, a scalar round trip for each.  Together, and past the
+    // cache's retention (fp16; fp32 rows measured 1.6 % slower that way): forward with fp16 partials, 64 heads x 32 x 512, d = 128
+    // 11.74 -> 10.70 ms, of which the merge was 2.4 ms; fp32 partials, 16 heads 3.74 -> 3.64 ms.
+    auto fetch = [&](int b, Batch& t) {
+      const int i0 = (b % n_groups) * G;
+      int at[R];
 #pragma unroll
-    for (int j = 0; j < R; ++j) at[j] = min(row_of(b, j), last_row) * (D * (PB / 8)) + c8 * PB;
+      for (int j = 0; j < R; ++j) at[j] = min(row_of(b, j), last_row) * (D * (PB / 8)) + c8 * PB;
 #pragma unroll
-    for (int u = 0; u < G; ++u) {
-      const char* base = (const char*)o_part + part_row(min(i0 + u, n_parts - 1)) * (D * (PB / 8));
+      for (int u = 0; u < G; ++u) {
+        if (G == 2 && u == 1 && n_parts == 1) break;  // (nothing is fetched ahead of it that a wait could include)
+        const char* base = (const char*)o_part + part_row(min(i0 + u, n_parts - 1)) * (D * (PB / 8));
 #pragma unroll
-      for (int j = 0; j < R; ++j)
+        for (int j = 0; j < R; ++j)
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-          const f32x4* src = (const f32x4*)(base + at[j] + 16 * v);
-          t.raw[j][u][v] = HP ? __builtin_nontemporal_load(src) : *src;
-        }
-    }
-  };
-  float mx[R], wsum[R], acc[R][8];
-  auto accumulate = [&](int b, const Batch& t) {
-    const int g = b % n_groups, i0 = g * G;
-    if (g == 0) {  // new rows: L = max over the parts first
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        mx[j] = -INFINITY;
-        wsum[j] = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[j][e] = 0.f;
+          for (int v = 0; v < NV; ++v) {
+            const f32x4* src = (const f32x4*)(base + at[j] + 16 * v);
+            t.raw[j][u][v] = HP ? __builtin_nontemporal_load(src) : *src;
+          }
       }
-      for (int i = 0; i < n_parts; ++i)
-#pragma unroll
-        for (int j = 0; j < R; ++j) mx[j] = fmaxf(mx[j], lse_s[i * BM + row_of(b, j)]);
-    }
-#pragma unroll
-    for (int u = 0; u < G; ++u)
-      if (i0 + u < n_parts) {
+    };
+    float mx[R], wsum[R], acc[R][8];
+    auto accumulate = [&](int b, const Batch& t) {
+      const int g = b % n_groups, i0 = g * G;
+      if (g == 0) {  // new rows: L = max over the parts first
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-          const float L = lse_s[(i0 + u) * BM + row_of(b, j)];
-          if (row0 + row_of(b, j) >= seg.q_len || L == -INFINITY) continue;  // identity element: its O may hold anything
-          const float w = __expf(L - mx[j]);
-          wsum[j] += w;
-          float x[8];
-          if (HP) {
-            const f16x8 hv = __builtin_bit_cast(f16x8, t.raw[j][u][0]);
+          mx[j] = -INFINITY;
+          wsum[j] = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = (float)hv[e];
-          } else {
+          for (int e = 0; e < 8; ++e) acc[j][e] = 0.f;
+        }
+        for (int i = 0; i < n_parts; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              x[e] = t.raw[j][u][0][e];
-              x[4 + e] = t.raw[j][u][NV - 1][e];
+          for (int j = 0; j < R; ++j) mx[j] = fmaxf(mx[j], lse_s[i * BM + row_of(b, j)]);
+      }
+#pragma unroll
+      for (int u = 0; u < G; ++u)
+        if (i0 + u < n_parts) {
+#pragma unroll
+          for (int j = 0; j < R; ++j) {
+            const float L = lse_s[(i0 + u) * BM + row_of(b, j)];
+            if (row0 + row_of(b, j) >= seg.q_len || L == -INFINITY) continue;  // identity element: its O may hold anything
+            const float w = __expf(L - mx[j]);
+            wsum[j] += w;
+            float x[8];
+            if (HP) {
+              const f16x8 hv = __builtin_bit_cast(f16x8, t.raw[j][u][0]);
+#pragma unroll
+              for (int e = 0; e < 8; ++e) x[e] = (float)hv[e];
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                x[e] = t.raw[j][u][0][e];
+                x[4 + e] = t.raw[j][u][NV - 1][e];
+              }
             }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[j][e] = __builtin_fmaf(w, x[e], acc[j][e]);
           }
+        }
+      if (g == n_groups - 1) {  // all parts in: normalise and store
 #pragma unroll
-          for (int e = 0; e < 8; ++e) acc[j][e] = __builtin_fmaf(w, x[e], acc[j][e]);
+        for (int j = 0; j < R; ++j) {
+          if (row0 + row_of(b, j) >= seg.q_len) continue;
+          if (mx[j] != -INFINITY) {
+            const float inv = 1.f / wsum[j];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[j][e] *= inv;
+          }
+          const int64_t out_row = (int64_t)bh * S + seg.q_start + row0 + row_of(b, j);
+          Store8<DT>::st((char*)out + (out_row * D + c8 * 8) * 2, acc[j]);
+          if (c8 == 0) lse[out_row] = (mx[j] == -INFINITY) ? -INFINITY : mx[j] + __logf(wsum[j]);
         }
       }
-    if (g == n_groups - 1) {  // all parts in: normalise and store
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        if (row0 + row_of(b, j) >= seg.q_len) continue;
-        if (mx[j] != -INFINITY) {
-          const float inv = 1.f / wsum[j];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) acc[j][e] *= inv;
-        }
-        const int64_t out_row = (int64_t)bh * S + seg.q_start + row0 + row_of(b, j);
-        Store8<DT>::st((char*)out + (out_row * D + c8 * 8) * 2, acc[j]);
-        if (c8 == 0) lse[out_row] = (mx[j] == -INFINITY) ? -INFINITY : mx[j] + __logf(wsum[j]);
-      }
+    };
+    // three batches in flight
+    Batch t0, t1, t2;
+    fetch(0, t0);
+    if (1 < n_batches) fetch(1, t1);
+    int b = 0;
+#pragma unroll 1
+    for (; b + 4 < n_batches; b += 3) {
+      fetch(b + 2, t2);
+      accumulate(b, t0);
+      fetch(b + 3, t0);
+      accumulate(b + 1, t1);
+      fetch(b + 4, t1);
+      accumulate(b + 2, t2);
+    }
+#pragma unroll 1
+    for (; b < n_batches; b += 3) {
+      if (b + 2 < n_batches) fetch(b + 2, t2);
+      accumulate(b, t0);
+      if (b + 3 < n_batches) fetch(b + 3, t0);
+      if (b + 1 < n_batches) accumulate(b + 1, t1);
+      if (b + 4 < n_batches) fetch(b + 4, t1);
+      if (b + 2 < n_batches) accumulate(b + 2, t2);
     }
   };
-  // three batches in flight
-  Batch t0, t1, t2;
-  fetch(0, t0);
-  if (1 < n_batches) fetch(1, t1);
-  int b = 0;
-#pragma unroll 1
-  for (; b + 4 < n_batches; b += 3) {
-    fetch(b + 2, t2);
-    accumulate(b, t0);
-    fetch(b + 3, t0);
-    accumulate(b + 1, t1);
-    fetch(b + 4, t1);
-    accumulate(b + 2, t2);
-  }
-#pragma unroll 1
-  for (; b < n_batches; b += 3) {
-    if (b + 2 < n_batches) fetch(b + 2, t2);
-    accumulate(b, t0);
-    if (b + 3 < n_batches) fetch(b + 3, t0);
-    if (b + 1 < n_batches) accumulate(b + 1, t1);
-    if (b + 4 < n_batches) fetch(b + 4, t1);
-    if (b + 2 < n_batches) accumulate(b + 2, t2);
-  }
+  // 64 registers a batch.  Of a segment with one part or two most of such a batch would be loads of rows that are there
+  // already, so these take twice the rows of two parts instead.  Forward with the steps apart, d = 128, us, one shape of batch ->
+  // two: 256 heads x 256 tokens, one part 36.8 -> 31.0, with fp16 partials 39.9 -> 25.2 (34.7 and 30.7 with loads under
+  // conditions); 2 x 256 tokens 108 -> 95 and 99 -> 73; causal 128 heads x 5 x 256 201 -> 187 and 163 -> 143.
+  if (n_parts <= 2) merge_in(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
+  else merge_in(std::integral_constant<int, 2>{}, std::integral_constant<int, HP ? 8 : 4>{});
 }
 
 }  // namespace ringattn
