@@ -34,13 +34,12 @@ def reference(q, k, v, hidden, causal, scale):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kernel", KERNELS)
-@pytest.mark.parametrize("d,dtype", [(64, "fp16"), (64, "bf16"), (128, "fp16"), (128, "bf16")])
+@pytest.mark.parametrize("kernel,d", [(k, d) for k in KERNELS for d in (64, 128)
+                                      if d == 128 or k != "ring_walk64_kernel, partials"])   # (partials at d = 128 only)
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 @pytest.mark.parametrize("hidden,causal", [(40, False), (130, False), (40, True), (130, True)])
 def test_rows_without_a_reference_in_their_first_tile(monkeypatch, kernel, d, dtype, hidden, causal):
     env, lens, options = KERNELS[kernel]
-    if d == 64 and options:
-        pytest.skip("ring_walk64_kernel emits partials at d = 128 only")
     for name in ("RINGATTN_WIDE", "RINGATTN_WIDE_D64", "RINGATTN_WIDE_PARTIALS", "RINGATTN_SPLIT", "RINGATTN_PAIR"):
         monkeypatch.delenv(name, raising=False)
     for name, value in env.items():
@@ -71,4 +70,4 @@ def test_rows_without_a_reference_in_their_first_tile(monkeypatch, kernel, d, dt
     u = 2.0 ** -(11 if dtype == "fp16" else 8)
     bound = 0.5 * storage_ulp(o_ref, dtype) + u * mean_abs_v + 2.0 ** -25 * S * np.abs(exact[2]).max() + 1e-5
     assert (np.abs(out - o_ref)[~blind] <= bound[~blind]).all()
-    assert (np.abs(lse - l_ref)[~blind] <= 1e-4 * np.abs(l_ref)[~blind]).all()
+    assert (np.abs(lse[~blind] - l_ref[~blind]) <= 1e-4 * np.abs(l_ref[~blind])).all()

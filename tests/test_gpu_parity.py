@@ -33,10 +33,24 @@ def to_dev(bits, dtype):
     return api.bits_to_tensor(bits, dtype)
 
 
-def forward(w, q, k, v, **kw):
+# What keeps a forward that carries the state on one kernel, whatever its size ("": the library's own choice, for the small
+# shapes of these tests ring_split_kernel or ring_pair_kernel).
+FORCE = {"": {}, "ring_walk_kernel": {"RINGATTN_WIDE": "0"}, "ring_walk64_kernel": {"RINGATTN_SPLIT": "0", "RINGATTN_PAIR": "0"}}
+
+
+def force(monkeypatch, kernel):
+    for name in ("RINGATTN_WIDE", "RINGATTN_WIDE_D64", "RINGATTN_WIDE_PARTIALS", "RINGATTN_SPLIT", "RINGATTN_PAIR"):
+        monkeypatch.delenv(name, raising=False)
+    for name, value in FORCE[kernel].items():
+        monkeypatch.setenv(name, value)
+
+
+def forward(w, q, k, v, kernel="", **kw):
+    """kernel: the one that has to run it (force() says so to the library)."""
     plan = api.RingAttention(w.npes, w.chunk, w.dim, w.batch, w.heads, w.dtype, w.causal, graph=w.graph,
                              half_partials=w.half_partials, **kw)
     try:
+        assert kernel in ("", plan.forward_kernel())
         out, lse = plan.forward(to_dev(q, w.dtype), to_dev(k, w.dtype), to_dev(v, w.dtype))
         torch.cuda.synchronize()
         return out, lse
@@ -212,9 +226,11 @@ def test_workload_whole_heads(oracle, name, step_partials):
     Workload("huge_logits_64", 1, 2, 64, 3, 384, "bf16", 29, True, sigma_qk=6.0),
     Workload("huge_logits_64h", 2, 1, 64, 2, 640, "fp16", 30, False, sigma_qk=6.0),
 ], ids=lambda w: w.name)
-def test_shapes_and_edges_full(oracle, w):
+@pytest.mark.parametrize("kernel", FORCE)
+def test_shapes_and_edges_full(oracle, monkeypatch, w, kernel):
+    force(monkeypatch, kernel)
     q, k, v = api.make_qkv_bits(w)
-    out, lse = forward(w, q, k, v)
+    out, lse = forward(w, q, k, v, kernel)
     check_rows(oracle, w, q, k, v, out, lse, np.arange(w.rows))
 
 
@@ -269,9 +285,11 @@ def test_unequal_rank_lengths(oracle, seqlen, causal, d, dtype):
     ((1026, 514), True, 64, "fp16", "zigzag"),             # d = 64: K and V tiles loaded by different halves of the workgroup
     ((640, 384, 896), False, 64, "bf16", "contiguous"),    # whole key tiles, chunk lengths that are no multiples of four tiles
 ])
-def test_ragged_lengths(oracle, seqlen, causal, d, dtype, layout):
+@pytest.mark.parametrize("kernel", ["", "ring_walk_kernel"])
+def test_ragged_lengths(oracle, monkeypatch, seqlen, causal, d, dtype, layout, kernel):
     # lengths that are no multiples of the 256-row q tile or the 32-key tile: the tail
     # predication the reference leaves open (csrc/ring_attention.cu:143-145)
+    force(monkeypatch, kernel)
     P, S, B, H = len(seqlen), sum(seqlen), 2, 2
     w = Workload("ragged", B, H, d, 1, S, dtype, 95, causal)
     q, k, v = api.make_qkv_bits(w)
@@ -283,6 +301,7 @@ def test_ragged_lengths(oracle, seqlen, causal, d, dtype, layout):
     lse_buf = torch.full((B * H * S + 64,), 7.0, dtype=torch.float32, device="cuda")
     out, lse = out_buf[:B * H * S].view(B, H, S, d), lse_buf[:B * H * S].view(B, H, S)
     plan = api.RingAttention(P, list(seqlen), d, B, H, dtype, causal, layout=layout)
+    assert kernel in ("", plan.forward_kernel())
     plan.forward(qd, kd, vd, out, lse)
     torch.cuda.synchronize()
     assert bool((out_buf[B * H * S:] == 7.0).all()) and bool((lse_buf[B * H * S:] == 7.0).all())
@@ -334,7 +353,9 @@ def test_grouped_query_heads(oracle, causal):
     ((1024,), 1, 2, 128, "fp16", 0),                  # one rank: zigzag degenerates to the plain causal mask
     ((256,) * 8, 1, 4, 128, "bf16", 2),               # with grouped-query heads
 ])
-def test_zigzag_layout(oracle, seqlen, B, H, d, dtype, hkv):
+@pytest.mark.parametrize("kernel", FORCE)
+def test_zigzag_layout(oracle, monkeypatch, seqlen, B, H, d, dtype, hkv, kernel):
+    force(monkeypatch, kernel)
     # The sequence is generated in sequence order, stored in zigzag memory order, and the
     # result (brought back to sequence order) must equal causal attention over the sequence.
     P, S = len(seqlen), sum(seqlen)
@@ -346,6 +367,7 @@ def test_zigzag_layout(oracle, seqlen, B, H, d, dtype, hkv):
     inv = torch.from_numpy(np.argsort(order)).cuda()
     qd, kd, vd = (to_dev(np.ascontiguousarray(x[:, :, order]), dtype) for x in (q, k, v))
     plan = api.RingAttention(P, list(seqlen), d, B, H, dtype, True, kv_heads=hkv, layout="zigzag")
+    assert kernel in ("", plan.forward_kernel())
     out, lse = plan.forward(qd, kd, vd)
     torch.cuda.synchronize()
     out_seq, lse_seq = out[:, :, inv].contiguous(), lse[:, :, inv].contiguous()
@@ -610,7 +632,9 @@ def test_host_api_checks_on_device():
         api.RingAttention(2, 101, 64, causal=True, layout="zigzag")   # the zigzag layout needs even lengths
 
 
-def test_random_plans_against_oracle(oracle):
+@pytest.mark.parametrize("kernel", ["", "ring_walk_kernel"])
+def test_random_plans_against_oracle(oracle, monkeypatch, kernel):
+    force(monkeypatch, kernel)
     # seeded sweep over the whole parameter space at small sizes: ranks, ragged lengths, batch,
     # heads, grouped KV heads, head dim, dtype, mask, layout, explicit scale, graph replay
     rng = np.random.default_rng(2024)
@@ -640,6 +664,7 @@ def test_random_plans_against_oracle(oracle):
         plan = api.RingAttention(P, lens, d, B, H, dtype, causal, softmax_scale=scale, graph=graph,
                                  kv_heads=hkv if group > 1 else 0, layout="zigzag" if zigzag else "contiguous",
                                  step_partials=steps_apart)
+        assert kernel in ("", plan.forward_kernel()), tag
         out, lse = plan.forward(qd, kd, vd)
         if graph:                                   # a replay of the captured graph must give the same bits
             out2, lse2 = plan.forward(qd, kd, vd, torch.empty_like(out), torch.empty_like(lse))

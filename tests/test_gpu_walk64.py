@@ -13,7 +13,7 @@ import torch
 from np_reference import bits_to_float64, float32_to_bits
 from ringattention_amd import api
 from ringattention_amd.configs import Workload
-from test_gpu_parity import check_rows, forward
+from test_gpu_parity import check_rows, force, forward
 
 pytestmark = pytest.mark.gpu
 
@@ -45,9 +45,10 @@ def rising_logits(w, slope, period=0):
     (Workload("rise64_c", 1, 2, 64, 4, 1024, "bf16", 46, True), 0.2, 0),
     (Workload("saw64_nc", 2, 1, 64, 3, 768, "fp16", 47, False), 0.3, 300),
 ], ids=lambda x: x.name if isinstance(x, Workload) else None)
-def test_reference_moves_inside_the_hand_scheduled_loop(oracle, w, slope, period):
+def test_reference_moves_inside_the_hand_scheduled_loop(oracle, monkeypatch, w, slope, period):
+    force(monkeypatch, "ring_walk64_kernel")
     q, k, v = rising_logits(w, slope, period)
-    out, lse = forward(w, q, k, v)
+    out, lse = forward(w, q, k, v, "ring_walk64_kernel")
     assert torch.isfinite(out).all() and torch.isfinite(lse).all()
     check_rows(oracle, w, q, k, v, out, lse, np.arange(w.rows))
 
@@ -66,15 +67,14 @@ def test_reference_moves_inside_the_hand_scheduled_loop(oracle, w, slope, period
     Workload("w64_big", 1, 2, 64, 2, 1024, "fp16", 61, False, sigma_qk=3.0),
 ], ids=lambda w: w.name)
 def test_both_kernels_agree(oracle, w, monkeypatch):
-    """The same forward with and without RINGATTN_WIDE=0 (which keeps it on ring_walk_kernel): both against the oracle,
-    and against each other within two units in the last place of the row's largest element (the two kernels move
+    """The same forward on ring_walk64_kernel and on ring_walk_kernel: both against the oracle, and against each other within two units in the last place of the row's largest element (the two kernels move
     their reference maxima at different times, so the probabilities are rounded at different scales)."""
     q, k, v = api.make_qkv_bits(w)
-    monkeypatch.delenv("RINGATTN_WIDE", raising=False)
-    out_w, lse_w = forward(w, q, k, v)
+    force(monkeypatch, "ring_walk64_kernel")
+    out_w, lse_w = forward(w, q, k, v, "ring_walk64_kernel")
     check_rows(oracle, w, q, k, v, out_w, lse_w, np.arange(w.rows))
-    monkeypatch.setenv("RINGATTN_WIDE", "0")
-    out_b, lse_b = forward(w, q, k, v)
+    force(monkeypatch, "ring_walk_kernel")
+    out_b, lse_b = forward(w, q, k, v, "ring_walk_kernel")
     check_rows(oracle, w, q, k, v, out_b, lse_b, np.arange(w.rows))
     a, b = out_w.double().cpu().numpy().reshape(-1, w.dim), out_b.double().cpu().numpy().reshape(-1, w.dim)
     big = np.maximum(np.abs(a), np.abs(b)).max(axis=1, keepdims=True)
@@ -84,15 +84,17 @@ def test_both_kernels_agree(oracle, w, monkeypatch):
     assert np.abs(lse_w.double().cpu().numpy() - lse_b.double().cpu().numpy()).max() <= 1e-4
 
 
-def test_wide_kernel_with_grouped_heads_and_unequal_ranks(oracle):
+def test_wide_kernel_with_grouped_heads_and_unequal_ranks(oracle, monkeypatch):
     """Shapes the kernel takes beyond plain equal chunks: grouped-query heads and ranks of different lengths
-    (multiples of 32, at least 128).  (The zigzag layout at d = 128 is covered by test_gpu_parity.test_zigzag_layout.)"""
+    (multiples of 32, at least 128).  (The zigzag layout is covered by test_gpu_parity.test_zigzag_layout.)"""
+    force(monkeypatch, "ring_walk64_kernel")
     # grouped-query heads
     w = Workload("w_gqa", 1, 4, 128, 4, 512, "bf16", 61, True)
     q, k, v = api.make_qkv_bits(w)
     k, v = k[:, :2].copy(), v[:, :2].copy()
     plan = api.RingAttention(w.npes, w.chunk, w.dim, w.batch, w.heads, w.dtype, w.causal, kv_heads=2)
     try:
+        assert plan.forward_kernel() == "ring_walk64_kernel"
         out, lse = plan.forward(*(api.bits_to_tensor(x, w.dtype) for x in (q, k, v)))
         torch.cuda.synchronize()
     finally:
@@ -106,6 +108,7 @@ def test_wide_kernel_with_grouped_heads_and_unequal_ranks(oracle):
     q, k, v = api.make_qkv_bits(wu)
     plan = api.RingAttention(len(seqlen), list(seqlen), 128, 1, 2, "fp16", True)
     try:
+        assert plan.forward_kernel() == "ring_walk64_kernel"
         out, lse = plan.forward(*(api.bits_to_tensor(x, "fp16") for x in (q, k, v)))
         torch.cuda.synchronize()
     finally:

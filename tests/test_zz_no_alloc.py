@@ -1,6 +1,6 @@
-"""The reference-shaped entry point that allocates nothing (its table of ring steps lives in a
-static device scratch) against the allocating one, through the C ABI: same bits, on two calls
-in a row, the second on a smaller input (the scratch keeps the first call's contents)."""
+"""The reference-shaped entry point that neither allocates nor synchronises (its one launch carries its key range in its
+arguments, so it holds no device memory of its own) against the blocking one, through the C ABI: same bits, on calls in
+a row, under capture, and with several in flight."""
 import numpy as np
 import pytest
 import torch
@@ -31,7 +31,7 @@ def _run_pair(npes, seqlen, dim, dtype, causal, mype, seed):
 
 
 def test_noalloc_entry_matches_allocating_entry_twice_in_a_row():
-    # first a larger call, then a smaller one on the same (dirty) scratch
+    # first a larger call, then smaller ones: nothing of a call is left for the next
     _run_pair(4, [640, 512, 384, 512], 128, torch.bfloat16, True, 3, seed=101)
     _run_pair(3, [100, 130, 77], 64, torch.float16, False, 1, seed=102)
     _run_pair(2, [256, 256], 128, torch.float16, True, 0, seed=103)
@@ -55,7 +55,7 @@ def test_noalloc_entry_without_lse_and_on_a_side_stream():
 def test_noalloc_entry_limits():
     lib = _lib.load()
     assert lib.ringattn_noalloc_scratch_bytes() == 4096
-    # the scratch holds the table of ring steps: 32 bytes + 32 per visible step, so 64 ranks fit ...
+    # (the bound it has always had; nothing of it is used)  The longest ring ...
     _run_pair(64, [64] * 64, 64, torch.float16, False, 17, seed=104)
     _run_pair(8, [4096] * 8, 128, torch.bfloat16, True, 7, seed=105)      # ... whatever the lengths
     # ... and a longer ring is refused as everywhere else
@@ -68,8 +68,8 @@ def test_noalloc_entry_limits():
 
 
 def test_noalloc_entry_under_stream_capture_allocates_nothing():
-    """What the entry is for: a caller that records it into a graph.  After one warm call outside the capture (the
-    first call on a device looks up the scratch address), the call is captured on a side stream -- an allocation, a
+    """What the entry is for: a caller that records it into a graph.  After one warm call outside the capture (which loads the
+    kernel), the call is captured on a side stream -- an allocation, a
     host copy or a synchronisation inside it would fail the capture --, the graph is replayed twice with eager work
     in between, and every replay gives the bits of the allocating entry point."""
     seqlen, dim, mype, npes = [512, 384, 512], 128, 2, 3
@@ -98,7 +98,7 @@ def test_noalloc_entry_under_stream_capture_allocates_nothing():
 
 
 def test_noalloc_calls_in_flight_on_several_streams():
-    """Each call's table takes its own slice of the scratch, so a handful of calls may be in flight at once."""
+    """Calls share no memory of the library's, so any number of them may be in flight at once."""
     dim, npes = 128, 4
     seqlen = [1024] * npes
     gen = torch.Generator(device="cpu").manual_seed(12)
