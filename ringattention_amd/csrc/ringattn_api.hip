@@ -295,7 +295,7 @@ struct TableSlice {
 };
 
 // ring_walk64_kernel walks whole 32-key tiles, and past the end of its sequence its load streams go round the first
-// four tiles of a head: a KV range must be a multiple of 32 keys and hold at least 128.
+// four tiles of a head: a KV range must be a multiple of 32 keys, hold at least 128 and begin within 4 GiB.
 static bool walk64_takes(const ringattn::SegItem& it, int dim) {
   return it.kv_len % 32 == 0 && it.kv_len >= 128 && begins_within_4g(it, dim);
 }

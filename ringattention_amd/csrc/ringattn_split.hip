@@ -118,7 +118,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel
     }
   };
 
-  // ---- the tiles of this wave: numbers wave, wave + 8, ... of the items' tiles laid end to end
+  // ---- the tiles of this wave: numbers wave, wave + WAVES, ... of the items' tiles laid end to end
   struct Pos {
     int item, t;  // item, tile within it
     int start, len, diag;
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel
       }
   }
   __syncthreads();
-  // a thread owns eight columns of a row (at d = 64 half the threads have none)
+  // a thread owns eight columns of a row (at d = 64 half the threads have none, with sixteen waves three quarters)
   const int row = tid / (D / 8), c8 = tid % (D / 8);
   if (row >= BM || q0 + row > q_last) return;  // (or the row lies beyond the query range)
   float top = -INFINITY, l = 0.f;
