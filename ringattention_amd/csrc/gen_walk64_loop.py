@@ -465,6 +465,10 @@ def loop_text(mfma, cvt):
     lines = k_prereads(0)
     # a wave whose walk is one tile has no second score tile to compute
     lines += ["s_cmp_ge_i32 %s, %s" % (S_C, S_STOP), "s_cbranch_scc1 700f"]
+    # Where the trip begins within 64 bytes of code decides how its eight-byte instructions fall on the instruction fetch, and would
+    # be up to whatever the compiler puts in front of it.  Words past the boundary 0, 3, 8, 12: causal 32 heads x 32 K tokens,
+    # d = 128, 6568, 6507, 6568, 6526 us; 64 heads x 16 K 6945, 6902, 6944, 6926; d = 64 and ring_pair_kernel the same for all.
+    lines += [".p2align 6"] + ["s_nop 0"] * _knob('PAD', 3)
     lines.append("200:")
     for i in range(UNROLL):
         lines += iteration(i, mfma, cvt)
