@@ -1,4 +1,4 @@
-"""Steps and merges of a plan whose first use they are, or that only forwards without tables in memory have warmed up, in a
+"""Steps, merges and forwards of a plan whose first use they are, or that only forwards without tables in memory have warmed up, in a
 stream capture: the plan's device tables are made then and there, and every replay gives the eager bits."""
 import pytest
 import torch
@@ -20,10 +20,14 @@ def rank_steps_and_merge(plan, t, o, l, out, lse, rank=2):
     return plan.rank_merge(rank, o, l, out, lse)
 
 
+def whole_forward(plan, t, o, l, out, lse):
+    return plan.forward(t["q"], t["k"], t["v"], out, lse)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["contiguous", "zigzag"])
 @pytest.mark.parametrize("warm", [True, False])
-@pytest.mark.parametrize("work", [steps_and_merge, rank_steps_and_merge])
+@pytest.mark.parametrize("work", [steps_and_merge, rank_steps_and_merge, whole_forward])
 def test_capture_after_forwards_only(layout, warm, work):
     P, c, H, d = 4, 96, 2, 64
     S, rank = P * c, 2
@@ -32,10 +36,10 @@ def test_capture_after_forwards_only(layout, warm, work):
     for r in range(P):
         for name in "qkv":
             t["%s_%d" % (name, r)] = t[name][:, :, r * c:(r + 1) * c].contiguous()
-    rows = S if work is steps_and_merge else c
+    rows = c if work is rank_steps_and_merge else S
 
     def buffers(plan):
-        o_shape, l_shape = plan.parts_shapes() if work is steps_and_merge else plan.rank_parts_shapes(rank)
+        o_shape, l_shape = plan.rank_parts_shapes(rank) if work is rank_steps_and_merge else plan.parts_shapes()
         return (torch.zeros(o_shape, device="cuda"), torch.full(l_shape, float("-inf"), device="cuda"),
                 torch.empty(1, H, rows, d, dtype=torch.float16, device="cuda"), torch.empty(1, H, rows, device="cuda"))
 
