@@ -329,16 +329,14 @@ static int pair_choice() {
   return !e ? -1 : (e[0] == '0' ? 0 : 1);
 }
 
-// A launch that carries the state has its choice of three kernels, with 256, 128 and 32 query rows per workgroup (kWalkM, kPairM,
-// kSplitM) -- the first of them ring_walk64_kernel where the ranges suit it (walk64_takes) and ring_walk_kernel elsewhere, 5 to
-// 11 % slower --, a workgroup per compute unit (at d = 64 two of ring_split_kernel and of ring_walk_kernel): the fewer the rows, the shorter the walks (the waves that do not own rows of their own share out the
+// Three kernels carry the state, with 256, 128 and 32 query rows per workgroup (kWalkM, kPairM, kSplitM), a workgroup per
+// compute unit: the fewer the rows, the shorter the walks (the waves that do not own rows of their own share out the
 // keys) and the more of them, but the more often a K/V tile is fetched from L2.  A launch of few q tiles takes as long as
 // its longest walk, one of many as all of them over the compute units, at a lower clock.  Each kernel by three measured
 // numbers: us per step of a walk (one, two and eight key tiles) with most compute units idle and with all of them busy,
-// and us per workgroup besides (Q, first tiles, result).  They give the time of 150 launches of whole tiles -- heads 1 to 64,
-// sequences of 320 to 32768, with and without the causal mask -- to 2-4 % rms where they were measured, and of 188 launches, most
-// of them ragged, on a slower card to 3-6 % about a common factor; us on ring_walk64_kernel and the 128- and 32-row kernel
-// at d = 128, and at d = 64:
+// and us per workgroup besides (Q, first tiles, result).  They give the time of 150 launches -- heads 1 to 64, sequences of
+// 320 to 32768, with and without the causal mask -- to 2-4 % rms; us measured on the 256-, 128- and 32-row kernel at
+// d = 128, and at d = 64:
 //     1 head x 2048                         44, 28, 17        34, 22, 13
 //     8 heads x 2048                        43, 29, 33        34, 22, 19
 //     8 heads x 4096, causal                79, 50, 65        61, 38, 35
@@ -350,9 +348,6 @@ static int pair_choice() {
 // Without a mask all walks are equally long and go round after round, ring_split_kernel's too.  us on it, and on
 // ring_pair_kernel: 1 head x 16385 at d = 64, one workgroup more than two to a compute unit, 148, 130; 4 x 4400, 552
 // workgroups, 46.7, 39.9; 2 x 4097 at d = 128, two more than one to a compute unit, 51.4, 48.3.
-// Ragged lengths, us on ring_walk_kernel, the 128- and the 32-row kernel, d = 128: 16 heads x 6001 288, 262, 446 (causal 154, 149,
-// 257); 32 x 4400 335, 318, 511 (causal 173, 169, 301); 16 x 8191 464, 471, 809; 64 x 2047 127, 144, 268.  d = 64: 8 x 16400 causal
-// 352, 317, 406; 64 x 1000 causal 23.5, 22.0, 30.4; 8 x 4400 71.6, 80.4, 73.9; 64 x 4400 350, 377, 499.
 enum class CarryKernel { kWhole, kPair, kSplit, kSplit16 };
 struct KernelRate {
   int tiles_per_step;
@@ -362,7 +357,6 @@ struct KernelRate {
 };
 constexpr KernelRate kRates128[3] = {{1, 0.55, 0.79, 5.3, 1, 0}, {2, 0.60, 0.84, 6.0, 1, 0}, {8, 1.15, 1.35, 4.9, 1, 0}};
 constexpr KernelRate kRates64[3] = {{1, 0.42, 0.49, 3.2, 1, 0}, {2, 0.46, 0.53, 4.0, 1, 0}, {8, 0.96, 0.71, 1.9, 2, 1.42}};
-constexpr KernelRate kWalkRate128 = {1, 0.57, 0.85, 8.0, 1, 0}, kWalkRate64 = {1, 0.46, 0.515, 5.5, 2, 0.90};
 
 static double carry_time(const WalkCost& w, const KernelRate& r, bool equal_walks) {
   const double longest = (double)w.tiles / r.tiles_per_step;
@@ -378,16 +372,14 @@ static double carry_time(const WalkCost& w, const KernelRate& r, bool equal_walk
   return std::sqrt(std::sqrt(x * x * x * x + y * y * y * y));
 }
 
-// `wide`: the 256-row kernel of this launch is ring_walk64_kernel
-static CarryKernel carry_kernel(const CarryCosts& c, int dim, bool wide) {
+static CarryKernel carry_kernel(const CarryCosts& c, int dim) {
   if (!walk64_enabled() || (dim == 64 && !walk64_d64_enabled()) || walk64_partials_choice() == 1) return CarryKernel::kWhole;
   if (c.pair && pair_choice() == 1) return CarryKernel::kPair;
   const int split = split_choice();
   if (split == 8 || split == 16) return split == 16 && dim == 64 ? CarryKernel::kSplit16 : CarryKernel::kSplit;
   const KernelRate* r = dim == 128 ? kRates128 : kRates64;
-  const KernelRate& whole = wide ? r[0] : dim == 128 ? kWalkRate128 : kWalkRate64;
   // the 256-row kernels unless another is ahead by more than these times are good for
-  double best = carry_time(c.whole, whole, !c.masked) * 0.95;
+  double best = carry_time(c.whole, r[0], !c.masked) * 0.95;
   CarryKernel kernel = CarryKernel::kWhole;
   if (c.pair && pair_choice() != 0) {
     const double t = carry_time(c.halves, r[1], !c.masked);
@@ -703,10 +695,9 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
     a.items = pl->d_segitems;
   }
   a.n_segs = sl.seg_count;
-  const bool wide = slice_takes_walk64(pl, sl, a.mode);
   const CarryKernel kernel =
-      a.mode == ringattn::kBlockCarryState ? carry_kernel(sl.costs, pl->p.dim, wide) : CarryKernel::kWhole;
-  RA_HIP(launch_q_tiles(a, kernel, wide, sl.q_len_max, pl->p.dtype, pl->p.dim, stream));
+      a.mode == ringattn::kBlockCarryState ? carry_kernel(sl.costs, pl->p.dim) : CarryKernel::kWhole;
+  RA_HIP(launch_q_tiles(a, kernel, slice_takes_walk64(pl, sl, a.mode), sl.q_len_max, pl->p.dtype, pl->p.dim, stream));
   return RINGATTN_OK;
 }
 
@@ -812,7 +803,7 @@ int run_rank_call(const RankCall& rc, const void* q, const void* k, const void* 
   const bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled() && walk64_takes(rc.item, dim);
   CarryCosts costs;
   costs.add(rc.seg, 1, dim, [&](int) -> const ringattn::SegItem& { return rc.item; });
-  RA_HIP(launch_q_tiles(a, carry_kernel(costs, dim, wide), wide, c, rc.p.dtype, dim, stream));
+  RA_HIP(launch_q_tiles(a, carry_kernel(costs, dim), wide, c, rc.p.dtype, dim, stream));
   return RINGATTN_OK;
 }
 
@@ -1061,12 +1052,11 @@ int ringattn_plan_launch_times(ringattn_plan* plan, float* ms, int capacity, int
 const char* ringattn_plan_forward_kernel(const ringattn_plan* plan) {
   if (!plan_ok(plan)) return nullptr;
   const int mode = step_partials(plan->p) ? ringattn::kBlockPartialsMerged : ringattn::kBlockCarryState;
-  const bool wide = slice_takes_walk64(plan, forward_slice(plan), mode);
   if (mode == ringattn::kBlockCarryState) {
-    const CarryKernel kernel = carry_kernel(plan->walk.costs, plan->p.dim, wide);
+    const CarryKernel kernel = carry_kernel(plan->walk.costs, plan->p.dim);
     if (kernel != CarryKernel::kWhole) return kernel == CarryKernel::kPair ? "ring_pair_kernel" : "ring_split_kernel";
   }
-  return wide ? "ring_walk64_kernel" : "ring_walk_kernel";
+  return slice_takes_walk64(plan, forward_slice(plan), mode) ? "ring_walk64_kernel" : "ring_walk_kernel";
 }
 
 int ringattn_plan_merge_regions(const ringattn_plan* plan, int* start, int* len, uint64_t* active, int capacity, int* n_out) {

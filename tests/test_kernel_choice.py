@@ -62,21 +62,3 @@ def test_switches_that_name_a_256_row_kernel(monkeypatch, lens, heads, causal):
 def test_a_round_of_few_workgroups_counts_as_one(monkeypatch, d, heads, tokens, kernel):
     """Where a launch has a few workgroups of ring_split_kernel more than the chip holds at once, the faster kernel as measured."""
     assert chosen(monkeypatch, (tokens,), d, heads) == kernel
-
-
-@pytest.mark.parametrize("d,heads,tokens,causal,kernel", [
-    (128, 16, 6001, False, "ring_pair_kernel"),    # us on ring_walk_kernel and ring_pair_kernel: 288, 262
-    (128, 16, 6001, True, "ring_pair_kernel"),     # 154, 149
-    (128, 32, 4400, False, "ring_pair_kernel"),    # 335, 318
-    (128, 16, 8191, False, "ring_walk_kernel"),    # 464, 471
-    (128, 64, 2047, False, "ring_walk_kernel"),    # 127, 144
-    (64, 8, 16400, True, "ring_pair_kernel"),      # 352, 317
-    (64, 64, 1000, True, "ring_pair_kernel"),      # 23.5, 22.0
-    (64, 8, 4400, False, "ring_walk_kernel"),      # 71.6, 80.4 (and 73.9 on ring_split_kernel)
-    (64, 64, 4400, False, "ring_walk_kernel"),     # 350, 377
-    (64, 16, 6001, False, "ring_pair_kernel"),     # 181, 169
-])
-def test_ragged_lengths_go_by_the_times_of_the_kernel_that_takes_them(monkeypatch, d, heads, tokens, causal, kernel):
-    """ring_walk64_kernel does not take a length that is no multiple of 32: the other kernels are weighed against
-    ring_walk_kernel there, and the faster one as measured is chosen."""
-    assert chosen(monkeypatch, (tokens,), d, heads, causal) == kernel
