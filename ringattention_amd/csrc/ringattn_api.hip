@@ -345,26 +345,20 @@ static int pair_choice() {
 //     8 heads x 8192                       211, 230, 389     131, 145, 198
 //     9 heads x 8192 (288 q tiles of 256)  355, 310, 437     244, 208, 223
 //     16 heads x 8192, causal              221, 245, 424     142, 159, 209
-// Without a mask all walks are equally long and go round after round, ring_split_kernel's too.  us on it, and on
-// ring_pair_kernel: 1 head x 16385 at d = 64, one workgroup more than two to a compute unit, 148, 130; 4 x 4400, 552
-// workgroups, 46.7, 39.9; 2 x 4097 at d = 128, two more than one to a compute unit, 51.4, 48.3.
 enum class CarryKernel { kWhole, kPair, kSplit, kSplit16 };
 struct KernelRate {
   int tiles_per_step;
   double lone, busy, job;
-  int per_cu;     // workgroups that a compute unit holds at once
-  double shared;  // per_cu == 2: us per step of walks that have a compute unit to two, with others idle
 };
-constexpr KernelRate kRates128[3] = {{1, 0.55, 0.79, 5.3, 1, 0}, {2, 0.60, 0.84, 6.0, 1, 0}, {8, 1.15, 1.35, 4.9, 1, 0}};
-constexpr KernelRate kRates64[3] = {{1, 0.42, 0.49, 3.2, 1, 0}, {2, 0.46, 0.53, 4.0, 1, 0}, {8, 0.96, 0.71, 1.9, 2, 1.42}};
+constexpr KernelRate kRates128[3] = {{1, 0.55, 0.79, 5.3}, {2, 0.60, 0.84, 6.0}, {8, 1.15, 1.35, 4.9}};
+constexpr KernelRate kRates64[3] = {{1, 0.42, 0.49, 3.2}, {2, 0.46, 0.53, 4.0}, {8, 0.96, 0.71, 1.9}};
 
 static double carry_time(const WalkCost& w, const KernelRate& r, bool equal_walks) {
   const double longest = (double)w.tiles / r.tiles_per_step;
   if (equal_walks) {  // round after round, the last one on what compute units it needs
-    const int64_t at_once = kComputeUnits * r.per_cu, rounds = w.jobs / at_once, rest = w.jobs % at_once;
-    const double t = (double)(rounds * r.per_cu) * (r.busy * longest + r.job);
-    const double slowest = rest > kComputeUnits ? r.shared : r.lone;
-    return rest == 0 ? t : t + r.job + longest * std::max(slowest, r.busy * (double)rest / kComputeUnits);
+    const int64_t rounds = w.jobs / kComputeUnits, rest = w.jobs % kComputeUnits;
+    const double t = (double)rounds * (r.busy * longest + r.job);
+    return rest == 0 ? t : t + r.job + longest * std::max(r.lone, r.busy * (double)rest / kComputeUnits);
   }
   // the longest walk and the even share of all of them; where these are alike, what is left at the end adds to both
   const double x = r.lone * longest + r.job;
@@ -385,7 +379,7 @@ static CarryKernel carry_kernel(const CarryCosts& c, int dim) {
     const double t = carry_time(c.halves, r[1], !c.masked);
     if (t < best) best = t, kernel = CarryKernel::kPair;
   }
-  if (split != 0 && carry_time(c.thin, r[2], !c.masked) < best) kernel = CarryKernel::kSplit;
+  if (split != 0 && carry_time(c.thin, r[2], false) < best) kernel = CarryKernel::kSplit;
   // At d = 64 two workgroups of ring_split_kernel fit on a compute unit.  A launch of no more workgroups than there are
   // compute units fills the other half with waves of the same workgroup, sixteen of them instead of eight, where the walk
   // is long enough to pay for the combination of twice the states.  us with eight and with sixteen waves, at 64, 128, 256

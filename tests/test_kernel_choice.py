@@ -48,17 +48,3 @@ def test_switches_that_name_a_256_row_kernel(monkeypatch, lens, heads, causal):
         assert chosen(monkeypatch, lens, d, heads, causal, env={"RINGATTN_WIDE": "0"}) == "ring_walk_kernel"
     assert chosen(monkeypatch, lens, 64, heads, causal, env={"RINGATTN_WIDE_D64": "0"}) == "ring_walk_kernel"
     assert chosen(monkeypatch, lens, 128, heads, causal, env={"RINGATTN_WIDE_D64": "0"}) == chosen(monkeypatch, lens, 128, heads, causal)
-
-
-@pytest.mark.parametrize("d,heads,tokens,kernel", [
-    (64, 1, 16385, "ring_pair_kernel"),    # us on ring_pair_kernel and ring_split_kernel: 130, 148
-    (64, 4, 4400, "ring_pair_kernel"),     # 39.9, 46.7
-    (64, 4, 16400, "ring_pair_kernel"),    # 413, 435
-    (128, 2, 4097, "ring_pair_kernel"),    # 48.3, 51.4
-    (64, 2, 4097, "ring_split_kernel"),    # 37.6, 26.7
-    (64, 8, 2047, "ring_split_kernel"),    # 21.9, 19.6
-    (128, 4, 2047, "ring_split_kernel"),   # 28.7, 19.4
-])
-def test_a_round_of_few_workgroups_counts_as_one(monkeypatch, d, heads, tokens, kernel):
-    """Where a launch has a few workgroups of ring_split_kernel more than the chip holds at once, the faster kernel as measured."""
-    assert chosen(monkeypatch, (tokens,), d, heads) == kernel
