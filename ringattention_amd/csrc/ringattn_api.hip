@@ -329,14 +329,15 @@ static int pair_choice() {
   return !e ? -1 : (e[0] == '0' ? 0 : 1);
 }
 
-// Three kernels carry the state, with 256, 128 and 32 query rows per workgroup (kWalkM, kPairM, kSplitM), a workgroup per
-// compute unit: the fewer the rows, the shorter the walks (the waves that do not own rows of their own share out the
+// A launch that carries the state has its choice of three kernels, with 256, 128 and 32 query rows per workgroup (kWalkM, kPairM,
+// kSplitM) -- the first of them ring_walk64_kernel where the ranges suit it (walk64_takes) and ring_walk_kernel elsewhere, 5 to
+// 11 % slower --, a workgroup per compute unit (at d = 64 two of ring_split_kernel and of ring_walk_kernel): the fewer the rows, the shorter the walks (the waves that do not own rows of their own share out the
 // keys) and the more of them, but the more often a K/V tile is fetched from L2.  A launch of few q tiles takes as long as
 // its longest walk, one of many as all of them over the compute units, at a lower clock.  Each kernel by three measured
 // numbers: us per step of a walk (one, two and eight key tiles) with most compute units idle and with all of them busy,
-// and us per workgroup besides (Q, first tiles, result).  They give the time of 150 launches -- heads 1 to 64, sequences of
-// 320 to 32768, with and without the causal mask -- to 2-4 % rms; us measured on the 256-, 128- and 32-row kernel at
-// d = 128, and at d = 64:
+// and us per workgroup besides (Q, first tiles, result).  They give the time of 150 launches of whole tiles -- heads 1 to 64,
+// sequences of 320 to 32768, with and without the causal mask, logits N(0, 1) -- to 2-4 % rms; us measured on ring_walk64_kernel
+// and the 128- and 32-row kernel at d = 128, and at d = 64:
 //     1 head x 2048                         44, 28, 17        34, 22, 13
 //     8 heads x 2048                        43, 29, 33        34, 22, 19
 //     8 heads x 4096, causal                79, 50, 65        61, 38, 35
@@ -349,16 +350,26 @@ enum class CarryKernel { kWhole, kPair, kSplit, kSplit16 };
 struct KernelRate {
   int tiles_per_step;
   double lone, busy, job;
+  int per_cu = 1;      // workgroups that a compute unit holds at once
+  double shared = 0;   // per_cu == 2: us per step of walks that have a compute unit to two, with others idle
 };
 constexpr KernelRate kRates128[3] = {{1, 0.55, 0.79, 5.3}, {2, 0.60, 0.84, 6.0}, {8, 1.15, 1.35, 4.9}};
 constexpr KernelRate kRates64[3] = {{1, 0.42, 0.49, 3.2}, {2, 0.46, 0.53, 4.0}, {8, 0.96, 0.71, 1.9}};
+// ring_walk_kernel on ragged lengths (4 % rms over 180 launches).  Its two waves per SIMD cover for each other when references move;
+// the one wave of ring_pair_kernel waits for itself.  With logits N(0, 81) a launch takes 8 to 15 % longer there, and 30 to 50 % on
+// ring_pair_kernel, which has to be ahead by 12 % on flat ones to be taken: at d = 64, where two workgroups of ring_walk_kernel
+// share a compute unit, it led by 1 to 9 % and fell back by 9 to 36 %.  us on ring_walk_kernel and ring_pair_kernel, logits N(0, 1)
+// and N(0, 81), d = 64: 24 heads x 3000 91, 90 and 103, 140; 16 x 6001 185, 174 and 204, 247; 12 x 6000 175, 165 and 193, 233; 8 x
+// 12001 363, 332 and 389, 423.  Still taken: d = 128 causal, 16 x 4400 123, 95 and 120, 129; d = 64, 9 x 8191 239, 220 and 257, 296.
+constexpr KernelRate kWalkRate128 = {1, 0.57, 0.85, 8.0}, kWalkRate64 = {1, 0.46, 0.515, 5.5, 2, 0.90};
 
 static double carry_time(const WalkCost& w, const KernelRate& r, bool equal_walks) {
   const double longest = (double)w.tiles / r.tiles_per_step;
   if (equal_walks) {  // round after round, the last one on what compute units it needs
-    const int64_t rounds = w.jobs / kComputeUnits, rest = w.jobs % kComputeUnits;
-    const double t = (double)rounds * (r.busy * longest + r.job);
-    return rest == 0 ? t : t + r.job + longest * std::max(r.lone, r.busy * (double)rest / kComputeUnits);
+    const int64_t at_once = kComputeUnits * r.per_cu, rounds = w.jobs / at_once, rest = w.jobs % at_once;
+    const double t = (double)(rounds * r.per_cu) * (r.busy * longest + r.job);
+    const double slowest = rest > kComputeUnits ? r.shared : r.lone;
+    return rest == 0 ? t : t + r.job + longest * std::max(slowest, r.busy * (double)rest / kComputeUnits);
   }
   // the longest walk and the even share of all of them; where these are alike, what is left at the end adds to both
   const double x = r.lone * longest + r.job;
@@ -366,7 +377,8 @@ static double carry_time(const WalkCost& w, const KernelRate& r, bool equal_walk
   return std::sqrt(std::sqrt(x * x * x * x + y * y * y * y));
 }
 
-static CarryKernel carry_kernel(const CarryCosts& c, int dim) {
+// `wide`: the 256-row kernel of this launch is ring_walk64_kernel
+static CarryKernel carry_kernel(const CarryCosts& c, int dim, bool wide) {
   if (!walk64_enabled() || (dim == 64 && !walk64_d64_enabled()) || walk64_partials_choice() == 1) return CarryKernel::kWhole;
   if (c.pair && pair_choice() == 1) return CarryKernel::kPair;
   const int split = split_choice();
@@ -374,6 +386,7 @@ static CarryKernel carry_kernel(const CarryCosts& c, int dim) {
   const KernelRate* r = dim == 128 ? kRates128 : kRates64;
   // the 256-row kernels unless another is ahead by more than these times are good for
   double best = carry_time(c.whole, r[0], !c.masked) * 0.95;
+  if (!wide) best = std::min(best, carry_time(c.whole, dim == 128 ? kWalkRate128 : kWalkRate64, !c.masked) * 0.88);
   CarryKernel kernel = CarryKernel::kWhole;
   if (c.pair && pair_choice() != 0) {
     const double t = carry_time(c.halves, r[1], !c.masked);
@@ -689,9 +702,10 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
     a.items = pl->d_segitems;
   }
   a.n_segs = sl.seg_count;
+  const bool wide = slice_takes_walk64(pl, sl, a.mode);
   const CarryKernel kernel =
-      a.mode == ringattn::kBlockCarryState ? carry_kernel(sl.costs, pl->p.dim) : CarryKernel::kWhole;
-  RA_HIP(launch_q_tiles(a, kernel, slice_takes_walk64(pl, sl, a.mode), sl.q_len_max, pl->p.dtype, pl->p.dim, stream));
+      a.mode == ringattn::kBlockCarryState ? carry_kernel(sl.costs, pl->p.dim, wide) : CarryKernel::kWhole;
+  RA_HIP(launch_q_tiles(a, kernel, wide, sl.q_len_max, pl->p.dtype, pl->p.dim, stream));
   return RINGATTN_OK;
 }
 
@@ -797,7 +811,7 @@ int run_rank_call(const RankCall& rc, const void* q, const void* k, const void* 
   const bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled() && walk64_takes(rc.item, dim);
   CarryCosts costs;
   costs.add(rc.seg, 1, dim, [&](int) -> const ringattn::SegItem& { return rc.item; });
-  RA_HIP(launch_q_tiles(a, carry_kernel(costs, dim), wide, c, rc.p.dtype, dim, stream));
+  RA_HIP(launch_q_tiles(a, carry_kernel(costs, dim, wide), wide, c, rc.p.dtype, dim, stream));
   return RINGATTN_OK;
 }
 
@@ -1046,11 +1060,12 @@ int ringattn_plan_launch_times(ringattn_plan* plan, float* ms, int capacity, int
 const char* ringattn_plan_forward_kernel(const ringattn_plan* plan) {
   if (!plan_ok(plan)) return nullptr;
   const int mode = step_partials(plan->p) ? ringattn::kBlockPartialsMerged : ringattn::kBlockCarryState;
+  const bool wide = slice_takes_walk64(plan, forward_slice(plan), mode);
   if (mode == ringattn::kBlockCarryState) {
-    const CarryKernel kernel = carry_kernel(plan->walk.costs, plan->p.dim);
+    const CarryKernel kernel = carry_kernel(plan->walk.costs, plan->p.dim, wide);
     if (kernel != CarryKernel::kWhole) return kernel == CarryKernel::kPair ? "ring_pair_kernel" : "ring_split_kernel";
   }
-  return slice_takes_walk64(plan, forward_slice(plan), mode) ? "ring_walk64_kernel" : "ring_walk_kernel";
+  return wide ? "ring_walk64_kernel" : "ring_walk_kernel";
 }
 
 int ringattn_plan_merge_regions(const ringattn_plan* plan, int* start, int* len, uint64_t* active, int capacity, int* n_out) {

@@ -1,7 +1,6 @@
 """The merge at the end of a workgroup of ring_walk_kernel (merge_job_rows in ringattn_device.h) where its batches can go
 wrong: one part and two, which go in batches of their own, fewer than a batch of four (fp32) or eight (fp16), one more, one
-less, up to the 64 a plan may have; a q tile
-that ends after one row, in the middle of a batch or exactly; rows that see only some of the parts.  The forward with the
+less, up to the 64 a plan may have; a q tile that ends after one row, in the middle of a batch or exactly; rows that see only some of the parts.  The forward with the
 steps apart is documented to give the bits of ringattn_block_fwd per step and ringattn_merge_ring, whose merge kernel is
 other code: the bound is equality."""
 import numpy as np

@@ -48,3 +48,20 @@ def test_switches_that_name_a_256_row_kernel(monkeypatch, lens, heads, causal):
         assert chosen(monkeypatch, lens, d, heads, causal, env={"RINGATTN_WIDE": "0"}) == "ring_walk_kernel"
     assert chosen(monkeypatch, lens, 64, heads, causal, env={"RINGATTN_WIDE_D64": "0"}) == "ring_walk_kernel"
     assert chosen(monkeypatch, lens, 128, heads, causal, env={"RINGATTN_WIDE_D64": "0"}) == chosen(monkeypatch, lens, 128, heads, causal)
+
+
+@pytest.mark.parametrize("d,heads,tokens,causal,kernel", [
+    # us on ring_walk_kernel and ring_pair_kernel, logits N(0, 1); the same with logits N(0, 81)
+    (64, 24, 3000, False, "ring_walk_kernel"),    # 91, 90; 103, 140
+    (64, 16, 6001, False, "ring_walk_kernel"),    # 185, 174; 204, 247
+    (64, 12, 6000, False, "ring_walk_kernel"),    # 175, 165; 193, 233
+    (64, 16, 4400, True, "ring_pair_kernel"),     # 78, 62; 87, 89
+    (64, 4, 8191, False, "ring_pair_kernel"),     # 129, 82; 146, 111
+    (128, 16, 4400, True, "ring_pair_kernel"),    # 123, 95; 120, 129
+    (128, 8, 8191, True, "ring_pair_kernel"),     # 180, 134; 204, 187
+    (128, 32, 4400, False, "ring_walk_kernel"),   # 337, 322; 380, 439
+])
+def test_ragged_lengths_leave_ring_walk_kernel_for_a_clear_lead_only(monkeypatch, d, heads, tokens, causal, kernel):
+    """Where the 256-row kernel is ring_walk_kernel (no multiple of 32), a small lead of ring_pair_kernel on flat logits is lost,
+    and more, on peaked ones."""
+    assert chosen(monkeypatch, (tokens,), d, heads, causal) == kernel
