@@ -17,6 +17,8 @@
 //       0.79 and 0.49 per tile of 256 rows.  us a pass, that kernel (or ring_split_kernel) before and this one after: d = 128,
 //       causal, 8 heads x 4096 65 -> 50, 8 heads x 8192 161 -> 124; no mask, 4 heads x 8192 151 -> 117, 9 heads x 8192 355 -> 310;
 //       16 heads x 4400, causal (not a multiple of 32: ring_walk_kernel) 100 -> 88.  carry_kernel in ringattn_api.hip chooses.
+//       Moves of the references (peaked logits) have no second wave to hide behind: that launch takes 129 us with N(0, 81) logits,
+//       ring_walk_kernel 120.
 //       Shapes it takes: every key range at least 128 keys, every one but the last walked a multiple of 32 keys, and none that
 //       begins beyond 4 GiB of its head.
 #include "ringattn_device.h"
