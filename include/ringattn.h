@@ -56,8 +56,8 @@ extern "C" {
                                       relative error per partial (fp32 partials add none); the partial LSE stays fp32.
                                       Applies wherever partials are written (ringattn_block_fwd, ringattn_rank_step_fwd,
                                       ringattn_fwd with RINGATTN_FLAG_STEP_PARTIALS) */
-#define RINGATTN_FLAG_STEP_PARTIALS 8 /* ringattn_fwd keeps the ring steps apart: a normalised partial (O, LSE) per step in
-                                      the workspace, merged at the end -- the arithmetic of ringattn_block_fwd +
+#define RINGATTN_FLAG_STEP_PARTIALS 8 /* ringattn_fwd keeps the ring steps apart: a normalised partial (O, LSE) per step, merged
+                                      on the chip or by way of the workspace -- the arithmetic of ringattn_block_fwd +
                                       ringattn_merge_ring, bit for bit, in one launch.  Without the flag (the default)
                                       the softmax state (max, sum, acc-O) runs through all steps in registers, as in the
                                       reference's kernel (csrc/ring_attention.cu:439-443,597), and no workspace is needed */
@@ -135,8 +135,8 @@ int ringattn_plan_destroy(ringattn_plan* plan);
  * (csrc/ring_attention.cu:706-722) run on every PE.  ONE block-attention launch: a workgroup
  * owns 256, 128 or 32 query rows and walks the keys of every ring step of those rows with the running max, sum and
  * acc-O in registers, like the reference's CTA (:439-443,456,597), then writes O = acc / sum
- * (:621-664) and the LSE.  (With RINGATTN_FLAG_STEP_PARTIALS: a partial (O, LSE) per step into
- * the workspace, merged at the end of the workgroup.)
+ * (:621-664) and the LSE.  (With RINGATTN_FLAG_STEP_PARTIALS: a partial (O, LSE) per step,
+ * merged where it arises or, by way of the workspace, at the end of the workgroup.)
  *   q, k, v : [batch, heads, S, dim] dtype     out : same shape and dtype
  *   lse     : [batch, heads, S] fp32, natural log (the reference never writes it)
  * Asynchronous on `stream` (a hipStream_t, or NULL for the default stream); the
@@ -171,7 +171,7 @@ int ringattn_merge(const float* o_parts, const float* lse_parts, int n_parts, in
 /*
  * The merge as ringattn_fwd runs it, on caller-held partials: o_parts
  * [npes, batch*heads*S, dim] and lse_parts [npes, batch*heads*S] as written by
- * ringattn_block_fwd for steps 0..npes-1.  With a causal plan, part s of a row is read
+ * ringattn_block_fwd for steps 0..npes-1, merged in this order, with a causal plan step 0 last.  With a causal plan, part s of a row is read
  * only if ringattn_block_fwd writes that row in step s (contiguous layout: s == 0 or
  * r + s >= npes for a row of rank r), so parts the step loop never wrote are never touched.  Like ringattn_merge, it has no counterpart
  * function in the reference (csrc/ring_attention.cu:207-245,621-633 pin the algebra).

@@ -12,7 +12,7 @@ LIB_PATH = os.environ.get("RINGATTN_LIB") or os.path.join(PKG_DIR, "libringattn.
 
 TORCH_LIB_PATH = os.path.join(PKG_DIR, "libringattn_torch.so")
 
-SOURCES = ["ringattn_kernels.hip", "ringattn_walk.hip", "ringattn_walk64.hip", "ringattn_pair.hip", "ringattn_split.hip", "ringattn_api.hip", "ringattn_datagen.cpp"]
+SOURCES = ["ringattn_kernels.hip", "ringattn_walk.hip", "ringattn_steps.hip", "ringattn_walk64.hip", "ringattn_pair.hip", "ringattn_split.hip", "ringattn_api.hip", "ringattn_datagen.cpp"]
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_*_f32 out of scalar float code.
 HIPCC_FLAGS = [
@@ -55,6 +55,7 @@ def source_id(paths):
 
 def library_sources():
     return [os.path.join(CSRC, s) for s in SOURCES] + [os.path.join(CSRC, "ringattn_kernels.h"), os.path.join(CSRC, "ringattn_device.h"),
+                                                       os.path.join(CSRC, "ringattn_walk_rows.h"),
                                                        os.path.join(CSRC, "ringattn_walk64_loop.inc"),
                                                        os.path.join(CSRC, "ringattn_walk64_loop_d64.inc"),
                                                        os.path.join(CSRC, "ringattn_pair_loop.inc"),

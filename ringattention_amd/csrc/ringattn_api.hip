@@ -831,6 +831,7 @@ int launch_regions(const ringattn_plan* pl, int first, int count, int max_len, i
   m.S = rows_per_head;
   m.part_stride_rows = part_stride_rows;
   m.half_partials = half_partials(pl->p) ? 1 : 0;
+  m.slot0_last = pl->p.causal ? 1 : 0;
   m.row_mul = row_partials(pl->p) ? pl->p.npes : 0;
   RA_HIP(ringattn::launch_merge(m, pl->p.dtype, pl->p.dim, stream));
   return RINGATTN_OK;

@@ -257,182 +257,38 @@ static __device__ __forceinline__ void store_block(const f32x16 (&acc)[D / 32], 
     }
 }
 
-// ---- merge of one job's rows (BM rows of a segment, one head) over the partials of the
-// segment's items.  The same arithmetic, in the same order, as merge_row; only the loads are
-// arranged differently: the attention kernel, which runs this at the end of a workgroup, has just two
-// waves per SIMD to hide memory latency with, and every round trip it waits for is time its
-// compute unit runs half empty.  So all partial LSEs are fetched in one sweep and parked in LDS
-// (lse_s: [items][BM] floats), and the partial O rows move in batches of 256 bytes per thread
-// (two output rows x four or eight parts), three batches in flight at any time.
-typedef __attribute__((address_space(3))) float lds_float;
-template <int DT, int D, bool HP, int BM, int THREADS>
-static __device__ __forceinline__ void merge_job_rows(const void* o_part, const float* lse_part, void* out, float* lse,
-                                                      const SegItem* items, const Segment& seg, int bh, int qt, int S,
-                                                      lds_float* lse_s) {
-  constexpr int WAVES = THREADS / 64;
-  constexpr int TPR = D / 8;  // threads per row, 8 columns each
-  constexpr int ROWS = THREADS / TPR;
-  constexpr int KMAX = kMaxParts / WAVES;  // parts per wave in the LSE sweep
-  constexpr int LR = BM / 64;              // rows per lane in the LSE sweep
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n_parts = seg.item_count;
-  const int row0 = qt * BM;  // first row of the job within the segment
-  const int last_row = min(BM, seg.q_len - row0) - 1;
-  // lane i keeps where the job's rows begin in the partials of item i
-  int64_t first_row = 0;
-  if (lane < n_parts) {
-    const SegItem* w = items + seg.item_begin + lane;
-    first_row = w->part_base + (int64_t)bh * w->part_bh_stride + row0;
+// Place in a segment's slice of the item table of the i-th item its workgroups walk: table order, except that item
+// `last_item` (the masked one) is moved to the end.
+static __device__ __forceinline__ int run_order(const Segment& seg, int i) {
+  if (seg.last_item < 0) return i;
+  return i == seg.item_count - 1 ? seg.last_item : (i >= seg.last_item ? i + 1 : i);
+}
+
+// ---- the merge of per-step partials of a row: L = logsumexp_s L_s, O = sum_s exp(L_s - L) O_s, one part after the other.  The
+// reference of the weights is the largest L_s so far; when it moves, the sums so far are scaled down to it (the rescale of
+// csrc/ring_attention.cu:226-232).  So a merge needs no look at all the L_s ahead of the first O_s, and a workgroup that
+// walks the steps of its rows merges each partial where it arises.  Every merge of the library (the merge kernel and
+// those in the attention kernels) is these operations on the same operands in the same order -- ring steps ascending, the
+// masked one last (a causal plan's step 0), as the attention kernels walk them --, so they give the same bits.  A part with
+// L_s = -inf is the identity: callers pass it by, whatever its O may hold.
+struct MergeState {
+  float top = -INFINITY, sum = 0.f;  // the reference; the weights' sum against it
+  // the weight of a part, and what the sums so far keep
+  __device__ __forceinline__ void weigh(float L, float& keep, float& w) {
+    constexpr float kLog2e = 1.4426950408889634f;
+    const float t = fmaxf(top, L);
+    keep = __builtin_amdgcn_exp2f((top - t) * kLog2e);  // 1 while the reference stays, 0 for the first part
+    w = __builtin_amdgcn_exp2f((L - t) * kLog2e);
+    sum = __builtin_fmaf(sum, keep, w);
+    top = t;
   }
-  auto part_row = [&](int i) -> int64_t {
-    return (int64_t)(((uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(first_row >> 32), i) << 32) |
-                     (unsigned)__builtin_amdgcn_readlane((int)first_row, i));
-  };
-  __syncthreads();  // the partial stores of all waves have completed and are visible to them; the LDS is idle
-  {
-    float v[KMAX][LR];
-#pragma unroll
-    for (int k = 0; k < KMAX; ++k) {
-      const int i = wave + WAVES * k;
-      if (i < n_parts) {
-        const int64_t prow = part_row(i);
-#pragma unroll
-        for (int r = 0; r < LR; ++r) v[k][r] = (row0 + lane + 64 * r < seg.q_len) ? lse_part[prow + lane + 64 * r] : -INFINITY;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < KMAX; ++k) {
-      const int i = wave + WAVES * k;
-      if (i < n_parts) {
-#pragma unroll
-        for (int r = 0; r < LR; ++r) lse_s[i * BM + lane + 64 * r] = v[k][r];
-      }
-    }
+  __device__ __forceinline__ float inverse() const { return top == -INFINITY ? 0.f : 1.f / sum; }
+  __device__ __forceinline__ float lse() const {
+    return top == -INFINITY ? -INFINITY : __builtin_fmaf(__builtin_amdgcn_logf(sum), 0.6931471805599453f, top);
   }
-  __syncthreads();
-  const int c8 = tid % TPR, rsub = tid / TPR;
-  // this thread's 8 columns of a partial row: 16 bytes as fp16, 32 as fp32
-  constexpr int PB = HP ? 16 : 32;
-  constexpr int NV = PB / 16;
-  // R rows and G parts of a thread per batch
-  auto merge_in = [&](auto rows_c, auto parts_c) {
-    constexpr int R = decltype(rows_c)::value, G = decltype(parts_c)::value;
-    constexpr int RSTEP = R * ROWS;
-    const int n_groups = (n_parts + G - 1) / G;
-    const int n_batches = (BM / RSTEP) * n_groups;  // batch b: rows of b / n_groups, parts of b % n_groups
-    struct Batch {
-      f32x4 raw[R][G][NV];  // as loaded; fp16 partials are widened when they are used
-    };
-    auto row_of = [&](int b, int j) { return (b / n_groups) * RSTEP + j * ROWS + rsub; };  // within the job
-    // Every load of a batch is made, those of parts and rows that do not exist from the last one that does: with loads under
-    // conditions the compiler cannot count those in flight, and waits for the batches fetched ahead as well.  Where the parts
-    // lie comes from a lane of first_row and not from the table, a scalar round trip for each.  Together, and past the
-    // cache's retention (fp16; fp32 rows measured 1.6 % slower that way): forward with fp16 partials, 64 heads x 32 x 512, d = 128
-    // 11.74 -> 10.70 ms, of which the merge was 2.4 ms; fp32 partials, 16 heads 3.74 -> 3.64 ms.
-    auto fetch = [&](int b, Batch& t) {
-      const int i0 = (b % n_groups) * G;
-      int at[R];
-#pragma unroll
-      for (int j = 0; j < R; ++j) at[j] = min(row_of(b, j), last_row) * (D * (PB / 8)) + c8 * PB;
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        if (G == 2 && u == 1 && n_parts == 1) break;  // (nothing is fetched ahead of it that a wait could include)
-        const char* base = (const char*)o_part + part_row(min(i0 + u, n_parts - 1)) * (D * (PB / 8));
-#pragma unroll
-        for (int j = 0; j < R; ++j)
-#pragma unroll
-          for (int v = 0; v < NV; ++v) {
-            const f32x4* src = (const f32x4*)(base + at[j] + 16 * v);
-            t.raw[j][u][v] = HP ? __builtin_nontemporal_load(src) : *src;
-          }
-      }
-    };
-    float mx[R], wsum[R], acc[R][8];
-    auto accumulate = [&](int b, const Batch& t) {
-      const int g = b % n_groups, i0 = g * G;
-      if (g == 0) {  // new rows: L = max over the parts first
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-          mx[j] = -INFINITY;
-          wsum[j] = 0.f;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) acc[j][e] = 0.f;
-        }
-        for (int i = 0; i < n_parts; ++i)
-#pragma unroll
-          for (int j = 0; j < R; ++j) mx[j] = fmaxf(mx[j], lse_s[i * BM + row_of(b, j)]);
-      }
-#pragma unroll
-      for (int u = 0; u < G; ++u)
-        if (i0 + u < n_parts) {
-#pragma unroll
-          for (int j = 0; j < R; ++j) {
-            const float L = lse_s[(i0 + u) * BM + row_of(b, j)];
-            if (row0 + row_of(b, j) >= seg.q_len || L == -INFINITY) continue;  // identity element: its O may hold anything
-            const float w = __expf(L - mx[j]);
-            wsum[j] += w;
-            float x[8];
-            if (HP) {
-              const f16x8 hv = __builtin_bit_cast(f16x8, t.raw[j][u][0]);
-#pragma unroll
-              for (int e = 0; e < 8; ++e) x[e] = (float)hv[e];
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                x[e] = t.raw[j][u][0][e];
-                x[4 + e] = t.raw[j][u][NV - 1][e];
-              }
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[j][e] = __builtin_fmaf(w, x[e], acc[j][e]);
-          }
-        }
-      if (g == n_groups - 1) {  // all parts in: normalise and store
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-          if (row0 + row_of(b, j) >= seg.q_len) continue;
-          if (mx[j] != -INFINITY) {
-            const float inv = 1.f / wsum[j];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[j][e] *= inv;
-          }
-          const int64_t out_row = (int64_t)bh * S + seg.q_start + row0 + row_of(b, j);
-          Store8<DT>::st((char*)out + (out_row * D + c8 * 8) * 2, acc[j]);
-          if (c8 == 0) lse[out_row] = (mx[j] == -INFINITY) ? -INFINITY : mx[j] + __logf(wsum[j]);
-        }
-      }
-    };
-    // three batches in flight
-    Batch t0, t1, t2;
-    fetch(0, t0);
-    if (1 < n_batches) fetch(1, t1);
-    int b = 0;
-#pragma unroll 1
-    for (; b + 4 < n_batches; b += 3) {
-      fetch(b + 2, t2);
-      accumulate(b, t0);
-      fetch(b + 3, t0);
-      accumulate(b + 1, t1);
-      fetch(b + 4, t1);
-      accumulate(b + 2, t2);
-    }
-#pragma unroll 1
-    for (; b < n_batches; b += 3) {
-      if (b + 2 < n_batches) fetch(b + 2, t2);
-      accumulate(b, t0);
-      if (b + 3 < n_batches) fetch(b + 3, t0);
-      if (b + 1 < n_batches) accumulate(b + 1, t1);
-      if (b + 4 < n_batches) fetch(b + 4, t1);
-      if (b + 2 < n_batches) accumulate(b + 2, t2);
-    }
-  };
-  // 64 registers a batch.  Of a segment with one part or two most of such a batch would be loads of rows that are there
-  // already, so these take twice the rows of two parts instead.  Forward with the steps apart, d = 128, us, one shape of batch ->
-  // two: 256 heads x 256 tokens, one part 36.8 -> 31.0, with fp16 partials 39.9 -> 25.2 (34.7 and 30.7 with loads under
-  // conditions); 2 x 256 tokens 108 -> 95 and 99 -> 73; causal 128 heads x 5 x 256 201 -> 187 and 163 -> 143.
-  if (n_parts <= 2) merge_in(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
-  else merge_in(std::integral_constant<int, 2>{}, std::integral_constant<int, HP ? 8 : 4>{});
+};
+static __device__ __forceinline__ float merge_in_part(float acc, float keep, float w, float x) {
+  return __builtin_fmaf(w, x, acc * keep);
 }
 
 }  // namespace ringattn

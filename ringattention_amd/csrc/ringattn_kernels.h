@@ -58,7 +58,8 @@ static_assert(sizeof(Segment) == 32, "Segment is read as two 16-byte scalar load
 // What a workgroup does with the softmax state (max, sum, acc-O) of its rows between the KV chunks it walks.
 enum BlockMode {
   kBlockPartials = 0,        // per chunk: emit the normalised partial (O, LSE), reset the state
-  kBlockPartialsMerged = 1,  // the same, and after the last chunk merge the partials of the rows into out / lse
+  kBlockPartialsMerged = 1,  // per chunk: the same partial, merged into out / lse.  ring_walk_kernel merges it on the spot;
+                             // ring_walk64_kernel emits it to o_part / lse_part and merges after the last chunk
   kBlockCarryState = 2,      // carry the state across the chunks, as the reference's CTA does across its ring
                              // steps (csrc/ring_attention.cu:439-443,597), and write out / lse once: no partials
 };
@@ -132,11 +133,14 @@ struct MergeArgs {
   int S;                  // rows per head
   int64_t part_stride_rows;  // rows between consecutive slots (>= heads * S)
   int half_partials;
+  int slot0_last;         // 1: slot 0, the masked step of a causal plan, is merged after the others, as the attention kernels walk it
   int row_mul;            // 0: slot-major partials as above; n > 0: [heads * S, n, D] / [heads * S, n], a row's slots adjacent
 };
 
 // dtype: 0 = fp16, 1 = bf16.  Return hipSuccess or the launch error.
 hipError_t launch_walk(BlockArgs a, int dtype, int dim, hipStream_t stream);  // ring_walk_kernel, any BlockMode
+// its kBlockPartialsMerged, the grid laid out (ringattn_steps.hip)
+hipError_t launch_steps(const BlockArgs& a, unsigned grid, int dtype, int dim, hipStream_t stream);
 // ring_walk64_kernel: the carried-state forward at d = 128 with 64 query rows per wave; only for tables that
 // walk64_takes() accepts
 hipError_t launch_walk64(BlockArgs a, int dtype, int dim, hipStream_t stream);

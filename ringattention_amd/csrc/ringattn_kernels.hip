@@ -11,77 +11,74 @@
 
 namespace ringattn {
 
-// ---- merge of one row: the merge kernel's arithmetic (the attention kernel's merge at the end of a workgroup follows it) -------
-// The parts of one row, in ascending slot order: the set bits of a mask over equally spaced slots.
+// ---- merge of one row (MergeState in ringattn_device.h) ---------------------------------------------------------------
+// The parts of one row: the set bits of a mask over equally spaced slots, ascending from slot `first` on, round to the slots before it.
 struct SlotParts {
-  uint64_t rest;
+  uint64_t rest;  // bit i: slot (first + i) mod 64
+  int first;
   int64_t row, stride;  // the row in slot 0, rows between slots
   __device__ __forceinline__ int left() const { return __builtin_popcountll(rest); }
   __device__ __forceinline__ int64_t take() {
-    const int64_t r = row + (int64_t)__builtin_ctzll(rest) * stride;
+    const int64_t r = row + (int64_t)((__builtin_ctzll(rest) + first) & 63) * stride;
     rest &= rest - 1;
     return r;
   }
 };
-// L = logsumexp_s L_s, O = sum_s exp(L_s - L) O_s over the parts of one row; this thread owns
-// columns [8 c8, 8 c8 + 8).  A part with L_s = -inf is the identity and its O is not used.
+// This thread owns columns [8 c8, 8 c8 + 8) of the row.
 template <int DT, int D, bool HP, class Parts>
-static __device__ __forceinline__ void merge_row(Parts parts, const void* o_parts, const float* lse_parts,
+static __device__ __forceinline__ void merge_row(Parts p, const void* o_parts, const float* lse_parts,
                                                  void* out, float* lse, int64_t out_row, int c8) {
   const typename PartRow<HP>::ptr o_base = (typename PartRow<HP>::ptr)o_parts + c8 * 8;
-  float mx = -INFINITY;
-  {
-    Parts p = parts;
-    while (p.left()) mx = fmaxf(mx, lse_parts[p.take()]);
-  }
+  MergeState st;
   float acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-  float wsum = 0.f;
-  if (mx != -INFINITY) {
-    // four parts per iteration: all their loads are issued before the first is consumed
-    Parts p = parts;
-    while (p.left() >= 4) {
-      float L[4];
-      f32x4 x0[4], x1[4];
+  auto merge_in = [&](float L, const f32x4& x0, const f32x4& x1) {
+    if (L == -INFINITY) return;  // identity element: its O may hold anything
+    float keep, w;
+    st.weigh(L, keep, w);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t r = p.take();
-        L[u] = lse_parts[r];
-        PartRow<HP>::ld(o_base + r * D, x0[u], x1[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float w = __expf(L[u] - mx);
-        if (L[u] == -INFINITY) continue;  // identity element: its O may hold anything
-        wsum += w;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          acc[e] = __builtin_fmaf(w, x0[u][e], acc[e]);
-          acc[4 + e] = __builtin_fmaf(w, x1[u][e], acc[4 + e]);
-        }
-      }
+    for (int e = 0; e < 4; ++e) {
+      acc[e] = merge_in_part(acc[e], keep, w, x0[e]);
+      acc[4 + e] = merge_in_part(acc[4 + e], keep, w, x1[e]);
     }
-    while (p.left()) {
+  };
+  // Two batches of four parts: one on its way while the other is merged.  With one pass over the parts and this, instead of a pass
+  // over the LSEs first and batches that were waited for, us: causal 32 heads x 8 x 4096, fp32 501 -> 493, fp16 297 -> 276, row-major 530 ->
+  // 523, d = 64 258 -> 252; 64 heads x 32 x 512, fp16 446 -> 420; 8 heads x 8 x 1024 49 -> 45.5.  (Batches of 1, 2 and 3: 520, 524, 510 in the
+  // first of these; one batch of four at a time 514, of eight 503.)
+  constexpr int kBatch = 4;
+  struct Batch {
+    float L[kBatch];
+    f32x4 x0[kBatch], x1[kBatch];
+  } even, odd;
+  const int n = p.left();
+  auto fetch = [&](Batch& t, int first) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (first + u >= n) break;
       const int64_t r = p.take();
-      const float Ls = lse_parts[r];
-      const float w = __expf(Ls - mx);
-      f32x4 x0, x1;
-      PartRow<HP>::ld(o_base + r * D, x0, x1);
-      if (Ls == -INFINITY) continue;
-      wsum += w;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[e] = __builtin_fmaf(w, x0[e], acc[e]);
-        acc[4 + e] = __builtin_fmaf(w, x1[e], acc[4 + e]);
-      }
+      t.L[u] = lse_parts[r];
+      PartRow<HP>::ld(o_base + r * D, t.x0[u], t.x1[u]);
     }
-    const float inv = 1.f / wsum;
+  };
+  auto merge_batch = [&](const Batch& t, int first) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] *= inv;
+    for (int u = 0; u < kBatch; ++u)
+      if (first + u < n) merge_in(t.L[u], t.x0[u], t.x1[u]);
+  };
+  fetch(even, 0);
+  for (int i = 0; i < n; i += 2 * kBatch) {
+    fetch(odd, i + kBatch);
+    merge_batch(even, i);
+    fetch(even, i + 2 * kBatch);
+    merge_batch(odd, i + kBatch);
   }
+  const float inv = st.inverse();
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] *= inv;
   Store8<DT>::st((char*)out + (out_row * D + c8 * 8) * 2, acc);
-  if (c8 == 0) lse[out_row] = (mx == -INFINITY) ? -INFINITY : mx + __logf(wsum);
+  if (c8 == 0) lse[out_row] = st.lse();
 }
 
 // ---- merge ------------------------------------------------------------------------
@@ -94,7 +91,8 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
   if (idx >= (int64_t)a.heads * reg.len) return;
   const int64_t row = (idx / reg.len) * a.S + reg.start + idx % reg.len;
   // slot-major partials: slot s of a row lies part_stride_rows rows further on; row-major: at entry row_mul row + s
-  SlotParts parts{reg.active, a.row_mul > 0 ? row * a.row_mul : row, a.row_mul > 0 ? (int64_t)1 : a.part_stride_rows};
+  const int first = a.slot0_last;
+  SlotParts parts{first ? reg.active >> 1 | reg.active << 63 : reg.active, first, a.row_mul > 0 ? row * a.row_mul : row, a.row_mul > 0 ? (int64_t)1 : a.part_stride_rows};
   merge_row<DT, D, HP>(parts, a.o_parts, a.lse_parts, a.out, a.lse, row, threadIdx.x % TPR);
 }
 

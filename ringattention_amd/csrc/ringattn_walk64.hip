@@ -27,8 +27,8 @@
 
 namespace ringattn {
 
-// Merge of the workgroup's 256 rows over the partials the workgroup has written (what merge_job_rows does for
-// ring_walk_kernel; the arithmetic and its order are merge_row's, so the bits are the merge kernel's).  With one wave
+// Merge of the workgroup's 256 rows over the partials the workgroup has written (the arithmetic and its order are
+// MergeState's, so the bits are the merge kernel's).  With one wave
 // per SIMD nobody covers for a wave that waits for memory, so the partial rows are not fetched into registers a
 // batch at a time but streamed through LDS, which the rings have left free: every wave merges eight rows of each
 // group of 32 and keeps six blocks (eight rows of one part: 4 KB, 2 KB as fp16) in flight in a ring of its own,
@@ -60,12 +60,13 @@ static __device__ __forceinline__ void merge_rows_staged(const BlockArgs& a, con
   int64_t* base_s = (int64_t*)(smem + kBaseAt);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();  // the partial stores of all waves have completed and are visible to them; the LDS is idle
-  for (int i0 = 0; i0 < n_parts; i0 += 8) {  // thread tid: the LSEs of row tid
+  for (int i0 = 0; i0 < n_parts; i0 += 8) {  // thread tid: the LSEs of row tid; parts in the order they were walked
     float v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (i0 + u < n_parts) {
-        const int64_t prow = its[i0 + u].part_base + (int64_t)bh * its[i0 + u].part_bh_stride + row0;
+        const SegItem* it = its + run_order(seg, i0 + u);
+        const int64_t prow = it->part_base + (int64_t)bh * it->part_bh_stride + row0;
         v[u] = tid < rows_here ? a.lse_part[prow + tid] : -INFINITY;
         if (tid == 0) base_s[i0 + u] = prow;
       }
@@ -100,7 +101,8 @@ static __device__ __forceinline__ void merge_rows_staged(const BlockArgs& a, con
   for (int t = 0; t < NS && t < total; ++t) issue_block(t);
 
   const int r8 = lane >> 3, c = lane & 7;
-  float mx = -INFINITY, wsum = 0.f, acc[NK * CPP];
+  MergeState st;
+  float acc[NK * CPP];
   int cg = 0, ci = 0;  // group and part of the block to consume
   int slot = 0;
   for (int t = 0; t < total; ++t) {
@@ -111,37 +113,33 @@ static __device__ __forceinline__ void merge_rows_staged(const BlockArgs& a, con
     const unsigned char* blk = smem + kRingAt + wave * (NS * SLOT) + slot * SLOT + r8 * RB;
 #pragma unroll
     for (int k = 0; k < NK; ++k) x[k] = *(const f32x4*)(blk + (((c + 8 * k) ^ (8 * (r8 & 1))) << 4));
-    if (ci == 0) {  // new rows: L = max over the parts first
-      mx = -INFINITY;
-      wsum = 0.f;
+    if (ci == 0) {  // new rows
+      st = MergeState();
 #pragma unroll
       for (int e = 0; e < NK * CPP; ++e) acc[e] = 0.f;
-      for (int i = 0; i < n_parts; ++i) mx = fmaxf(mx, lse_s[i * BM + row]);
     }
     const float L = lse_s[ci * BM + row];
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the block is in registers: its slot takes the block NS further on
     if (t + NS < total) issue_block(slot);
     if (row < rows_here && L != -INFINITY) {  // (-inf: the identity element, its O may hold anything)
-      const float w = __expf(L - mx);
-      wsum += w;
+      float keep, w;
+      st.weigh(L, keep, w);
 #pragma unroll
       for (int k = 0; k < NK; ++k) {
         if (HP) {
           const f16x8 hv = __builtin_bit_cast(f16x8, x[k]);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) acc[8 * k + e] = __builtin_fmaf(w, (float)hv[e], acc[8 * k + e]);
+          for (int e = 0; e < 8; ++e) acc[8 * k + e] = merge_in_part(acc[8 * k + e], keep, w, (float)hv[e]);
         } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[4 * k + e] = __builtin_fmaf(w, x[k][e], acc[4 * k + e]);
+          for (int e = 0; e < 4; ++e) acc[4 * k + e] = merge_in_part(acc[4 * k + e], keep, w, x[k][e]);
         }
       }
     }
     if (ci == n_parts - 1 && row < rows_here) {  // all parts in: normalise and store
-      if (mx != -INFINITY) {
-        const float inv = 1.f / wsum;
+      const float inv = st.inverse();
 #pragma unroll
-        for (int e = 0; e < NK * CPP; ++e) acc[e] *= inv;
-      }
+      for (int e = 0; e < NK * CPP; ++e) acc[e] *= inv;
       const int64_t out_row = (int64_t)bh * a.S + seg.q_start + row0 + row;
       typename Elem<DT>::type* orow = (typename Elem<DT>::type*)a.out + out_row * D;
 #pragma unroll
@@ -155,13 +153,171 @@ static __device__ __forceinline__ void merge_rows_staged(const BlockArgs& a, con
           *(typename Elem<DT>::vec4*)(orow + (c + 8 * k) * 4) = o4;
         }
       }
-      if (c == 0) a.lse[out_row] = (mx == -INFINITY) ? -INFINITY : mx + __logf(wsum);
+      if (c == 0) a.lse[out_row] = st.lse();
     }
     if (++ci == n_parts) {
       ci = 0;
       ++cg;
     }
     slot = slot + 1 == NS ? 0 : slot + 1;
+  }
+}
+
+// The same merge where the LSEs of the parts leave no room for the staging rings: all of them are parked in LDS (lse_s:
+// [items][256] floats), and the partial O rows move through registers in batches of 256 bytes per thread
+// (two output rows x four or eight parts), three batches in flight at any time.
+typedef __attribute__((address_space(3))) float lds_float;
+template <int DT, bool HP>
+static __device__ __forceinline__ void merge_job_rows(const void* o_part, const float* lse_part, void* out, float* lse,
+                                                      const SegItem* items, const Segment& seg, int bh, int qt, int S,
+                                                      lds_float* lse_s) {
+  constexpr int D = 128, BM = kWalkM, WAVES = 4, THREADS = 64 * WAVES;
+  constexpr int TPR = D / 8;  // threads per row, 8 columns each
+  constexpr int ROWS = THREADS / TPR;
+  constexpr int KMAX = kMaxParts / WAVES;  // parts per wave in the LSE sweep
+  constexpr int LR = BM / 64;              // rows per lane in the LSE sweep
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n_parts = seg.item_count;
+  const int row0 = qt * BM;  // first row of the job within the segment
+  const int last_row = min(BM, seg.q_len - row0) - 1;
+  // lane i keeps where the job's rows begin in the partials of the i-th item walked
+  int64_t first_row = 0;
+  if (lane < n_parts) {
+    const SegItem* w = items + seg.item_begin + run_order(seg, lane);
+    first_row = w->part_base + (int64_t)bh * w->part_bh_stride + row0;
+  }
+  auto part_row = [&](int i) -> int64_t {
+    return (int64_t)(((uint64_t)(unsigned)__builtin_amdgcn_readlane((int)(first_row >> 32), i) << 32) |
+                     (unsigned)__builtin_amdgcn_readlane((int)first_row, i));
+  };
+  __syncthreads();  // the partial stores of all waves have completed and are visible to them; the LDS is idle
+  {
+    float v[KMAX][LR];
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k) {
+      const int i = wave + WAVES * k;
+      if (i < n_parts) {
+        const int64_t prow = part_row(i);
+#pragma unroll
+        for (int r = 0; r < LR; ++r) v[k][r] = (row0 + lane + 64 * r < seg.q_len) ? lse_part[prow + lane + 64 * r] : -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k) {
+      const int i = wave + WAVES * k;
+      if (i < n_parts) {
+#pragma unroll
+        for (int r = 0; r < LR; ++r) lse_s[i * BM + lane + 64 * r] = v[k][r];
+      }
+    }
+  }
+  __syncthreads();
+  const int c8 = tid % TPR, rsub = tid / TPR;
+  // this thread's 8 columns of a partial row: 16 bytes as fp16, 32 as fp32
+  constexpr int PB = HP ? 16 : 32;
+  constexpr int NV = PB / 16;
+  // R rows and G parts of a thread per batch: 64 registers
+  constexpr int R = 2, G = HP ? 8 : 4;
+  constexpr int RSTEP = R * ROWS;
+  const int n_groups = (n_parts + G - 1) / G;
+  const int n_batches = (BM / RSTEP) * n_groups;  // batch b: rows of b / n_groups, parts of b % n_groups
+  struct Batch {
+    f32x4 raw[R][G][NV];  // as loaded; fp16 partials are widened when they are used
+  };
+  auto row_of = [&](int b, int j) { return (b / n_groups) * RSTEP + j * ROWS + rsub; };  // within the job
+  // Every load of a batch is made, those of parts and rows that do not exist from the last one that does: with loads under
+  // conditions the compiler cannot count those in flight, and waits for the batches fetched ahead as well.  Where the parts
+  // lie comes from a lane of first_row and not from the table, a scalar round trip for each.
+  auto fetch = [&](int b, Batch& t) {
+    const int i0 = (b % n_groups) * G;
+    int at[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) at[j] = min(row_of(b, j), last_row) * (D * (PB / 8)) + c8 * PB;
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      const char* base = (const char*)o_part + part_row(min(i0 + u, n_parts - 1)) * (D * (PB / 8));
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const f32x4* src = (const f32x4*)(base + at[j] + 16 * v);
+          t.raw[j][u][v] = HP ? __builtin_nontemporal_load(src) : *src;
+        }
+    }
+  };
+  MergeState st[R];
+  float acc[R][8];
+  auto accumulate = [&](int b, const Batch& t) {
+    const int g = b % n_groups, i0 = g * G;
+    if (g == 0) {  // new rows
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        st[j] = MergeState();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[j][e] = 0.f;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < G; ++u)
+      if (i0 + u < n_parts) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          const float L = lse_s[(i0 + u) * BM + row_of(b, j)];
+          if (row0 + row_of(b, j) >= seg.q_len || L == -INFINITY) continue;  // identity element: its O may hold anything
+          float keep, w;
+          st[j].weigh(L, keep, w);
+          float x[8];
+          if (HP) {
+            const f16x8 hv = __builtin_bit_cast(f16x8, t.raw[j][u][0]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = (float)hv[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              x[e] = t.raw[j][u][0][e];
+              x[4 + e] = t.raw[j][u][NV - 1][e];
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[j][e] = merge_in_part(acc[j][e], keep, w, x[e]);
+        }
+      }
+    if (g == n_groups - 1) {  // all parts in: normalise and store
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        if (row0 + row_of(b, j) >= seg.q_len) continue;
+        const float inv = st[j].inverse();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[j][e] *= inv;
+        const int64_t out_row = (int64_t)bh * S + seg.q_start + row0 + row_of(b, j);
+        Store8<DT>::st((char*)out + (out_row * D + c8 * 8) * 2, acc[j]);
+        if (c8 == 0) lse[out_row] = st[j].lse();
+      }
+    }
+  };
+  // three batches in flight
+  Batch t0, t1, t2;
+  fetch(0, t0);
+  if (1 < n_batches) fetch(1, t1);
+  int b = 0;
+#pragma unroll 1
+  for (; b + 4 < n_batches; b += 3) {
+    fetch(b + 2, t2);
+    accumulate(b, t0);
+    fetch(b + 3, t0);
+    accumulate(b + 1, t1);
+    fetch(b + 4, t1);
+    accumulate(b + 2, t2);
+  }
+#pragma unroll 1
+  for (; b < n_batches; b += 3) {
+    if (b + 2 < n_batches) fetch(b + 2, t2);
+    accumulate(b, t0);
+    if (b + 3 < n_batches) fetch(b + 3, t0);
+    if (b + 1 < n_batches) accumulate(b + 1, t1);
+    if (b + 4 < n_batches) fetch(b + 4, t1);
+    if (b + 2 < n_batches) accumulate(b + 2, t2);
   }
 }
 
@@ -200,11 +356,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   const int all_items = seg.item_count;
   const ItemPtr items = items_of(a);
   // items in run order: table order, except that item `last_item` (the diagonal one) is moved to the end
-  auto item_in_order = [&](int i) -> ItemPtr {
-    int idx = i;
-    if (seg.last_item >= 0) idx = (i == all_items - 1) ? seg.last_item : (i >= seg.last_item ? i + 1 : i);
-    return items + seg.item_begin + idx;
-  };
+  auto item_in_order = [&](int i) -> ItemPtr { return items + seg.item_begin + run_order(seg, i); };
   const int64_t head_off = (int64_t)bh * a.bh_stride;
   const int kv_bh = (bh / a.heads) * (a.heads / a.kv_group) + (bh % a.heads) / a.kv_group;
   const int64_t kv_head_off = (int64_t)kv_bh * a.kv_bh_stride;
@@ -472,8 +624,8 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
       if (all_items <= kStagedMergeMaxParts)
         merge_rows_staged<DT, HP>(a, seg, bh, qt, smem, smem_base);
       else
-        merge_job_rows<DT, D, HP, BM, 64 * WAVES>(a.o_part, a.lse_part, a.out, a.lse, a.items, seg, bh, qt, a.S,
-                                                  (lds_float*)(__attribute__((address_space(3))) void*)smem);
+        merge_job_rows<DT, HP>(a.o_part, a.lse_part, a.out, a.lse, a.items, seg, bh, qt, a.S,
+                               (lds_float*)(__attribute__((address_space(3))) void*)smem);
     }
   }
 }
