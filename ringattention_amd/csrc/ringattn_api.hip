@@ -346,6 +346,10 @@ static int pair_choice() {
 //     8 heads x 8192                       211, 230, 389     131, 145, 198
 //     9 heads x 8192 (288 q tiles of 256)  355, 310, 437     244, 208, 223
 //     16 heads x 8192, causal              221, 245, 424     142, 159, 209
+// ring_split_kernel has since become 5 to 30 % faster where compute units idle (its file) and 5 % elsewhere; its numbers are left, because the lines
+// they draw are those between equals: with new ones d = 64 launches moved to it that both kernels run alike (us on
+// ring_split_kernel and ring_pair_kernel: causal 8 x 4928 47, 48; 12 x 3054 33, 34; 4 x 10816 97, 94; no mask 6 x 3394 39, 38; 1 x
+// 20971 184, 164), and at d = 128 some whose second round of workgroups is mostly empty (4 x 3328 43.5, 40.6).
 enum class CarryKernel { kWhole, kPair, kSplit, kSplit16 };
 struct KernelRate {
   int tiles_per_step;
@@ -393,12 +397,12 @@ static CarryKernel carry_kernel(const CarryCosts& c, int dim, bool wide) {
     if (t < best) best = t, kernel = CarryKernel::kPair;
   }
   if (split != 0 && carry_time(c.thin, r[2], false) < best) kernel = CarryKernel::kSplit;
-  // At d = 64 two workgroups of ring_split_kernel fit on a compute unit.  A launch of no more workgroups than there are
-  // compute units fills the other half with waves of the same workgroup, sixteen of them instead of eight, where the walk
+  // At d = 64 two workgroups of ring_split_kernel fit on a compute unit.  A launch that leaves half of the compute units idle
+  // may as well fill that place with waves of the same workgroup, sixteen of them instead of eight, where the walk
   // is long enough to pay for the combination of twice the states.  us with eight and with sixteen waves, at 64, 128, 256
-  // and 512 tiles: 2048 rows 12.8, 13.7; 4096 rows 20.4, 18.9; 8192 rows 36.9, 33.1; 8192 rows x 16384 keys 64.1, 58.2, 4096 of
-  // them 63.1, 48.5; causal 4096 rows 19.8, 18.6.  More workgroups than compute units: 8 heads x 2048 19.2, 25.6.
-  if (kernel == CarryKernel::kSplit && dim == 64 && c.thin.jobs <= kComputeUnits && c.thin.tiles >= 96)
+  // and 512 tiles: 2048 rows 11.3, 12.9; 4096 rows, causal 15.1, 16.6; 8192 rows 30.8, 31.6; 2048, 4096 and 8192 rows x 16384
+  // keys 44.1, 41.8; 43.9, 42.0; 53.7, 55.3.
+  if (kernel == CarryKernel::kSplit && dim == 64 && 2 * c.thin.jobs <= kComputeUnits && c.thin.tiles >= 384)
     kernel = CarryKernel::kSplit16;
   return kernel;
 }

@@ -13,13 +13,16 @@
 //       the fragments of this one are in registers and has the softmax and the PV product to arrive in, the next V tile
 //       has the QK^T product and the softmax; two (d = 64: four) waves per SIMD overlap one another's matrix and vector
 //       phases without any coordination.
-//       What bounds it: a K/V tile fetched from L2 feeds 32 query rows instead of 256.  At d = 128 a compute unit would
-//       have to take in 128 B per clock to keep its matrix pipes full, twice what its path to L2 carries; without the
-//       loads (timing only) the loop runs 25 % faster.  A full device reaches 690 TFLOP/s at d = 128 and 640 at d = 64
-//       (ring_walk64_kernel 1260 and 940), so this kernel is for launches that leave it compute units idle: the host
-//       weighs the kernels (carry_kernel in ringattn_api.hip).  One head of 8192 tokens, us: 152 -> 54 at d = 128, 114 -> 38 at
-//       d = 64; one head of 512 tokens 19.2 -> 10.2 and 13.6 -> 10.7 (with the host's share of the launch).  With sixteen waves, four
-//       per SIMD, for the 256 workgroups of 8192 rows x 16384 keys at d = 64: 64.1 -> 58.2, and for half as many rows 63.1 -> 48.5.
+//       What bounds it: a K/V tile fetched from L2 feeds 32 query rows instead of 256, and a compute unit takes in 46 (d = 64) to
+//       50 (d = 128) of the 64 bytes per clock that its path to L2 carries.  A full device reaches 730 TFLOP/s at d = 128 and
+//       690 at d = 64 (ring_walk64_kernel 1260 and 940), so this kernel is for launches that leave it compute units idle: the
+//       host weighs the kernels (carry_kernel in ringattn_api.hip).  Up to there it was the instructions around a tile: with
+//       the next tile's place worked out by a search through the ranges in registers, an M0 write and a base address per 1 KB
+//       piece, and the choice to move the references in scalar logic, a tile cost a wave 100 scalar and 93 vector instructions
+//       and some twenty branches.  Now a tile's place is a count that only the end of a range sends to the table, pieces within
+//       4 KB share M0 and address, and the first score of a row overflows into the branch that moves its reference.  us before and
+//       after: d = 64, 8192 rows x 16384 keys 58.2 -> 53.7, 2048 x 16384 48.5 -> 42, 4096 x 4096 causal 18.7 -> 15.1, 8 heads x 4096 causal
+//       36 -> 33.5; d = 128, 8192 x 8192 57 -> 53, 4096 x 4096 causal 27 -> 22.3, 512 x 2048 causal 16.6 -> 14.3, 8 heads x 2048 34 -> 31.
 #include "ringattn_device.h"
 
 namespace ringattn {
@@ -52,16 +55,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel
   const int n_items = seg.item_count;
   const int q0 = qt * BM;  // first row of the tile within the segment
   const int q_last = min(q0 + BM, seg.q_len) - 1;
-  // lane i keeps item i of the segment (kMaxParts = 64 at most); the order they are walked in does not matter here
-  int it_start = 0, it_len = 0, it_diag = -1;
-  if (lane < n_items) {
-    const ItemPtr w = items_of(a) + seg.item_begin + lane;
-    it_start = w->kv_start;
-    it_len = w->kv_len;
-    it_diag = w->diag_off;
-  }
-  int it_tiles = (it_len + BN - 1) / BN;
-  if (it_diag >= 0) it_tiles = min(it_tiles, (it_diag + q_last) / BN + 1);
+  const ItemPtr items = items_of(a) + seg.item_begin;  // the order they are walked in does not matter here
 
   const int64_t head_off = (int64_t)bh * a.bh_stride;
   // grouped-query attention: query head h of a batch entry reads KV head h / kv_group
@@ -93,7 +87,8 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel
       voff[db] = TILE + row8 * ROWB + ((c ^ v_swizzle<D>(row8)) << 4) + ((s & 1) << 3);
     }
   }
-  // offsets of this lane's 16 bytes within a 1 KB piece of a tile; the swizzles repeat after a few pieces
+  // Offsets of this lane's 16 bytes within a 1 KB piece of a tile; the swizzles repeat after a few pieces.  A load instruction's
+  // own offset moves both ends, so pieces up to 4 KB apart share a base address and an M0 (d = 128 needs two of each).
   constexpr int NPK = D == 128 ? 4 : 2, NPV = D == 128 ? 2 : 1;
   const int prow = lane / CPR;
   int goff_k[NPK], goff_v[NPV];
@@ -106,8 +101,13 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel
     constexpr int NP = sizeof(goff) / sizeof(int);
     if (rows >= BN) {
 #pragma unroll
-      for (int j = 0; j < PIECES; ++j)
-        load_lds_16_settled(base + 1024 * j, goff[j % NP], __builtin_amdgcn_readfirstlane(dst + 1024 * j));
+      for (int j = 0; j < PIECES; j += 4)
+        asm volatile(
+            "s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %5\n\tglobal_load_lds_dwordx4 %2, %5 offset:1024\n\t"
+            "global_load_lds_dwordx4 %3, %5 offset:2048\n\tglobal_load_lds_dwordx4 %4, %5 offset:3072" ::"s"(
+                __builtin_amdgcn_readfirstlane(dst + 1024 * j)),
+            "v"(goff[0]), "v"(goff[1 % NP]), "v"(goff[2 % NP]), "v"(goff[3 % NP]), "s"(base + 1024 * j)
+            : "m0");
     } else {
       int row = prow;
       asm volatile("" : "+v"(row));  // (keeps this seldom taken arithmetic from being done ahead of the loop, in registers)
@@ -119,33 +119,25 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel
   };
 
   // ---- the tiles of this wave: numbers wave, wave + WAVES, ... of the items' tiles laid end to end
-  struct Pos {
-    int item, t;  // item, tile within it
-    int start, len, diag;
-  };
-  auto settle = [&](Pos& p) {  // p.t may lie beyond the item: on to the item that holds it; false past the last one
-    while (p.item < n_items) {
-      const int tiles = __builtin_amdgcn_readlane(it_tiles, p.item);
-      if (p.t < tiles) {
-        p.start = __builtin_amdgcn_readlane(it_start, p.item);
-        p.len = __builtin_amdgcn_readlane(it_len, p.item);
-        p.diag = __builtin_amdgcn_readlane(it_diag, p.item);
-        return true;
-      }
-      p.t -= tiles;
-      ++p.item;
+  int item = 0, t = wave, tiles = 0;   // the tile whose K is loaded next: tile t of `tiles` of item `item`
+  int len = 0, diag = -1;
+  int64_t start = 0;
+  auto enter = [&]() {  // t may lie beyond the item: on to the one that holds it; false past the last
+    for (; item < n_items; ++item) {
+      const ItemPtr w = items + item;
+      len = w->kv_len;
+      diag = w->diag_off;
+      start = w->kv_start;
+      tiles = (len + BN - 1) / BN;
+      if (diag >= 0) tiles = min(tiles, (diag + q_last) / BN + 1);
+      if (t < tiles) return true;
+      t -= tiles;
     }
     return false;
   };
-  auto issue_k = [&](const Pos& p) {
-    load_tile(k_head + ((int64_t)p.start + p.t * BN) * ROWB, k_lds, p.len - p.t * BN, goff_k);
-  };
-  auto issue_v = [&](const Pos& p) {
-    load_tile(v_head + ((int64_t)p.start + p.t * BN) * ROWB, k_lds + TILE, p.len - p.t * BN, goff_v);
-  };
 
   float m = -INFINITY;  // reference max (raw score units)
-  float ms = 0.f;       // m * k2, 0 while m is -inf (guard of csrc/ring_attention.cu:183)
+  float ms = kNoReference;  // m * k2, kNoReference while m is -inf (guard of csrc/ring_attention.cu:183): a first finite score overflows
   float ls[4] = {0.f, 0.f, 0.f, 0.f};
   f32x16 oacc[DB];
 #pragma unroll
@@ -153,106 +145,135 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel
 #pragma unroll
     for (int e = 0; e < 16; ++e) oacc[db][e] = 0.f;
 
-  Pos cur;
-  cur.item = 0;
-  cur.t = wave;
-  bool have = settle(cur);
-  bool fresh = true;  // no tile done yet: no reference to take exponentials against
-  if (have) {
+  // a tile's place and mask, carried from its loads to its scores
+  struct Tile {
+    int64_t at;    // byte offset of its first row from the head's
+    int rows;      // keys from its first on to the end of its item
+    int visible;   // keys from its first on that the first row of the q tile sees (with `rows`, what the mask goes by)
+  };
+  auto tile_here = [&]() {
+    Tile x;
+    x.at = (start + (int64_t)t * BN) * ROWB;
+    x.rows = len - t * BN;
+    x.visible = diag >= 0 ? diag + q0 + 1 - t * BN : INT32_MAX - BM;
+    return x;
+  };
+  auto issue_k = [&](const Tile& x) { load_tile(k_head + x.at, k_lds, x.rows, goff_k); };
+  auto issue_v = [&](const Tile& x) { load_tile(v_head + x.at, k_lds + TILE, x.rows, goff_v); };
+  // P = exp2(S k2 - m k2) and the sums of four: from the unrounded values (:242); rounded for the MFMA (:604)
+  f32x16 sacc;
+  s16x8 pf[2];
+  float sums[4];
+  auto exponentials = [&]() {
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      typename E::vec8 pv;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[8 * t2 + e], a.scale_log2, -ms));
+        sums[e & 3] = t2 == 0 && e < 4 ? p : sums[e & 3] + p;
+        pv[e] = (typename E::type)p;
+      }
+      pf[t2] = __builtin_bit_cast(s16x8, pv);
+    }
+  };
+  auto move_reference = [&]() {  // rescale of l and acc-O as in :226-232
+    float m0 = m, m1 = m;
+#pragma unroll
+    for (int e = 0; e < 16; e += 4) {
+      m0 = fmaxf(fmaxf(m0, sacc[e]), sacc[e + 1]);
+      m1 = fmaxf(fmaxf(m1, sacc[e + 2]), sacc[e + 3]);
+    }
+    m = cross_half_max(fmaxf(m0, m1));
+    const float cs = (m == -INFINITY) ? kNoReference : m * a.scale_log2;
+    const float alpha = __builtin_amdgcn_exp2f(ms - cs);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ls[i] *= alpha;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
+    ms = cs;
+  };
+
+  Tile cur{}, nxt{};
+  bool more = enter();
+  if (more) {
+    cur = tile_here();
     issue_k(cur);
     issue_v(cur);
   }
   __builtin_amdgcn_s_waitcnt(0);  // retire the Q loads with a wait the compiler can see (and the first tiles)
-  while (have) {
-    Pos nxt = cur;
-    nxt.t += WAVES;
-    const bool more = settle(nxt);
+  for (int pass = 1; more; pass = 0) {  // pass: 1 while there is no reference to take exponentials against
+    t += WAVES;
+    more = t < tiles;
+    if (!more) {
+      t -= tiles;
+      ++item;
+      more = enter();
+    }
     // ---- S^T = K Q^T (csrc/ring_attention.cu:565): K(t) is in, V(t) may still be on its way
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
-    f32x16 sacc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) sacc[e] = 0.f;
     {
       s16x8 kfr[KS];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) kfr[ks] = *(const s16x8*)(my + koff[ks]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sacc[e] = 0.f;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) sacc = E::mma(kfr[ks], qf[ks], sacc);
     }
+    __builtin_amdgcn_sched_barrier(0);
     // the fragments are in registers: the K buffer takes the next tile
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (more) issue_k(nxt);
+    if (more) {
+      nxt = tile_here();
+      issue_k(nxt);
+    }
     // key visible iff inside the KV range and key_local <= query_local + diag_off
-    const int t0 = cur.t * BN;
-    if (t0 + BN > cur.len || (cur.diag >= 0 && t0 + BN - 1 > cur.diag + q0)) {
-      int lim = cur.len - 1 - t0 - 4 * h;
-      if (cur.diag >= 0) lim = min(lim, cur.diag + q0 + n - t0 - 4 * h);
+    if (min(cur.rows, cur.visible) < BN) {
+      const int lim = min(cur.rows, cur.visible + n) - 4 * h;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int key = 8 * (e >> 2) + (e & 3);
-        if (key > lim) sacc[e] = -INFINITY;
-      }
+      for (int e = 0; e < 16; ++e)
+        if (8 * (e >> 2) + (e & 3) >= lim) sacc[e] = -INFINITY;
     }
     // ---- softmax (:194-245): exponentials against the reference as it stands; the row maximum is only looked at when a
-    // sum of four exponentials is above 2^14 (or not a number), or a row has no reference yet
-    s16x8 pf[2];
-    float sums[4];
-    bool move = fresh;
-    fresh = false;
+    // sum of four exponentials is above 2^14 (or not a number)
 #pragma unroll 1
-    for (;;) {
-      if (move) {  // rescale of l and acc-O as in :226-232
-        float m0 = m, m1 = m;
-#pragma unroll
-        for (int e = 0; e < 16; e += 4) {
-          m0 = fmaxf(fmaxf(m0, sacc[e]), sacc[e + 1]);
-          m1 = fmaxf(fmaxf(m1, sacc[e + 2]), sacc[e + 3]);
-        }
-        const float cand = cross_half_max(fmaxf(m0, m1));
-        const float cs = (cand == -INFINITY) ? 0.f : cand * a.scale_log2;
-        const float alpha = __builtin_amdgcn_exp2f(m * a.scale_log2 - cs);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ls[i] *= alpha;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
-        m = cand;
-        ms = cs;
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sums[i] = 0.f;
-#pragma unroll
-      for (int t2 = 0; t2 < 2; ++t2) {
-        typename E::vec8 pv;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[8 * t2 + e], a.scale_log2, -ms));
-          sums[e & 3] += p;             // from the unrounded p (:242)
-          pv[e] = (typename E::type)p;  // rounded for the MFMA (:604)
-        }
-        pf[t2] = __builtin_bit_cast(s16x8, pv);
-      }
-      const bool again = !(fmaxf(fmaxf(sums[0], sums[1]), fmaxf(sums[2], sums[3])) <= 16384.f) || m == -INFINITY;
-      if (move || __builtin_amdgcn_ballot_w64(again) == 0) break;
-      move = true;
+    for (;; pass = 1) {
+      if (pass) move_reference();
+      exponentials();
+      const bool large = !(fmaxf(fmaxf(sums[0], sums[1]), fmaxf(sums[2], sums[3])) <= 16384.f);
+      if (pass || __builtin_amdgcn_ballot_w64(large) == 0) break;
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) ls[i] += sums[i];
     // ---- O^T += V^T P^T (:609): V(t) is in, K of the next tile may still be on its way
     if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const unsigned char* vrow = my + 16 * t2 * ROWB + voff[db];
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      constexpr int AHEAD = 2;  // fragments read ahead of the MFMA that consumes one
+      s16x8 vfr[2 * DB];
+      auto read_v = [&](int f) {
+        if (f >= 2 * DB) return;
+        const unsigned char* vrow = my + 16 * (f / DB) * ROWB + voff[f % DB];
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow));
         const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow + 8 * ROWB));
-        oacc[db] = E::mma(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pf[t2], oacc[db]);
+        vfr[f] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      };
+#pragma unroll
+      for (int f = 0; f < AHEAD; ++f) read_v(f);
+#pragma unroll
+      for (int f = 0; f < 2 * DB; ++f) {
+        read_v(f + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+        oacc[f % DB] = E::mma(vfr[f], pf[f / DB], oacc[f % DB]);
+        __builtin_amdgcn_sched_barrier(0);
       }
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (more) issue_v(nxt);
     cur = nxt;
-    have = more;
   }
 
   // ---- combine the states: a common reference, every wave's factor against it, and the sums
