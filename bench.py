@@ -41,7 +41,7 @@ MEASURED_TRAFFIC = {
 }
 KERNEL_SOURCES = {
     "ring_walk64_kernel": ("ringattn_walk64.hip", "ringattn_walk64_loop.inc", "ringattn_walk64_loop_d64.inc", "ringattn_device.h"),
-    "ring_walk_kernel": ("ringattn_walk.hip", "ringattn_steps.hip", "ringattn_walk_rows.h", "ringattn_device.h"),
+    "ring_walk_kernel": ("ringattn_walk.hip", "ringattn_steps.hip", "ringattn_thin.hip", "ringattn_walk_rows.h", "ringattn_device.h"),
 }
 BASELINE_METRIC = "ring-attn fwd TFLOP/s + % bf16 MFMA peak, S=32K d=128 8-step ring, 1 GPU"
 

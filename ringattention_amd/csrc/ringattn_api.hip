@@ -666,6 +666,17 @@ bool slice_takes_walk64(const ringattn_plan* pl, const TableSlice& sl, int mode)
   return pl->p.dim == 128 || (pl->p.dim == 64 && walk64_d64_enabled());
 }
 
+// thin::ring_walk_kernel gives the bits of ring_walk_kernel with one wave per SIMD on half the rows, so a launch may have either.  It is the
+// faster one, at d = 64, while there are compute units to spare (figures in ringattn_thin.hip); places within a
+// range are 32-bit offsets there.  RINGATTN_THIN=0 and 1 in the environment: never, and whatever the size (comparisons, tests).
+constexpr int64_t kThinMaxJobs = 128;  // 256-row q tiles
+bool takes_thin(const ringattn_plan* pl, const TableSlice& sl) {
+  if (pl->p.dim != 64 || pl->d.S * 2 * pl->p.dim > INT32_MAX) return false;
+  const char* e = std::getenv("RINGATTN_THIN");
+  if (e) return e[0] != '0';
+  return (int64_t)sl.seg_count * q_tiles_of(sl.q_len_max) * pl->d.BH <= kThinMaxJobs;
+}
+
 // the slice ringattn_fwd launches
 const TableSlice& forward_slice(const ringattn_plan* pl) { return step_partials(pl->p) ? pl->fwd : pl->walk; }
 
@@ -707,6 +718,11 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
   }
   a.n_segs = sl.seg_count;
   const bool wide = slice_takes_walk64(pl, sl, a.mode);
+  if (a.mode != ringattn::kBlockCarryState && !wide && takes_thin(pl, sl)) {
+    a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kThinM);
+    RA_HIP(ringattn::launch_thin(a, pl->p.dtype, stream));
+    return RINGATTN_OK;
+  }
   const CarryKernel kernel =
       a.mode == ringattn::kBlockCarryState ? carry_kernel(sl.costs, pl->p.dim, wide) : CarryKernel::kWhole;
   RA_HIP(launch_q_tiles(a, kernel, wide, sl.q_len_max, pl->p.dtype, pl->p.dim, stream));

@@ -9,6 +9,7 @@ namespace ringattn {
 constexpr int kWalkM = 256;   // query rows per workgroup of ring_walk_kernel (8 waves x 32 rows)
 constexpr int kSplitM = 32;   // query rows per workgroup of ring_split_kernel
 constexpr int kPairM = 128;  // query rows per workgroup of ring_pair_kernel
+constexpr int kThinM = 128;  // query rows per workgroup of thin::ring_walk_kernel
 constexpr int kMaxParts = 64; // partial slots a merge can combine
 
 // One unit of block-attention work as the host layer lists it: the queries
@@ -141,6 +142,8 @@ struct MergeArgs {
 hipError_t launch_walk(BlockArgs a, int dtype, int dim, hipStream_t stream);  // ring_walk_kernel, any BlockMode
 // its kBlockPartialsMerged, the grid laid out (ringattn_steps.hip)
 hipError_t launch_steps(const BlockArgs& a, unsigned grid, int dtype, int dim, hipStream_t stream);
+// the same at d = 64 for launches that leave compute units idle, the ring steps apart (a.q_tiles_max counts tiles of kThinM rows)
+hipError_t launch_thin(BlockArgs a, int dtype, hipStream_t stream);
 // ring_walk64_kernel: the carried-state forward at d = 128 with 64 query rows per wave; only for tables that
 // walk64_takes() accepts
 hipError_t launch_walk64(BlockArgs a, int dtype, int dim, hipStream_t stream);

@@ -57,6 +57,49 @@
 
 namespace ringattn {
 
+static __device__ __forceinline__ float partial_lse(float l, float ms) {
+  return (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
+}
+// An entry of a normalised partial row as it is stored: as fp16 rounded twice, not by a fused multiply-and-convert.
+template <bool HP> static __device__ __forceinline__ float partial_entry(float x, float inv) {
+  float p = x * inv;
+  if (HP) {
+    asm("" : "+v"(p));
+    p = (float)(_Float16)p;
+  }
+  return p;
+}
+// A chunk's partial (csrc/ring_attention.cu:621-633) of a wave's 32 rows, the first of them row0 of the segment: normalised, with
+// its LSE, to the rows the item says.  l: the row sum of the lane's row.
+template <int D, bool HP>
+static __device__ __forceinline__ void store_partial(const BlockArgs& a, ItemPtr w, const f32x16 (&oacc)[D / 32], float l, float ms,
+                                                     int bh, int row0, int q_len) {
+  const int lane = threadIdx.x & 63, n = lane & 31, h = lane >> 5;
+  const float inv = (l > 0.f) ? 1.f / l : 0.f;
+  if constexpr (HP) {  // fp16 partials: |O_part| <= max |V|, the caller vouches that this fits
+    const int step = w->part_row_mul > 0 ? w->part_row_mul : 1;  // n: a row's steps next to each other
+    const int64_t prow = (w->part_base + (int64_t)bh * w->part_bh_stride + row0) * step + (w->part_row_mul > 0 ? w->slot : 0);
+    store_block<0, D>(oacc, inv, (char*)a.o_part + prow * (D * 2), (int64_t)step * (D * 2), q_len - row0);
+    if (h == 0 && row0 + n < q_len) a.lse_part[prow + (int64_t)n * step] = partial_lse(l, ms);
+    return;
+  }
+  // fp32 rows come out 32 bytes at a time as they are; with store_block's 64 a forward over many chunks of a few tiles
+  // (ranks of 32 to 192 tokens, d = 64) measured 127 -> 133 us, longer chunks the same
+  if (row0 + n >= q_len) return;  // a row beyond the query range
+  int64_t prow = w->part_base + (int64_t)bh * w->part_bh_stride + row0 + n;
+  if (w->part_row_mul > 0) prow = prow * w->part_row_mul + w->slot;  // a row's steps next to each other
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      f32x4 val;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) val[e] = oacc[db][4 * q4 + e] * inv;
+      *(f32x4*)((float*)a.o_part + prow * D + 32 * db + 8 * q4 + 4 * h) = val;
+    }
+  if (h == 0) a.lse_part[prow] = partial_lse(l, ms);
+}
+
 // LDS of a workgroup: K ring, V ring; and at d = 128 with the steps merged as they come half of the rows' merged O (64 of the
 // 128 columns of 256 rows as fp32; the other half takes 32 registers a lane, which with the 32 of this half would not
 // fit).  (Where partials are stored at d = 64 half of it lies idle: two workgroups a compute unit, by their registers.)
@@ -374,37 +417,6 @@ static __device__ __forceinline__ void walk_rows(const BlockArgs& a, unsigned ch
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   };
-  // a chunk's partial (csrc/ring_attention.cu:621-633): normalise, emit O and LSE
-  auto emit_partial = [&](ItemPtr w) {
-    const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
-    const float inv = (l > 0.f) ? 1.f / l : 0.f;
-    if constexpr (HP) {  // fp16 partials: |O_part| <= max |V|, the caller vouches that this fits
-      const int row0 = qt * BM + 32 * wave;
-      const int step = w->part_row_mul > 0 ? w->part_row_mul : 1;  // n: a row's steps next to each other
-      const int64_t prow = (w->part_base + (int64_t)bh * w->part_bh_stride + row0) * step + (w->part_row_mul > 0 ? w->slot : 0);
-      store_block<0, D>(oacc, inv, (char*)a.o_part + prow * (D * 2), (int64_t)step * (D * 2), q_len - row0);
-      if (h == 0 && row0 + n < q_len)
-        a.lse_part[prow + (int64_t)n * step] = (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
-      return;
-    }
-    // fp32 rows come out 32 bytes at a time as they are; with store_block's 64 a forward over many chunks of a few tiles
-    // (ranks of 32 to 192 tokens, d = 64) measured 127 -> 133 us, longer chunks the same
-    const int row_l = qt * BM + 32 * wave + n;
-    if (row_l >= q_len) return;  // a row beyond the query range
-    int64_t prow = w->part_base + (int64_t)bh * w->part_bh_stride + row_l;
-    if (w->part_row_mul > 0) prow = prow * w->part_row_mul + w->slot;  // a row's steps next to each other
-    const int64_t opos = prow * D;
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        f32x4 val;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) val[e] = oacc[db][4 * q4 + e] * inv;
-        *(f32x4*)((float*)a.o_part + opos + 32 * db + 8 * q4 + 4 * h) = val;
-      }
-    if (h == 0) a.lse_part[prow] = (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
-  };
   // MERGE: partials that are stored and read back at the end of the workgroup cost, of 10.7 ms (64 heads x 32 x 512 tokens, d = 128, fp16
   // partials), 1.0 for the stores and 1.2 for the merge; merged on the spot that forward takes 8.45 ms (fp32 partials, 16 heads x
   // 32 x 256: 1366 -> 543 us; d = 64: 715 -> 381).  The result of this lane's row so far, in acc-O's places: a reference, the sum of the weights against it, and the
@@ -423,20 +435,11 @@ static __device__ __forceinline__ void walk_rows(const BlockArgs& a, unsigned ch
   }
   auto merge_partial = [&]() {
     const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
-    const float inv = (l > 0.f) ? 1.f / l : 0.f;
-    const float L = (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
+    const float inv = (l > 0.f) ? 1.f / l : 0.f, L = partial_lse(l, ms);
     if (L == -INFINITY) return;  // the identity
     float keep, w;
     mst.weigh(L, keep, w);
-    // the entry of the partial row as it would be stored: as fp16 rounded twice, not by a fused multiply-and-convert
-    auto part = [&](float x) {
-      float p = x * inv;
-      if (HP) {
-        asm("" : "+v"(p));
-        p = (float)(_Float16)p;
-      }
-      return p;
-    };
+    auto part = [&](float x) { return partial_entry<HP>(x, inv); };
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -634,7 +637,7 @@ static __device__ __forceinline__ void walk_rows(const BlockArgs& a, unsigned ch
         __syncthreads();
         synced = true;
       }
-      emit_partial(w);
+      store_partial<D, HP>(a, w, oacc, cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3])), ms, bh, qt * BM + 32 * wave, q_len);
       reset_state();
     }
   };
@@ -665,7 +668,7 @@ static __device__ __forceinline__ void walk_rows(const BlockArgs& a, unsigned ch
     } else {
       const float l = cross_half_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
       inv = (l > 0.f) ? 1.f / l : 0.f;
-      out_lse = (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
+      out_lse = partial_lse(l, ms);
 #pragma unroll
       for (int db = 0; db < DB; ++db) res[db] = oacc[db];
     }
