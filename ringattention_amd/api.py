@@ -24,14 +24,28 @@ FLAG_ROW_PARTIALS = 16
 LAYOUT_CODE = {"contiguous": 0, "zigzag": 1}
 
 
+# What a call costs besides its launch counts: a ring of some hundred tokens is a few microseconds of GPU work.  So the checks take
+# one look per tensor and describe what is wrong in a second one, shapes are a plan's own, addresses go to ctypes as they are
+# (every pointer argument is declared c_void_p), and the current stream is asked for without making an object of it.  us a call
+# of forward() on the host, before and after: 10.5, 6.3.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr(stream=None):
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+def _fits(t, dtype, shape):
+    """What _check_tensors checks, without saying what is wrong."""
+    return t.shape == shape and t.dtype == dtype and t.is_cuda and t.is_contiguous()
 
 
 def _check_meta(t, name, dtype=None, shape=None):
@@ -109,6 +123,10 @@ class RingAttention:
                                   | (FLAG_STEP_PARTIALS if step_partials else 0)
                                   | (FLAG_ROW_PARTIALS if row_partials else 0), kv_heads,
                                   LAYOUT_CODE[layout])
+        b, h, hkv, d = batch, heads, self.kv_heads, dim
+        self._q_shape, self._kv_shape, self._lse_shape = (b, h, self.seq, d), (b, hkv, self.seq, d), (b, h, self.seq)
+        # of one rank's rows
+        self._rank_shapes = [((b, h, n, d), (b, hkv, n, d), (b, h, n)) for n in self.seqlen]
         self.handle = ctypes.c_void_p()
         ws_ptr, ws_bytes = (None, 0) if workspace is None else (ctypes.c_void_p(int(workspace[0])), int(workspace[1]))
         check(self.lib.ringattn_plan_create(ctypes.byref(self.params), ws_ptr, ws_bytes, ctypes.byref(self.handle)),
@@ -148,14 +166,17 @@ class RingAttention:
                 (v, "v", self.torch_dtype, kv_shape)]
 
     def forward(self, q, k, v, out=None, lse=None, stream=None):
-        _check_tensors(*self._qkv_specs(q, k, v))
+        dtype, kv_shape = self.torch_dtype, self._kv_shape
+        if not (_fits(q, dtype, self._q_shape) and _fits(k, dtype, kv_shape) and _fits(v, dtype, kv_shape)):
+            _check_tensors(*self._qkv_specs(q, k, v))
         if out is None:
             out = torch.empty_like(q)
         if lse is None:
-            lse = torch.empty(self._shape()[:3], dtype=torch.float32, device=q.device)
-        _check_tensors((out, "out", self.torch_dtype, self._shape()), (lse, "lse", torch.float32, self._shape()[:3]))
-        check(self.lib.ringattn_fwd(self.handle, _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _stream_ptr(stream)),
-              "ringattn_fwd")
+            lse = torch.empty(self._lse_shape, dtype=torch.float32, device=q.device)
+        if not (_fits(out, dtype, self._q_shape) and _fits(lse, torch.float32, self._lse_shape)):
+            _check_tensors((out, "out", dtype, self._shape()), (lse, "lse", torch.float32, self._shape()[:3]))
+        check(self.lib.ringattn_fwd(self.handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
+                                    _stream_ptr(stream)), "ringattn_fwd")
         return out, lse
 
     def block_forward(self, step, q, k, v, o_part=None, lse_part=None, stream=None):
@@ -181,24 +202,27 @@ class RingAttention:
         o_part and lse_part are the rank's whole [B, H, rows, npes, d] / [B, H, rows, npes] buffers at every step."""
         if not (0 <= rank < self.npes and 0 <= step < self.npes):
             raise ValueError("rank and step must be in [0, npes)")
-        rows, kv_rows = self.seqlen[rank], self.seqlen[(rank + step) % self.npes]
-        o_shape, l_shape = (self.batch, self.heads, rows, self.dim), (self.batch, self.heads, rows)
+        q_shape, _, l_shape = self._rank_shapes[rank]
+        o_shape = q_shape
+        kv_shape = self._rank_shapes[(rank + step) % self.npes][1]
         if self.row_partials:
             o_shape, l_shape = self.rank_parts_shapes(rank)
-        specs = [(q, "q", self.torch_dtype, (self.batch, self.heads, rows, self.dim)),
-                 (k_chunk, "k_chunk", self.torch_dtype, (self.batch, self.kv_heads, kv_rows, self.dim)),
-                 (v_chunk, "v_chunk", self.torch_dtype, (self.batch, self.kv_heads, kv_rows, self.dim))]
-        if o_part is not None:
-            specs.append((o_part, "o_part", self.part_dtype, o_shape))
-        if lse_part is not None:
-            specs.append((lse_part, "lse_part", torch.float32, l_shape))
-        _check_tensors(*specs)
+        dtype = self.torch_dtype
+        if not (_fits(q, dtype, q_shape) and _fits(k_chunk, dtype, kv_shape) and _fits(v_chunk, dtype, kv_shape)
+                and (o_part is None or _fits(o_part, self.part_dtype, o_shape))
+                and (lse_part is None or _fits(lse_part, torch.float32, l_shape))):
+            specs = [(q, "q", dtype, q_shape), (k_chunk, "k_chunk", dtype, kv_shape), (v_chunk, "v_chunk", dtype, kv_shape)]
+            if o_part is not None:
+                specs.append((o_part, "o_part", self.part_dtype, o_shape))
+            if lse_part is not None:
+                specs.append((lse_part, "lse_part", torch.float32, l_shape))
+            _check_tensors(*specs)
         if o_part is None:
             o_part = torch.zeros(o_shape, dtype=self.part_dtype, device=q.device)
         if lse_part is None:
             lse_part = torch.full(l_shape, float("-inf"), dtype=torch.float32, device=q.device)
-        check(self.lib.ringattn_rank_step_fwd(self.handle, int(rank), int(step), _ptr(q), _ptr(k_chunk), _ptr(v_chunk),
-                                              _ptr(o_part), _ptr(lse_part), _stream_ptr(stream)), "ringattn_rank_step_fwd")
+        check(self.lib.ringattn_rank_step_fwd(self.handle, int(rank), int(step), q.data_ptr(), k_chunk.data_ptr(), v_chunk.data_ptr(),
+                                              o_part.data_ptr(), lse_part.data_ptr(), _stream_ptr(stream)), "ringattn_rank_step_fwd")
         return o_part, lse_part
 
     def rank_merge(self, rank, o_parts, lse_parts, out=None, lse=None, stream=None):
@@ -305,6 +329,10 @@ def _check_rank_call(q, k, v, out, lse, npes, mype, seqlen, dim):
     if len(seqlen) != npes or not 0 <= mype < npes:
         raise ValueError("seqlen must hold npes lengths and mype must be in [0, npes)")
     rows, total = int(seqlen[mype]), int(sum(seqlen))
+    dtype = q.dtype
+    if (_fits(q, dtype, (rows, dim)) and _fits(k, dtype, (total, dim)) and _fits(v, dtype, (total, dim))
+            and _fits(out, dtype, (rows, dim)) and (lse is None or _fits(lse, torch.float32, (rows,)))):
+        return
     specs = [(q, "q", None, (rows, dim)), (k, "k", q.dtype, (total, dim)), (v, "v", q.dtype, (total, dim)),
              (out, "out", q.dtype, (rows, dim))]
     if lse is not None:
