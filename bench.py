@@ -34,10 +34,10 @@ PEAK_HBM_GBS = 8000.0
 # (bytes, summary under profiles/, kernel, kernel_source_id(kernel) when it was measured).  The figure is only printed
 # while the forward still runs that kernel and its source is still the one that was profiled.
 MEASURED_TRAFFIC = {
-    "cfg4": (2336e6, "profiles/ring_walk64_kernel_cfg4.md", "ring_walk64_kernel", "5b8957e9240ce0ad"),
-    "cfg3": (1623e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "5b8957e9240ce0ad"),
-    "cfg5": (41862e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "5b8957e9240ce0ad"),
-    "cfg2": (34.2e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "5b8957e9240ce0ad"),
+    "cfg4": (2280e6, "profiles/ring_walk64_kernel_cfg4.md", "ring_walk64_kernel", "fb6cfad5d7b6f313"),
+    "cfg3": (1623e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "fb6cfad5d7b6f313"),
+    "cfg5": (47323e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "fb6cfad5d7b6f313"),
+    "cfg2": (34.3e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "fb6cfad5d7b6f313"),
 }
 KERNEL_SOURCES = {
     "ring_walk64_kernel": ("ringattn_walk64.hip", "ringattn_walk64_loop.inc", "ringattn_walk64_loop_d64.inc", "ringattn_device.h"),

@@ -14,7 +14,7 @@
 //       has the QK^T product and the softmax; two (d = 64: four) waves per SIMD overlap one another's matrix and vector
 //       phases without any coordination.
 //       What bounds it: a K/V tile fetched from L2 feeds 32 query rows instead of 256, and a compute unit takes in 46 (d = 64) to
-//       50 (d = 128) of the 64 bytes per clock that its path to L2 carries.  A full device reaches 730 TFLOP/s at d = 128 and
+//       50 (d = 128) of the 64 bytes per clock that its path to L2 carries (34 with all of them busy).  A full device reaches 730 TFLOP/s at d = 128 and
 //       690 at d = 64 (ring_walk64_kernel 1260 and 940), so this kernel is for launches that leave it compute units idle: the
 //       host weighs the kernels (carry_kernel in ringattn_api.hip).  Up to there it was the instructions around a tile: with
 //       the next tile's place worked out by a search through the ranges in registers, an M0 write and a base address per 1 KB
