@@ -168,6 +168,7 @@ __global__ __launch_bounds__(256, 2) void ring_walk_kernel(const BlockArgs a) {
     s16x8 kfr[KS];  // the K fragments of tile u+1
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) kfr[ks] = *(const s16x8*)(smem + TILE + koff[ks]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // tile 0 is in registers: its place is given away behind the first barrier
 
     auto iteration = [&](auto slot_c, auto first_c, int u) {
       constexpr int SLOT = decltype(slot_c)::value;      // u mod NBUF
