@@ -397,12 +397,14 @@ static CarryKernel carry_kernel(const CarryCosts& c, int dim, bool wide) {
     if (t < best) best = t, kernel = CarryKernel::kPair;
   }
   if (split != 0 && carry_time(c.thin, r[2], false) < best) kernel = CarryKernel::kSplit;
-  // At d = 64 two workgroups of ring_split_kernel fit on a compute unit.  A launch that leaves half of the compute units idle
-  // may as well fill that place with waves of the same workgroup, sixteen of them instead of eight, where the walk
-  // is long enough to pay for the combination of twice the states.  us with eight and with sixteen waves, at 64, 128, 256
-  // and 512 tiles: 2048 rows 11.3, 12.9; 4096 rows, causal 15.1, 16.6; 8192 rows 30.8, 31.6; 2048, 4096 and 8192 rows x 16384
-  // keys 44.1, 41.8; 43.9, 42.0; 53.7, 55.3.
-  if (kernel == CarryKernel::kSplit && dim == 64 && 2 * c.thin.jobs <= kComputeUnits && c.thin.tiles >= 384)
+  // At d = 64 two workgroups of ring_split_kernel fit on a compute unit.  A launch of no more workgroups than there are compute
+  // units fills the other half with waves of the same workgroup, sixteen of them instead of eight, where the walk has 96
+  // tiles or more.  A row's keys then meet twice as many references, and its probabilities are rounded closer: relative error of
+  // O against float64, eight and sixteen waves, 48 calls of 96 to 500 tiles, fp16 2.79e-4, 2.76e-4 (N(0, 1) logits) and 2.34e-4,
+  // 2.24e-4 (N(0, 81)), bf16 2.23e-3, 2.21e-3 and 1.85e-3, 1.77e-3.  That is what draws the line, not the time, us: 4096 rows x
+  // 4096 keys 15.0, 16.7; 8192 x 8192 28.4, 30.3, causal 24.3, 24.8; 8192 x 16384 53.3, 54.4; 4096 x 16384 43.5, 42.0; 2048 x 16384 42.6,
+  // 41.3; the last three with N(0, 81) logits 56.2, 55.9; 48.0, 44.2; 47.1, 43.4.
+  if (kernel == CarryKernel::kSplit && dim == 64 && c.thin.jobs <= kComputeUnits && c.thin.tiles >= 96)
     kernel = CarryKernel::kSplit16;
   return kernel;
 }

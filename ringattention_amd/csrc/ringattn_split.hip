@@ -21,7 +21,7 @@
 //       piece, and the choice to move the references in scalar logic, a tile cost a wave 100 scalar and 93 vector instructions
 //       and some twenty branches.  Now a tile's place is a count that only the end of a range sends to the table, pieces within
 //       4 KB share M0 and address, and the first score of a row overflows into the branch that moves its reference.  us before and
-//       after: d = 64, 8192 rows x 16384 keys 58.2 -> 53.7, 2048 x 16384 48.5 -> 42, 4096 x 4096 causal 18.7 -> 15.1, 8 heads x 4096 causal
+//       after: d = 64, 8192 rows x 16384 keys 60.2 -> 54.4, 2048 x 16384 48.5 -> 41.3, 4096 x 4096 causal 18.3 -> 16.4, 8 heads x 4096 causal
 //       36 -> 33.5; d = 128, 8192 x 8192 57 -> 53, 4096 x 4096 causal 27 -> 22.3, 512 x 2048 causal 16.6 -> 14.3, 8 heads x 2048 34 -> 31.
 #include "ringattn_device.h"
 

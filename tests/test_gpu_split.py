@@ -10,6 +10,7 @@ import torch
 from ringattention_amd import api
 from ringattention_amd.configs import Workload
 from test_gpu_parity import check_rows
+from launched import launched
 from test_gpu_walk64 import rising_logits
 from test_kernel_resources import test_no_lds_transfer_reads_a_scalar_register_fresh_from_a_vector_instruction as _hazards
 from test_kernel_resources import compile_to_asm
@@ -72,7 +73,70 @@ def test_split_kernel_with_sixteen_waves(oracle, monkeypatch, lens, B, H, hkv, d
         monkeypatch.delenv(name, raising=False)
     if forced:
         monkeypatch.setenv("RINGATTN_SPLIT", "16")
+    else:
+        plan = api.RingAttention(len(lens), list(lens), 64, B, H, dtype, causal, kv_heads=hkv)
+        x, kv = (torch.zeros(B, h, sum(lens), 64, dtype=torch.float16, device="cuda") for h in (H, hkv))
+        out, lse = torch.empty_like(x), torch.empty(B, H, sum(lens), device="cuda")
+        assert launched(lambda stream: plan.forward(x, kv, kv, out, lse, stream)) == [(1024, 0)]
+        plan.close()
     check_forward(oracle, lens, B, H, hkv, dtype, causal, zigzag, slope, 64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,rank,causal,waves", [
+    ((3137,), 0, True, 16),          # 99 tiles
+    ((3072,), 0, False, 16),         # 96
+    ((3040,), 0, False, 8),          # 95
+    ((8192, 8192), 0, False, 16),    # 256 workgroups
+    ((333, 11968), 0, False, 16),    # 385 tiles, the last of 13 keys
+    ((12000, 300), 1, True, 16),     # 385 tiles, diagonal in the last ten
+])
+def test_how_many_waves_share_the_keys(oracle, monkeypatch, lens, rank, causal, waves):
+    """d = 64: sixteen waves where a launch leaves no compute unit a second workgroup and the walk has 96 tiles or more.  The keys of
+    a row then meet sixteen references instead of eight: the result is bit for bit that of the switch that asks for as many
+    waves, and another than that of the other number."""
+    for name in ("RINGATTN_WIDE", "RINGATTN_WIDE_D64", "RINGATTN_WIDE_PARTIALS", "RINGATTN_SPLIT", "RINGATTN_PAIR"):
+        monkeypatch.delenv(name, raising=False)
+    d, S, first, rows = 64, sum(lens), sum(lens[:rank]), lens[rank]
+    w = Workload("waves", 1, 1, d, 1, S, "fp16", 4000 + S, causal)
+    bits = api.make_qkv_bits(w)
+    q, k, v = (api.bits_to_tensor(np.ascontiguousarray(x[0, 0]), w.dtype) for x in bits)
+    q = q[first:first + rows].contiguous()
+    out, lse = torch.zeros(S, d, dtype=q.dtype, device="cuda"), torch.zeros(S, device="cuda")
+
+    def call(stream=None):
+        api.ring_attention_noalloc(q, k, v, out[first:first + rows], len(lens), rank, lens, d, max(lens), lse=lse[first:first + rows],
+                                   causal=causal, stream=stream)
+
+    def result():
+        call()
+        torch.cuda.synchronize()
+        return out.clone(), lse.clone()
+
+    assert launched(call) == [(64 * waves, 0)]
+    got, results = result(), {}
+    for n in (8, 16):
+        monkeypatch.setenv("RINGATTN_SPLIT", str(n))
+        assert launched(call) == [(64 * n, 0)]
+        results[n] = result()
+    assert torch.equal(got[0], results[waves][0]) and torch.equal(got[1], results[waves][1])
+    assert not torch.equal(got[0], results[24 - waves][0])
+    some = first + np.unique(np.concatenate([np.arange(0, rows, max(1, rows // 100)), [rows - 1]]))
+    check_rows(oracle, w, *bits, *got, some)
+
+
+@pytest.mark.gpu
+def test_eight_waves_where_two_workgroups_share_a_compute_unit(monkeypatch):
+    for name in ("RINGATTN_WIDE", "RINGATTN_WIDE_D64", "RINGATTN_WIDE_PARTIALS", "RINGATTN_SPLIT", "RINGATTN_PAIR"):
+        monkeypatch.delenv(name, raising=False)
+    plan = api.RingAttention(1, 4096, 64, 1, 8, "fp16", True)   # 128 tiles, 1024 workgroups
+    try:
+        x = torch.zeros(1, 8, 4096, 64, dtype=torch.float16, device="cuda")
+        out, lse = torch.empty_like(x), torch.empty(1, 8, 4096, device="cuda")
+        assert plan.forward_kernel() == "ring_split_kernel"
+        assert launched(lambda stream: plan.forward(x, x, x, out, lse, stream)) == [(512, 0)]
+    finally:
+        plan.close()
 
 
 def test_split_kernel_resources_and_hazards(tmp_path):
