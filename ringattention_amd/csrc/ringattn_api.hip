@@ -264,7 +264,7 @@ static void add_walks(WalkCost& c, const ringattn::Segment& seg, int rows, int64
 // (A range may reach beyond that: the loops add whole tiles to 64-bit addresses.)
 static bool begins_within_4g(const ringattn::SegItem& it, int dim) { return ((int64_t)it.kv_start + 32) * 2 * dim <= UINT32_MAX; }
 
-constexpr int kComputeUnits = 256;
+using ringattn::kComputeUnits;
 struct CarryCosts {
   WalkCost whole, halves, thin;  // with q tiles of kWalkM, kPairM and kSplitM rows
   bool pair = true;              // every segment suits ring_pair_kernel
@@ -291,6 +291,7 @@ struct TableSlice {
   int q_len_max = 0;    // rows of the longest segment
   bool wide = false;    // every KV range of the slice suits ring_walk64_kernel
   int min_kv = 0;       // the shortest KV range of the slice
+  ringattn::Walks walks;
   CarryCosts costs;     // pl->walk only
 };
 
@@ -505,6 +506,14 @@ void push_segment(ringattn_plan* pl, TableSlice& slice, int q_start, int q_len,
   bool wide = true;
   for (size_t i = 0; i < items.size(); ++i) wide = wide && walk64_takes(pl->h_segitems[(size_t)sg.item_begin + i], pl->p.dim);
   slice.wide = slice.seg_count == 0 ? wide : (slice.wide && wide);
+  int keys = 0;
+  for (const auto& w : items) {
+    keys += (w.kv_len + 31) / 32;
+    if (w.diag_off >= 0) slice.walks.masked = slice.walks.uneven = true;
+  }
+  if (slice.seg_count > 0 && keys != slice.walks.longest) slice.walks.uneven = true;
+  slice.walks.longest = std::max(slice.walks.longest, keys);
+  slice.walks.tiles += q_tiles_of(q_len);
   for (size_t i = 0; i < items.size(); ++i) {
     const int kv = pl->h_segitems[(size_t)sg.item_begin + i].kv_len;
     slice.min_kv = (slice.seg_count == 0 && i == 0) ? kv : std::min(slice.min_kv, kv);
@@ -690,7 +699,8 @@ bool in_arguments(const ringattn_plan* pl, const TableSlice& sl, int mode) {
 }
 
 // the launch of `kernel` over q tiles of its size; `wide`: kWhole is ring_walk64_kernel
-hipError_t launch_q_tiles(ringattn::BlockArgs& a, CarryKernel kernel, bool wide, int q_len, int dtype, int dim, hipStream_t stream) {
+hipError_t launch_q_tiles(ringattn::BlockArgs& a, CarryKernel kernel, bool wide, const ringattn::Walks& walks, int q_len, int dtype, int dim,
+                          hipStream_t stream) {
   switch (kernel) {
     case CarryKernel::kPair:
       a.q_tiles_max = q_tiles_of(q_len, ringattn::kPairM);
@@ -701,7 +711,7 @@ hipError_t launch_q_tiles(ringattn::BlockArgs& a, CarryKernel kernel, bool wide,
       return ringattn::launch_split(a, dtype, dim, kernel == CarryKernel::kSplit16, stream);
     default:
       a.q_tiles_max = q_tiles_of(q_len);
-      return wide ? ringattn::launch_walk64(a, dtype, dim, stream) : ringattn::launch_walk(a, dtype, dim, stream);
+      return wide ? ringattn::launch_walk64(a, dtype, dim, stream) : ringattn::launch_walk(a, walks, dtype, dim, stream);
   }
 }
 
@@ -727,7 +737,7 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
   }
   const CarryKernel kernel =
       a.mode == ringattn::kBlockCarryState ? carry_kernel(sl.costs, pl->p.dim, wide) : CarryKernel::kWhole;
-  RA_HIP(launch_q_tiles(a, kernel, wide, sl.q_len_max, pl->p.dtype, pl->p.dim, stream));
+  RA_HIP(launch_q_tiles(a, kernel, wide, sl.walks, sl.q_len_max, pl->p.dtype, pl->p.dim, stream));
   return RINGATTN_OK;
 }
 
@@ -833,7 +843,7 @@ int run_rank_call(const RankCall& rc, const void* q, const void* k, const void* 
   const bool wide = (dim == 128 || (dim == 64 && walk64_d64_enabled())) && walk64_enabled() && walk64_takes(rc.item, dim);
   CarryCosts costs;
   costs.add(rc.seg, 1, dim, [&](int) -> const ringattn::SegItem& { return rc.item; });
-  RA_HIP(launch_q_tiles(a, carry_kernel(costs, dim, wide), wide, c, rc.p.dtype, dim, stream));
+  RA_HIP(launch_q_tiles(a, carry_kernel(costs, dim, wide), wide, {}, c, rc.p.dtype, dim, stream));
   return RINGATTN_OK;
 }
 

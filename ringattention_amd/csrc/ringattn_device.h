@@ -107,17 +107,27 @@ static __device__ __forceinline__ SegPtr segs_of(const BlockArgs& a) {
   return a.items ? (SegPtr)(uintptr_t)a.segs : (SegPtr)(args + offsetof(BlockArgs, one_seg));
 }
 
+// An XCD hands its workgroups to its 32 compute units in turn.  Where a compute unit holds two, the first 32 jobs, longest walk first,
+// are the first ones of the compute units and the next 32 the second ones: those run shortest first (a.second_lap: how many
+// of the XCD's first 64 there are; 0: as they come), so that long walks share a compute unit with short ones.
+static __device__ __forceinline__ int lap_order(const BlockArgs& a, int w) {
+  constexpr int lap = kComputeUnits / kXcds;
+  return w >= lap && w < a.second_lap ? a.second_lap + lap - 1 - w : w;
+}
+
 // workgroup -> job (segment, head, q tile); false for the holes of the grid.  blockIdx mod 8 is the XCD.  Heads are dealt
 // to the XCDs round-robin, and an XCD runs the segments of a head one after the other (busiest first), the q tiles of a
 // segment as consecutive workgroups: everything that reads a head's K and V follows each other through that XCD's L2.
 // The batch * heads mod 8 heads that do not deal out evenly are shared: with rem of them, gcd(8, rem) sets of XCDs take
 // rem / gcd heads each and split their tiles round-robin, so that one head (or any number) still fills all XCDs.  The last
 // a.tail_heads heads of an XCD and its part of the shared ones are interleaved (job_grid says why).
-template <int TILE_ROWS>
+// LAPS: compute units hold two workgroups (lap_order).
+template <int TILE_ROWS, bool LAPS = false>
 static __device__ __forceinline__ bool decode_job(const BlockArgs& a, Segment& seg, int& bh, int& qt) {
   const int q_tiles = a.q_tiles_max;
   const int per_head = a.n_segs * q_tiles;
-  const int xcd = blockIdx.x & 7, w = blockIdx.x >> 3;
+  const int xcd = blockIdx.x & 7, place = blockIdx.x >> 3;
+  const int w = LAPS ? lap_order(a, place) : place;
   const int full = a.BH >> 3, rem = a.BH & 7;
   const int lead = (full - a.tail_heads) * per_head;
   int job;  // its number among those of its head

@@ -11,6 +11,7 @@ constexpr int kSplitM = 32;   // query rows per workgroup of ring_split_kernel
 constexpr int kPairM = 128;  // query rows per workgroup of ring_pair_kernel
 constexpr int kThinM = 128;  // query rows per workgroup of thin::ring_walk_kernel
 constexpr int kMaxParts = 64; // partial slots a merge can combine
+constexpr int kComputeUnits = 256, kXcds = 8;
 
 // One unit of block-attention work as the host layer lists it: the queries
 // [q_start, q_start + q_len) of every head against the keys/values
@@ -88,6 +89,7 @@ struct BlockArgs {
   int mode;            // BlockMode
   int causal;          // some item is masked
   int tail_heads;      // see job_grid
+  int second_lap;      // see lap_order in ringattn_device.h
   Segment one_seg;
   SegItem one_item;
 };
@@ -139,7 +141,14 @@ struct MergeArgs {
 };
 
 // dtype: 0 = fp16, 1 = bf16.  Return hipSuccess or the launch error.
-hipError_t launch_walk(BlockArgs a, int dtype, int dim, hipStream_t stream);  // ring_walk_kernel, any BlockMode
+// The walks of a launch, for what ring_walk_kernel makes of their number and lengths.
+struct Walks {
+  int tiles = 0;        // 256-row q tiles of a head that there are (the grid has as many for every segment)
+  int longest = 0;      // 32-key tiles of the longest
+  bool uneven = false;  // they differ in length
+  bool masked = false;  // ... by a causal diagonal, so that those of a segment come longest first
+};
+hipError_t launch_walk(BlockArgs a, const Walks& walks, int dtype, int dim, hipStream_t stream);  // ring_walk_kernel, any BlockMode
 // its kBlockPartialsMerged, the grid laid out (ringattn_steps.hip)
 hipError_t launch_steps(const BlockArgs& a, unsigned grid, int dtype, int dim, hipStream_t stream);
 // the same at d = 64 for launches that leave compute units idle, the ring steps apart (a.q_tiles_max counts tiles of kThinM rows)

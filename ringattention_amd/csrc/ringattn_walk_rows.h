@@ -134,7 +134,7 @@ static __device__ __forceinline__ void walk_rows(const BlockArgs& a, unsigned ch
 
   Segment seg;
   int bh, qt;
-  if (!decode_job<BM>(a, seg, bh, qt)) return;
+  if (!decode_job<BM, D == 64 && MODE == kBlockPartials>(a, seg, bh, qt)) return;
   const int q_start = seg.q_start, q_len = seg.q_len;
   const int n_items = seg.item_count;
   const ItemPtr items = items_of(a);
