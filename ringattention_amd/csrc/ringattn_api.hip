@@ -862,6 +862,10 @@ int launch_regions(const ringattn_plan* pl, int first, int count, int max_len, i
   m.heads = (int)pl->d.BH;
   m.S = rows_per_head;
   m.part_stride_rows = part_stride_rows;
+  for (int i = first; i < first + count; ++i) {
+    const ringattn::MergeRegion& reg = pl->regions[(size_t)i];
+    m.part_rows += (int64_t)m.heads * reg.len * __builtin_popcountll(reg.active);
+  }
   m.half_partials = half_partials(pl->p) ? 1 : 0;
   m.slot0_last = pl->p.causal ? 1 : 0;
   m.row_mul = row_partials(pl->p) ? pl->p.npes : 0;
@@ -1139,6 +1143,7 @@ int ringattn_merge(const float* o_parts, const float* lse_parts, int n_parts, in
     m.heads = 1;
     m.S = len;
     m.part_stride_rows = rows;
+    m.part_rows = (int64_t)len * n_parts;
     RA_HIP(ringattn::launch_merge(m, dtype, dim, (hipStream_t)stream));
   }
   return RINGATTN_OK;

@@ -135,6 +135,7 @@ struct MergeArgs {
   int heads;              // batch * heads: every region is merged for each of them
   int S;                  // rows per head
   int64_t part_stride_rows;  // rows between consecutive slots (>= heads * S)
+  int64_t part_rows;         // rows of partials the launch reads, all regions and slots together
   int half_partials;
   int slot0_last;         // 1: slot 0, the masked step of a causal plan, is merged after the others, as the attention kernels walk it
   int row_mul;            // 0: slot-major partials as above; n > 0: [heads * S, n, D] / [heads * S, n], a row's slots adjacent

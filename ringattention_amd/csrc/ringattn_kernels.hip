@@ -25,7 +25,7 @@ struct SlotParts {
   }
 };
 // This thread owns columns [8 c8, 8 c8 + 8) of the row.
-template <int DT, int D, bool HP, class Parts>
+template <int DT, int D, bool HP, bool AHEAD, class Parts>
 static __device__ __forceinline__ void merge_row(Parts p, const void* o_parts, const float* lse_parts,
                                                  void* out, float* lse, int64_t out_row, int c8) {
   const typename PartRow<HP>::ptr o_base = (typename PartRow<HP>::ptr)o_parts + c8 * 8;
@@ -43,15 +43,15 @@ static __device__ __forceinline__ void merge_row(Parts p, const void* o_parts, c
       acc[4 + e] = merge_in_part(acc[4 + e], keep, w, x1[e]);
     }
   };
-  // Two batches of four parts: one on its way while the other is merged.  With one pass over the parts and this, instead of a pass
-  // over the LSEs first and batches that were waited for, us: causal 32 heads x 8 x 4096, fp32 501 -> 493, fp16 297 -> 276, row-major 530 ->
-  // 523, d = 64 258 -> 252; 64 heads x 32 x 512, fp16 446 -> 420; 8 heads x 8 x 1024 49 -> 45.5.  (Batches of 1, 2 and 3: 520, 524, 510 in the
-  // first of these; one batch of four at a time 514, of eight 503.)
+  // Batches of four parts.  AHEAD: one on its way while another is merged, in 98 to 107 registers, for launches whose parts come from HBM;
+  // without it 60, and twice as many waves to wait for memory, for those whose parts the Infinity Cache may hold (launch_merge).
+  // 32 heads x 8 x 4096 under the causal mask, fp32 parts, us: batches of one, two, three and four ahead 520, 524, 510, 489, one of four at a
+  // time 518, of eight 503.
   constexpr int kBatch = 4;
   struct Batch {
     float L[kBatch];
     f32x4 x0[kBatch], x1[kBatch];
-  } even, odd;
+  } batch;
   const int n = p.left();
   auto fetch = [&](Batch& t, int first) {
 #pragma unroll
@@ -67,12 +67,21 @@ static __device__ __forceinline__ void merge_row(Parts p, const void* o_parts, c
     for (int u = 0; u < kBatch; ++u)
       if (first + u < n) merge_in(t.L[u], t.x0[u], t.x1[u]);
   };
-  fetch(even, 0);
-  for (int i = 0; i < n; i += 2 * kBatch) {
-    fetch(odd, i + kBatch);
-    merge_batch(even, i);
-    fetch(even, i + 2 * kBatch);
-    merge_batch(odd, i + kBatch);
+  if constexpr (AHEAD) {
+    Batch odd;
+    fetch(batch, 0);
+    for (int i = 0; i < n; i += 2 * kBatch) {
+      fetch(odd, i + kBatch);
+      merge_batch(batch, i);
+      fetch(batch, i + 2 * kBatch);
+      merge_batch(odd, i + kBatch);
+    }
+  } else {
+#pragma unroll 1
+    for (int i = 0; i < n; i += kBatch) {
+      fetch(batch, i);
+      merge_batch(batch, i);
+    }
   }
   const float inv = st.inverse();
 #pragma unroll
@@ -82,7 +91,7 @@ static __device__ __forceinline__ void merge_row(Parts p, const void* o_parts, c
 }
 
 // ---- merge ------------------------------------------------------------------------
-template <int DT, int D, bool HP>
+template <int DT, int D, bool HP, bool AHEAD>
 __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
   constexpr int TPR = D / 8;  // threads per row, 8 columns each
   constexpr int ROWS = 256 / TPR;
@@ -93,26 +102,38 @@ __global__ __launch_bounds__(256) void merge_kernel(const MergeArgs a) {
   // slot-major partials: slot s of a row lies part_stride_rows rows further on; row-major: at entry row_mul row + s
   const int first = a.slot0_last;
   SlotParts parts{first ? reg.active >> 1 | reg.active << 63 : reg.active, first, a.row_mul > 0 ? row * a.row_mul : row, a.row_mul > 0 ? (int64_t)1 : a.part_stride_rows};
-  merge_row<DT, D, HP>(parts, a.o_parts, a.lse_parts, a.out, a.lse, row, threadIdx.x % TPR);
+  merge_row<DT, D, HP, AHEAD>(parts, a.o_parts, a.lse_parts, a.out, a.lse, row, threadIdx.x % TPR);
 }
 
 // ---- host launchers -----------------------------------------------------------------
+// us with 60 registers and with a batch ahead, 8 ranks unless said, under the causal mask: fp32 partials, d = 128, 8 heads x 1024 (152 MB of
+// parts) 26.7, 27.3, 16 x 1024 (304 MB) 58.1, 59.1, 16 x 4096 (1.2 GB) 266, 246; d = 64, 8 x 2048 (153 MB) 27.1, 27.9, 16 x 4096 (613 MB) 132, 125;
+// fp16, d = 128, 8 heads x 4 x 2048 (43 MB) 10.9, 12.3, 16 x 3 x 5160 (129 MB) 30.3, 34.9, 3 x 11384 (320 MB) 72.7, 74.5, 32 x 4096 (1.2 GB) 297, 277;
+// no mask, 3 heads x 12 x 7312 (821 MB) 171, 163, 16 x 5 x 3352, causal (196 MB) 45.5, 53.1.  Between 256 and 512 MB either may be ahead.
+constexpr int64_t kMergeAheadBytes = (int64_t)256 << 20;
 hipError_t launch_merge(const MergeArgs& a, int dtype, int dim, hipStream_t stream) {
   if (a.n_regions <= 0 || a.max_len <= 0 || a.heads <= 0) return hipSuccess;
   const int rows_per_block = 256 / (dim / 8);
   const int64_t cols = ((int64_t)a.heads * a.max_len + rows_per_block - 1) / rows_per_block;
   if (cols > INT32_MAX || a.n_regions > 65535) return hipErrorInvalidValue;
   const dim3 grid((unsigned)cols, (unsigned)a.n_regions);
-#define RA_LAUNCH_MERGE(DT_, D_)                                                 \
-  do {                                                                        \
-    if (a.half_partials) merge_kernel<DT_, D_, true><<<grid, 256, 0, stream>>>(a);  \
-    else merge_kernel<DT_, D_, false><<<grid, 256, 0, stream>>>(a);                \
+  const bool ahead = a.part_rows * (dim * (a.half_partials ? 2 : 4) + (int64_t)sizeof(float)) > kMergeAheadBytes;
+#define RA_LAUNCH_MERGE_OF(DT_, D_, HP_)                                                     \
+  do {                                                                                      \
+    if (ahead) merge_kernel<DT_, D_, HP_, true><<<grid, 256, 0, stream>>>(a);                \
+    else merge_kernel<DT_, D_, HP_, false><<<grid, 256, 0, stream>>>(a);                     \
+  } while (0)
+#define RA_LAUNCH_MERGE(DT_, D_)                           \
+  do {                                                    \
+    if (a.half_partials) RA_LAUNCH_MERGE_OF(DT_, D_, true); \
+    else RA_LAUNCH_MERGE_OF(DT_, D_, false);               \
   } while (0)
   if (dtype == 0 && dim == 64) RA_LAUNCH_MERGE(0, 64);
   else if (dtype == 0 && dim == 128) RA_LAUNCH_MERGE(0, 128);
   else if (dtype == 1 && dim == 64) RA_LAUNCH_MERGE(1, 64);
   else if (dtype == 1 && dim == 128) RA_LAUNCH_MERGE(1, 128);
 #undef RA_LAUNCH_MERGE
+#undef RA_LAUNCH_MERGE_OF
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

@@ -24,6 +24,15 @@ def _hip():
 
 def launched(call):
     """(threads per workgroup, bytes of dynamic LDS) of every kernel that call(stream) launches on the stream, in order."""
+    return [(p.block.x, p.shared) for p in _nodes(call)]
+
+
+def kernels(call):
+    """What tells the kernels of call(stream) apart, in order."""
+    return [p.func for p in _nodes(call)]
+
+
+def _nodes(call):
     hip = _hip()
 
     def ok(code):
@@ -31,7 +40,7 @@ def launched(call):
 
     stream, graph = torch.cuda.Stream(), ctypes.c_void_p()
     torch.cuda.synchronize()
-    ok(hip.hipStreamBeginCapture(ctypes.c_void_p(stream.cuda_stream), 1))   # hipStreamCaptureModeThreadLocal
+    ok(hip.hipStreamBeginCapture(ctypes.c_void_p(stream.cuda_stream), 2))   # hipStreamCaptureModeRelaxed: outputs may be allocated
     try:
         call(stream)
     finally:
@@ -48,7 +57,7 @@ def launched(call):
             assert kind.value == 0   # hipGraphNodeTypeKernel
             p = _KernelNodeParams()
             ok(hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)))
-            found.append((p.block.x, p.shared))
+            found.append(p)
     finally:
         ok(hip.hipGraphDestroy(graph))
     return found
