@@ -85,7 +85,7 @@ static __device__ __forceinline__ void merge_row(Parts p, const void* o_parts, c
   }
   const float inv = st.inverse();
 #pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] *= inv;
+  for (int e = 0; e < 8; ++e) acc[e] = inv == 0.f ? 0.f : acc[e] * inv;  // (0: no finite LSE, but perhaps a NaN, which is in the sums)
   Store8<DT>::st((char*)out + (out_row * D + c8 * 8) * 2, acc);
   if (c8 == 0) lse[out_row] = st.lse();
 }

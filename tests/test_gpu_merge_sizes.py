@@ -53,3 +53,24 @@ def test_merge_of_all_ranks_and_of_one(half, rows_first, d):
         if rank == 0:
             assert kernels(lambda s: plan.merge_ring(o, l, out, lse, s)) != kernels(lambda s: plan.rank_merge(0, o_r, l_r, out_r, lse_r, s))
     plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+def test_rows_whose_lses_are_no_numbers(d):
+    """A row without any finite LSE has seen nothing: O = 0, LSE = -inf, whether its LSEs are -inf or NaN; one NaN next to a finite LSE
+    makes both NaN, whichever comes first."""
+    inf, nan = float("inf"), float("nan")
+    nothing = [(-inf, -inf, -inf), (nan, nan, nan), (nan, -inf, nan), (-inf, nan, -inf)]
+    broken = [(nan, 0.5, 0.25), (0.5, nan, -inf), (-inf, 0.5, nan), (nan, -inf, 0.5)]
+    l = torch.tensor(nothing + broken, device="cuda").T.contiguous()
+    o = torch.randn(3, 8, d, device="cuda")
+    plan = api.RingAttention(3, [8, 2, 2], d, 1, 1, "fp16")   # (the rows of its first rank)
+    o_parts, l_parts = torch.zeros(3, 1, 1, 12, d, device="cuda"), torch.zeros(3, 1, 1, 12, device="cuda")
+    o_parts[:, 0, 0, :8], l_parts[:, 0, 0, :8] = o, l
+    ring = [x[0, 0, :8] for x in plan.merge_ring(o_parts, l_parts)]
+    rank = [x[0, 0] for x in plan.rank_merge(0, o[:, None, None].contiguous(), l[:, None, None].contiguous())]
+    for out, lse in (api.merge(o, l, "fp16"), ring, rank):
+        assert bool((out[:4] == 0).all()) and bool((lse[:4] == -inf).all())
+        assert bool(out[4:].isnan().all()) and bool(lse[4:].isnan().all())
+    plan.close()
