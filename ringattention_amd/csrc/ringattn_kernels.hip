@@ -85,7 +85,10 @@ static __device__ __forceinline__ void merge_row(Parts p, const void* o_parts, c
   }
   const float inv = st.inverse();
 #pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = inv == 0.f ? 0.f : acc[e] * inv;  // (0: no finite LSE, but perhaps a NaN, which is in the sums)
+  for (int e = 0; e < 8; ++e) {
+    if (inv == 0.f) acc[e] = 0.f;  // no finite LSE, but perhaps a NaN, which is in the sums
+    acc[e] *= inv;  // (the last thing before the store: product and conversion are one rounding in every merge)
+  }
   Store8<DT>::st((char*)out + (out_row * D + c8 * 8) * 2, acc);
   if (c8 == 0) lse[out_row] = st.lse();
 }
