@@ -102,8 +102,8 @@ static __device__ __forceinline__ void store_partial(const BlockArgs& a, ItemPtr
 
 // LDS of a workgroup: K ring, V ring; and at d = 128 with the steps merged as they come half of the rows' merged O (64 of the
 // 128 columns of 256 rows as fp32; the other half takes 32 registers a lane, which with the 32 of this half would not
-// fit).  (Where partials are stored at d = 64 half of it lies idle: two workgroups a compute unit, by their registers.)
-template <int D, int MODE> constexpr int kWalkLds = MODE == kBlockCarryState ? 512 * D : MODE == kBlockPartials || D == 64 ? 65536 : 131072;
+// fit).
+template <int D, int MODE> constexpr int kWalkLds = 512 * D + (MODE == kBlockPartialsMerged && D == 128 ? 65536 : 0);
 
 // MODE: the softmax state is carried through the chunks (kBlockCarryState), or a partial is formed per chunk and stored
 // (kBlockPartials) or merged into the rows' result (kBlockPartialsMerged); HP: partial O rounded to fp16.
@@ -125,7 +125,7 @@ static __device__ __forceinline__ void walk_rows(const BlockArgs& a, unsigned ch
   static_assert(BM == 32 * WAVES, "one 32-row block per wave");
   static_assert(PIECES == WAVES || 2 * PIECES == WAVES, "a tile is loaded by all waves, or K and V by half of them each");
   constexpr int kRingBytes = 2 * NBUF * TILE;
-  static_assert(kRingBytes + (MERGE && D == 128 ? 64 * BM * 4 : 0) <= kWalkLds<D, MODE>, "rings and merged columns");
+  static_assert(kRingBytes + (MERGE && D == 128 ? 64 * BM * 4 : 0) == kWalkLds<D, MODE>, "rings and merged columns");
 
   const unsigned smem_base = lds_offset(smem);
   const int tid = threadIdx.x, lane = tid & 63;

@@ -1,8 +1,8 @@
-"""What the compiler made of the attention kernel: every instantiation must fit two waves per
-SIMD (256 registers), the carried-state ones without scratch memory, and the steady key loops of
-the d = 128 ones -- the loops that hold 64 MFMAs, four 32-key blocks -- must carry one barrier per
-two tiles and no scratch access.
-Compiles the kernel to assembly for gfx950; needs hipcc but no GPU."""
+"""What the compiler made of the attention kernels: every instantiation must fit two waves per
+SIMD (256 registers) without scratch memory in its loops, and the steady key loops of the d = 128
+ones -- the loops that hold 64 MFMAs, four 32-key blocks -- must carry one barrier per two tiles and
+read their fragments ahead of the MFMAs.
+Compiles the kernels to assembly for gfx950; needs hipcc but no GPU."""
 import os
 import re
 import shutil
@@ -74,6 +74,21 @@ def steady_loops(asm, kernel):
     return [(lab, ins) for lab, ins in loops_of(asm[start:end]) if sum(i.startswith("v_mfma") for i in ins) == 64]
 
 
+def body_of(asm, kernel):
+    start = asm.index("\n" + kernel + ":")
+    return asm[start:asm.index(".amdhsa_kernel " + kernel, start)]
+
+
+def check_steady_loops(asm, n, barriers):
+    """The four loops of a d = 128 instantiation: plain and masked groups, for each half of the workgroup."""
+    steady = steady_loops(asm, n)
+    assert len(steady) == 4, (n, len(steady))
+    for lab, ins in steady:
+        assert sum(i.startswith("s_barrier") for i in ins) in barriers, (n, lab)   # one per two tiles
+        # fragments are read six and more ahead: a wait for the last read comes at the end of a phase and not at every MFMA
+        assert sum(bool(re.match(r"s_waitcnt .*lgkmcnt\(0\)", i)) for i in ins) <= 12, (n, lab)
+
+
 def test_walk_kernel_runs_two_waves_per_simd_without_spills(tmp_path):
     asm, usage = compile_to_asm("ringattn_walk.hip", tmp_path / "walk.s")
     walks = {n: u for n, u in usage.items() if "ring_walk_kernel" in n}
@@ -81,22 +96,43 @@ def test_walk_kernel_runs_two_waves_per_simd_without_spills(tmp_path):
     assert len(walks) == 12
     for n, u in walks.items():
         carried = n.endswith("Lb0ELb1EEEvNS_9BlockArgsE")
-        # the carried-state variants must not spill at all; the others (which also hold the merge of a workgroup's
-        # partials, three 64-register batches in flight) may around that merge, never in the steady loops
-        assert u["ScratchSize [bytes/lane]"] == 0 or not carried, (n, u)
-        assert u["VGPRs"] <= 256, (n, u)                       # eight waves per workgroup, one workgroup per compute unit
-        if carried and "Li64E" in n:
-            assert u["VGPRs"] <= 128, (n, u)                   # d = 64: two workgroups per compute unit (+12 % measured)
-        # K and V rings; the variants that merge park the partial LSEs of their 256 rows there afterwards
-        assert u["LDS Size [bytes/block]"] == (32768 if carried and "Li64E" in n else 65536), (n, u)
-        if "Li128E" in n:
-            steady = steady_loops(asm, n)
-            assert len(steady) == 4, (n, len(steady))          # plain and masked groups, for each half of the workgroup
-            for lab, ins in steady:
-                # one barrier per two tiles (where partials are emitted the first one of a chunk may have been
-                # taken before the stores, which puts it on a side path of the loop)
-                assert sum(i.startswith("s_barrier") for i in ins) in ((2,) if carried else (1, 2)), (n, lab)
-                assert not any(i.startswith("scratch_") for i in ins), (n, lab)
+        d64 = "Li64E" in n
+        # (a register of the d = 64 variants that store partials waits in scratch from the start to the stores)
+        assert u["ScratchSize [bytes/lane]"] <= (8 if d64 and not carried else 0), (n, u)
+        assert not any(i.startswith("scratch_") for _, ins in loops_of(body_of(asm, n)) for i in ins), n
+        # eight waves per workgroup; d = 64: two workgroups per compute unit (+12 % measured)
+        assert u["VGPRs"] <= (128 if d64 else 256), (n, u)
+        assert u["LDS Size [bytes/block]"] == (32768 if d64 else 65536), (n, u)   # K and V rings, four tiles of 32 keys each
+        if not d64:
+            # (where partials are stored the first barrier of a chunk may have been taken before the stores, which puts
+            # it on a side path of the loop)
+            check_steady_loops(asm, n, (2,) if carried else (1, 2))
+
+
+def test_walk_kernel_that_merges_its_steps(tmp_path):
+    """The same program with the result of the rows in 32 registers more and, at d = 128, 64 KB of LDS."""
+    asm, usage = compile_to_asm("ringattn_steps.hip", tmp_path / "steps.s")
+    kernels = {n: u for n, u in usage.items() if "ring_walk_kernel" in n}
+    assert len(kernels) == 8   # {fp16, bf16} x {64, 128} x {partials rounded to fp16 or not}
+    for n, u in kernels.items():
+        d64 = "Li64E" in n
+        assert u["ScratchSize [bytes/lane]"] == 0 and u["VGPRs"] <= 256, (n, u)
+        assert u["LDS Size [bytes/block]"] == (32768 if d64 else 131072), (n, u)
+        if not d64:
+            check_steady_loops(asm, n, (2,))
+
+
+def test_thin_walk_kernel(tmp_path):
+    """thin::ring_walk_kernel: four waves that a compute unit may hold twice, rings of eight tiles, and one loop of eight tiles (64
+    MFMAs) with a barrier per two."""
+    asm, usage = compile_to_asm("ringattn_thin.hip", tmp_path / "thin.s")
+    kernels = {n: u for n, u in usage.items() if "ring_walk_kernel" in n}
+    assert len(kernels) == 8   # {fp16, bf16} x {fp32, fp16 partials} x {stored, merged}
+    for n, u in kernels.items():
+        assert u["ScratchSize [bytes/lane]"] == 0 and u["VGPRs"] <= 256, (n, u)
+        assert u["LDS Size [bytes/block]"] == 65536, (n, u)
+        (_, ins), = steady_loops(asm, n)
+        assert sum(i.startswith("s_barrier") for i in ins) == 4, n
 
 
 def test_walk64_kernel_runs_one_wave_per_simd(tmp_path):
@@ -137,7 +173,7 @@ def test_every_wave_of_the_workgroup_enters_the_hand_scheduled_loop(tmp_path):
                 assert not m or at[m.group(1)] < end, (n, l)
 
 
-@pytest.mark.parametrize("source", ["ringattn_walk.hip", "ringattn_walk64.hip"])
+@pytest.mark.parametrize("source", ["ringattn_walk.hip", "ringattn_steps.hip", "ringattn_thin.hip", "ringattn_walk64.hip"])
 def test_no_lds_transfer_reads_a_scalar_register_fresh_from_a_vector_instruction(source, tmp_path):
     """A vector instruction that writes a scalar register (v_readfirstlane, v_readlane, a compare into a register
     pair) must be five wait states ahead of a memory instruction that reads that register as its base address; the
