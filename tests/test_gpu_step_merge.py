@@ -1,18 +1,19 @@
-"""The merge at the end of a workgroup of ring_walk_kernel (merge_job_rows in ringattn_device.h) where its batches can go
-wrong: one part and two, which go in batches of their own, fewer than a batch of four (fp32) or eight (fp16), one more, one
-less, up to the 64 a plan may have; a q tile that ends after one row, in the middle of a batch or exactly; rows that see only some of the parts.  The forward with the
-steps apart is documented to give the bits of ringattn_block_fwd per step and ringattn_merge_ring, whose merge kernel is
-other code: the bound is equality."""
+"""The forward with the steps apart on ring_walk_kernel, which merges the partial of a step where it arises (ringattn_steps.hip; at d = 64
+thin::ring_walk_kernel as well), where the walk from step to step can go wrong: one part and two, up to the 64 a plan may
+have; a q tile that ends after one row, in the middle of a wave or exactly; chunks of less than a tile; rows that see only some of
+the parts; the masked part last.  It is documented to give the bits of ringattn_block_fwd per step and
+ringattn_merge_ring, whose merge kernel is other code: the bound is equality."""
 import numpy as np
 import pytest
 import torch
 
+from launched import launched
 from ringattention_amd import api
 from ringattention_amd.configs import Workload
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("d,thin", [(64, False), (64, True), (128, False)])
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("lens,causal,zigzag", [
     ((257,), False, False),
@@ -27,8 +28,9 @@ from ringattention_amd.configs import Workload
     ((9,) * 63 + (321,), False, False),
     ((17,) * 64, True, False),
 ])
-def test_forward_with_the_steps_apart_gives_the_bits_of_steps_and_merge(monkeypatch, lens, causal, zigzag, half, d):
+def test_forward_with_the_steps_apart_gives_the_bits_of_steps_and_merge(monkeypatch, lens, causal, zigzag, half, d, thin):
     monkeypatch.setenv("RINGATTN_WIDE_PARTIALS", "0")
+    monkeypatch.setenv("RINGATTN_THIN", "1" if thin else "0")
     P, S, B, H = len(lens), sum(lens), 1, 3
     w = Workload("step_merge", B, H, d, 1, S, "fp16" if d == 128 else "bf16", 700 + S, causal)
     q, k, v = (api.bits_to_tensor(np.ascontiguousarray(x), w.dtype) for x in api.make_qkv_bits(w))
@@ -37,6 +39,7 @@ def test_forward_with_the_steps_apart_gives_the_bits_of_steps_and_merge(monkeypa
     try:
         assert plan.forward_kernel() == "ring_walk_kernel"
         out, lse = plan.forward(q, k, v)
+        assert launched(lambda stream: plan.forward(q, k, v, out, lse, stream)) == [(256 if thin else 512, 0)]
         o_shape, l_shape = plan.parts_shapes()
         o_parts = torch.full(o_shape, float("nan"), dtype=plan.part_dtype, device="cuda")   # nobody may read what no step wrote
         l_parts = torch.full(l_shape, float("-inf"), dtype=torch.float32, device="cuda")

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from launched import launched
 from ringattention_amd import api
 from ringattention_amd.configs import Workload
 
@@ -50,9 +51,36 @@ def test_bits_of_ring_walk_kernel(monkeypatch, lens, causal, zigzag, kind, half)
             l_parts = torch.full(l_shape, 7.0, dtype=torch.float32, device="cuda")
             for s in range(P):
                 plan.block_forward(s, q, k, v, o_parts[s], l_parts[s])
+            threads = 256 if choice == "1" else 512
+            assert [t for t, _ in launched(lambda stream: plan.forward(q, k, v, out, lse, stream))] == [threads]
+            assert [t for t, _ in launched(lambda stream: plan.block_forward(0, q, k, v, o_parts[0], l_parts[0], stream))] == [threads]
             torch.cuda.synchronize()
             plan.close()
             results.append((out, lse, o_parts, l_parts))
         for x, y in zip(*results):
             ints = torch.int32 if x.dtype == torch.float32 else torch.int16
             assert torch.equal(x.view(ints), y.view(ints)), dtype
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,tokens,heads,thin", [
+    (64, 512, 64, True),     # 128 q tiles of 256 rows in all
+    (64, 512, 66, False),
+    (64, 257, 64, True),     # as many, the second of a head one row long
+    (128, 512, 2, False),
+])
+def test_which_launches_it_is_chosen_for(monkeypatch, d, tokens, heads, thin):
+    for name in ("RINGATTN_WIDE", "RINGATTN_WIDE_PARTIALS", "RINGATTN_THIN"):
+        monkeypatch.delenv(name, raising=False)
+    x = torch.zeros(1, heads, 2 * tokens, d, dtype=torch.float16, device="cuda")
+    own = x[:, :, :tokens].contiguous()
+    plan = api.RingAttention(2, tokens, d, 1, heads, "fp16")
+    o, l = plan.rank_step_forward(0, 1, own, own, own)
+    assert [t for t, _ in launched(lambda stream: plan.rank_step_forward(0, 1, own, own, own, o, l, stream))] == [256 if thin else 512]
+    plan.close()
+    if heads % 2 == 0:   # two ranks of half as many heads are as many q tiles
+        half = x[:, :heads // 2].contiguous()
+        plan = api.RingAttention(2, tokens, d, 1, heads // 2, "fp16", step_partials=True)
+        out, lse = plan.forward(half, half, half)
+        assert [t for t, _ in launched(lambda stream: plan.forward(half, half, half, out, lse, stream))] == [256 if thin else 512]
+        plan.close()
