@@ -163,7 +163,9 @@ int ringattn_block_fwd(ringattn_plan* plan, int step, const void* q, const void*
  * carrying max / sum / acc-O across steps, csrc/ring_attention.cu:207-245,621-633):
  *   lse = logsumexp_s lse_parts[s];  out = sum_s exp(lse_parts[s] - lse) * o_parts[s]
  * o_parts [n_parts, rows, dim] fp32, lse_parts [n_parts, rows] fp32 (a part with
- * lse = -inf is the identity); out [rows, dim] dtype; lse [rows] fp32.
+ * lse = -inf is the identity); out [rows, dim] dtype; lse [rows] fp32.  The parts are merged in
+ * ascending order, where ringattn_merge_ring takes step 0 of a causal plan last: on such a plan's
+ * parts the two agree to the rounding of fp32, not bit for bit.
  */
 int ringattn_merge(const float* o_parts, const float* lse_parts, int n_parts, int64_t rows, int dim,
                    int dtype, void* out, float* lse, void* stream);

@@ -97,7 +97,7 @@ class RingAttention:
         grouped-query attention (0 = same as `heads`).  `layout`: "contiguous" (rank r holds
         the tokens after those of rank r-1) or "zigzag" (rank r holds a low and a high
         half-chunk; see zigzag_order).  `step_partials`: forward() keeps the ring steps apart (a
-        partial (O, LSE) per step in the workspace, merged at the end: the arithmetic of
+        partial (O, LSE) per step, merged on the chip or by way of the workspace: the arithmetic of
         block_forward + merge_ring) instead of carrying the softmax state through all steps in
         registers.  `half_partials`: keep per-step partial O in fp16 (half the workspace and merge
         traffic; needs |V| < 65504).  `workspace`: a (device address, bytes) pair the caller owns

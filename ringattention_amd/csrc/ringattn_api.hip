@@ -336,9 +336,9 @@ static int pair_choice() {
 // keys) and the more of them, but the more often a K/V tile is fetched from L2.  A launch of few q tiles takes as long as
 // its longest walk, one of many as all of them over the compute units, at a lower clock.  Each kernel by three measured
 // numbers: us per step of a walk (one, two and eight key tiles) with most compute units idle and with all of them busy,
-// and us per workgroup besides (Q, first tiles, result).  They give the time of 150 launches of whole tiles -- heads 1 to 64,
-// sequences of 320 to 32768, with and without the causal mask, logits N(0, 1) -- to 2-4 % rms; us measured on ring_walk64_kernel
-// and the 128- and 32-row kernel at d = 128, and at d = 64:
+// and us per workgroup besides (Q, first tiles, result).  When they were fitted they gave the time of 150 launches of whole tiles -- heads
+// 1 to 64, sequences of 320 to 32768, with and without the causal mask, logits N(0, 1) -- to 2-4 % rms, from these and others; us
+// measured on ring_walk64_kernel and the 128- and 32-row kernel at d = 128, and at d = 64:
 //     1 head x 2048                         44, 28, 17        34, 22, 13
 //     8 heads x 2048                        43, 29, 33        34, 22, 19
 //     8 heads x 4096, causal                79, 50, 65        61, 38, 35
@@ -347,8 +347,9 @@ static int pair_choice() {
 //     8 heads x 8192                       211, 230, 389     131, 145, 198
 //     9 heads x 8192 (288 q tiles of 256)  355, 310, 437     244, 208, 223
 //     16 heads x 8192, causal              221, 245, 424     142, 159, 209
-// ring_split_kernel has since become 5 to 30 % faster where compute units idle (its file) and 5 % elsewhere; its numbers are left, because the lines
-// they draw are those between equals: with new ones d = 64 launches moved to it that both kernels run alike (us on
+// ring_split_kernel has since become 5 to 30 % faster where compute units idle (its file) and 5 % elsewhere, so the third row of either table
+// below overstates it by that much and draws lines, but does not give its times.  It is left, because the lines
+// are those between equals: with new numbers d = 64 launches moved to it that both kernels run alike (us on
 // ring_split_kernel and ring_pair_kernel: causal 8 x 4928 47, 48; 12 x 3054 33, 34; 4 x 10816 97, 94; no mask 6 x 3394 39, 38; 1 x
 // 20971 184, 164), and at d = 128 some whose second round of workgroups is mostly empty (4 x 3328 43.5, 40.6).
 enum class CarryKernel { kWhole, kPair, kSplit, kSplit16 };
@@ -660,11 +661,16 @@ int ensure_tables(ringattn_plan* pl, hipStream_t stream) {
 
 // ring_walk64_kernel runs the launch of a slice when every KV range suits it and d = 128.  The launches that emit
 // partials go by the forward's ranges, so that the forward and the steps run one by one keep giving the same bits.
-// A chunk walked on its own costs ring_walk64_kernel a start and a drain of its pipeline, and its four waves move the
-// partials (stores, merge) more slowly than the eight of ring_walk_kernel.  It wins where its loop is well ahead --
-// causal forwards, whose masked tiles it skips wave by wave -- and the chunks are long; measured with per-step
-// partials, ring_walk64_kernel against ring_walk_kernel: cfg4 (causal, 4096 keys per chunk) 1130 against 1050
-// TFLOP/s, cfg5 (not causal, 8192) 1060 against 1145, cfg3 (not causal, 512) 590 against 700.
+// A chunk walked on its own costs ring_walk64_kernel a start and a drain of its pipeline, and it writes its partials to memory and
+// reads them back where ring_walk_kernel merges them on the chip; its loop is the faster one, also because it skips masked
+// tiles wave by wave.  Whichever is taken runs the forward and the single steps of a plan.  us on ring_walk_kernel and on
+// ring_walk64_kernel, fp16, fp32 partials (in brackets fp16 partials), causal forwards of 4 ranks, 4 and 32 heads: chunks of 1024
+// 89, 120 (90, 110) and 145, 186 (146, 164); of 2048 166, 193 (167, 184) and 541, 580 (544, 557); of 4096 349, 362 (353, 356) and 1992, 1978
+// (1989, 1909); of 8192 981, 937 and 7702, 7317.  One step of a rank of them, masked, 8 and 32 heads: chunks of 1024 30, 29 and
+// 32, 30; of 2048 50, 47 and 57, 52; of 4096 89, 84 and 144, 132; any other step 28, 29 and 31, 31; 47, 47 and 69, 66; 88, 85 and 253,
+// 237.  So from 2048 keys on a ring run step by step gains up to 9 %, and the forward in one launch loses up to 14 % at 2048, 4 % at
+// 4096 where heads are few, and gains beyond.  Without a mask ring_walk64_kernel lies 0 to 6 % ahead at 4096 keys and 3 to 8 % at 8192, and is
+// not taken.
 constexpr int kWidePartialsMinKeys = 2048;
 bool slice_takes_walk64(const ringattn_plan* pl, const TableSlice& sl, int mode) {
   if (!sl.wide || !walk64_enabled()) return false;
@@ -744,7 +750,8 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
 // The ring step loop (csrc/ring_attention.cu:456-620) and the epilogue (:621-664), ONE launch:
 // every workgroup walks the ring steps of its 256 rows with the softmax state carried in
 // registers, like the reference's CTA (:439-443,597).  With RINGATTN_FLAG_STEP_PARTIALS it
-// writes a partial (O, LSE) per step instead and merges them at the end.
+// makes a partial (O, LSE) per step instead: ring_walk_kernel merges each where it arises,
+// ring_walk64_kernel writes them to the workspace and merges them at the end.
 int run_forward(ringattn_plan* pl, const void* q, const void* k, const void* v, void* out,
                 float* lse, hipStream_t stream) {
   const bool timing = (pl->p.flags & RINGATTN_FLAG_TIMING) && !(pl->p.flags & RINGATTN_FLAG_GRAPH);

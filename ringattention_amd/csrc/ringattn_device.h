@@ -277,10 +277,10 @@ static __device__ __forceinline__ int run_order(const Segment& seg, int i) {
 // ---- the merge of per-step partials of a row: L = logsumexp_s L_s, O = sum_s exp(L_s - L) O_s, one part after the other.  The
 // reference of the weights is the largest L_s so far; when it moves, the sums so far are scaled down to it (the rescale of
 // csrc/ring_attention.cu:226-232).  So a merge needs no look at all the L_s ahead of the first O_s, and a workgroup that
-// walks the steps of its rows merges each partial where it arises.  Every merge of the library (the merge kernel and
+// walks the steps of its rows merges each partial where it arises.  Every merge of a plan's steps (the merge kernel and
 // those in the attention kernels) is these operations on the same operands in the same order -- ring steps ascending, the
-// masked one last (a causal plan's step 0), as the attention kernels walk them --, so they give the same bits.  A part with
-// L_s = -inf is the identity: callers pass it by, whatever its O may hold.
+// masked one last (a causal plan's step 0), as the attention kernels walk them --, so they give the same bits.  ringattn_merge knows
+// no plan and takes its parts as they come.  A part with L_s = -inf is the identity: callers pass it by, whatever its O may hold.
 struct MergeState {
   float top = -INFINITY, sum = 0.f;  // the reference; the weights' sum against it
   // the weight of a part, and what the sums so far keep
