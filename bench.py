@@ -11,8 +11,8 @@ over the wall time of K steps; `roofline` prices the block-attention launch of t
 against the dense MFMA peak, timed by an event pair on the launch stream (a second pass of K
 forwards on a plan with the timing flag); `sustained` is the same forward run back to back for a few
 seconds more, the figure of its last second; `forward_with_step_partials` is the same forward on a
-plan that keeps the ring steps apart (a fp32 partial (O, LSE) per step in a workspace, merged at
-the end of each workgroup: another instantiation of the kernel, so a kernel trace keeps the two
+plan that keeps the ring steps apart (a fp32 partial (O, LSE) per step, merged on the
+chip or by way of a workspace: another instantiation of the kernel, so a kernel trace keeps the two
 apart; --step-partials makes that one the headline, --one-forward skips the other one); `merge`
 times the merge kernel alone, on
 caller-held per-step partials, against HBM bandwidth; `cpu_baseline` is the CPU oracle timed on
@@ -34,10 +34,10 @@ PEAK_HBM_GBS = 8000.0
 # (bytes, summary under profiles/, kernel, kernel_source_id(kernel) when it was measured).  The figure is only printed
 # while the forward still runs that kernel and its source is still the one that was profiled.
 MEASURED_TRAFFIC = {
-    "cfg4": (2280e6, "profiles/ring_walk64_kernel_cfg4.md", "ring_walk64_kernel", "fb6cfad5d7b6f313"),
-    "cfg3": (1623e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "fb6cfad5d7b6f313"),
-    "cfg5": (47323e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "fb6cfad5d7b6f313"),
-    "cfg2": (34.3e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "fb6cfad5d7b6f313"),
+    "cfg4": (2282e6, "profiles/ring_walk64_kernel_cfg4.md", "ring_walk64_kernel", "0f7fdaa0c1c3f628"),
+    "cfg3": (1623e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "0f7fdaa0c1c3f628"),
+    "cfg5": (46836e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "0f7fdaa0c1c3f628"),
+    "cfg2": (34.2e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "0f7fdaa0c1c3f628"),
 }
 KERNEL_SOURCES = {
     "ring_walk64_kernel": ("ringattn_walk64.hip", "ringattn_walk64_loop.inc", "ringattn_walk64_loop_d64.inc", "ringattn_device.h"),
@@ -86,8 +86,8 @@ def main():
     ap.add_argument("--one-forward", action="store_true",
                     help="skip the forward of the other kind (see --step-partials), which is timed as well by default")
     ap.add_argument("--step-partials", action="store_true",
-                    help="time the forward that keeps the ring steps apart (per-step partials in a workspace, merged at "
-                         "the end) instead of the one that carries the softmax state through the steps")
+                    help="time the forward that keeps the ring steps apart (per-step partials, merged "
+                         "in the same launch) instead of the one that carries the softmax state through the steps")
     ap.add_argument("--operands", default="workload", choices=["workload", "zeros"],
                     help="diagnostic: 'zeros' runs the same launches on all-zero Q, K, V (same instruction stream, no operand "
                          "toggling: shows what the power manager leaves of the clock); not a valid headline")
