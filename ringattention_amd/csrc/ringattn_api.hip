@@ -463,8 +463,7 @@ void fill_geometry(ringattn::BlockArgs& a, const ringattn_params& p, const Deriv
   a.kv_bh_stride = d.S * p.dim;
   a.S = (int)d.S;
   a.BH = (int)d.BH;
-  a.heads = p.heads;
-  a.kv_group = p.kv_heads > 0 ? p.heads / p.kv_heads : 1;
+  a.by_group = ringattn::divisor(p.kv_heads > 0 ? p.heads / p.kv_heads : 1);
   a.scale_log2 = d.scale * kLog2e;
   a.half_partials = half_partials(p) ? 1 : 0;
   a.causal = p.causal != 0;

@@ -117,51 +117,23 @@ static __device__ __forceinline__ int lap_order(const BlockArgs& a, int w) {
 
 // workgroup -> job (segment, head, q tile); false for the holes of the grid.  blockIdx mod 8 is the XCD.  Heads are dealt
 // to the XCDs round-robin, and an XCD runs the segments of a head one after the other (busiest first), the q tiles of a
-// segment as consecutive workgroups: everything that reads a head's K and V follows each other through that XCD's L2.
-// The batch * heads mod 8 heads that do not deal out evenly are shared: with rem of them, gcd(8, rem) sets of XCDs take
-// rem / gcd heads each and split their tiles round-robin, so that one head (or any number) still fills all XCDs.  The last
-// a.tail_heads heads of an XCD and its part of the shared ones are interleaved (job_grid says why).
+// segment as consecutive workgroups: everything that reads a head's K and V follows each other through that XCD's L2
+// (job_map in ringattn_jobs.h).
 // LAPS: compute units hold two workgroups (lap_order).
 template <int TILE_ROWS, bool LAPS = false>
 static __device__ __forceinline__ bool decode_job(const BlockArgs& a, Segment& seg, int& bh, int& qt) {
-  const int q_tiles = a.q_tiles_max;
-  const int per_head = a.n_segs * q_tiles;
-  const int xcd = blockIdx.x & 7, place = blockIdx.x >> 3;
-  const int w = LAPS ? lap_order(a, place) : place;
-  const int full = a.BH >> 3, rem = a.BH & 7;
-  const int lead = (full - a.tail_heads) * per_head;
+  const int place = blockIdx.x >> 3;
   int job;  // its number among those of its head
-  if (w < lead) {
-    bh = (w / per_head) * 8 + xcd;
-    job = w % per_head;
-  } else {
-    int p = w - lead;
-    const int own = a.tail_heads * per_head;  // jobs of whole heads
-    const int sets = rem & -rem;
-    const int share = rem ? 8 / sets : 1, sub = rem ? xcd / sets : 0, heads = rem ? rem / sets : 0;
-    const int shared = (heads * per_head - sub + share - 1) / share;  // this XCD's jobs of the shared heads
-    if (p >= own + shared) return false;
-    // p-th of both lists merged in proportion
-    const int from_shared = rem ? (int)((int64_t)p * shared / (own + shared)) : 0;
-    const int with_this = rem ? (int)((int64_t)(p + 1) * shared / (own + shared)) : 0;
-    if (with_this > from_shared) {
-      const int j = from_shared * share + sub;
-      job = a.causal ? j / heads : j % per_head;
-      bh = (a.BH & ~7) + (xcd & (sets - 1)) + sets * (a.causal ? j % heads : j / per_head);
-    } else {
-      p -= from_shared;
-      job = p / a.tail_heads;
-      bh = (full - a.tail_heads + p % a.tail_heads) * 8 + xcd;
-    }
-  }
-  const SegPtr sp = segs_of(a) + job / q_tiles;
+  if (!job_of(a.map, a.causal, blockIdx.x & 7, LAPS ? lap_order(a, place) : place, bh, job)) return false;
+  const int nth = quotient(job, a.by_q_tiles);
+  const SegPtr sp = segs_of(a) + nth;
   seg.q_start = sp->q_start;
   seg.q_len = sp->q_len;
   seg.item_begin = sp->item_begin;
   seg.item_count = sp->item_count;
   seg.last_item = sp->last_item;
   seg.reverse_tiles = sp->reverse_tiles;
-  qt = job % q_tiles;
+  qt = job - nth * a.q_tiles_max;
   if (qt * TILE_ROWS >= seg.q_len) return false;  // segments shorter than the longest one
   if (seg.reverse_tiles) qt = (seg.q_len + TILE_ROWS - 1) / TILE_ROWS - 1 - qt;  // most keys first
   return true;

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "ringattn_jobs.h"
 
 namespace ringattn {
 
@@ -82,37 +83,23 @@ struct BlockArgs {
   int q_tiles_max;     // kWalkM-row q tiles of the longest segment (grid dimension)
   int n_segs;
   int BH;              // batch * heads
-  int heads;           // query heads per batch entry
-  int kv_group;        // query heads per KV head (1 = one KV head per query head)
+  Divisor by_group;    // query heads per KV head: head bh of all batch entries reads K and V of head bh / that
   float scale_log2;    // softmax_scale * log2(e)
   int half_partials;   // partial O stored as fp16 instead of fp32
   int mode;            // BlockMode
   int causal;          // some item is masked
-  int tail_heads;      // see job_grid
+  Divisor by_q_tiles;  // q_tiles_max, and the jobs: job_grid
+  JobMap map;
   int second_lap;      // see lap_order in ringattn_device.h
   Segment one_seg;
   SegItem one_item;
 };
 
-// Workgroups of a launch: 8 x the jobs (head, segment, q tile) of the busiest XCD (decode_job in ringattn_device.h is the
-// other half of this).  Heads are dealt to the eight XCDs and run one after the other; what is left of them, batch * heads
-// mod 8, is shared out tile by tile.  `masked`: the q tiles of a head differ in length, longest first.  Then the last heads
-// of an XCD, as many as make up 64 jobs (two for each of its 32 compute units), and its part of the shared ones go through
-// their tiles together: one after the other, the longest tile of the last head would start when little else is left.
+// Workgroups of a launch over n_segs segments of q_tiles_max q tiles each, for every head (decode_job in ringattn_device.h is the other
+// half of this).
 inline int64_t job_grid(BlockArgs& a, bool masked) {
-  const int64_t per_head = (int64_t)a.n_segs * a.q_tiles_max;
-  const int full = a.BH / 8, rem = a.BH & 7;
-  a.tail_heads = 0;
-  if (masked && per_head > 0) {
-    const int64_t g = (64 + per_head - 1) / per_head;
-    a.tail_heads = (int)(g < full ? g : full);
-  }
-  int64_t per_xcd = full * per_head;
-  if (rem) {
-    const int sets = rem & -rem;  // gcd(8, rem): groups of 8 / sets XCDs with rem / sets heads each
-    per_xcd += ((rem / sets) * per_head * sets + 7) / 8;
-  }
-  return 8 * per_xcd;
+  a.by_q_tiles = divisor(a.q_tiles_max > 0 ? a.q_tiles_max : 1);
+  return job_map(a.map, a.BH, (int64_t)a.n_segs * a.q_tiles_max, masked);
 }
 
 // Merge of (O, LSE) partials into the final O (storage dtype) and LSE, for row ranges of every

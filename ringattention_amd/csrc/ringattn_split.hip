@@ -58,8 +58,8 @@ __global__ __launch_bounds__(64 * WAVES, D == 64 ? 4 : 2) void ring_split_kernel
   const ItemPtr items = items_of(a) + seg.item_begin;  // the order they are walked in does not matter here
 
   const int64_t head_off = (int64_t)bh * a.bh_stride;
-  // grouped-query attention: query head h of a batch entry reads KV head h / kv_group
-  const int kv_bh = (bh / a.heads) * (a.heads / a.kv_group) + (bh % a.heads) / a.kv_group;
+  // grouped-query attention: query head h of a batch entry reads KV head h / kv_group, and heads are whole groups
+  const int kv_bh = quotient(bh, a.by_group);
   const char* k_head = (const char*)a.k + (int64_t)kv_bh * a.kv_bh_stride * 2;
   const char* v_head = (const char*)a.v + (int64_t)kv_bh * a.kv_bh_stride * 2;
 

@@ -61,8 +61,8 @@ __global__ __launch_bounds__(256, 2) void ring_walk_kernel(const BlockArgs a) {
   const ItemPtr items = items_of(a);
 
   const int64_t head_off = (int64_t)bh * a.bh_stride;
-  // grouped-query attention: query head h of a batch entry reads KV head h / kv_group
-  const int kv_bh = (bh / a.heads) * (a.heads / a.kv_group) + (bh % a.heads) / a.kv_group;
+  // grouped-query attention: query head h of a batch entry reads KV head h / kv_group, and heads are whole groups
+  const int kv_bh = quotient(bh, a.by_group);
   const int64_t kv_head_off = (int64_t)kv_bh * a.kv_bh_stride;
 
   // this lane's query row; rows beyond the range read the last valid row

@@ -358,7 +358,7 @@ __global__ __launch_bounds__(256, 1) void ring_walk64_kernel(const BlockArgs a) 
   // items in run order: table order, except that item `last_item` (the diagonal one) is moved to the end
   auto item_in_order = [&](int i) -> ItemPtr { return items + seg.item_begin + run_order(seg, i); };
   const int64_t head_off = (int64_t)bh * a.bh_stride;
-  const int kv_bh = (bh / a.heads) * (a.heads / a.kv_group) + (bh % a.heads) / a.kv_group;
+  const int kv_bh = quotient(bh, a.by_group);
   const int64_t kv_head_off = (int64_t)kv_bh * a.kv_bh_stride;
   const char* qbase = (const char*)a.q + (head_off + (int64_t)(q_start + qt * BM) * D) * 2;
   const char* k_head = (const char*)a.k + kv_head_off * 2;

@@ -141,8 +141,8 @@ static __device__ __forceinline__ void walk_rows(const BlockArgs& a, unsigned ch
   auto item_at = [&](int i) -> ItemPtr { return items + seg.item_begin + run_order(seg, i); };
 
   const int64_t head_off = (int64_t)bh * a.bh_stride;
-  // grouped-query attention: query head h of a batch entry reads KV head h / kv_group
-  const int kv_bh = (bh / a.heads) * (a.heads / a.kv_group) + (bh % a.heads) / a.kv_group;
+  // grouped-query attention: query head h of a batch entry reads KV head h / kv_group, and heads are whole groups
+  const int kv_bh = quotient(bh, a.by_group);
   const int64_t kv_head_off = (int64_t)kv_bh * a.kv_bh_stride;
   const char* qbase = (const char*)a.q + (head_off + (int64_t)(q_start + qt * BM) * D) * 2;
 
