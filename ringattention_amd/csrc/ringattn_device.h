@@ -246,6 +246,19 @@ static __device__ __forceinline__ int run_order(const Segment& seg, int i) {
   return i == seg.item_count - 1 ? seg.last_item : (i >= seg.last_item ? i + 1 : i);
 }
 
+static __device__ __forceinline__ float partial_lse(float l, float ms) {
+  return (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
+}
+// An entry of a normalised partial row as it is stored: as fp16 rounded twice, not by a fused multiply-and-convert.
+template <bool HP> static __device__ __forceinline__ float partial_entry(float x, float inv) {
+  float p = x * inv;
+  if (HP) {
+    asm("" : "+v"(p));
+    p = (float)(_Float16)p;
+  }
+  return p;
+}
+
 // ---- the merge of per-step partials of a row: L = logsumexp_s L_s, O = sum_s exp(L_s - L) O_s, one part after the other.  The
 // reference of the weights is the largest L_s so far; when it moves, the sums so far are scaled down to it (the rescale of
 // csrc/ring_attention.cu:226-232).  So a merge needs no look at all the L_s ahead of the first O_s, and a workgroup that

@@ -57,18 +57,6 @@
 
 namespace ringattn {
 
-static __device__ __forceinline__ float partial_lse(float l, float ms) {
-  return (l > 0.f) ? (ms + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
-}
-// An entry of a normalised partial row as it is stored: as fp16 rounded twice, not by a fused multiply-and-convert.
-template <bool HP> static __device__ __forceinline__ float partial_entry(float x, float inv) {
-  float p = x * inv;
-  if (HP) {
-    asm("" : "+v"(p));
-    p = (float)(_Float16)p;
-  }
-  return p;
-}
 // A chunk's partial (csrc/ring_attention.cu:621-633) of a wave's 32 rows, the first of them row0 of the segment: normalised, with
 // its LSE, to the rows the item says.  l: the row sum of the lane's row.
 template <int D, bool HP>
