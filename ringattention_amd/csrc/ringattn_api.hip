@@ -418,6 +418,7 @@ struct ringattn_plan {
   void* ws = nullptr;
   size_t ws_bytes = 0;
   bool own_ws = false;
+  bool small_steps = false;    // launches that keep the ring steps apart: steps::ring_split_kernel
   void* o_parts = nullptr;     // partial O rows, fp32 (fp16 with RINGATTN_FLAG_HALF_PARTIALS)
   float* lse_parts = nullptr;  // partial LSE rows
   // Segment / item tables (host copies; device copies made by ensure_tables).  Three
@@ -693,6 +694,33 @@ bool takes_thin(const ringattn_plan* pl, const TableSlice& sl) {
   return (int64_t)sl.seg_count * q_tiles_of(sl.q_len_max) * pl->d.BH <= kThinMaxJobs;
 }
 
+// steps::ring_split_kernel runs the launches of a plan that keep the ring steps apart -- single steps of one rank and of all, and
+// the forward with RINGATTN_FLAG_STEP_PARTIALS -- where even the largest of them are small.  Its partials have other bits than those of the
+// 256-row kernels, and all launches of a plan give the same: so it is for plans that lose nothing by it in any of
+// the three, whichever a program calls.  Those of one step stop gaining where there are more 32-row q tiles than a round of
+// workgroups, but the longer their walks the later, the forward where the 256-row kernels fill the device.  Over 6500 drawn
+// plans (P 1 to 32, 600 to 60 000 rows, logits N(0, 1) and N(0, 81)) the lines leave these shares of the time on the kernels
+// before, geometric mean (the worst of fifty in brackets) of a rank's step, a step of all and the forward: d = 64 0.69 (1.05), 0.75 (1.08), 0.63 (0.95), under the
+// mask 0.67 (1.04), 0.69 (1.08), 0.57 (0.93); d = 128 0.59 (1.08), 0.64 (1.10), 0.51 (0.88), under the mask 0.56 (1.08), 0.60 (1.08), 0.45 (0.74).  us before and after: d = 64,
+// 4 heads x 4 x 512 9.9, 10.1, 29.9 and 6.2, 6.9, 17.7, 2 x 4 x 2048 25.6, 27.6, 94 and 10.1, 19.1, 65; d = 128, 8 heads x 8 x 256 12.9, 14.3,
+// 56 and 7.0, 14.8, 47, causal 4 x 4 x 777 29.5, 29.7, 100 and 11.9, 11.8, 42.  Beyond them, d = 64, 8 heads x 8 x 1024: 15.6, 30.3, 181 and 8.4, 45, 296.
+// RINGATTN_SPLIT_STEPS=0 and 1 in the environment: never, and always (comparisons, tests); the switches that name one of the
+// other kernels for these launches, or all launches, take this one out.
+bool small_steps(const ringattn_params& p, const Derived& d) {
+  int64_t tiles = 0;
+  for (int r = 0; r < p.npes; ++r) tiles += d.BH * ((d.start[r + 1] - d.start[r] + ringattn::kSplitM - 1) / ringattn::kSplitM);
+  const double chunk = (double)d.S / p.npes;
+  if (chunk < (p.npes == 1 ? 192 : 64)) return false;  // (a tile or two: one wave's work)
+  const double more = p.dim == 64 ? 1.03 * std::pow(std::max(1.0, chunk / 128), 0.25) : std::min(2.5, std::max(1.0, std::sqrt(chunk / 512)));
+  const double masked = p.causal && (p.dim == 64 || chunk >= 512) ? 1.4 : 1.0;
+  return (double)tiles <= ringattn::kComputeUnits * more * masked;
+}
+bool takes_split_steps(const ringattn_plan* pl) {
+  const char* e = std::getenv("RINGATTN_SPLIT_STEPS");
+  if (e) return e[0] != '0';
+  return pl->small_steps && walk64_enabled() && walk64_partials_choice() < 0 && split_choice() != 0 && !std::getenv("RINGATTN_THIN");
+}
+
 // the slice ringattn_fwd launches
 const TableSlice& forward_slice(const ringattn_plan* pl) { return step_partials(pl->p) ? pl->fwd : pl->walk; }
 
@@ -734,6 +762,11 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
     a.items = pl->d_segitems;
   }
   a.n_segs = sl.seg_count;
+  if (a.mode != ringattn::kBlockCarryState && takes_split_steps(pl)) {
+    a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kSplitM);
+    RA_HIP(ringattn::launch_split_steps(a, pl->p.dtype, pl->p.dim, stream));
+    return RINGATTN_OK;
+  }
   const bool wide = slice_takes_walk64(pl, sl, a.mode);
   if (a.mode != ringattn::kBlockCarryState && !wide && takes_thin(pl, sl)) {
     a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kThinM);
@@ -921,6 +954,7 @@ int ringattn_plan_create(const ringattn_params* params, void* workspace, size_t 
     pl->own_ws = true;
   }
   build_schedule(pl);
+  pl->small_steps = small_steps(pl->p, d);
   const size_t part_rows = need / ((size_t)params->dim * (half_partials(*params) ? 2 : 4) + sizeof(float));
   pl->o_parts = pl->ws;
   pl->lse_parts = (float*)((char*)pl->ws + part_rows * params->dim * (half_partials(*params) ? 2 : 4));
@@ -1103,6 +1137,7 @@ int ringattn_plan_launch_times(ringattn_plan* plan, float* ms, int capacity, int
 const char* ringattn_plan_forward_kernel(const ringattn_plan* plan) {
   if (!plan_ok(plan)) return nullptr;
   const int mode = step_partials(plan->p) ? ringattn::kBlockPartialsMerged : ringattn::kBlockCarryState;
+  if (mode != ringattn::kBlockCarryState && takes_split_steps(plan)) return "ring_split_kernel";
   const bool wide = slice_takes_walk64(plan, forward_slice(plan), mode);
   if (mode == ringattn::kBlockCarryState) {
     const CarryKernel kernel = carry_kernel(plan->walk.costs, plan->p.dim, wide);

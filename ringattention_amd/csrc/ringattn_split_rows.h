@@ -1,5 +1,5 @@
-// gfx950 (CDNA4) kernel: block attention for launches with few query rows.  The workgroup's program; ringattn_split.hip wraps it into
-// kernels.
+// gfx950 (CDNA4) kernel: block attention for launches with few query rows.  The workgroup's program; ringattn_split.hip and
+// ringattn_split_steps.hip wrap it into kernels.
 //
 //   ring_split_kernel : the forward of ring_walk_kernel and ring_walk64_kernel (the reference's CTA that walks its ring
 //       steps with max / sum / acc-O in registers, csrc/ring_attention.cu:439-443,456-620, epilogue :621-664) with the
@@ -36,6 +36,14 @@ namespace ringattn {
 
 // LDS of a wave: its K tile and its V tile; at the end its acc-O.
 template <int D> constexpr int kSplitWaveLds = 128 * D;
+// LDS of a workgroup that merges the steps of its rows: eight waves', the ranges, and ten numbers to eight columns of a row
+template <int D> constexpr int kSplitStepsLds = 8 * kSplitWaveLds<D> + 16 * kMaxParts + 4 * 10 * kSplitM * (D / 8);
+
+// The steps apart: the waves that share a key range of so many tiles, each with a run of up to four of them while there are waves; one,
+// two, four or all eight, so that whole ranges fill the workgroup.  It goes by the range alone: its partial has the same bits
+// in every launch.
+static __device__ __forceinline__ int split_units(int tiles) { return tiles <= 4 ? 1 : tiles <= 8 ? 2 : tiles <= 16 ? 4 : 8; }
+
 // MODE: one state of the rows through all of their keys (kBlockCarryState), or one per key range, whose partial is stored
 // (kBlockPartials) or merged into the rows' result (kBlockPartialsMerged); HP: partial O rounded to fp16.
 template <int DT, int D, int WAVES, bool HP, int MODE>
@@ -54,6 +62,7 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
   constexpr int WREG = kSplitWaveLds<D>;
   static_assert(WREG == 2 * TILE && WREG == BM * D * 4, "acc-O of a wave as fp32 takes the place of its tiles");
   constexpr bool KEEP = MODE == kBlockCarryState, MERGE = MODE == kBlockPartialsMerged;
+  static_assert(KEEP || WAVES == 8, "split_units");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -370,6 +379,127 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
     return;
   }
 
+  // a run of tiles: run `unit` of `units` of a range that begins at row `start`
+  auto enter_unit = [&](int unit, int units) {
+    const int all = (len + BN - 1) / BN;
+    t = unit * all / units;
+    tiles = (unit + 1) * all / units;
+    if (diag >= 0) tiles = min(tiles, (diag + q_last) / BN + 1);
+    return t < tiles;
+  };
+  if constexpr (MODE == kBlockPartials) {  // one range
+    start = items->kv_start;
+    len = items->kv_len;
+    diag = items->diag_off;
+    const int units = split_units((len + BN - 1) / BN);
+    const bool seen = wave < units && enter_unit(wave, units);
+    walk(seen);
+    show_state();
+    __syncthreads();
+    if (!owner()) return;
+    combine(0, units);
+    const int row = tid / TPR, c8 = tid % TPR;
+    // its partial (:621-633)
+    const float inv = (l > 0.f) ? 1.f / l : 0.f;
+    int64_t prow = items->part_base + (int64_t)bh * items->part_bh_stride + q0 + row;
+    if (items->part_row_mul > 0) prow = prow * items->part_row_mul + items->slot;  // a row's steps next to each other
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = partial_entry<HP>(o[e], inv);
+    if constexpr (HP) {  // fp16 partials: |O_part| <= max |V|, the caller vouches that this fits
+      Store8<0>::st((char*)a.o_part + (prow * D + c8 * 8) * 2, o);
+    } else {
+      float* to = (float*)a.o_part + prow * D + c8 * 8;
+      *(f32x4*)to = f32x4{o[0], o[1], o[2], o[3]};
+      *(f32x4*)(to + 4) = f32x4{o[4], o[5], o[6], o[7]};
+    }
+    if (c8 == 0) a.lse_part[prow] = partial_lse(l, top);
+    return;
+  }
+
+  if constexpr (MERGE) {
+    // rounds of as many whole ranges as there are waves for.  What lasts from round to round -- the ranges in the order of the walk, and
+    // the rows' result so far -- waits in LDS: in registers it would be more than two workgroups on a compute unit can have at d = 64.
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    i32x4* its = (i32x4*)(smem + WAVES * WREG);  // first row, rows, diag_off, units
+    constexpr int kStride = BM * TPR;
+    auto kept = [&](int i) -> float& { return ((float*)(its + kMaxParts))[i * kStride + fresh(tid)]; };  // of owners
+    static_assert(WAVES * WREG + 16 * kMaxParts + 4 * 10 * kStride == kSplitStepsLds<D>, "tiles, ranges, results");
+    if (lane < n_items) {  // (every wave writes all of them, the same: it reads none but after its own)
+      const ItemPtr w = items + run_order(seg, lane);
+      its[lane] = i32x4{w->kv_start, w->kv_len, w->diag_off, split_units((w->kv_len + BN - 1) / BN)};
+    }
+    auto range = [&](int i) {
+      i32x4 x = its[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = __builtin_amdgcn_readfirstlane(x[e]);
+      return x;
+    };
+    MergeState mst;  // the result of the row so far, and this thread's columns of it
+    float macc[8];
+    for (int round = 0; round < n_items;) {
+      int end = round, used = 0;
+      bool seen = false;
+      for (; end < n_items; ++end) {
+        const i32x4 x = range(end);
+        if (used + x[3] > WAVES) break;
+        if (wave >= used && wave < used + x[3]) {
+          start = x[0];
+          len = x[1];
+          diag = x[2];
+          seen = enter_unit(wave - used, x[3]);
+        }
+        used += x[3];
+      }
+      if (round > 0) {
+        reset();
+        __syncthreads();  // the states of the round before have been read
+      }
+      walk(seen);
+      show_state();
+      __syncthreads();
+      if (owner()) {
+        mst = MergeState();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) macc[e] = 0.f;
+        if (round > 0) {
+          mst.top = kept(0);
+          mst.sum = kept(1);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) macc[e] = kept(2 + e);
+        }
+      }
+      int first = 0;  // the wave that has the first run of a range
+      for (int i = round; i < end; ++i) {
+        const int g = range(i)[3];
+        if (owner()) {
+          combine(first, g);
+          const float inv = (l > 0.f) ? 1.f / l : 0.f, L = partial_lse(l, top);
+          if (L != -INFINITY) {  // (-inf: the identity)
+            float keep, wt;
+            mst.weigh(L, keep, wt);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) macc[e] = merge_in_part(macc[e], keep, wt, partial_entry<HP>(o[e], inv));
+          }
+        }
+        first += g;
+      }
+      round = end;
+      if (owner() && round < n_items) {
+        kept(0) = mst.top;
+        kept(1) = mst.sum;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) kept(2 + e) = macc[e];
+      }
+    }
+    if (!owner()) return;
+    const int row = fresh(tid) / TPR, c8 = fresh(tid) % TPR;
+    const float inv = mst.inverse();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) macc[e] *= inv;
+    const int64_t orow = (int64_t)bh * a.S + seg.q_start + q0 + row;
+    Store8<DT>::st((char*)a.out + (orow * D + c8 * 8) * 2, macc);
+    if (c8 == 0) a.lse[orow] = mst.lse();
+  }
 }
 
 }  // namespace ringattn
