@@ -325,6 +325,20 @@ static int split_choice() {  // -1: unset
   const char* e = std::getenv("RINGATTN_SPLIT");
   return e ? std::atoi(e) : -1;
 }
+// The columns of V and O that a workgroup of ring_split_kernel has.  A launch of few row tiles gains from fewer of them while their
+// workgroups find compute units of their own; with all of these busy they share what L2 delivers, and every one of them asks for the
+// whole of K.  us with all, 64 and 32 columns, d = 128: 16 row tiles x 16 key tiles 8.0, 7.1, 6.7, x 256 37.5, 29.7, 27.8; 32 x 32 10.1,
+// 8.7, 8.4, x 256 37.8, 30.2, 29.3; 64 x 64 14.5, 12.3, 12.4, x 512 75.6, 59.6, 67.6; 96 x 96 18.8, 16.3, 28.1; 128 x 128 22.6, 21.6,
+// 37.1; 256 x 64 17.3, 24.8.  d = 64, all and 32: 32 x 32 6.9, 6.4; 64 x 64 9.4, 9.1, x 512 40.7, 39.5; 75 x 25 6.5, 6.2; 96 x 96 12.0, 11.9;
+// 128 x 128 14.4, 14.6, x 256 23.7, 25.3.
+// RINGATTN_SPLIT_COLUMNS in the environment: 32, 64 or 128, at most the head dimension (comparisons, tests).
+static int split_columns(int64_t row_tiles, int dim) {
+  const char* e = std::getenv("RINGATTN_SPLIT_COLUMNS");
+  const int asked = e ? std::atoi(e) : 0;
+  if (asked == 32 || asked == 64 || asked == 128) return std::min(asked, dim);
+  if (dim == 64) return row_tiles <= 96 ? 32 : 64;
+  return row_tiles <= 32 ? 32 : row_tiles <= 128 ? 64 : 128;
+}
 static int pair_choice() {
   const char* e = std::getenv("RINGATTN_PAIR");
   return !e ? -1 : (e[0] == '0' ? 0 : 1);
@@ -741,7 +755,7 @@ hipError_t launch_q_tiles(ringattn::BlockArgs& a, CarryKernel kernel, bool wide,
     case CarryKernel::kSplit:
     case CarryKernel::kSplit16:
       a.q_tiles_max = q_tiles_of(q_len, ringattn::kSplitM);
-      return ringattn::launch_split(a, dtype, dim, kernel == CarryKernel::kSplit16, stream);
+      return ringattn::launch_split(a, dtype, dim, kernel == CarryKernel::kSplit16, split_columns((int64_t)a.n_segs * a.q_tiles_max * a.BH, dim), stream);
     default:
       a.q_tiles_max = q_tiles_of(q_len);
       return wide ? ringattn::launch_walk64(a, dtype, dim, stream) : ringattn::launch_walk(a, walks, dtype, dim, stream);
@@ -764,7 +778,8 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
   a.n_segs = sl.seg_count;
   if (a.mode != ringattn::kBlockCarryState && takes_split_steps(pl)) {
     a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kSplitM);
-    RA_HIP(ringattn::launch_split_steps(a, pl->p.dtype, pl->p.dim, stream));
+    const int columns = a.mode == ringattn::kBlockPartials ? split_columns((int64_t)a.n_segs * a.q_tiles_max * a.BH, pl->p.dim) : pl->p.dim;
+    RA_HIP(ringattn::launch_split_steps(a, pl->p.dtype, pl->p.dim, columns, stream));
     return RINGATTN_OK;
   }
   const bool wide = slice_takes_walk64(pl, sl, a.mode);

@@ -84,6 +84,7 @@ template <int D> static __device__ __forceinline__ int k_swizzle(int row) {
   return D == 128 ? (row & 15) : ((row >> 1) & 7);
 }
 template <int D> static __device__ __forceinline__ int v_swizzle(int row) {
+  if (D == 32) return 0;  // (four rows of 64 bytes are all banks)
   return D == 128 ? (((row & 3) << 2) | (((row >> 2) & 1) << 1))
                   : ((((row >> 1) & 1) << 2) | (((row >> 2) & 1) << 1));
 }

@@ -145,10 +145,12 @@ hipError_t launch_thin(BlockArgs a, int dtype, hipStream_t stream);
 // walk64_takes() accepts
 hipError_t launch_walk64(BlockArgs a, int dtype, int dim, hipStream_t stream);
 // ring_split_kernel: kSplitM query rows per workgroup (a.q_tiles_max counts tiles of that many rows), the keys split over
-// its waves (eight; `many_waves`, d = 64 only: sixteen); kBlockCarryState
-hipError_t launch_split(BlockArgs a, int dtype, int dim, bool many_waves, hipStream_t stream);
-// the same with the ring steps apart, kBlockPartials and kBlockPartialsMerged; eight waves
-hipError_t launch_split_steps(BlockArgs a, int dtype, int dim, hipStream_t stream);
+// its waves (eight; `many_waves`, d = 64 only: sixteen), `columns` of V and O (32, 64 or all) in a workgroup; kBlockCarryState
+hipError_t launch_split(BlockArgs a, int dtype, int dim, bool many_waves, int columns, hipStream_t stream);
+// the same with the ring steps apart, kBlockPartials and kBlockPartialsMerged (which has all columns); eight waves
+hipError_t launch_split_steps(BlockArgs a, int dtype, int dim, int columns, hipStream_t stream);
+// either with fewer columns than all, the grid laid out
+hipError_t launch_split_columns(const BlockArgs& a, unsigned grid, int dtype, int dim, bool many_waves, int columns, hipStream_t stream);
 // ring_pair_kernel: kPairM query rows per workgroup (a.q_tiles_max counts tiles of that many rows), the keys dealt to two
 // pairs of waves; kBlockCarryState, tables that CarryCosts::add finds fit for it
 hipError_t launch_pair(BlockArgs a, int dtype, int dim, hipStream_t stream);

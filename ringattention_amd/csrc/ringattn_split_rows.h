@@ -29,13 +29,19 @@
 //       factor of a state comes with its reader, which spares a barrier, and the next K tile is asked for behind the first product of the
 //       chain and not behind the last: 5.46 us; 256 rows x 256 keys 5.45 -> 4.84, 640 x 640 6.76 -> 6.15, 1280 x 8960 causal 24.9 -> 24.0;
 //       d = 128, 4 heads x 256 7.18 -> 6.89, 512 x 2048 causal 13.8 -> 13.5.
+//       Where a launch has so few row tiles that it leaves compute units idle, the COLUMNS of V and O are dealt to workgroups
+//       as well: each takes all of K and 64 or 32 columns of V.  A compute unit then takes in three quarters (d = 128, half
+//       the columns) of the bytes a tile, has half or a quarter of the products of P V to do, and as much less to put together at
+//       the end; scores are computed once per workgroup.  The columns of a row do not meet, so the bits are the same.  us before and after:
+//       d = 128, 512 rows x 2048 causal 13.5 -> 11.0, 512 x 512 8.0 -> 6.7, 1024 x 1024 10.1 -> 8.4, 512 x 8192 37.5 -> 27.8;
+//       d = 64, 512 x 512 5.5 -> 5.2, 1024 x 1024 6.9 -> 6.4; how many columns: split_columns in ringattn_api.hip.
 #pragma once
 #include "ringattn_device.h"
 
 namespace ringattn {
 
-// LDS of a wave: its K tile and its V tile; at the end its acc-O.
-template <int D> constexpr int kSplitWaveLds = 128 * D;
+// LDS of a wave: its K tile and C columns of its V tile; at the end its acc-O.
+template <int D, int C = D> constexpr int kSplitWaveLds = 64 * D + 64 * C;
 // LDS of a workgroup that merges the steps of its rows: eight waves', the ranges, and ten numbers to eight columns of a row
 template <int D> constexpr int kSplitStepsLds = 8 * kSplitWaveLds<D> + 16 * kMaxParts + 4 * 10 * kSplitM * (D / 8);
 
@@ -46,23 +52,25 @@ static __device__ __forceinline__ int split_units(int tiles) { return tiles <= 4
 
 // MODE: one state of the rows through all of their keys (kBlockCarryState), or one per key range, whose partial is stored
 // (kBlockPartials) or merged into the rows' result (kBlockPartialsMerged); HP: partial O rounded to fp16.
-template <int DT, int D, int WAVES, bool HP, int MODE>
+// C: the columns of V and O that a workgroup has, blockIdx.y the how many-th of them.
+template <int DT, int D, int C, int WAVES, bool HP, int MODE>
 static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned char* smem, float2 (*stat)[kSplitM]) {
   using E = Elem<DT>;
   constexpr int BM = kSplitM;      // query rows per workgroup, all of them in every wave
   constexpr int BN = 32;           // keys per tile
   constexpr int CPR = D / 8;       // 16-byte chunks per row
   constexpr int ROWB = D * 2;      // bytes per row
-  constexpr int TILE = BN * ROWB;  // bytes per tile
+  constexpr int TILE = BN * ROWB;  // bytes per K tile
+  constexpr int ROWV = C * 2;      // bytes per row of a V tile
   constexpr int KS = D / 16;       // contraction slices of QK^T
-  constexpr int DB = D / 32;       // 32-wide blocks of the head dim in PV
-  constexpr int PIECES = TILE / 1024;  // 1 KB wave-loads per tile
-  constexpr int RPP = 1024 / ROWB;     // rows per piece
+  constexpr int DB = C / 32;       // 32-wide blocks of the head dim in PV
+  constexpr int PIECES_K = TILE / 1024, PIECES_V = BN * ROWV / 1024;  // 1 KB wave-loads per tile
   static_assert(BM == 32, "one 32-row block");
-  constexpr int WREG = kSplitWaveLds<D>;
-  static_assert(WREG == 2 * TILE && WREG == BM * D * 4, "acc-O of a wave as fp32 takes the place of its tiles");
+  constexpr int WREG = kSplitWaveLds<D, C>;
+  static_assert(WREG == TILE + BN * ROWV && WREG >= BM * C * 4, "acc-O of a wave as fp32 takes the place of its tiles");
   constexpr bool KEEP = MODE == kBlockCarryState, MERGE = MODE == kBlockPartialsMerged;
   static_assert(KEEP || WAVES == 8, "split_units");
+  static_assert(C == D || !MERGE, "kSplitStepsLds");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -80,7 +88,8 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
   // grouped-query attention: query head h of a batch entry reads KV head h / kv_group, and heads are whole groups
   const int kv_bh = quotient(bh, a.by_group);
   const char* k_head = (const char*)a.k + (int64_t)kv_bh * a.kv_bh_stride * 2;
-  const char* v_head = (const char*)a.v + (int64_t)kv_bh * a.kv_bh_stride * 2;
+  const int column = C == D ? 0 : blockIdx.y * C;  // this workgroup's first
+  const char* v_head = (const char*)a.v + ((int64_t)kv_bh * a.kv_bh_stride + column) * 2;
 
   // Q of this lane's row (B operands for the whole launch); rows beyond the range read the last valid row
   s16x8 qf[KS];
@@ -103,36 +112,50 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
       const int c = 2 * (2 * db + g1) + ((s & 3) >> 1);
-      voff[db] = TILE + row8 * ROWB + ((c ^ v_swizzle<D>(row8)) << 4) + ((s & 1) << 3);
+      voff[db] = TILE + row8 * ROWV + ((c ^ v_swizzle<C>(row8)) << 4) + ((s & 1) << 3);
     }
   }
   // Offsets of this lane's 16 bytes within a 1 KB piece of a tile; the swizzles repeat after a few pieces.  A load instruction's
-  // own offset moves both ends, so pieces up to 4 KB apart share a base address and an M0 (d = 128 needs two of each).
-  constexpr int NPK = D == 128 ? 4 : 2, NPV = D == 128 ? 2 : 1;
-  const int prow = lane / CPR;
+  // own offset moves both ends, so pieces up to 4 KB apart share a base address and an M0 (d = 128 needs two of each).  With
+  // some of the columns of V its pieces lie further apart in memory than in LDS: the difference is in the offsets.
+  constexpr int NPK = D == 128 ? 4 : 2, NPV = C < D ? PIECES_V : D == 128 ? 2 : 1;
   int goff_k[NPK], goff_v[NPV];
 #pragma unroll
-  for (int j = 0; j < NPK; ++j) goff_k[j] = prow * ROWB + (((lane % CPR) ^ k_swizzle<D>(RPP * j + prow)) << 4);
+  for (int j = 0; j < NPK; ++j) {
+    const int row = lane / CPR;
+    goff_k[j] = row * ROWB + (((lane % CPR) ^ k_swizzle<D>(1024 / ROWB * j + row)) << 4);
+  }
 #pragma unroll
-  for (int j = 0; j < NPV; ++j) goff_v[j] = prow * ROWB + (((lane % CPR) ^ v_swizzle<D>(RPP * j + prow)) << 4);
-  // the tile at `base` to `dst`; `rows` of it exist (if fewer than 32, the others read the last one of them)
-  auto load_tile = [&](const char* base, unsigned dst, int rows, const auto& goff) {
-    constexpr int NP = sizeof(goff) / sizeof(int);
+  for (int j = 0; j < NPV; ++j) {
+    const int row = lane / (C / 8);
+    goff_v[j] = row * ROWB + (((lane % (C / 8)) ^ v_swizzle<C>(1024 / ROWV * j + row)) << 4);
+    if (C < D) goff_v[j] += j * (1024 / ROWV * ROWB - 1024);
+  }
+  // the tile at `base` to `dst`, its rows of ROW bytes; `rows` of it exist (if fewer than 32, the others read the last one of them)
+  auto load_tile = [&](const char* base, unsigned dst, int rows, const auto& goff, auto row_bytes) {
+    constexpr int NP = sizeof(goff) / sizeof(int), ROW = decltype(row_bytes)::value, PIECES = BN * ROW / 1024;
     if (rows >= BN) {
+      if constexpr (PIECES == 2) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %3\n\tglobal_load_lds_dwordx4 %2, %3 offset:1024" ::"s"(
+                         __builtin_amdgcn_readfirstlane(dst)),
+                     "v"(goff[0]), "v"(goff[1 % NP]), "s"(base)
+                     : "m0");
+      } else {
 #pragma unroll
-      for (int j = 0; j < PIECES; j += 4)
-        asm volatile(
-            "s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %5\n\tglobal_load_lds_dwordx4 %2, %5 offset:1024\n\t"
-            "global_load_lds_dwordx4 %3, %5 offset:2048\n\tglobal_load_lds_dwordx4 %4, %5 offset:3072" ::"s"(
-                __builtin_amdgcn_readfirstlane(dst + 1024 * j)),
-            "v"(goff[0]), "v"(goff[1 % NP]), "v"(goff[2 % NP]), "v"(goff[3 % NP]), "s"(base + 1024 * j)
-            : "m0");
+        for (int j = 0; j < PIECES; j += 4)
+          asm volatile(
+              "s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %5\n\tglobal_load_lds_dwordx4 %2, %5 offset:1024\n\t"
+              "global_load_lds_dwordx4 %3, %5 offset:2048\n\tglobal_load_lds_dwordx4 %4, %5 offset:3072" ::"s"(
+                  __builtin_amdgcn_readfirstlane(dst + 1024 * j)),
+              "v"(goff[j % NP]), "v"(goff[(j + 1) % NP]), "v"(goff[(j + 2) % NP]), "v"(goff[(j + 3) % NP]), "s"(base + 1024 * j)
+              : "m0");
+      }
     } else {
-      int row = prow;
+      int row = 16 * lane / ROW;
       asm volatile("" : "+v"(row));  // (keeps this seldom taken arithmetic from being done ahead of the loop, in registers)
 #pragma unroll
       for (int j = 0; j < PIECES; ++j)
-        load_lds_16_settled(base, goff[j % NP] + 1024 * j - max(0, RPP * j + row - (rows - 1)) * ROWB,
+        load_lds_16_settled(base, goff[j % NP] + 1024 * j - max(0, 1024 / ROW * j + row - (rows - 1)) * ROWB,
                             __builtin_amdgcn_readfirstlane(dst + 1024 * j));
     }
   };
@@ -190,8 +213,8 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
     x.visible = diag >= 0 ? diag + q0 + 1 - t * BN : INT32_MAX - BM;
     return x;
   };
-  auto issue_k = [&](const Tile& x) { load_tile(k_head + x.at, my_lds, x.rows, goff_k); };
-  auto issue_v = [&](const Tile& x) { load_tile(v_head + x.at, my_lds + TILE, x.rows, goff_v); };
+  auto issue_k = [&](const Tile& x) { load_tile(k_head + x.at, my_lds, x.rows, goff_k, std::integral_constant<int, ROWB>{}); };
+  auto issue_v = [&](const Tile& x) { load_tile(v_head + x.at, my_lds + TILE, x.rows, goff_v, std::integral_constant<int, ROWV>{}); };
   // P = exp2(S k2 - m k2) and the sums of four: from the unrounded values (:242); rounded for the MFMA (:604)
   f32x16 sacc;
   s16x8 pf[2];
@@ -239,7 +262,7 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
     for (int pass = 1; more; pass = 0) {  // pass: 1 while there is no reference to take exponentials against
       more = advance();
       // ---- S^T = K Q^T (csrc/ring_attention.cu:565): K(t) is in, V(t) may still be on its way
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES_V) : "memory");
       {
         s16x8 kfr[KS];
 #pragma unroll
@@ -282,7 +305,7 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
 #pragma unroll
       for (int i = 0; i < 4; ++i) ls[i] += sums[i];
       // ---- O^T += V^T P^T (:609): V(t) is in, K of the next tile may still be on its way
-      if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
+      if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES_K) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
       {
@@ -290,9 +313,9 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
         s16x8 vfr[2 * DB];
         auto read_v = [&](int f) {
           if (f >= 2 * DB) return;
-          const unsigned char* vrow = my + 16 * (f / DB) * ROWB + voff[f % DB];
+          const unsigned char* vrow = my + 16 * (f / DB) * ROWV + voff[f % DB];
           const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow + 8 * ROWB));
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow + 8 * ROWV));
           vfr[f] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         };
 #pragma unroll
@@ -330,11 +353,11 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
 #pragma unroll
         for (int e = 0; e < 4; ++e) val[e] = oacc[db][4 * q4 + e];
         const int c = 8 * db + 2 * q4 + h;
-        *(f32x4*)(my + n * (D * 4) + ((c ^ (n & (D / 4 - 1))) << 4)) = val;
+        *(f32x4*)(my + n * (C * 4) + ((c ^ (n & (C / 4 - 1))) << 4)) = val;
       }
   };
   // The states of `count` waves from `first` on put together, for eight columns of a row: their reference, row sum and acc-O.
-  constexpr int TPR = D / 8;  // threads of a row (at d = 64 half the threads have none, with sixteen waves three quarters)
+  constexpr int TPR = C / 8;  // threads of a row (at 64 columns half the threads have none, with sixteen waves three quarters)
   auto owner = [&]() { return (MERGE ? fresh(tid) : tid) / TPR < min(BM, q_last + 1 - q0); };
   float top, l, o[8];
   auto combine = [&](int first, auto count) {
@@ -349,9 +372,9 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
 #pragma unroll(WAVES > 8 || MERGE ? 4 : 8)  // (else they would not fit the registers)
     for (int w = 0; w < count; ++w) {
       const float2 st = stat[first + w][row];
-      const unsigned char* src = smem + (first + w) * WREG + row * (D * 4);
-      const f32x4 x0 = *(const f32x4*)(src + (((2 * c8) ^ (row & (D / 4 - 1))) << 4));
-      const f32x4 x1 = *(const f32x4*)(src + (((2 * c8 + 1) ^ (row & (D / 4 - 1))) << 4));
+      const unsigned char* src = smem + (first + w) * WREG + row * (C * 4);
+      const f32x4 x0 = *(const f32x4*)(src + (((2 * c8) ^ (row & (C / 4 - 1))) << 4));
+      const f32x4 x1 = *(const f32x4*)(src + (((2 * c8 + 1) ^ (row & (C / 4 - 1))) << 4));
       const float f = st.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(st.x - top);
       l = __builtin_fmaf(st.y, f, l);
 #pragma unroll
@@ -374,8 +397,8 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] *= inv;
     const int64_t orow = (int64_t)bh * a.S + seg.q_start + q0 + row;
-    Store8<DT>::st((char*)a.out + (orow * D + c8 * 8) * 2, o);
-    if (c8 == 0 && a.lse) a.lse[orow] = partial_lse(l, top);
+    Store8<DT>::st((char*)a.out + (orow * D + column + c8 * 8) * 2, o);
+    if (column + c8 == 0 && a.lse) a.lse[orow] = partial_lse(l, top);
     return;
   }
 
@@ -406,13 +429,13 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = partial_entry<HP>(o[e], inv);
     if constexpr (HP) {  // fp16 partials: |O_part| <= max |V|, the caller vouches that this fits
-      Store8<0>::st((char*)a.o_part + (prow * D + c8 * 8) * 2, o);
+      Store8<0>::st((char*)a.o_part + (prow * D + column + c8 * 8) * 2, o);
     } else {
-      float* to = (float*)a.o_part + prow * D + c8 * 8;
+      float* to = (float*)a.o_part + prow * D + column + c8 * 8;
       *(f32x4*)to = f32x4{o[0], o[1], o[2], o[3]};
       *(f32x4*)(to + 4) = f32x4{o[4], o[5], o[6], o[7]};
     }
-    if (c8 == 0) a.lse_part[prow] = partial_lse(l, top);
+    if (column + c8 == 0) a.lse_part[prow] = partial_lse(l, top);
     return;
   }
 

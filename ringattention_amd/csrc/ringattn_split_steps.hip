@@ -16,16 +16,17 @@ template <int DT, int D, bool HP, int MODE>
 __global__ __launch_bounds__(512, D == 64 ? 4 : 2) void ring_split_kernel(const BlockArgs a) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[MODE == kBlockPartialsMerged ? kSplitStepsLds<D> : 8 * kSplitWaveLds<D>];
   __shared__ float2 stat[8][kSplitM];
-  split_rows<DT, D, 8, HP, MODE>(a, smem, stat);
+  split_rows<DT, D, D, 8, HP, MODE>(a, smem, stat);
 }
 
 }  // namespace steps
 
-hipError_t launch_split_steps(BlockArgs a, int dtype, int dim, hipStream_t stream) {
+hipError_t launch_split_steps(BlockArgs a, int dtype, int dim, int columns, hipStream_t stream) {
   if (a.n_segs <= 0) return hipSuccess;
   const int64_t blocks = job_grid(a, a.causal != 0);
   if (a.q_tiles_max <= 0 || blocks > INT32_MAX || a.mode == kBlockCarryState) return hipErrorInvalidValue;
   const unsigned grid = (unsigned)blocks;
+  if (columns != dim) return launch_split_columns(a, grid, dtype, dim, false, columns, stream);
 #define RA_LAUNCH_OF(DT_, D_, HP_)                                                                                      \
   do {                                                                                                                 \
     if (a.mode == kBlockPartials) steps::ring_split_kernel<DT_, D_, HP_, kBlockPartials><<<grid, 512, 0, stream>>>(a);  \
