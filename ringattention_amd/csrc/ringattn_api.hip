@@ -708,6 +708,19 @@ bool takes_thin(const ringattn_plan* pl, const TableSlice& sl) {
   return (int64_t)sl.seg_count * q_tiles_of(sl.q_len_max) * pl->d.BH <= kThinMaxJobs;
 }
 
+// Of the launches that thin::ring_walk_kernel may have, dealt::ring_walk_kernel, which gives the same bits again, takes single steps of no more
+// 32-row q tiles than there are compute units, each of which holds one of its workgroups; under the diagonal, where the short walks of
+// a second round fill in behind the long ones, of twice as many.  us on thin and dealt: 8 heads x 1024 x 1024 15.6, 10.7 (256 workgroups), 6 x
+// 1500 x 1500 21.1, 23.9 (282), 16 x 1024 x 1024 16.1, 19.2 (512); causal 8 x 2048 x 2048 27.1, 19.2 (512).
+// RINGATTN_DEALT=0 and 1 in the environment: never, and whatever the size (comparisons, tests); RINGATTN_THIN names the other two.
+bool takes_dealt(const ringattn_plan* pl, const TableSlice& sl) {
+  if (std::getenv("RINGATTN_THIN")) return false;
+  const char* e = std::getenv("RINGATTN_DEALT");
+  if (e) return e[0] != '0';
+  const int64_t tiles = (int64_t)sl.seg_count * q_tiles_of(sl.q_len_max, ringattn::kDealtM) * pl->d.BH;
+  return tiles <= ringattn::kComputeUnits * (sl.walks.masked ? 2 : 1);
+}
+
 // steps::ring_split_kernel runs the launches of a plan that keep the ring steps apart -- single steps of one rank and of all, and
 // the forward with RINGATTN_FLAG_STEP_PARTIALS -- where even the largest of them are small.  Its partials have other bits than those of the
 // 256-row kernels, and all launches of a plan give the same: so it is for plans that lose nothing by it in any of
@@ -784,6 +797,11 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
   }
   const bool wide = slice_takes_walk64(pl, sl, a.mode);
   if (a.mode != ringattn::kBlockCarryState && !wide && takes_thin(pl, sl)) {
+    if (a.mode == ringattn::kBlockPartials && takes_dealt(pl, sl)) {
+      a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kDealtM);
+      RA_HIP(ringattn::launch_dealt(a, pl->p.dtype, stream));
+      return RINGATTN_OK;
+    }
     a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kThinM);
     RA_HIP(ringattn::launch_thin(a, pl->p.dtype, stream));
     return RINGATTN_OK;

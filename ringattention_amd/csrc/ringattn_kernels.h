@@ -11,6 +11,7 @@ constexpr int kWalkM = 256;   // query rows per workgroup of ring_walk_kernel (8
 constexpr int kSplitM = 32;   // query rows per workgroup of ring_split_kernel
 constexpr int kPairM = 128;  // query rows per workgroup of ring_pair_kernel
 constexpr int kThinM = 128;  // query rows per workgroup of thin::ring_walk_kernel
+constexpr int kDealtM = 32;  // query rows per workgroup of dealt::ring_walk_kernel
 constexpr int kMaxParts = 64; // partial slots a merge can combine
 constexpr int kComputeUnits = 256, kXcds = 8;
 
@@ -141,6 +142,8 @@ hipError_t launch_walk(BlockArgs a, const Walks& walks, int dtype, int dim, hipS
 hipError_t launch_steps(const BlockArgs& a, unsigned grid, int dtype, int dim, hipStream_t stream);
 // the same at d = 64 for launches that leave compute units idle, the ring steps apart (a.q_tiles_max counts tiles of kThinM rows)
 hipError_t launch_thin(BlockArgs a, int dtype, hipStream_t stream);
+// the same, kBlockPartials only, for launches of a few row tiles (a.q_tiles_max counts tiles of kDealtM rows)
+hipError_t launch_dealt(BlockArgs a, int dtype, hipStream_t stream);
 // ring_walk64_kernel: the carried-state forward at d = 128 with 64 query rows per wave; only for tables that
 // walk64_takes() accepts
 hipError_t launch_walk64(BlockArgs a, int dtype, int dim, hipStream_t stream);
