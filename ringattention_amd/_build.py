@@ -11,6 +11,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.environ.get("RINGATTN_LIB") or os.path.join(PKG_DIR, "libringattn.so")
 
 TORCH_LIB_PATH = os.path.join(PKG_DIR, "libringattn_torch.so")
+CALLS_PATH = os.path.join(PKG_DIR, "ringattn_calls.so")
 
 SOURCES = ["ringattn_kernels.hip", "ringattn_walk.hip", "ringattn_steps.hip", "ringattn_thin.hip", "ringattn_dealt.hip", "ringattn_walk64.hip", "ringattn_pair.hip", "ringattn_split.hip", "ringattn_split_steps.hip", "ringattn_split_columns.hip", "ringattn_api.hip", "ringattn_datagen.cpp"]
 
@@ -134,6 +135,36 @@ def build_torch_shim(verbose=False):
     return TORCH_LIB_PATH
 
 
+def calls_sources():
+    return [os.path.join(CSRC, "ringattn_calls.cpp")]
+
+
+def build_calls():
+    """Compile csrc/ringattn_calls.cpp (Python module, the host's part of a call) against the installed torch.  Host code only; the entry
+    points it calls come to it as addresses, so it links nothing of this package.  Always recompiles."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("g++ not found: cannot build ringattn_calls.so")
+    tmp = CALLS_PATH + ".tmp"
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}"]
+    for inc in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", inc]
+    cmd += [os.path.join(CSRC, "ringattn_calls.cpp"), "-o", tmp, "-L", torch_lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+            f"-Wl,-rpath,{torch_lib}"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("ringattn_calls build failed:\n" + " ".join(cmd) + "\n" + res.stdout + res.stderr)
+    os.replace(tmp, CALLS_PATH)
+    write_stamp(CALLS_PATH, calls_sources())
+    return CALLS_PATH
+
+
 def sanitizer_runtime():
     """Path of the AddressSanitizer runtime of hipcc's clang (to be preloaded into a python that
     loads a sanitized library)."""
@@ -184,3 +215,4 @@ if __name__ == "__main__":
     print(build_library(verbose=True))
     print(build_harness())
     print(build_torch_shim(verbose=True))
+    print(build_calls())

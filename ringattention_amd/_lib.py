@@ -6,11 +6,14 @@ The library must have been built (ringattention_amd._build.build_library or
 __graft_entry__.build); there is no fallback implementation.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
-from ._build import LIB_PATH
+from ._build import CALLS_PATH, LIB_PATH
 
 _lib = None
+_calls = None
 
 c_int_p = ctypes.POINTER(ctypes.c_int)
 c_float_p = ctypes.POINTER(ctypes.c_float)
@@ -87,6 +90,22 @@ def load():
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+def load_calls():
+    """The module ringattn_calls (csrc/ringattn_calls.cpp); raise if it has not been built."""
+    global _calls
+    if _calls is None:
+        if not os.path.exists(CALLS_PATH):
+            raise RuntimeError(
+                f"{CALLS_PATH} is missing: the call path has not been built. "
+                "Run `python -c 'import __graft_entry__ as g; g.build()'` at the repository root.")
+        loader = importlib.machinery.ExtensionFileLoader("ringattn_calls", CALLS_PATH)
+        spec = importlib.util.spec_from_file_location("ringattn_calls", CALLS_PATH, loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        _calls = module
+    return _calls
 
 
 class RingattnError(RuntimeError):

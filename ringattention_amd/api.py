@@ -27,7 +27,8 @@ LAYOUT_CODE = {"contiguous": 0, "zigzag": 1}
 # What a call costs besides its launch counts: a ring of some hundred tokens is a few microseconds of GPU work.  So the checks take
 # one look per tensor and describe what is wrong in a second one, shapes are a plan's own, addresses go to ctypes as they are
 # (every pointer argument is declared c_void_p), and the current stream is asked for without making an object of it.  us a call
-# of forward() on the host, before and after: 10.5, 6.3.
+# of forward() on the host, before and after: 10.5, 6.3.  Calls that are launched again and again with tensors of the caller's --
+# forward(), rank_step_forward() -- are checked and made by ringattn_calls (csrc/ringattn_calls.cpp) where everything fits: 6.8, 4.4.
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
@@ -131,8 +132,14 @@ class RingAttention:
         ws_ptr, ws_bytes = (None, 0) if workspace is None else (ctypes.c_void_p(int(workspace[0])), int(workspace[1]))
         check(self.lib.ringattn_plan_create(ctypes.byref(self.params), ws_ptr, ws_bytes, ctypes.byref(self.handle)),
               "ringattn_plan_create")
+        self._call_type = _lib.load_calls().Call
+        qkv = tuple((self.torch_dtype, s) for s in (self._q_shape, self._kv_shape, self._kv_shape))
+        self._forward_call = self._call_type(ctypes.cast(self.lib.ringattn_fwd, ctypes.c_void_p).value, self.handle.value, -1, 0,
+                                             qkv + ((self.torch_dtype, self._q_shape), (torch.float32, self._lse_shape)))
+        self._step_calls = {}   # by (rank, step), made when first asked for
 
     def close(self):
+        self._forward_call, self._step_calls = None, {}
         if self.handle:
             check(self.lib.ringattn_plan_destroy(self.handle), "ringattn_plan_destroy")
             self.handle = ctypes.c_void_p()
@@ -166,6 +173,12 @@ class RingAttention:
                 (v, "v", self.torch_dtype, kv_shape)]
 
     def forward(self, q, k, v, out=None, lse=None, stream=None):
+        call = self._forward_call
+        if out is not None and lse is not None and call is not None:
+            rc = call(q, k, v, out, lse, stream)
+            if rc is not None:
+                check(rc, "ringattn_fwd")
+                return out, lse
         dtype, kv_shape = self.torch_dtype, self._kv_shape
         if not (_fits(q, dtype, self._q_shape) and _fits(k, dtype, kv_shape) and _fits(v, dtype, kv_shape)):
             _check_tensors(*self._qkv_specs(q, k, v))
@@ -202,6 +215,11 @@ class RingAttention:
         o_part and lse_part are the rank's whole [B, H, rows, npes, d] / [B, H, rows, npes] buffers at every step."""
         if not (0 <= rank < self.npes and 0 <= step < self.npes):
             raise ValueError("rank and step must be in [0, npes)")
+        if o_part is not None and lse_part is not None and self.handle:
+            rc = (self._step_calls.get((rank, step)) or self._step_call(rank, step))(q, k_chunk, v_chunk, o_part, lse_part, stream)
+            if rc is not None:
+                check(rc, "ringattn_rank_step_fwd")
+                return o_part, lse_part
         q_shape, _, l_shape = self._rank_shapes[rank]
         o_shape = q_shape
         kv_shape = self._rank_shapes[(rank + step) % self.npes][1]
@@ -224,6 +242,15 @@ class RingAttention:
         check(self.lib.ringattn_rank_step_fwd(self.handle, int(rank), int(step), q.data_ptr(), k_chunk.data_ptr(), v_chunk.data_ptr(),
                                               o_part.data_ptr(), lse_part.data_ptr(), _stream_ptr(stream)), "ringattn_rank_step_fwd")
         return o_part, lse_part
+
+    def _step_call(self, rank, step):
+        q_shape, _, l_shape = self._rank_shapes[rank]
+        kv = (self.torch_dtype, self._rank_shapes[(rank + step) % self.npes][1])
+        o_shape, l_shape = self.rank_parts_shapes(rank) if self.row_partials else (q_shape, l_shape)
+        call = self._call_type(ctypes.cast(self.lib.ringattn_rank_step_fwd, ctypes.c_void_p).value, self.handle.value, int(rank), int(step),
+                               ((self.torch_dtype, q_shape), kv, kv, (self.part_dtype, o_shape), (torch.float32, l_shape)))
+        self._step_calls[int(rank), int(step)] = call
+        return call
 
     def rank_merge(self, rank, o_parts, lse_parts, out=None, lse=None, stream=None):
         """Merge of one rank's per-step partials [npes, B, H, rows, d] / [npes, B, H, rows]
