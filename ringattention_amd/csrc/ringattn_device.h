@@ -121,11 +121,15 @@ static __device__ __forceinline__ int lap_order(const BlockArgs& a, int w) {
 // segment as consecutive workgroups: everything that reads a head's K and V follows each other through that XCD's L2
 // (job_map in ringattn_jobs.h).
 // LAPS: compute units hold two workgroups (lap_order).
+// Launches of few workgroups do without that table (job_grid).
 template <int TILE_ROWS, bool LAPS = false>
 static __device__ __forceinline__ bool decode_job(const BlockArgs& a, Segment& seg, int& bh, int& qt) {
   const int place = blockIdx.x >> 3;
   int job;  // its number among those of its head
-  if (!job_of(a.map, a.causal, blockIdx.x & 7, LAPS ? lap_order(a, place) : place, bh, job)) return false;
+  if (a.few) {
+    job = quotient(blockIdx.x, a.by_heads);
+    bh = blockIdx.x - job * a.BH;
+  } else if (!job_of(a.map, a.causal, blockIdx.x & 7, LAPS ? lap_order(a, place) : place, bh, job)) return false;
   const int nth = quotient(job, a.by_q_tiles);
   const SegPtr sp = segs_of(a) + nth;
   seg.q_start = sp->q_start;
