@@ -246,8 +246,8 @@ int ringattn_plan_launch_times(ringattn_plan* plan, float* ms, int capacity, int
  * plan; others:
  * "ring_walk64_kernel" (every KV range a multiple of 32 keys, at least 128 and beginning within 4 GiB of its head; with
  * RINGATTN_FLAG_STEP_PARTIALS only at d = 128 in causal plans with at least 2048 keys per chunk) or "ring_walk_kernel".
- * RINGATTN_SPLIT, RINGATTN_SPLIT_STEPS, RINGATTN_PAIR, RINGATTN_THIN, RINGATTN_WIDE, RINGATTN_WIDE_D64 and RINGATTN_WIDE_PARTIALS in the
- * environment override.
+ * RINGATTN_SPLIT, RINGATTN_SPLIT_COLUMNS, RINGATTN_SPLIT_STEPS, RINGATTN_PAIR, RINGATTN_THIN, RINGATTN_DEALT, RINGATTN_WIDE,
+ * RINGATTN_WIDE_D64 and RINGATTN_WIDE_PARTIALS in the environment override.
  * All are restatements of the reference's one kernel (csrc/ring_attention.cu:398-666) with its tiling
  * (csrc/kernel_traits.h:11-177) replaced; the last two differ in how the 256 query rows of a workgroup are laid out over waves
  * (64 rows per wave at one wave per SIMD, or 32 rows per wave at two).  NULL for an invalid plan.

@@ -2,7 +2,7 @@
 //
 // A forward of a few hundred tokens, or one step of a short ring, is some 5 us of GPU work, and a launch costs the host 4.3 us of
 // its own.  The checks of five tensors, their addresses and the stream took Python another 2.2 (6.8 us a call of forward()); here they take
-// 0.3.  A Call holds one entry point of the C ABI with its plan and the shapes and types it expects.  Called with five tensors and a stream it
+// 0.2 (4.4).  A Call holds one entry point of the C ABI with its plan and the shapes and types it expects.  Called with five tensors and a stream it
 // returns the entry point's code, or None, without having done anything, where the arguments are not plainly what it
 // expects: the caller then goes the general way, which says what is wrong, or serves what is merely unusual (tensor subclasses).
 // Only addresses of this call's tensors are handed on; nothing of a tensor is kept.
