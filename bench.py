@@ -34,10 +34,10 @@ PEAK_HBM_GBS = 8000.0
 # (bytes, summary under profiles/, kernel, kernel_source_id(kernel) when it was measured).  The figure is only printed
 # while the forward still runs that kernel and its source is still the one that was profiled.
 MEASURED_TRAFFIC = {
-    "cfg4": (2282e6, "profiles/ring_walk64_kernel_cfg4.md", "ring_walk64_kernel", "0f7fdaa0c1c3f628"),
-    "cfg3": (1623e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "0f7fdaa0c1c3f628"),
-    "cfg5": (46836e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "0f7fdaa0c1c3f628"),
-    "cfg2": (34.2e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "0f7fdaa0c1c3f628"),
+    "cfg4": (2318e6, "profiles/ring_walk64_kernel_cfg4.md", "ring_walk64_kernel", "f5cf3ad4e6b41949"),
+    "cfg3": (1623e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "f5cf3ad4e6b41949"),
+    "cfg5": (47589e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "f5cf3ad4e6b41949"),
+    "cfg2": (34.2e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "f5cf3ad4e6b41949"),
 }
 KERNEL_SOURCES = {
     "ring_walk64_kernel": ("ringattn_walk64.hip", "ringattn_walk64_loop.inc", "ringattn_walk64_loop_d64.inc", "ringattn_device.h"),

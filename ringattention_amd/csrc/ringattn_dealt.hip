@@ -54,6 +54,7 @@ __global__ __launch_bounds__(64 * (kScoreWaves + 2), 2) void ring_walk_kernel(co
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
 
+  fetch_arguments(a);
   Segment seg;
   int bh, qt;
   if (!decode_job<BM>(a, seg, bh, qt)) return;

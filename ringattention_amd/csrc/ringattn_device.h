@@ -108,6 +108,16 @@ static __device__ __forceinline__ SegPtr segs_of(const BlockArgs& a) {
   return a.items ? (SegPtr)(uintptr_t)a.segs : (SegPtr)(args + offsetof(BlockArgs, one_seg));
 }
 
+// Asks for the arguments that the start of a workgroup goes by, all at once: left to itself the compiler asks for each where it needs it, six
+// round trips one after the other in front of the first tile load.  us a step before and after: 4 heads x 512 rows, d = 64 5.91, 5.77, 8 x 1024 10.35, 10.19;
+// 8 x 256, d = 128 7.22, 7.11.  (ring_split_kernel with the state carried: no difference, and none made.)
+static __device__ __forceinline__ void fetch_arguments(const BlockArgs& a) {
+  asm volatile("" ::"s"(a.q), "s"(a.k), "s"(a.v), "s"(a.segs), "s"(a.items), "s"(a.bh_stride), "s"(a.kv_bh_stride), "s"(a.q_tiles_max), "s"(a.BH),
+               "s"(a.by_group.mul), "s"(a.by_group.shift), "s"(a.scale_log2), "s"(a.by_q_tiles.mul), "s"(a.by_q_tiles.shift), "s"(a.few),
+               "s"(a.by_heads.mul), "s"(a.by_heads.shift), "s"(a.one_seg.q_start), "s"(a.one_seg.q_len), "s"(a.one_seg.item_begin), "s"(a.one_seg.item_count),
+               "s"(a.one_seg.reverse_tiles), "s"(a.one_item.kv_start), "s"(a.one_item.kv_len), "s"(a.one_item.diag_off));
+}
+
 // An XCD hands its workgroups to its 32 compute units in turn.  Where a compute unit holds two, the first 32 jobs, longest walk first,
 // are the first ones of the compute units and the next 32 the second ones: those run shortest first (a.second_lap: how many
 // of the XCD's first 64 there are; 0: as they come), so that long walks share a compute unit with short ones.
@@ -131,13 +141,17 @@ static __device__ __forceinline__ bool decode_job(const BlockArgs& a, Segment& s
     bh = blockIdx.x - job * a.BH;
   } else if (!job_of(a.map, a.causal, blockIdx.x & 7, LAPS ? lap_order(a, place) : place, bh, job)) return false;
   const int nth = quotient(job, a.by_q_tiles);
-  const SegPtr sp = segs_of(a) + nth;
-  seg.q_start = sp->q_start;
-  seg.q_len = sp->q_len;
-  seg.item_begin = sp->item_begin;
-  seg.item_count = sp->item_count;
-  seg.last_item = sp->last_item;
-  seg.reverse_tiles = sp->reverse_tiles;
+  if (!a.items) {
+    seg = a.one_seg;
+  } else {
+    const SegPtr sp = segs_of(a) + nth;
+    seg.q_start = sp->q_start;
+    seg.q_len = sp->q_len;
+    seg.item_begin = sp->item_begin;
+    seg.item_count = sp->item_count;
+    seg.last_item = sp->last_item;
+    seg.reverse_tiles = sp->reverse_tiles;
+  }
   qt = job - nth * a.q_tiles_max;
   if (qt * TILE_ROWS >= seg.q_len) return false;  // segments shorter than the longest one
   if (seg.reverse_tiles) qt = (seg.q_len + TILE_ROWS - 1) / TILE_ROWS - 1 - qt;  // most keys first

@@ -76,6 +76,7 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
 
+  if (!KEEP) fetch_arguments(a);
   Segment seg;
   int bh, qt;
   if (!decode_job<BM>(a, seg, bh, qt)) return;
@@ -168,9 +169,9 @@ static __device__ __forceinline__ void split_rows(const BlockArgs& a, unsigned c
   auto enter = [&]() {  // t may lie beyond the item: on to the one that holds it; false past the last
     for (; item < n_items; ++item) {
       const ItemPtr w = items + item;
-      len = w->kv_len;
-      diag = w->diag_off;
-      start = w->kv_start;
+      len = a.items ? w->kv_len : a.one_item.kv_len;
+      diag = a.items ? w->diag_off : a.one_item.diag_off;
+      start = a.items ? w->kv_start : a.one_item.kv_start;
       tiles = (len + BN - 1) / BN;
       if (diag >= 0) tiles = min(tiles, (diag + q_last) / BN + 1);
       if (t < tiles) return true;
