@@ -712,14 +712,16 @@ bool takes_thin(const ringattn_plan* pl, const TableSlice& sl) {
 // 32-row q tiles than there are compute units, each of which holds one of its workgroups; under the diagonal, where the short walks of
 // a second round fill in behind the long ones, of twice as many.  us on thin and dealt: 8 heads x 1024 x 1024 15.6, 10.7 (256 workgroups), 6 x
 // 1500 x 1500 21.1, 23.9 (282), 16 x 1024 x 1024 16.1, 19.2 (512); causal 8 x 2048 x 2048 27.1, 19.2 (512).
-// A walk that is over within a round has nothing to share out: 64 heads x 64 x 64 4.8, 5.4, 8 x 60 x 60 5.0, 5.2; 32 x 128 x 128 5.9, 5.3.
+// A walk that is over within a round has nothing to share out: 64 heads x 64 x 64 4.8, 5.4, 8 x 60 x 60 5.0, 5.2; 32 x 128 x 128 5.9, 5.3.  And a
+// move of the references costs a round of short walks more than it gains, with N(0, 81) logits: 32 x 128 x 128 6.6, 6.9, 8 x 256 x 256 8.4, 8.8,
+// 4 x 384 x 384 10.3, 9.6; under the diagonal 32 x 128 x 128 7.3, 6.9, 8 x 256 x 256 8.9, 8.5.
 // RINGATTN_DEALT=0 and 1 in the environment: never, and whatever the size (comparisons, tests); RINGATTN_THIN names the other two.
 bool takes_dealt(const ringattn_plan* pl, const TableSlice& sl) {
   if (std::getenv("RINGATTN_THIN")) return false;
   const char* e = std::getenv("RINGATTN_DEALT");
   if (e) return e[0] != '0';
   const int64_t tiles = (int64_t)sl.seg_count * q_tiles_of(sl.q_len_max, ringattn::kDealtM) * pl->d.BH;
-  return sl.walks.longest >= 4 && tiles <= ringattn::kComputeUnits * (sl.walks.masked ? 2 : 1);
+  return sl.walks.longest >= (sl.walks.masked ? 4 : 12) && tiles <= ringattn::kComputeUnits * (sl.walks.masked ? 2 : 1);
 }
 
 // steps::ring_split_kernel runs the launches of a plan that keep the ring steps apart -- single steps of one rank and of all, and

@@ -100,8 +100,10 @@ def test_bits_of_ring_walk_kernel(monkeypatch, lens, causal, zigzag, kind, half,
 @pytest.mark.parametrize("tokens,heads,step,threads", [
     (1024, 8, 1, 384),     # 256 q tiles of 32 rows
     (1024, 9, 1, 256),     # thin::ring_walk_kernel
-    (97, 8, 1, 384),       # four tiles
-    (96, 8, 1, 256),       # three
+    (353, 8, 1, 384),      # twelve tiles
+    (352, 8, 1, 256),
+    (97, 8, 0, 384),       # four, under the diagonal
+    (96, 8, 0, 256),
     (1024, 16, 0, 384),    # 512 under the diagonal
     (1056, 16, 0, 256),
 ])
