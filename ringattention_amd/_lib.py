@@ -88,6 +88,8 @@ def load():
         fn = getattr(lib, name)
         fn.restype = restype
         fn.argtypes = argtypes
+    # where the entry points lie that ringattn_calls calls
+    lib.addresses = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in ("ringattn_fwd", "ringattn_rank_step_fwd")}
     _lib = lib
     return lib
 

@@ -7,6 +7,7 @@
 the stream; every computation goes through libringattn.so.
 """
 import ctypes
+from operator import index
 
 import numpy as np
 import torch
@@ -133,10 +134,7 @@ class RingAttention:
         check(self.lib.ringattn_plan_create(ctypes.byref(self.params), ws_ptr, ws_bytes, ctypes.byref(self.handle)),
               "ringattn_plan_create")
         self._call_type = _lib.load_calls().Call
-        qkv = tuple((self.torch_dtype, s) for s in (self._q_shape, self._kv_shape, self._kv_shape))
-        self._forward_call = self._call_type(ctypes.cast(self.lib.ringattn_fwd, ctypes.c_void_p).value, self.handle.value, -1, 0,
-                                             qkv + ((self.torch_dtype, self._q_shape), (torch.float32, self._lse_shape)))
-        self._step_calls = {}   # by (rank, step), made when first asked for
+        self._forward_call, self._step_calls = None, {}   # made when first asked for; the steps' by (rank, step)
 
     def close(self):
         self._forward_call, self._step_calls = None, {}
@@ -173,9 +171,8 @@ class RingAttention:
                 (v, "v", self.torch_dtype, kv_shape)]
 
     def forward(self, q, k, v, out=None, lse=None, stream=None):
-        call = self._forward_call
-        if out is not None and lse is not None and call is not None:
-            rc = call(q, k, v, out, lse, stream)
+        if out is not None and lse is not None and self.handle:
+            rc = (self._forward_call or self._make_forward_call())(q, k, v, out, lse, stream)
             if rc is not None:
                 check(rc, "ringattn_fwd")
                 return out, lse
@@ -191,6 +188,12 @@ class RingAttention:
         check(self.lib.ringattn_fwd(self.handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
                                     _stream_ptr(stream)), "ringattn_fwd")
         return out, lse
+
+    def _make_forward_call(self):
+        q, kv = (self.torch_dtype, self._q_shape), (self.torch_dtype, self._kv_shape)
+        self._forward_call = call = self._call_type(self.lib.addresses["ringattn_fwd"], self.handle.value, -1, 0,
+                                                    (q, kv, kv, q, (torch.float32, self._lse_shape)))
+        return call
 
     def block_forward(self, step, q, k, v, o_part=None, lse_part=None, stream=None):
         specs = self._qkv_specs(q, k, v)
@@ -216,7 +219,8 @@ class RingAttention:
         if not (0 <= rank < self.npes and 0 <= step < self.npes):
             raise ValueError("rank and step must be in [0, npes)")
         if o_part is not None and lse_part is not None and self.handle:
-            rc = (self._step_calls.get((rank, step)) or self._step_call(rank, step))(q, k_chunk, v_chunk, o_part, lse_part, stream)
+            at = (index(rank), index(step))
+            rc = (self._step_calls.get(at) or self._step_call(*at))(q, k_chunk, v_chunk, o_part, lse_part, stream)
             if rc is not None:
                 check(rc, "ringattn_rank_step_fwd")
                 return o_part, lse_part
@@ -247,9 +251,9 @@ class RingAttention:
         q_shape, _, l_shape = self._rank_shapes[rank]
         kv = (self.torch_dtype, self._rank_shapes[(rank + step) % self.npes][1])
         o_shape, l_shape = self.rank_parts_shapes(rank) if self.row_partials else (q_shape, l_shape)
-        call = self._call_type(ctypes.cast(self.lib.ringattn_rank_step_fwd, ctypes.c_void_p).value, self.handle.value, int(rank), int(step),
+        call = self._call_type(self.lib.addresses["ringattn_rank_step_fwd"], self.handle.value, rank, step,
                                ((self.torch_dtype, q_shape), kv, kv, (self.part_dtype, o_shape), (torch.float32, l_shape)))
-        self._step_calls[int(rank), int(step)] = call
+        self._step_calls[rank, step] = call
         return call
 
     def rank_merge(self, rank, o_parts, lse_parts, out=None, lse=None, stream=None):

@@ -3,6 +3,7 @@ expects: everything else must fare as on the general way -- what was refused is 
 and a closed plan is out of its reach."""
 import threading
 
+import numpy as np
 import pytest
 import torch
 
@@ -30,13 +31,17 @@ def steps_of(plan, tensors):
 
 def test_host_tensors_are_refused_in_words():
     plan, t = plan_and_tensors("cpu")
-    assert plan._forward_call(*t, None) is None
     with pytest.raises(ValueError, match="q must be a device tensor"):
         plan.forward(*t)
+    assert plan._forward_call(*t, None) is None
     with pytest.raises(ValueError, match="q must be a device tensor"):
         plan.rank_step_forward(1, 1, *steps_of(plan, t))
     with pytest.raises(ValueError, match="rank and step"):
         plan.rank_step_forward(2, 0, *t)
+    with pytest.raises(TypeError):
+        plan.rank_step_forward(1.0, 1, *steps_of(plan, t))
+    with pytest.raises(ValueError, match="q must be a device tensor"):
+        plan.rank_step_forward(np.array(1), True, *steps_of(plan, t))
     plan.close()
     assert plan._forward_call is None
 
@@ -132,6 +137,7 @@ def test_both_ways_give_the_same():
 @pytest.mark.gpu
 def test_batched_tensors_have_no_address():
     plan, t = plan_and_tensors("cuda")
+    plan.forward(*t)
     stacked = torch.stack([t[0], t[0]])
 
     def one(q):
