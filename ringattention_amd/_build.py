@@ -55,7 +55,7 @@ def source_id(paths):
 
 
 def library_sources():
-    return [os.path.join(CSRC, s) for s in SOURCES] + [os.path.join(CSRC, "ringattn_kernels.h"), os.path.join(CSRC, "ringattn_jobs.h"), os.path.join(CSRC, "ringattn_device.h"),
+    return [os.path.join(CSRC, s) for s in SOURCES] + [os.path.join(CSRC, "ringattn_kernels.h"), os.path.join(CSRC, "ringattn_jobs.h"), os.path.join(CSRC, "ringattn_news.h"), os.path.join(CSRC, "ringattn_device.h"),
                                                        os.path.join(CSRC, "ringattn_walk_rows.h"),
                                                        os.path.join(CSRC, "ringattn_split_rows.h"),
                                                        os.path.join(CSRC, "ringattn_walk64_loop.inc"),

@@ -13,7 +13,10 @@
 //           waves 0-3, round r :  S(r+1) = K Q^T  |  P(r), its sums, the wish   -> LDS, barrier, whose wish?
 //           waves 4-5, round r :  barrier, whose wish?  O += P(r) V(r), read V(r+1)
 //       probs, row_sums, factors and news are double-buffered by round: those of round r are read before the barrier of round r+1, and
-//       written again behind it.  K tiles belong to the wave that loads them; V tiles are loaded half by one, half by the other wave of P V: a
+//       those of a round without a move are written again behind it.  In a round with one the tile that moves writes its probs, row_sums and
+//       news again, and the tiles behind it theirs a barrier later, while others may still be reading what stood there: of the first two
+//       they then have something of each, and read again behind the last barrier of the round; the news say the same to who
+//       reads early and who reads late (ringattn_news.h).  K tiles belong to the wave that loads them; V tiles are loaded half by one, half by the other wave of P V: a
 //       wave passes the barrier of round r with its part of V(r+1) landed, and with V(r) in its registers.
 //       A step of 8 heads x 1024 rows is 64 workgroups of thin::ring_walk_kernel whose waves walk 32 tiles each; here it is 256, with eight
 //       rounds.  us on thin::ring_walk_kernel and here: 8 heads x 1024 rows x 1024 keys 15.6, 10.7; 4 x 2048 x 2048 26.3, 16.0; 2 x 4096
@@ -23,6 +26,7 @@
 //       exponentials at 16 cycles, and 54 scalar ones) and spends the rest on the way through LDS: P out, barrier, wishes in.  Eight tiles a
 //       round with eight waves, and V loaded column by column, took as long a tile.
 #include "ringattn_walk_rows.h"
+#include "ringattn_news.h"
 
 #include <utility>
 
@@ -47,7 +51,7 @@ __global__ __launch_bounds__(64 * (kScoreWaves + 2), 2) void ring_walk_kernel(co
   __shared__ s16x8 probs[2][W][2][64];   // the probabilities of a round, as the lanes hold them
   __shared__ f32x4 row_sums[2][W][64];   // their sums of four
   __shared__ float factors[2][W][BM];    // where a tile moved the references: what the sums so far are multiplied by
-  __shared__ __attribute__((aligned(16))) int news[2][W];  // bit 0: its tile wants to move the references, bit 8: it has done so
+  __shared__ __attribute__((aligned(16))) int news[2][W];  // kNewsWish, kNewsMoved or neither
   __shared__ float reference[BM];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -75,9 +79,8 @@ __global__ __launch_bounds__(64 * (kScoreWaves + 2), 2) void ring_walk_kernel(co
   auto barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
   typedef int i32x4 __attribute__((ext_vector_type(4)));
   auto read_news = [&](int r) { return *(const i32x4*)news[r & 1]; };
-  auto bits_of = [&](const i32x4& x) { return __builtin_amdgcn_readfirstlane(x[0] | x[1] << 1 | x[2] << 2 | x[3] << 3); };
-  // which tile of the round is the first, from tile `from` on, that wants to move the references: W for none
-  auto first_wish = [&](int bits, int from) { return from + __builtin_ctz(((bits & ((1 << W) - 1)) | 1 << W) >> from); };
+  static_assert(W == kNewsTiles, "news_of_round");
+  auto bits_of = [&](const i32x4& x) { return __builtin_amdgcn_readfirstlane(news_of_round(x[0], x[1], x[2], x[3])); };
 
   if (wave < W) {
     // ---- a wave of scores
@@ -220,7 +223,7 @@ __global__ __launch_bounds__(64 * (kScoreWaves + 2), 2) void ring_walk_kernel(co
 #pragma unroll
         for (int k = kHead + (kSteps - kHead) * ks / KS; k < kHead + (kSteps - kHead) * (ks + 1) / KS; ++k) exp_step(k);
       }
-      hand_over(u < n_tiles && wish());
+      hand_over(u < n_tiles && wish() ? kNewsWish : 0);
       // K of the round after the next one: two rounds' loads may be in flight
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kAhead - 2) * PIECES) : "memory");
       barrier();
@@ -236,7 +239,7 @@ __global__ __launch_bounds__(64 * (kScoreWaves + 2), 2) void ring_walk_kernel(co
           const float alpha = __builtin_amdgcn_exp2f(m * a.scale_log2 - cs);
           set_reference(cand);
           exponentials();
-          hand_over(1 << 8);
+          hand_over(kNewsMoved);
           if (h == 0) {
             factors[r & 1][wave][n] = alpha;
             reference[n] = m;
@@ -248,7 +251,7 @@ __global__ __launch_bounds__(64 * (kScoreWaves + 2), 2) void ring_walk_kernel(co
         if (from == W) break;
         if (wave >= from) {
           exponentials();
-          hand_over(u < n_tiles && wish());
+          hand_over(u < n_tiles && wish() ? kNewsWish : 0);
         }
         barrier();
       }
@@ -344,7 +347,7 @@ __global__ __launch_bounds__(64 * (kScoreWaves + 2), 2) void ring_walk_kernel(co
       read_p();
       if (from == W) break;
     }
-    const int moves = bits_of(said >> 8);
+    const int moves = bits_of(said >> kNewsMovedBit);
     read_v(r + 1, vfr[ODD ^ 1]);
 #pragma unroll
     for (int i = 0; i < W; ++i) {
