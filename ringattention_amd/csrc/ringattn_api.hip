@@ -331,8 +331,12 @@ static int split_choice() {  // -1: unset
 // 8.7, 8.4, x 256 37.8, 30.2, 29.3; 64 x 64 14.5, 12.3, 12.4, x 512 75.6, 59.6, 67.6; 96 x 96 18.8, 16.3, 28.1; 128 x 128 22.6, 21.6,
 // 37.1; 256 x 64 17.3, 24.8.  d = 64, all and 32: 32 x 32 6.9, 6.4; 64 x 64 9.4, 9.1, x 512 40.7, 39.5; 75 x 25 6.5, 6.2; 96 x 96 12.0, 11.9;
 // 128 x 128 14.4, 14.6, x 256 23.7, 25.3.
+// A caller may have O, or fp16 partials, written over Q.  That is all right while one workgroup reads a row of Q and writes it; with the columns
+// dealt out one of them could have stored its part before another has read the row, so such a launch keeps all columns.
 // RINGATTN_SPLIT_COLUMNS in the environment: 32, 64 or 128, at most the head dimension (comparisons, tests).
-static int split_columns(int64_t row_tiles, int dim) {
+static int split_columns(const ringattn::BlockArgs& a, int dim) {
+  if ((a.mode == ringattn::kBlockCarryState ? a.out : a.o_part) == a.q) return dim;
+  const int64_t row_tiles = (int64_t)a.n_segs * a.q_tiles_max * a.BH;
   const char* e = std::getenv("RINGATTN_SPLIT_COLUMNS");
   const int asked = e ? std::atoi(e) : 0;
   if (asked == 32 || asked == 64 || asked == 128) return std::min(asked, dim);
@@ -771,7 +775,7 @@ hipError_t launch_q_tiles(ringattn::BlockArgs& a, CarryKernel kernel, bool wide,
     case CarryKernel::kSplit:
     case CarryKernel::kSplit16:
       a.q_tiles_max = q_tiles_of(q_len, ringattn::kSplitM);
-      return ringattn::launch_split(a, dtype, dim, kernel == CarryKernel::kSplit16, split_columns((int64_t)a.n_segs * a.q_tiles_max * a.BH, dim), stream);
+      return ringattn::launch_split(a, dtype, dim, kernel == CarryKernel::kSplit16, split_columns(a, dim), stream);
     default:
       a.q_tiles_max = q_tiles_of(q_len);
       return wide ? ringattn::launch_walk64(a, dtype, dim, stream) : ringattn::launch_walk(a, walks, dtype, dim, stream);
@@ -794,7 +798,7 @@ int launch_slice(ringattn_plan* pl, const TableSlice& sl, ringattn::BlockArgs& a
   a.n_segs = sl.seg_count;
   if (a.mode != ringattn::kBlockCarryState && takes_split_steps(pl)) {
     a.q_tiles_max = q_tiles_of(sl.q_len_max, ringattn::kSplitM);
-    const int columns = a.mode == ringattn::kBlockPartials ? split_columns((int64_t)a.n_segs * a.q_tiles_max * a.BH, pl->p.dim) : pl->p.dim;
+    const int columns = a.mode == ringattn::kBlockPartials ? split_columns(a, pl->p.dim) : pl->p.dim;
     RA_HIP(ringattn::launch_split_steps(a, pl->p.dtype, pl->p.dim, columns, stream));
     return RINGATTN_OK;
   }

@@ -126,6 +126,37 @@ def test_how_many_columns(monkeypatch, dim, tokens, columns):
         plan.close()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["forward", "call", "step", "block"])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_results_over_q(monkeypatch, dim, kind):
+    """O, or fp16 partials, written over Q: a row of Q is read by the workgroup that writes it, so all columns are its own."""
+    H, S = (1 if kind == "call" else 3), 300
+    (q, k, v), lse = tensors(dim, torch.float16, *[(S,) if kind == "call" else (1, H, S)] * 3), torch.empty(1, H, S, device="cuda")
+    plan = api.RingAttention(1, S, dim, 1, H, "fp16", True, half_partials=True)
+    call = {
+        "forward": lambda q, out, stream=None: plan.forward(q, k, v, out, lse, stream),
+        "call": lambda q, out, stream=None: api.ring_attention_noalloc(q, k, v, out, 1, 0, [S], dim, S, causal=True, stream=stream),
+        "step": lambda q, out, stream=None: plan.rank_step_forward(0, 0, q, k, v, out, lse, stream),
+        "block": lambda q, out, stream=None: plan.block_forward(0, q, k, v, out, lse, stream),
+    }[kind]
+    monkeypatch.setenv(*(("RINGATTN_SPLIT", "8") if kind in ("forward", "call") else ("RINGATTN_SPLIT_STEPS", "1")))
+    out = torch.empty_like(q)
+    try:
+        some, over = kernels(lambda stream: call(q, out, stream)), kernels(lambda stream: call(q, q, stream))
+        monkeypatch.setenv("RINGATTN_SPLIT_COLUMNS", "32")
+        assert kernels(lambda stream: call(q, out, stream)) == some != over and kernels(lambda stream: call(q, q, stream)) == over
+        monkeypatch.setenv("RINGATTN_SPLIT_COLUMNS", "128")
+        assert kernels(lambda stream: call(q, out, stream)) == over
+        call(q, out)
+        monkeypatch.delenv("RINGATTN_SPLIT_COLUMNS")
+        call(q, q)
+        torch.cuda.synchronize()
+        assert torch.equal(q.view(torch.int16), out.view(torch.int16))
+    finally:
+        plan.close()
+
+
 def test_resources_and_hazards(tmp_path):
     """Two waves per SIMD at d = 128, four at d = 64 (two workgroups of eight waves on a compute unit), no scratch; and the wait states
     in front of the direct-to-LDS loads."""
