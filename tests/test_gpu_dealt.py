@@ -106,6 +106,10 @@ def test_bits_of_ring_walk_kernel(monkeypatch, lens, causal, zigzag, kind, half,
     (96, 8, 0, 256),
     (1024, 16, 0, 384),    # 512 under the diagonal
     (1056, 16, 0, 256),
+    (512, 16, 0, 384),     # 256
+    (512, 17, 0, 256),     # 272 of sixteen tiles
+    (544, 16, 0, 384),     # 272 of seventeen
+    (223, 64, 0, 256),     # 448 of seven
 ])
 def test_which_launches_it_is_chosen_for(monkeypatch, tokens, heads, step, threads):
     monkeypatch.setenv("RINGATTN_SPLIT_STEPS", "0")
