@@ -9,11 +9,12 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import warnings
 
 from ._build import CALLS_PATH, LIB_PATH
 
 _lib = None
-_calls = None
+_calls = None   # the module, once loaded; False where it cannot be
 
 c_int_p = ctypes.POINTER(ctypes.c_int)
 c_float_p = ctypes.POINTER(ctypes.c_float)
@@ -95,19 +96,20 @@ def load():
 
 
 def load_calls():
-    """The module ringattn_calls (csrc/ringattn_calls.cpp); raise if it has not been built."""
+    """The module ringattn_calls (csrc/ringattn_calls.cpp), or None: a library that was built without it (make needs no Python), or next
+    to one made for another torch, is called by way of ctypes alone, some 2 us a call slower on the host."""
     global _calls
-    if _calls is None:
-        if not os.path.exists(CALLS_PATH):
-            raise RuntimeError(
-                f"{CALLS_PATH} is missing: the call path has not been built. "
-                "Run `python -c 'import __graft_entry__ as g; g.build()'` at the repository root.")
-        loader = importlib.machinery.ExtensionFileLoader("ringattn_calls", CALLS_PATH)
-        spec = importlib.util.spec_from_file_location("ringattn_calls", CALLS_PATH, loader=loader)
-        module = importlib.util.module_from_spec(spec)
-        loader.exec_module(module)
-        _calls = module
-    return _calls
+    if _calls is None and os.path.exists(CALLS_PATH):
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("ringattn_calls", CALLS_PATH)
+            spec = importlib.util.spec_from_file_location("ringattn_calls", CALLS_PATH, loader=loader)
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+            _calls = module
+        except ImportError as e:
+            warnings.warn(f"{CALLS_PATH} cannot be loaded ({e}): calls go by way of ctypes")
+            _calls = False
+    return _calls or None
 
 
 class RingattnError(RuntimeError):

@@ -133,11 +133,12 @@ class RingAttention:
         ws_ptr, ws_bytes = (None, 0) if workspace is None else (ctypes.c_void_p(int(workspace[0])), int(workspace[1]))
         check(self.lib.ringattn_plan_create(ctypes.byref(self.params), ws_ptr, ws_bytes, ctypes.byref(self.handle)),
               "ringattn_plan_create")
-        self._call_type = _lib.load_calls().Call
+        calls = _lib.load_calls()
+        self._call_type = calls and calls.Call   # None: every call goes the general way
         self._forward_call, self._step_calls = None, {}   # made when first asked for; the steps' by (rank, step)
 
     def close(self):
-        self._forward_call, self._step_calls = None, {}
+        self._call_type, self._forward_call, self._step_calls = None, None, {}
         if self.handle:
             check(self.lib.ringattn_plan_destroy(self.handle), "ringattn_plan_destroy")
             self.handle = ctypes.c_void_p()
@@ -171,7 +172,7 @@ class RingAttention:
                 (v, "v", self.torch_dtype, kv_shape)]
 
     def forward(self, q, k, v, out=None, lse=None, stream=None):
-        if out is not None and lse is not None and self.handle:
+        if out is not None and lse is not None and self._call_type:
             rc = (self._forward_call or self._make_forward_call())(q, k, v, out, lse, stream)
             if rc is not None:
                 check(rc, "ringattn_fwd")
@@ -218,7 +219,7 @@ class RingAttention:
         o_part and lse_part are the rank's whole [B, H, rows, npes, d] / [B, H, rows, npes] buffers at every step."""
         if not (0 <= rank < self.npes and 0 <= step < self.npes):
             raise ValueError("rank and step must be in [0, npes)")
-        if o_part is not None and lse_part is not None and self.handle:
+        if o_part is not None and lse_part is not None and self._call_type:
             at = (index(rank), index(step))
             rc = (self._step_calls.get(at) or self._step_call(*at))(q, k_chunk, v_chunk, o_part, lse_part, stream)
             if rc is not None:

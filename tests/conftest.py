@@ -41,6 +41,8 @@ def built_artifacts():
         _build.build_library()
     if not _build.is_current(_build.TORCH_LIB_PATH, _build.torch_shim_sources()):
         _build.build_torch_shim()
+    if not _build.is_current(_build.CALLS_PATH, _build.calls_sources()):
+        _build.build_calls()
     if not _build.is_current(_build.HARNESS_PATH, _build.harness_sources()):
         _build.build_harness()
     from oracle import build as oracle_build

@@ -59,6 +59,40 @@ def test_arguments_of_a_call():
     assert call(1, 2, 3, 4, 5, None) is None and call(*(None,) * 6) is None
 
 
+@pytest.fixture(params=["not built", "not loadable"])
+def without_module(request, monkeypatch, tmp_path):
+    """A library made by make, which does not build the module, or next to a module made for another torch."""
+    path = tmp_path / "ringattn_calls.so"
+    if request.param == "not loadable":
+        path.write_bytes(b"not a library")
+    monkeypatch.setattr(_lib, "CALLS_PATH", str(path))
+    monkeypatch.setattr(_lib, "_calls", None)
+
+
+@pytest.mark.filterwarnings("ignore:.*cannot be loaded")
+def test_a_plan_does_without_the_module(without_module):
+    plan, t = plan_and_tensors("cpu")
+    for call, args in ((plan.forward, t), (lambda *a: plan.rank_step_forward(1, 1, *a), steps_of(plan, t))):
+        with pytest.raises(ValueError, match="q must be a device tensor"):
+            call(*args)
+    plan.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:.*cannot be loaded")
+def test_results_without_the_module(without_module):
+    plan, t = plan_and_tensors("cuda")
+    s = steps_of(plan, t)
+    plan.forward(*t)
+    plan.rank_step_forward(1, 1, *s)
+    assert plan._forward_call is None and not plan._step_calls
+    o, l = plan.forward(*t[:3])
+    p, m = plan.rank_step_forward(1, 1, *s[:3])
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(t[3:] + s[3:], (o, l, p, m)))
+    plan.close()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 def test_what_does_not_fit_is_refused_as_ever(dtype):
