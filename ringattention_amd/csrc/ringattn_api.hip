@@ -366,7 +366,8 @@ static int pair_choice() {
 //     9 heads x 8192 (288 q tiles of 256)  355, 310, 437     244, 208, 223
 //     16 heads x 8192, causal              221, 245, 424     142, 159, 209
 // ring_split_kernel has since become 5 to 30 % faster where compute units idle (its file) and 5 % elsewhere, so the third row of either table
-// below overstates it by that much and draws lines, but does not give its times.  It is left, because the lines
+// below overstates it by that much and draws lines, but does not give its times.  (What the columns gain on top of that, split_columns, is no matter to the
+// lines: of 56 000 drawn forwards of so few row tiles every one is on ring_split_kernel.)  It is left, because the lines
 // are those between equals: with new numbers d = 64 launches moved to it that both kernels run alike (us on
 // ring_split_kernel and ring_pair_kernel: causal 8 x 4928 47, 48; 12 x 3054 33, 34; 4 x 10816 97, 94; no mask 6 x 3394 39, 38; 1 x
 // 20971 184, 164), and at d = 128 some whose second round of workgroups is mostly empty (4 x 3328 43.5, 40.6).
@@ -735,14 +736,18 @@ bool takes_dealt(const ringattn_plan* pl, const TableSlice& sl) {
 
 // steps::ring_split_kernel runs the launches of a plan that keep the ring steps apart -- single steps of one rank and of all, and
 // the forward with RINGATTN_FLAG_STEP_PARTIALS -- where even the largest of them are small.  Its partials have other bits than those of the
-// 256-row kernels, and all launches of a plan give the same: so it is for plans that lose nothing by it in any of
-// the three, whichever a program calls.  Those of one step stop gaining where there are more 32-row q tiles than a round of
-// workgroups, but the longer their walks the later, the forward where the 256-row kernels fill the device.  Over 6500 drawn
-// plans (P 1 to 32, 600 to 60 000 rows, logits N(0, 1) and N(0, 81)) the lines leave these shares of the time on the kernels
-// before, geometric mean (the worst of fifty in brackets) of a rank's step, a step of all and the forward: d = 64 0.69 (1.05), 0.75 (1.08), 0.63 (0.95), under the
-// mask 0.67 (1.04), 0.69 (1.08), 0.57 (0.93); d = 128 0.59 (1.08), 0.64 (1.10), 0.51 (0.88), under the mask 0.56 (1.08), 0.60 (1.08), 0.45 (0.74).  us before and after: d = 64,
-// 4 heads x 4 x 512 9.9, 10.1, 29.9 and 6.2, 6.9, 17.7, 2 x 4 x 2048 25.6, 27.6, 94 and 10.1, 19.1, 65; d = 128, 8 heads x 8 x 256 12.9, 14.3,
-// 56 and 7.0, 14.8, 47, causal 4 x 4 x 777 29.5, 29.7, 100 and 11.9, 11.8, 42.  Beyond them, d = 64, 8 heads x 8 x 1024: 15.6, 30.3, 181 and 8.4, 45, 296.
+// 256-row kernels, and all launches of a plan give the same, so there is one choice for the three, whichever a program
+// calls.  Those of one step stop gaining where there are more 32-row q tiles than a round of workgroups, but the longer their walks the later,
+// the forward where the 256-row kernels fill the device.  2780 of 4100 drawn plans (P 1 to 32, 600 to 60 000 rows, logits N(0, 1) and N(0, 81), 2700 of
+// them around the lines) are within the lines.  What these leave of the time on the kernels that had the launches before it (ring_walk_kernel, at d = 64
+// thin::), geometric mean (the worst of fifty in brackets) of a rank's step, a step of all and the forward: d = 64 0.51 (0.93), 0.58 (0.98), 0.52 (0.88), under
+// the mask 0.52 (0.93), 0.55 (1.01), 0.48 (0.82); d = 128 0.39 (0.86), 0.47 (0.94), 0.44 (0.84), under the mask 0.38 (0.89), 0.43 (0.99), 0.37 (0.65).
+// A rank's step lost in none of them.  A step of all lost in 25, up to 16 %, nearly all of them with chunks of up to 128 keys, which are one wave's
+// work (2 ranks x 41 heads x 128, zigzag, 5.5, 6.4), and in one, whose short segments leave holes in a grid larger than the device, 46 % (23 x 3
+// heads x 76 on average, d = 128: 9.0, 13.1); their forwards take 0.33 to 1.01 of the time.  The forward lost in two, of one rank: d = 64, 38 heads x 256 7.4, 8.3, 35 x
+// 256 8.8, 9.4.  us before and after: d = 64, 4 heads x 4 x 512 9.9, 10.1, 29.9 and 6.2, 6.9, 17.7, 2 x 4 x 2048 25.6, 27.6, 94 and 10.1, 19.1, 65;
+// d = 128, 2 heads x 4 x 2048 46, 49, 163 and 15.3, 36, 123, causal 4 x 4 x 777 29.5, 29.7, 100 and 11.9, 11.8, 42.  Beyond them, d = 64, 8 heads x 8 x
+// 1024: 15.6, 30.3, 181 and 8.4, 45, 296; d = 128, 8 x 8 x 256 12.9, 14.3, 56 and 7.0, 14.8, 47.
 // RINGATTN_SPLIT_STEPS=0 and 1 in the environment: never, and always (comparisons, tests); the switches that name one of the
 // other kernels for these launches, or all launches, take this one out.
 bool small_steps(const ringattn_params& p, const Derived& d) {

@@ -1,5 +1,5 @@
-// gfx950 (CDNA4) kernel: block attention for launches with few query rows.  The workgroup's program; ringattn_split.hip and
-// ringattn_split_steps.hip wrap it into kernels.
+// gfx950 (CDNA4) kernel: block attention for launches with few query rows.  The workgroup's program; ringattn_split.hip,
+// ringattn_split_steps.hip and ringattn_split_columns.hip wrap it into kernels.
 //
 //   ring_split_kernel : the forward of ring_walk_kernel and ring_walk64_kernel (the reference's CTA that walks its ring
 //       steps with max / sum / acc-O in registers, csrc/ring_attention.cu:439-443,456-620, epilogue :621-664) with the

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from launched import launched
+from launched import kernels
 from ringattention_amd import api
 from ringattention_amd.configs import Workload
 from test_gpu_parity import check_rows
@@ -96,19 +96,29 @@ def test_steps_and_forward_give_the_same_bits_and_the_oracles_numbers(oracle, mo
     (64, (100,), 4, False, False),           # one range of few tiles
     (64, (40,) * 6, 2, False, False),
 ])
-def test_which_plans_run_on_it(d, lens, heads, causal, taken):
-    """One choice for all launches of a plan, whether or not its forward keeps the steps apart."""
+def test_which_plans_run_on_it(monkeypatch, d, lens, heads, causal, taken):
+    """One choice for all launches of a plan, whether or not its forward keeps the steps apart: single steps of all ranks and of one, and
+    the forward that merges them, launch what they do with the choice forced to what it should be, and not what they do with the other."""
     x = torch.zeros(1, heads, sum(lens), d, dtype=torch.float16, device="cuda")
-    names = []
+    r = len(lens) - 1
+    own = x[:, :, :lens[r]].contiguous()
     for apart in (True, False):
         plan = api.RingAttention(len(lens), list(lens), d, 1, heads, "fp16", causal, step_partials=apart)
         o, l = plan.block_forward(0, x, x, x)
-        (threads, _), = launched(lambda stream: plan.block_forward(0, x, x, x, o, l, stream))
-        names.append((plan.forward_kernel() == "ring_split_kernel") if apart else (threads == 512))
-        if not apart and taken:
-            assert threads == 512   # eight waves
+        o_r, l_r = plan.rank_step_forward(r, 0, own, own, own)
+        out, lse = plan.forward(x, x, x)
+        calls = [lambda stream: plan.block_forward(0, x, x, x, o, l, stream), lambda stream: plan.rank_step_forward(r, 0, own, own, own, o_r, l_r, stream)]
+        if apart:
+            calls.append(lambda stream: plan.forward(x, x, x, out, lse, stream))
+            assert (plan.forward_kernel() == "ring_split_kernel") == taken
+        for call in calls:
+            chosen = kernels(call)
+            monkeypatch.setenv("RINGATTN_SPLIT_STEPS", "1" if taken else "0")
+            assert kernels(call) == chosen
+            monkeypatch.setenv("RINGATTN_SPLIT_STEPS", "0" if taken else "1")
+            assert kernels(call) != chosen
+            monkeypatch.delenv("RINGATTN_SPLIT_STEPS")
         plan.close()
-    assert names[0] == taken
 
 
 def test_resources_and_hazards(tmp_path):
