@@ -34,14 +34,16 @@ PEAK_HBM_GBS = 8000.0
 # (bytes, summary under profiles/, kernel, kernel_source_id(kernel) when it was measured).  The figure is only printed
 # while the forward still runs that kernel and its source is still the one that was profiled.
 MEASURED_TRAFFIC = {
-    "cfg4": (2318e6, "profiles/ring_walk64_kernel_cfg4.md", "ring_walk64_kernel", "f5cf3ad4e6b41949"),
-    "cfg3": (1623e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "f5cf3ad4e6b41949"),
-    "cfg5": (47589e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "f5cf3ad4e6b41949"),
-    "cfg2": (34.2e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "f5cf3ad4e6b41949"),
+    "cfg4": (2279e6, "profiles/ring_walk64_kernel_cfg4.md", "ring_walk64_kernel", "4171ab4a9e5823d4"),
+    "cfg3": (1623e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "4171ab4a9e5823d4"),
+    "cfg5": (47061e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "4171ab4a9e5823d4"),
+    "cfg2": (34.2e6, "profiles/ring_walk64_kernel_other_workloads.md", "ring_walk64_kernel", "4171ab4a9e5823d4"),
 }
 KERNEL_SOURCES = {
-    "ring_walk64_kernel": ("ringattn_walk64.hip", "ringattn_walk64_loop.inc", "ringattn_walk64_loop_d64.inc", "ringattn_device.h"),
-    "ring_walk_kernel": ("ringattn_walk.hip", "ringattn_steps.hip", "ringattn_thin.hip", "ringattn_walk_rows.h", "ringattn_device.h"),
+    "ring_walk64_kernel": ("ringattn_walk64.hip", "ringattn_walk64_loop.inc", "ringattn_walk64_loop_d64.inc", "ringattn_device.h",
+                           "ringattn_jobs.h", "ringattn_kernels.h"),   # (these two: which workgroup does what, and so what meets in L2)
+    "ring_walk_kernel": ("ringattn_walk.hip", "ringattn_steps.hip", "ringattn_thin.hip", "ringattn_walk_rows.h", "ringattn_device.h",
+                         "ringattn_jobs.h", "ringattn_kernels.h"),
 }
 BASELINE_METRIC = "ring-attn fwd TFLOP/s + % bf16 MFMA peak, S=32K d=128 8-step ring, 1 GPU"
 
