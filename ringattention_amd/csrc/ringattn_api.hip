@@ -718,12 +718,12 @@ bool takes_thin(const ringattn_plan* pl, const TableSlice& sl) {
 // a second round fill in behind the long ones, of twice as many.  us on thin and dealt: 8 heads x 1024 x 1024 15.6, 10.7 (256 workgroups), 6 x
 // 1500 x 1500 21.1, 23.9 (282), 16 x 1024 x 1024 16.1, 19.2 (512); causal 8 x 2048 x 2048 27.1, 19.2 (512).
 // With a second round the walks have to be the longer the more of it there is, or it costs more than dealing the tiles gains: time on dealt over
-// that on thin with N(0, 1) logits, 260 to 512 workgroups, 0.94 to 1.40 below 16 key tiles, and above the line of the rule, a tile to sixteen
-// workgroups, 0.50 to 0.94 (900 drawn steps).  64 heads x 223 8.4, 12.2 (448), 35 x 342 10.7, 13.4 (385), 29 x 512 11.4, 12.2 (464).
+// that on thin, 257 to 512 workgroups, above the line of the rule, a tile to sixteen workgroups, 0.52 to 0.92 with N(0, 1) logits and up to 0.96 with
+// N(0, 9), below it 0.91 to 1.40 and 0.92 to 1.42 (1100 drawn steps).  64 heads x 223 8.4, 12.2 (448), 35 x 342 10.7, 13.4 (385), 29 x 512 11.4, 12.2 (464).
 // A walk that is over within a round has nothing to share out: 64 heads x 64 x 64 4.8, 5.4, 8 x 60 x 60 5.0, 5.2; 32 x 128 x 128 5.9, 5.3.
-// A move of the references costs a round of short walks more than it gains.  With N(0, 81) logits the lines leave 0.56 to 1.10 of the time on thin
-// without a mask, 1.00 to 1.10 of it at twelve to sixteen tiles, and 0.55 to 1.18 under the diagonal, 0.9 to 1.18 of it up to nine tiles; N(0, 9) logits lose
-// nowhere (1500 drawn steps).
+// A move of the references costs a round of short walks more than it gains.  With N(0, 81) logits the lines leave 0.57 to 1.10 of the time on thin
+// without a mask, where twelve to sixteen tiles have 0.91 to 1.10, and 0.55 to 1.18 under the diagonal, where up to nine have 0.89 to 1.18; with N(0, 1) the
+// same take 0.76 to 0.87 and 0.76 to 0.93, and N(0, 9) logits lose nowhere (1700 drawn steps within the lines).
 // RINGATTN_DEALT=0 and 1 in the environment: never, and whatever the size (comparisons, tests); RINGATTN_THIN names the other two.
 bool takes_dealt(const ringattn_plan* pl, const TableSlice& sl) {
   if (std::getenv("RINGATTN_THIN")) return false;
